@@ -72,20 +72,23 @@ constexpr float kGrazingCos = 0.35f;
 // shadow rays per bounce at or below which one wave traces each ray
 constexpr uint32_t kSparseShadowRays = 8192;
 // Lanes per shadow ray above that threshold when the settings leave it at 0:
-// 16 up to kGroupShadowRays rays, one lane per ray beyond.  On the
-// 4M-triangle NEE frame's first bounce (412 K shadow rays) 16 lanes take
-// 0.76 ms against 0.95 with one lane per ray (0.80 with 8, 0.85 with 32);
-// on the 4096-environment batch (about 3 M shadow rays of small scenes) one
-// lane per ray is fastest.
+// 16 up to kGroupShadowRays rays, one lane per ray beyond.  On a 4M-triangle
+// NEE frame's first bounce 416 K shadow rays take 0.74 ms with 16 lanes and
+// 0.95 with one, 600 K of another mesh 0.84 and 0.66; 67 K 0.12 and 0.34; on
+// the 4096-environment batch (about 3 M shadow rays of small scenes) one lane
+// per ray is fastest.
 constexpr uint32_t kDefaultShadowGroup = 16;
-constexpr uint32_t kGroupShadowRays = 1u << 20;
+constexpr uint32_t kGroupShadowRays = 1u << 19;
 // Lanes per path of the tail when the settings leave it at 0: 32 up to
-// kGroupTailPaths live paths (the tail takes over at a few thousand), one lane
-// per path above.  Four nodes per step shorten the slowest paths' chains: the
-// 4M-triangle frame's tail takes 0.29 ms (NEE) and 0.23 ms (PATH) against
-// 0.36 and 0.29 with 16 lanes, and 0.36 and 0.31 with 64.
-constexpr uint32_t kDefaultTailGroup = 32;
-constexpr uint32_t kGroupTailPaths = 1u << 15;
+// kWideTailPaths live paths, 16 up to kGroupTailPaths; above that the
+// wavefront goes on.  (4M-triangle mesh, frame times: 959 live paths 1.00 ms
+// with 32 lanes, 1.08 with 16; 3,785: 1.37 and 1.39; material box 5,792: 0.49
+// and 0.43, 23,150: 0.73 and 0.56 (0.58 one lane per path); mesh 33,748: 5.67
+// and 5.45 (5.91 one lane per path, 6.48 wavefront).  With 149,294 paths the
+// one-lane tail took 1.54 ms a frame against 1.00 with the bounce traced by
+// the wavefront and the tail taking the 959 paths left.)
+constexpr uint32_t kWideTailPaths = 2048;
+constexpr uint32_t kGroupTailPaths = 49152;
 constexpr int kCounterWords = 16;
 constexpr uint32_t kStatusPathOverflow = 1, kStatusShadowOverflow = 3;
 constexpr int kMaxBounces = 64;
@@ -532,16 +535,6 @@ BJ_D bool direct_light(const SceneView& sc, uint64_t seed, uint32_t path_id, uin
   return true;
 }
 
-// Wave-aggregated maximum of a per-lane count.
-BJ_D void wave_max(unsigned long long* dst, uint32_t v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    const uint32_t o = (uint32_t)__shfl_xor((int)v, off, 64);
-    v = o > v ? o : v;
-  }
-  if (lane_id() == 0 && v) atomicMax(dst, (unsigned long long)v);
-}
-
 // Wave-aggregated 64-bit add of a per-lane count.
 BJ_D void wave_add(unsigned long long* dst, uint32_t v) {
   uint64_t x = v;
@@ -549,6 +542,35 @@ BJ_D void wave_add(unsigned long long* dst, uint32_t v) {
   for (int off = 32; off >= 1; off >>= 1) x += __shfl_xor(x, off, 64);
   if (lane_id() == 0 && x) atomicAdd(dst, (unsigned long long)x);
 }
+
+// A tail block's per-bounce statistics, gathered in LDS and added to the
+// frame's once per block: extension rays, shadow rays, and the largest
+// node-visit count of one extension and of one shadow ray.
+struct BounceStats {
+  uint32_t count[kMaxBounces][2];
+  uint32_t visits[kMaxBounces][2];
+  BJ_D void clear() {
+    for (uint32_t i = threadIdx.x; i < 2 * kMaxBounces; i += blockDim.x) (&count[0][0])[i] = (&visits[0][0])[i] = 0;
+    __syncthreads();
+  }
+  BJ_D void rays(uint32_t bounce, int kind, bool p) {
+    const uint64_t m = ballot(p);
+    if (bounce < (uint32_t)kMaxBounces && m && lane_id() == (uint32_t)__builtin_ctzll(m))
+      atomicAdd(&count[bounce][kind], (uint32_t)__builtin_popcountll(m));
+  }
+  BJ_D void longest(uint32_t bounce, int kind, uint32_t v) {
+    if (bounce < (uint32_t)kMaxBounces && v) atomicMax(&visits[bounce][kind], v);
+  }
+  // Every thread of the block calls it once its paths are done.
+  BJ_D void flush(unsigned long long* __restrict__ stats) const {
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < 2 * kMaxBounces; i += blockDim.x) {
+      const uint32_t c = (&count[0][0])[i], v = (&visits[0][0])[i];
+      if (c) atomicAdd(stats + i, (unsigned long long)c);
+      if (v) atomicMax(stats + kMaxVisitBase + i, (unsigned long long)v);
+    }
+  }
+};
 
 // Surface facts of an extension hit (rt/geometry.mojo:20-30: the outward
 // normal is oriented against the ray).
@@ -936,12 +958,14 @@ __global__ void __launch_bounds__(kRtBlock) tail_kernel(SceneView sc, Queues q, 
                                                         unsigned long long* __restrict__ stats,
                                                         uint32_t* __restrict__ spill) {
   __shared__ uint32_t s_stack[kLdsStack * kRtBlock];
+  __shared__ BounceStats s_bounce;
   const uint32_t tag = q.counters[kTailDone];
   if (tag != 0 && tag != bounce + 1u) return;
   const uint64_t cap = q.capacity;
   const uint32_t active = q.counters[kActive] < cap ? q.counters[kActive] : (uint32_t)cap;
   if (active <= lo || active > threshold) return;  // (lo: the lane-group tail takes those)
   if (blockIdx.x == 0 && threadIdx.x == 0) q.counters[kTailDone] = bounce + 1u;
+  s_bounce.clear();
   const uint32_t lane = lane_id();
   const uint64_t gtid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   Stack st{s_stack + threadIdx.x, spill + gtid, (uint64_t)gridDim.x * blockDim.x, 0};
@@ -996,7 +1020,7 @@ __global__ void __launch_bounds__(kRtBlock) tail_kernel(SceneView sc, Queues q, 
       const uint32_t b = bounce + k;
       const bool ext_step = k < nb;
       if (!ext_step) alive = false;  // a path still going after the last bounce ends here
-      if (ext_step && b < kMaxBounces) wave_add(stats + 2 * b, alive ? 1u : 0u);
+      s_bounce.rays(b, 0, alive);
       uint32_t ext_max = 0, sh_max = 0;
       // one traversal call for both lane kinds, so the path's extension ray
       // and its mate's shadow ray step through the same instructions
@@ -1067,11 +1091,9 @@ __global__ void __launch_bounds__(kRtBlock) tail_kernel(SceneView sc, Queues q, 
 #pragma unroll
       for (int p = 0; p < kShadowPlanes; ++p) sf[p] = __shfl(nsf[p], (int)mate, 64);
       sh_live = mine && !is_path && mate_cast;
-      if (ext_step && b < kMaxBounces) {
-        wave_add(stats + 2 * b + 1, cast ? 1u : 0u);
-        wave_max(stats + kMaxVisitBase + 2 * b, ext_max);
-      }
-      if (k > 0 && b - 1 < kMaxBounces) wave_max(stats + kMaxVisitBase + 2 * (b - 1) + 1, sh_max);
+      s_bounce.rays(b, 1, cast);
+      s_bounce.longest(b, 0, ext_max);
+      if (k > 0) s_bounce.longest(b - 1, 1, sh_max);
       if (!ballot(alive || sh_live)) break;
     }
     if (mine && is_path) {
@@ -1083,12 +1105,13 @@ __global__ void __launch_bounds__(kRtBlock) tail_kernel(SceneView sc, Queues q, 
   wave_add(stats + kWorkBase + 1, (uint32_t)ext_leaves);
   wave_add(stats + kWorkBase + 2, (uint32_t)sh_visits);
   wave_add(stats + kWorkBase + 3, (uint32_t)sh_leaves);
+  s_bounce.flush(stats);
 }
 
 // The tail with G lanes per path (triangle and batch scenes, 4- and 8-wide):
 // each group carries one path through the remaining bounces -- its extension
-// ray by GroupClosest (Walk8 on the group's leader for the rare near ties),
-// shading on the leader, then the bounce's shadow ray by GroupWalk -- so the
+// ray by GroupWalk8 (Walk8 on the group's leader for the rare near ties),
+// shading on the leader, then the bounce's shadow ray by GroupWalk8 -- so the
 // sample receives the wavefront's additions in its order (extension, then
 // shadow, bounce by bounce) and images equal the per-lane tail's.  The last
 // few thousand paths of a chunk walk long serial chains (over 100 node
@@ -1100,15 +1123,19 @@ __global__ void __launch_bounds__(kRtBlock) tail_group_kernel(SceneView sc, Queu
                                                               uint32_t depth, uint32_t lo, uint32_t hi,
                                                               unsigned long long* __restrict__ stats) {
   constexpr int kGroups = kRtBlock / G;
-  static_assert(GroupWalk<G>::kStack <= 2 * GroupClosest<G>::kStack, "the walks share one LDS stack area");
-  __shared__ uint32_t s_stack[kGroups][2 * GroupClosest<G>::kStack];
-  __shared__ uint32_t s_recs[kGroups][GroupWalk<G>::kRecs];
+  using Ext = Wide8<G, false>;
+  using Shadow = GroupWalk8<G, true, false>;
+  static_assert(Ext::kStackWords <= Shadow::kStackWords && Ext::kRecs <= Shadow::kRecs, "the walks share one LDS area");
+  __shared__ uint32_t s_stack[kGroups][Shadow::kStackWords];
+  __shared__ uint32_t s_recs[kGroups][Shadow::kRecs];
+  __shared__ BounceStats s_bounce;
   const uint32_t tag = q.counters[kTailDone];
   if (tag != 0 && tag != bounce + 1u) return;
   const uint64_t cap = q.capacity;
   const uint32_t active = q.counters[kActive] < cap ? q.counters[kActive] : (uint32_t)cap;
   if (active <= lo || active > hi) return;
   if (blockIdx.x == 0 && threadIdx.x == 0) q.counters[kTailDone] = bounce + 1u;
+  s_bounce.clear();
   const uint32_t lane = lane_id(), grp = threadIdx.x / G, gl = lane % G;
   const int lead = (int)((lane / G) * G);  // the group's leader lane in the wave
   const bool leader = gl == 0;
@@ -1152,28 +1179,20 @@ __global__ void __launch_bounds__(kRtBlock) tail_group_kernel(SceneView sc, Queu
       first = alive ? (uint32_t)sc.seg_off[env] : 0u;
     }
     for (uint32_t b = bounce; b < depth; ++b) {
-      if (b < kMaxBounces) wave_add(stats + 2 * b, (leader && alive) ? 1u : 0u);
+      s_bounce.rays(b, 0, leader && alive);
       // the extension ray
       const Ray ray{mk(f[0], f[1], f[2]), mk(f[4], f[5], f[6]), f[3], f[7]};
-      GroupClosest<G> gc;
+      Ext gc;
       uint32_t ev = 0, et = 0;
-      if (alive) gc.begin(wv, ray, stack);
+      if (alive) gc.begin(wv, ray);
       bool walking = alive;
       while (__ballot(walking) != 0) {
         if (walking && gc.step(wv, stack, recs, ev, et)) walking = false;
       }
       Hit h = miss(ray.tmax);
+      if (alive) h = gc.finish(wv, stack, recs, ev, et);
       if (alive && leader) {
-        if (gc.near_tie()) {
-          // Walk8 decides; its stack lives in the group's (now free) LDS area
-          Stack fst{stack, nullptr, 0, 0, kMaxStack, 1};
-          TraceCounters tc;
-          h = traverse8<BAJO_TRACE_CLOSEST_HIT, true>(wv, ray, fst, &tc);
-          ev += tc.visits;
-          et += tc.leaves;
-        } else {
-          h = gc.finish(wv);
-        }
+
         if constexpr (kGeo == kGeoBatch)
           if (h.prim != kEmpty) h.prim += first;
       }
@@ -1181,7 +1200,7 @@ __global__ void __launch_bounds__(kRtBlock) tail_group_kernel(SceneView sc, Queu
         ext_visits += ev;
         ext_leaves += et;
       }
-      if (b < kMaxBounces) wave_max(stats + kMaxVisitBase + 2 * b, leader ? ev : 0u);
+      s_bounce.longest(b, 0, leader ? ev : 0u);
       // shading on the leader
       bool cast = false, next = false;
       float sf[kShadowPlanes];
@@ -1211,24 +1230,22 @@ __global__ void __launch_bounds__(kRtBlock) tail_group_kernel(SceneView sc, Queu
           delta = (np.id & kPathDelta) != 0;
         }
       }
-      if (b < kMaxBounces) wave_add(stats + 2 * b + 1, (leader && cast) ? 1u : 0u);
+      s_bounce.rays(b, 1, leader && cast);
       // the bounce's shadow ray, traced by the whole group
       cast = __shfl(cast, lead, 64);
 #pragma unroll
       for (int p = 0; p < kShadowPlanes; ++p) sf[p] = __shfl(sf[p], lead, 64);
-      GroupWalk<G> gw;
+      Shadow gw;
       uint32_t sv = 0, stt = 0;
       bool occluded = false;
-      if (cast) gw.begin(wv, Ray{mk(sf[0], sf[1], sf[2]), mk(sf[4], sf[5], sf[6]), sf[3], sf[7]}, stack);
+      if (cast) gw.begin(wv, Ray{mk(sf[0], sf[1], sf[2]), mk(sf[4], sf[5], sf[6]), sf[3], sf[7]});
       bool shadowing = cast;
       while (__ballot(shadowing) != 0) {
-        if (shadowing) {
-          bool occ = false;
-          if (gw.step(wv, stack, recs, sv, stt, occ)) {
-            shadowing = false;
-            occluded = occ;
-          }
-        }
+        if (shadowing && gw.step(wv, stack, recs, sv, stt)) shadowing = false;
+      }
+      if (cast) {
+        const Hit sh = gw.finish(wv, stack, recs, sv, stt);
+        occluded = sh.prim == kEmpty && sh.t == 0.0f;
       }
       if (cast && leader && (kAlg == BAJO_RENDER_AO || !occluded)) {
         const v3 cs = shadow_radiance<kAlg>(occluded, sf);
@@ -1240,7 +1257,7 @@ __global__ void __launch_bounds__(kRtBlock) tail_group_kernel(SceneView sc, Queu
         sh_visits += sv;
         sh_leaves += stt;
       }
-      if (b < kMaxBounces) wave_max(stats + kMaxVisitBase + 2 * b + 1, leader ? sv : 0u);
+      s_bounce.longest(b, 1, leader ? sv : 0u);
       // the next segment, from the leader (a path still going after the last bounce ends)
       alive = __shfl(next, lead, 64) && b + 1 < depth;
 #pragma unroll
@@ -1258,6 +1275,7 @@ __global__ void __launch_bounds__(kRtBlock) tail_group_kernel(SceneView sc, Queu
   wave_add(stats + kWorkBase + 1, (uint32_t)ext_leaves);
   wave_add(stats + kWorkBase + 2, (uint32_t)sh_visits);
   wave_add(stats + kWorkBase + 3, (uint32_t)sh_leaves);
+  s_bounce.flush(stats);
 }
 
 // kWalk: the shadow walk form (traverse8_any: bit 0 two nodes per step, bit 1
@@ -1311,7 +1329,7 @@ shadow_kernel(SceneView sc, Queues q, uint32_t bounce,
   store_block_work(work, work_visits, work_leaves, ray_max);
 }
 
-// Shadow rays with G lanes per ray (GroupWalk) when the bounce's shadow count
+// Shadow rays with G lanes per ray (GroupWalk8) when the bounce's shadow count
 // lies in (lo, hi] -- decided on the device from the queue length, so exactly
 // one shadow launch of a bounce traces its rays.  After the first bounce only
 // a few thousand shadow rays remain, and the per-lane kernel's time is the
@@ -1322,8 +1340,9 @@ template <int kAlg, int kGeo, int G>
 __global__ void __launch_bounds__(kRtBlock) shadow_group_kernel(SceneView sc, Queues q, uint32_t bounce, uint32_t lo,
                                                                 uint32_t hi, unsigned long long* __restrict__ work) {
   constexpr int kGroups = kRtBlock / G;
-  __shared__ uint32_t s_stack[kGroups][GroupWalk<G>::kStack];
-  __shared__ uint32_t s_recs[kGroups][GroupWalk<G>::kRecs];
+  using Walk = GroupWalk8<G, true, false>;
+  __shared__ uint32_t s_stack[kGroups][Walk::kStackWords];
+  __shared__ uint32_t s_recs[kGroups][Walk::kRecs];
   const uint64_t cap = q.capacity;
   const uint32_t count =
       q.counters[kTailDone] ? 0u : (q.counters[kShadow] < cap ? q.counters[kShadow] : (uint32_t)cap);
@@ -1335,31 +1354,36 @@ __global__ void __launch_bounds__(kRtBlock) shadow_group_kernel(SceneView sc, Qu
   const uint32_t groups = gridDim.x * kGroups;
   uint32_t idx = blockIdx.x * kGroups + grp;
   uint32_t visits = 0, tests = 0, ray_max = 0, rv = 0;
-  GroupWalk<G> walk;
+  Walk walk;
   WideView wv = sc.bvh.wide;
-  float f[kShadowPlanes];
-  uint32_t slot = 0;
   bool have = false;
   for (;;) {
     if (!have && idx < count) {
+      // the ray's planes now, its radiance planes (8..10) and id after the walk
+      float f[8];
 #pragma unroll
-      for (int p = 0; p < kShadowPlanes; ++p) f[p] = q.shadow_fields[plane_at<kShadowPlanes>(idx, p)];
-      const uint32_t sid = q.shadow_ids[idx];
-      slot = sid - q.sample_base;
-      if constexpr (kGeo == kGeoBatch) wv.root = sid / sc.env_paths;  // segment roots lead the node array
-      walk.begin(wv, Ray{mk(f[0], f[1], f[2]), mk(f[4], f[5], f[6]), f[3], f[7]}, stack);
+      for (int p = 0; p < 8; ++p) f[p] = q.shadow_fields[plane_at<kShadowPlanes>(idx, p)];
+      if constexpr (kGeo == kGeoBatch) wv.root = q.shadow_ids[idx] / sc.env_paths;  // segment roots lead the node array
+      walk.begin(wv, Ray{mk(f[0], f[1], f[2]), mk(f[4], f[5], f[6]), f[3], f[7]});
       rv = 0;
       have = true;
     }
     if (__ballot(have) == 0) break;  // every group of the wave is out of rays
     if (have) {
-      bool occluded = false;
-      if (walk.step(wv, stack, recs, rv, tests, occluded)) {
-        if (gl == 0 && (kAlg == BAJO_RENDER_AO || !occluded)) {
-          const v3 c = shadow_radiance<kAlg>(occluded, f);
-          accumulate(q.sample, slot, c);
-          if constexpr (kAlg == BAJO_RENDER_GUIDED)
-            if (q.contrib) contrib_add(q.contrib, slot, q.depth, bounce, c);
+      if (walk.step(wv, stack, recs, rv, tests)) {
+        const Hit h = walk.finish(wv, stack, recs, rv, tests);
+        if (gl == 0) {
+          const bool occluded = h.prim == kEmpty && h.t == 0.0f;
+          if (kAlg == BAJO_RENDER_AO || !occluded) {
+            float f[kShadowPlanes];
+#pragma unroll
+            for (int p = 8; p < kShadowPlanes; ++p) f[p] = q.shadow_fields[plane_at<kShadowPlanes>(idx, p)];
+            const uint32_t slot = q.shadow_ids[idx] - q.sample_base;
+            const v3 c = shadow_radiance<kAlg>(occluded, f);
+            accumulate(q.sample, slot, c);
+            if constexpr (kAlg == BAJO_RENDER_GUIDED)
+              if (q.contrib) contrib_add(q.contrib, slot, q.depth, bounce, c);
+          }
         }
         visits += rv;
         ray_max = rv > ray_max ? rv : ray_max;
@@ -1688,6 +1712,10 @@ struct LaunchEvents {
     (void)hipEventCreate(&e);
     return e;
   }
+  void mark(std::vector<hipEvent_t>& v, hipStream_t stream) {
+    v.push_back(make());
+    (void)hipEventRecord(v.back(), stream);
+  }
   ~LaunchEvents() {
     for (auto e : ext) (void)hipEventDestroy(e);
     for (auto e : sh) (void)hipEventDestroy(e);
@@ -1761,9 +1789,6 @@ int32_t run_render(bajo_ctx* ctx, bajo_scene* s, RenderArena& a, const bajo_rend
   constexpr bool kTail = kAlg == BAJO_RENDER_PATH || kAlg == BAJO_RENDER_NEE || kAlg == BAJO_RENDER_MIS;
   const uint64_t cap = shape.cap;
   const unsigned g_ext = shape.g_ext, g_sh = g_ext, g_tail = shape.g_tail, simds = shape.simds;
-  // the tail takes over when the remaining paths fit one pass of its resident
-  // threads, or at the schedule's own threshold
-  const uint32_t tail_threshold = st->tail_paths ? st->tail_paths : g_tail * kRtBlock;
   BJ_REQUIRE(st->extend_waves == 0 || st->extend_waves == 4 || st->extend_waves == 6 || st->extend_waves == 8,
              "bajo_render: extend_waves must be 0, 4, 6 or 8 (got %u)", st->extend_waves);
   // extension kernels compiled for other occupancies (the hot renders only)
@@ -1787,11 +1812,21 @@ int32_t run_render(bajo_ctx* ctx, bajo_scene* s, RenderArena& a, const bajo_rend
   BJ_REQUIRE(st->tail_group == 0 || st->tail_group == 1 || st->tail_group == 16 || st->tail_group == 32 ||
                  st->tail_group == 64,
              "bajo_render: tail_group must be 0, 1, 16, 32 or 64 (got %u)", st->tail_group);
+  // The tail takes over at `tail_threshold` live paths: with lane groups those
+  // in (0, wide_hi] by `wide_lanes` and those in (wide_hi, group_hi] by 16
+  // lanes, the rest one lane per path.
   constexpr bool kGroupTail = kWide && kGeo != kGeoMixed;
-  const uint32_t tail_group = st->tail_group ? st->tail_group : kDefaultTailGroup;
-  uint32_t group_tail_hi = 0;
-  if (kGroupTail && (tail_group == 16 || tail_group == 32 || tail_group == 64))
-    group_tail_hi = st->tail_group ? tail_threshold : (kGroupTailPaths < tail_threshold ? kGroupTailPaths : tail_threshold);
+  const uint32_t resident_paths = g_tail * kRtBlock;
+  uint32_t tail_threshold = st->tail_paths ? st->tail_paths : resident_paths;
+  uint32_t wide_hi = 0, group_hi = 0, wide_lanes = 32;
+  if (kGroupTail && st->tail_group > 1) {
+    wide_lanes = st->tail_group;
+    wide_hi = group_hi = tail_threshold;
+  } else if (kGroupTail && st->tail_group == 0) {
+    if (!st->tail_paths) tail_threshold = kGroupTailPaths;
+    group_hi = tail_threshold < kGroupTailPaths ? tail_threshold : kGroupTailPaths;
+    wide_hi = group_hi < kWideTailPaths ? group_hi : kWideTailPaths;
+  }
   const bool adaptive_group = st->shadow_group == 0;
   const uint32_t shadow_group = adaptive_group ? kDefaultShadowGroup : st->shadow_group;
   // the lane-group shadow kernel loops over its rays with a fixed stride, so
@@ -1893,27 +1928,38 @@ int32_t run_render(bajo_ctx* ctx, bajo_scene* s, RenderArena& a, const bajo_rend
         q.contrib = gr->train ? gr->g->contrib : nullptr;
         q.depth = depth;
       }
-      if (ev) { ev->ext.push_back(ev->make()); (void)hipEventRecord(ev->ext.back(), stream); }
+      if (ev) { ev->mark(ev->ext, stream); }
       if constexpr (kTail) {
         if (b > 0) {
-          // lane groups up to group_tail_hi live paths, one lane per path above
-          uint32_t lo = 0;
           if constexpr (kGroupTail) {
             constexpr int kTG = kGroupTail ? kGeo : kGeoTriangles;
-            if (group_tail_hi && tail_group == 32)
+            if (wide_hi && wide_lanes == 32)
               tail_group_kernel<kAlg, kTG, 32><<<g_tgroup, kRtBlock, 0, stream>>>(sv, q, st->rng_seed, b, depth, 0u,
-                                                                                 group_tail_hi, a.stats);
-            else if (group_tail_hi && tail_group == 64)
+                                                                                 wide_hi, a.stats);
+            else if (wide_hi && wide_lanes == 64)
               tail_group_kernel<kAlg, kTG, 64><<<g_tgroup, kRtBlock, 0, stream>>>(sv, q, st->rng_seed, b, depth, 0u,
-                                                                                 group_tail_hi, a.stats);
-            else if (group_tail_hi)
-              tail_group_kernel<kAlg, kTG, 16><<<g_tgroup, kRtBlock, 0, stream>>>(sv, q, st->rng_seed, b, depth, 0u,
-                                                                                 group_tail_hi, a.stats);
-            if (group_tail_hi) lo = group_tail_hi;
+                                                                                 wide_hi, a.stats);
+            const uint32_t lo16 = wide_lanes == 16 ? 0u : wide_hi;
+            if (group_hi > lo16)
+              tail_group_kernel<kAlg, kTG, 16><<<g_tgroup, kRtBlock, 0, stream>>>(sv, q, st->rng_seed, b, depth, lo16,
+                                                                                 group_hi, a.stats);
           }
-          tail_kernel<kAlg, kWide, kGeo><<<g_tail, kRtBlock, 0, stream>>>(sv, q, st->rng_seed, b, depth, lo,
-                                                                    tail_threshold, simds, a.stats, a.spill);
+          if (tail_threshold > group_hi)
+            tail_kernel<kAlg, kWide, kGeo><<<g_tail, kRtBlock, 0, stream>>>(sv, q, st->rng_seed, b, depth, group_hi,
+                                                                      tail_threshold, simds, a.stats, a.spill);
           BJ_HIP(hipGetLastError());
+          // a chunk no larger than the threshold ends in this tail: nothing is
+          // left to launch for its later bounces (the material box at
+          // 160 x 120 x 2 spp, depth 8, launched 48 kernels that returned at once)
+          if (chunk <= tail_threshold) {
+            if (ev) {
+              // the event pairs of the launches left out
+              const bool shadows = kAlg != BAJO_RENDER_PATH && kAlg != BAJO_RENDER_NORMALS;
+              for (uint32_t k = 2 * b + 1; k < 2 * depth; ++k) ev->mark(ev->ext, stream);
+              for (uint32_t k = 2 * b; shadows && k < 2 * depth; ++k) ev->mark(ev->sh, stream);
+            }
+            break;
+          }
         }
       }
       if (b == 0)
@@ -1929,23 +1975,23 @@ int32_t run_render(bajo_ctx* ctx, bajo_scene* s, RenderArena& a, const bajo_rend
         extend_kernel<kAlg, kWide, false, kGeo><<<g_ext, kRtBlock, 0, stream>>>(sv, q, st->rng_seed, b, pa, a.spill,
                                                                           a.work_ext, a.stats);
       BJ_HIP(hipGetLastError());
-      if (ev) { ev->ext.push_back(ev->make()); (void)hipEventRecord(ev->ext.back(), stream); }
+      if (ev) { ev->mark(ev->ext, stream); }
       if constexpr (kAlg == BAJO_RENDER_GUIDED) {
         // the network over this bounce's guided vertices, then their
         // continuations (none after the last bounce)
-        if (b + 1 < depth && ev) { ev->inf.push_back(ev->make()); (void)hipEventRecord(ev->inf.back(), stream); }
+        if (b + 1 < depth && ev) { ev->mark(ev->inf, stream); }
         if (b + 1 < depth) {
           rc = guide_infer_vertices(stream, gr->g, gr->g->vertices, a.counters + kVertex, cap, gr->bounds,
                                     gr->g->outputs);
           if (rc) return rc;
-          if (ev) { ev->inf.push_back(ev->make()); (void)hipEventRecord(ev->inf.back(), stream); }
+          if (ev) { ev->mark(ev->inf, stream); }
           guide_sample_kernel<<<g_ext, kRtBlock, 0, stream>>>(sv, q, st->rng_seed, b, gr->g->outputs,
                                                              gr->train ? gr->g->records : nullptr);
           BJ_HIP(hipGetLastError());
         }
       }
       if (kAlg != BAJO_RENDER_PATH && kAlg != BAJO_RENDER_NORMALS) {
-        if (ev) { ev->sh.push_back(ev->make()); (void)hipEventRecord(ev->sh.back(), stream); }
+        if (ev) { ev->mark(ev->sh, stream); }
         // sparse bounces: one wave per ray; dense ones: lane groups or one
         // lane per ray (triangle and batch scenes, 4- and 8-wide)
         constexpr bool kSparse = kWide && kGeo != kGeoMixed;
@@ -1985,7 +2031,7 @@ int32_t run_render(bajo_ctx* ctx, bajo_scene* s, RenderArena& a, const bajo_rend
             shadow_group_kernel<kAlg, kG, 64><<<g_wave, kRtBlock, 0, stream>>>(sv, q, b, 0u, sparse, a.work_sh);
         }
         BJ_HIP(hipGetLastError());
-        if (ev) { ev->sh.push_back(ev->make()); (void)hipEventRecord(ev->sh.back(), stream); }
+        if (ev) { ev->mark(ev->sh, stream); }
       }
       const bool traced_shadows = kAlg != BAJO_RENDER_PATH && kAlg != BAJO_RENDER_NORMALS;
       partials_sum_kernel<<<kSumBlocks, 256, 0, stream>>>(a.counters, (uint32_t)cap, a.work_ext, g_ext, a.work_sh,

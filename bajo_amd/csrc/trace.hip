@@ -176,6 +176,80 @@ __global__ void __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_e
   }
 }
 
+// Short launches: G lanes per ray (OrderedWalk8, GroupWalk8 or GroupWalk2),
+// each group taking every `groups`-th ray.  With one lane per ray a launch
+// lasts as long as its slowest lane's chain of node and record loads, whatever
+// its size: 4,096 closest-hit rays through a 65,536-triangle soup took 377 us
+// at widths 2 and 8; with 32 (binary) or 64 (8-wide) lanes per ray 43 and 27.
+// Five waves per SIMD: the walk holds about 85 VGPRs, the rare fallback more.
+template <int kMode, bool kCamera, bool kWide, bool kSeg, int G>
+__global__ void __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(5)))
+trace_group_kernel(const AccelView av, const float* __restrict__ rays,
+                                                                  const float* __restrict__ cams, uint32_t cam_w,
+                                                                  uint32_t cam_h, float inv_height,
+                                                                  float* __restrict__ hits, uint64_t R,
+                                                                  const uint64_t* __restrict__ seg_off) {
+  constexpr bool kAny = kMode == BAJO_TRACE_ANY_HIT;
+  constexpr int kGroups = kTraceBlock / G;
+  using Walk = std::conditional_t<kWide, Wide8<G < 8 ? 8 : G, kAny>, GroupWalk2<G, kAny>>;
+  __shared__ uint32_t s_stack[kGroups][Walk::kStackWords];
+  __shared__ uint32_t s_recs[kWide ? kGroups : 1][kWide ? Wide8<G < 8 ? 8 : G, kAny>::kRecs : 1];
+  const uint32_t grp = threadIdx.x / G, gl = lane_id() % G;
+  uint32_t* stack = s_stack[grp];
+  uint32_t* recs = s_recs[kWide ? grp : 0];
+  const uint64_t groups = (uint64_t)gridDim.x * kGroups;
+  uint64_t r = (uint64_t)blockIdx.x * kGroups + grp;
+  AccelView v = av;
+  Walk walk;
+  // A finished ray's record and the next ray's start cost a few loads that the
+  // other groups of the wave would wait for, so they are done once a quarter
+  // of the groups are finished or none is left walking (262,144 closest-hit
+  // rays, 8 lanes each: 279 us against 294 with every group on its own).
+  constexpr uint32_t kRefill = G < 16 ? 64 / G / 4 : 1;
+  bool have = false, walking = false;
+  uint32_t visits = 0, tests = 0;
+  for (;;) {
+    const uint64_t busy = ballot(walking);
+    if (64u - (uint32_t)__builtin_popcountll(busy) >= kRefill * G || busy == 0) {
+      if (have && !walking) {
+        Hit h;
+        if constexpr (kWide) {
+          h = walk.finish(v.wide, stack, recs, visits, tests);
+          if (gl == 0) store_hit(hits, r, h);
+        } else if (gl == 0) {
+          store_hit(hits, r, walk.finish(v.bin, stack));
+        }
+        have = false;
+        r += groups;
+      }
+      if (!have && r < R) {
+        Ray ray;
+        if constexpr (kCamera) {
+          ray = camera_ray(cams, r, cam_w, cam_h, inv_height);
+        } else {
+          ray.o = mk(rays[0 * R + r], rays[1 * R + r], rays[2 * R + r]);
+          ray.tmin = rays[3 * R + r];
+          ray.d = mk(rays[4 * R + r], rays[5 * R + r], rays[6 * R + r]);
+          ray.tmax = rays[7 * R + r];
+        }
+        if constexpr (kSeg) {
+          const uint32_t root = segment_root<kWide>(seg_off, r / ((uint64_t)cam_w * cam_h));
+          if constexpr (kWide) v.wide.root = root;
+          else v.bin.root = root;
+        }
+        if constexpr (kWide) walk.begin(v.wide, ray);
+        else walk.begin(v.bin, ray);
+        have = walking = true;
+      }
+      if (ballot(have) == 0) break;  // every group of the wave is out of rays
+    }
+    if (walking) {
+      if constexpr (kWide) walking = !walk.step(v.wide, stack, recs, visits, tests);
+      else walking = !walk.step(v.bin, stack);
+    }
+  }
+}
+
 __global__ void trace_init_kernel(uint32_t* counter, uint32_t* status) {
   if (threadIdx.x == 0) { *counter = 0; *status = 0; }
 }
@@ -208,9 +282,76 @@ int32_t occupancy_grid(unsigned* grid) {
   return BAJO_OK;
 }
 
+// Lanes per ray of a launch of R rays (1: the per-lane kernels).  More lanes
+// shorten the serial chain of a ray but spend more instructions on it, so
+// each width pays until the chip is full.  Measured over 65,536-triangle and
+// 1M-triangle soups and 100K / 4M-triangle closed meshes, random and camera
+// rays (us, one lane per ray against the choice): 8-wide closest 16,384 rays
+// 343 -> 64, 65,536: 293 -> 137, 131,072: 332 -> 249, 262,144: 433 -> 458;
+// 8-wide any 16,384: 194 -> 31, 131,072: 214 -> 165, 262,144: 289 -> 306;
+// binary closest 4,096: 377 -> 43, 16,384: 395 -> 66, 65,536: 405 -> 160,
+// 131,072: 437 -> 306, 262,144: 515 -> 475, 524,288: 471 -> 622 (camera).
+int lanes_per_ray(bool wide, bool any, uint64_t R) {
+  if (wide) {
+    if (R <= (any ? 32768u : 24576u)) return 64;
+    return R <= 196608u ? (any ? 16 : 8) : 1;
+  }
+  if (R <= 8192u) return 32;
+  if (R <= 32768u) return 16;
+  if (R <= 98304u) return 8;
+  return R <= (any ? 196608u : 294912u) ? 4 : 1;
+}
+
+// A launch with G lanes per ray on its resident blocks.
+template <int kMode, bool kCamera, bool kWide, bool kSeg, int G>
+int32_t launch_groups(bajo_ctx* ctx, const bajo_bvh* h, const float* rays, const float* cams, uint32_t w, uint32_t hh,
+                      float* hits, uint64_t R) {
+  static unsigned resident = 0;
+  if (!resident) {
+    int dev = 0, cus = 0, per_cu = 0;
+    BJ_HIP(hipGetDevice(&dev));
+    BJ_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    BJ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, trace_group_kernel<kMode, kCamera, kWide, kSeg, G>,
+                                                        kTraceBlock, 0));
+    resident = (unsigned)(cus * (per_cu < 1 ? 1 : per_cu));
+  }
+  const uint64_t need = (R * G + kTraceBlock - 1) / kTraceBlock;
+  const unsigned grid = need < resident ? (unsigned)need : resident;
+  void* scratch = nullptr;
+  const int32_t rc = ctx_scratch(ctx, 256, &scratch);
+  if (rc) return rc;
+  const AccelView av = accel_view(h, (uint32_t*)scratch);
+  trace_group_kernel<kMode, kCamera, kWide, kSeg, G><<<grid, kTraceBlock, 0, ctx->stream>>>(
+      av, rays, cams, w, hh, hh ? 1.0f / (float)hh : 0.0f, hits, R, kSeg ? h->seg_off : nullptr);
+  BJ_HIP(hipGetLastError());
+  return BAJO_OK;
+}
+
 template <int kMode, bool kStats, bool kCamera, bool kWide, bool kSeg = false, bool kSph = false>
 int32_t launch_width(bajo_ctx* ctx, const bajo_bvh* h, const float* rays, const float* cams, uint32_t w, uint32_t hh,
                      float* hits, uint64_t R, uint32_t* stats) {
+  if constexpr (!kStats && !kSph) {
+    switch (lanes_per_ray(kWide, kMode == BAJO_TRACE_ANY_HIT, R)) {
+      case 4:
+        if constexpr (!kWide) return launch_groups<kMode, kCamera, kWide, kSeg, 4>(ctx, h, rays, cams, w, hh, hits, R);
+        break;
+      case 8:
+        if constexpr (!kWide || kMode == BAJO_TRACE_CLOSEST_HIT)
+          return launch_groups<kMode, kCamera, kWide, kSeg, 8>(ctx, h, rays, cams, w, hh, hits, R);
+        break;
+      case 16:
+        if constexpr (!kWide || kMode == BAJO_TRACE_ANY_HIT)
+          return launch_groups<kMode, kCamera, kWide, kSeg, 16>(ctx, h, rays, cams, w, hh, hits, R);
+        break;
+      case 32:
+        if constexpr (!kWide) return launch_groups<kMode, kCamera, kWide, kSeg, 32>(ctx, h, rays, cams, w, hh, hits, R);
+        break;
+      case 64:
+        if constexpr (kWide) return launch_groups<kMode, kCamera, kWide, kSeg, 64>(ctx, h, rays, cams, w, hh, hits, R);
+        break;
+      default: break;
+    }
+  }
   unsigned grid = 0;
   int32_t rc = occupancy_grid<kMode, kStats, kCamera, kWide, kSeg, kSph>(&grid);
   if (rc) return rc;

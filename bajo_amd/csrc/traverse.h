@@ -12,6 +12,8 @@
 // suffice.
 #pragma once
 
+#include <type_traits>
+
 #include "bvh_internal.h"
 
 namespace bj {
@@ -884,368 +886,666 @@ BJ_D void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Any hit with G lanes per ray (G = 8, 16, 32 or 64): the walk of rays whose
-// chains are long and serial when one lane carries a ray, such as shadow
-// rays (they leave a surface and pass many boxes and leaves near it).  A
-// step takes up to G/8 nodes off the group's LDS stack, lane 8j + i tests
-// child i of node j (the same quantized slab test as Walk8), entered inner
-// children are pushed, and the records of all entered leaves are tested one
-// per lane.  A step therefore waits for one round of node loads and one of
-// record loads whatever the width of the ray's frontier.  The records tested
-// are every record whose leaf box the ray enters, as in every other any-hit
-// walk, so occlusion comes out the same.
-//
-// GroupWalk holds one group's state; every lane of the group holds the same
-// copy.  step() is called by the group's lanes together (other groups of the
-// wave may be stepping their own rays at the same time).
+// Ballots and lane masks of a group of G lanes: 32 bits wide where they fit.
 template <int G>
-struct GroupWalk {
-  static constexpr int kStack = 16 * G;  // a level pushes at most 7G/8 net; 18 levels fit
-  static constexpr int kRecs = 8 * G;    // G entered leaves of up to 8 records
-  Ray ray;
-  v3 rcp;
-  bool px, py, pz;
-  int sp;
-  uint32_t steps;
-  // The frontier of the next step, taken off the stack and loaded while the
-  // previous step's records were tested: how many nodes it holds, whether
-  // this lane's node is one of them, its first four 16-byte words and this
-  // lane's child reference.  Every step issues these loads at one place (a
-  // dummy node 0 where no node is taken), so they stay in flight across the
-  // record tests.
-  int nf;
-  bool mine;
-  uint4 w0, w1, w2, w3;
-  uint32_t ref;
+using GroupBits = std::conditional_t<G == 64, uint64_t, uint32_t>;
 
-  BJ_D uint64_t group_mask() const {
-    const uint32_t lane = lane_id();
-    return (G == 64 ? ~0ull : ((1ull << G) - 1ull)) << ((lane / G) * G);
+template <int G>
+BJ_D GroupBits<G> group_ballot(bool p) {
+  const uint64_t b = ballot(p);
+  if constexpr (G == 64) return b;
+  else return (uint32_t)(b >> (lane_id() & (64u - G))) & (uint32_t)((1ull << G) - 1ull);
+}
+BJ_D uint32_t bit_count(uint32_t m) { return (uint32_t)__builtin_popcount(m); }
+BJ_D uint32_t bit_count(uint64_t m) { return (uint32_t)__builtin_popcountll(m); }
+BJ_D uint32_t low_bit(uint32_t m) { return (uint32_t)__builtin_ctz(m); }
+BJ_D uint32_t low_bit(uint64_t m) { return (uint32_t)__builtin_ctzll(m); }
+
+template <int kCtrl>
+BJ_D uint32_t dpp_mov(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, 0xF, 0xF, true);
+}
+
+// Within each aligned group of 8 lanes: how many lanes with a nonzero key come
+// before this one when keys are ordered from the largest down (equal keys:
+// higher lane first).  Lanes exchange keys through quad permutes and the
+// half-row mirror, so nothing waits on LDS.
+BJ_D uint32_t far_rank8(uint32_t key) {
+  const uint32_t lane = lane_id();
+  // a partner above this lane comes first at an equal key, one below does not
+  const uint32_t t1 = key + (lane & 1u), t2 = key + ((lane >> 1) & 1u), t4 = key + ((lane >> 2) & 1u);
+  const uint32_t m = dpp_mov<0x141>(key);  // lane ^ 7
+  uint32_t r = 0;
+  r += dpp_mov<0xB1>(key) >= t1 ? 1u : 0u;  // ^ 1
+  r += dpp_mov<0x4E>(key) >= t2 ? 1u : 0u;  // ^ 2
+  r += dpp_mov<0x1B>(key) >= t2 ? 1u : 0u;  // ^ 3
+  r += dpp_mov<0x1B>(m) >= t4 ? 1u : 0u;    // ^ 4
+  r += dpp_mov<0x4E>(m) >= t4 ? 1u : 0u;    // ^ 5
+  r += dpp_mov<0xB1>(m) >= t4 ? 1u : 0u;    // ^ 6
+  r += m >= t4 ? 1u : 0u;                   // ^ 7
+  return r;
+}
+
+// The two nearest candidates a group has met.  A one-lane walk accepts a
+// triangle when its scaled distance beats the best so far
+// (ts < t_best * det) and enters boxes up to the best so far, so which of two
+// triangles wins can depend on their order when their distances lie within
+// rounding of each other (or of a box's entry); a group visits nodes in
+// another order.  So the group keeps the two smallest candidate distances it
+// has seen (t1 with its record, t2; candidates pass the walk's own test
+// against the ray's t_max), culls only boxes entered beyond t1 plus a slack
+// and reports a near tie when t2 lies within that slack of t1: the caller
+// then runs the one-lane order for that ray.  The slack is 4e-6 t1 (ten times
+// the rounding of the scaled test at distances like the triangle's own) plus
+// 1e-6 of the origin's coordinates (t of a near triangle carries the rounding
+// of o - v0).  Beyond it the comparisons have their exact outcome and the
+// one-lane walk ends at the unique nearest candidate; its hit record is
+// formed by testing it again (the same arithmetic that formed it in the
+// walk).  A candidate at t < 0 (only rays with a negative t_min have them)
+// closes every box to the one-lane walk, so what it had found by then
+// decides: that is left to it as well.
+struct NearTwo {
+  static constexpr float kRelative = 4e-6f, kAbsolute = 1e-6f;
+  float t1, t2, slack;
+  uint32_t best;  // record of t1 (kEmpty: no candidate)
+  BJ_D void clear(const Ray& r) {
+    t1 = t2 = kFltMax;
+    best = kEmpty;
+    const float d = fmaxf(fabsf(r.d.x), fmaxf(fabsf(r.d.y), fabsf(r.d.z)));
+    slack = kAbsolute * (fabsf(r.o.x) + fabsf(r.o.y) + fabsf(r.o.z)) / d;
   }
-
-  // Starts a ray with the root as its first frontier (loaded here); a root
-  // outside the hierarchy ends the ray at once with a status word.
-  BJ_D void begin(const WideView& wv, const Ray& r, uint32_t* stack) {
-    ray = r;
-    rcp = rcp_dir(r.d);
-    px = rcp.x >= 0.0f;
-    py = rcp.y >= 0.0f;
-    pz = rcp.z >= 0.0f;
-    steps = 1;
-    sp = 0;
-    const bool ok = wv.node_count != 0 && wv.root < wv.node_count;
-    if (wv.node_count != 0 && !ok && lane_id() % G == 0) atomicOr(wv.status, (uint32_t)BAJO_STATUS_BAD_NODE);
-    nf = ok ? 1 : 0;
-    mine = ok && (lane_id() % G) < 8;
-    if (wv.node_count != 0) load(wv, ok ? wv.root : 0u);
-  }
-
-  BJ_D void load(const WideView& wv, uint32_t node) {
-    const uint4* np = reinterpret_cast<const uint4*>(wv.nodes + node);
-    w0 = np[0];
-    w1 = np[1];
-    w2 = np[2];
-    w3 = np[3];
-    ref = reinterpret_cast<const uint32_t*>(wv.nodes + node)[16 + (lane_id() & 7u)];
-  }
-
-  // One step; returns true once the ray is finished (then *occluded says how).
-  BJ_D bool step(const WideView& wv, uint32_t* stack, uint32_t* recs, uint32_t& visits, uint32_t& tests,
-                 bool& occluded) {
-    occluded = false;
-    if (nf == 0) return true;
-    visits += (uint32_t)nf;
-    const uint32_t gl = lane_id() % G, j = gl >> 3, i = gl & 7;
-    const uint64_t gm = group_mask();
-    bool hit = false;
-    const uint32_t cref = ref;
-    if (mine) {
-      const uint32_t meta = w0.w;
-      const uint32_t n = meta >> 24;
-      const float sx = __builtin_bit_cast(float, (meta & 0xFFu) << 23);
-      const float sy = __builtin_bit_cast(float, ((meta >> 8) & 0xFFu) << 23);
-      const float sz = __builtin_bit_cast(float, ((meta >> 16) & 0xFFu) << 23);
-      const float ax = (__builtin_bit_cast(float, w0.x) - ray.o.x) * rcp.x;
-      const float ay = (__builtin_bit_cast(float, w0.y) - ray.o.y) * rcp.y;
-      const float az = (__builtin_bit_cast(float, w0.z) - ray.o.z) * rcp.z;
-      const float bx = sx * rcp.x, by = sy * rcp.y, bz = sz * rcp.z;
-      // byte i of lo_x (w1.xy), lo_y (w1.zw), lo_z (w2.xy), hi_x (w2.zw), hi_y (w3.xy), hi_z (w3.zw)
-      const bool hiw = i >= 4;
-      const int bt = (int)(i & 3u);
-      const uint32_t lox = hiw ? w1.y : w1.x, loy = hiw ? w1.w : w1.z, loz = hiw ? w2.y : w2.x;
-      const uint32_t hix = hiw ? w2.w : w2.z, hiy = hiw ? w3.y : w3.x, hiz = hiw ? w3.w : w3.z;
-      const uint32_t qnx = px ? lox : hix, qfx = px ? hix : lox;
-      const uint32_t qny = py ? loy : hiy, qfy = py ? hiy : loy;
-      const uint32_t qnz = pz ? loz : hiz, qfz = pz ? hiz : loz;
-      const float tnx = fmaf(ubyte_f(qnx, bt), bx, ax), tfx = fmaf(ubyte_f(qfx, bt), bx, ax);
-      const float tny = fmaf(ubyte_f(qny, bt), by, ay), tfy = fmaf(ubyte_f(qfy, bt), by, ay);
-      const float tnz = fmaf(ubyte_f(qnz, bt), bz, az), tfz = fmaf(ubyte_f(qfz, bt), bz, az);
-      const float tmin = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, 0.0f));
-      const float tmax = fminf(fminf(tfx, tfy), fminf(tfz, ray.tmax));
-      hit = i < n && tmin <= tmax;
-    }
-    const bool is_leaf = hit && (cref & kLeafFlag) != 0;
-    const bool is_inner = hit && (cref & kLeafFlag) == 0;
-    // entered inner children onto the group's stack
-    const uint64_t inner = __ballot(is_inner) & gm;
-    const int n_inner = __builtin_popcountll(inner);
-    if (sp + n_inner > kStack) {
-      if (gl == 0) atomicOr(wv.status, (uint32_t)BAJO_STATUS_STACK_OVERFLOW);
-      sp = 0;
-      nf = 0;
-      return true;
-    }
-    if (is_inner) stack[sp + (int)mask_rank(inner)] = cref;
-    sp += n_inner;
-    // the entered leaves' records, one per lane
-    uint32_t start = 0, k = 0;
-    if (is_leaf) {
-      start = cref & kWideLeafStartMask;
-      const uint32_t e = start + ((cref >> 28) & 7u) + 1u;
-      k = (e > wv.prim_count ? wv.prim_count : e) - (start < wv.prim_count ? start : wv.prim_count);
-    }
-    uint32_t incl = k;
-#pragma unroll
-    for (int off = 1; off < G; off <<= 1) {
-      const uint32_t y = __shfl_up(incl, off, G);
-      if (gl >= (uint32_t)off) incl += y;
-    }
-    const uint32_t total = __shfl(incl, G - 1, G);
-    for (uint32_t m = 0; m < k; ++m) recs[incl - k + m] = start + m;
-    wave_lds_sync();
-    tests += total;
-    // the first round of records is loaded, then the next frontier (up to G/8
-    // nodes off the stack), so its node loads are in flight while the
-    // records are tested
-    LeafRec rec;
-    const bool has = gl < total;
-    if (has) rec = load_rec<false>(wv.tris, recs[gl]);
-    nf = sp < G / 8 ? sp : G / 8;
-    mine = (int)j < nf;
-    // lanes without a node of their own load their group's first node (the
-    // same cache lines as its owners)
-    const int at = sp - 1 - (mine ? (int)j : 0);
-    const uint32_t top = stack[at > 0 ? at : 0];
-    wave_lds_sync();
-    sp -= nf;
-    const bool bad = (__ballot(mine && top >= wv.node_count) & gm) != 0 || (nf > 0 && ++steps > wv.node_count);
-    load(wv, mine && top < wv.node_count ? top : 0u);
-    if ((__ballot(has && rec_any<false>(rec, ray)) & gm) != 0) {
-      occluded = true;
-      nf = 0;
-      return true;
-    }
-    for (uint32_t base = G; base < total; base += G) {
-      bool occ = false;
-      if (base + gl < total) {
-        const LeafRec r2 = load_rec<false>(wv.tris, recs[base + gl]);
-        occ = rec_any<false>(r2, ray);
-      }
-      if ((__ballot(occ) & gm) != 0) {
-        occluded = true;
-        nf = 0;
-        return true;
+  BJ_D float reach() const { return fmaf(t1, kRelative, t1 + slack); }
+  BJ_D float cull(float tmax) const { return fminf(tmax, reach()); }
+  BJ_D bool tie() const { return best != kEmpty && (!(t2 > reach()) || t1 < 0.0f); }
+  // Takes the candidates of the group's lanes (record `s` at distance `t`
+  // where `on`); every lane of the group holds the same state.
+  template <int G>
+  BJ_D void take(bool on, float t, uint32_t s) {
+    const uint32_t base = lane_id() & (64u - G);
+    for (GroupBits<G> m = group_ballot<G>(on); m; m &= m - 1) {
+      const int p = (int)(base + low_bit(m));
+      const float tp = __shfl(t, p, 64);
+      const uint32_t sp = (uint32_t)__shfl((int)s, p, 64);
+      if (best == kEmpty || tp < t1) {
+        t2 = t1;
+        t1 = tp;
+        best = sp;
+      } else {
+        t2 = fminf(t2, tp);
       }
     }
-    wave_lds_sync();
-    if (bad) {
-      if (gl == 0) atomicOr(wv.status, (uint32_t)BAJO_STATUS_BAD_NODE);
-      nf = 0;
-      return true;
-    }
-    return nf == 0;
   }
 };
 
-// Closest hit with G lanes per ray (the tail kernel's extension rays), equal
-// to the one-lane Walk8 result.  Walk8 accepts a triangle when its scaled
-// distance beats the best so far (ts < t_best * det), so which of two
-// triangles wins can depend on their test order when their distances lie
-// within rounding of each other; the group visits nodes in another order.
-// So the group keeps the two smallest candidate distances it has seen (t1
-// with its record, t2; candidates pass Walk8's own test against the ray's
-// t_max), culls only boxes entered beyond t1 * (1 + margin),
-// and reports a near tie when t2 <= t1 * (1 + margin); the caller then runs
-// Walk8 for that ray.  Without a near tie every pairwise comparison Walk8
-// makes has the exact outcome (the margin, 4e-6, is ten times the rounding of
-// the scaled test), so Walk8 ends at the unique nearest candidate, which is
-// t1's record; its hit record is formed by testing it again (the same
-// arithmetic that formed it in the walk).
+// Lane 8j + i's share of an 8-wide node: the header, child i's six plane bytes
+// and its reference.  Each lane loads its own bytes (eight lanes' bytes of a
+// plane are contiguous), so nothing is shifted out of wider words.
+struct ChildLane {
+  uint4 h;
+  uint32_t lx, ly, lz, hx, hy, hz, ref;
+
+  BJ_D void load(const BjWide* __restrict__ nodes, uint32_t node) {
+    const BjWide* nd = nodes + node;
+    const uint32_t i = lane_id() & 7u;
+    h = *reinterpret_cast<const uint4*>(nd);
+    lx = nd->lo_x[i];
+    ly = nd->lo_y[i];
+    lz = nd->lo_z[i];
+    hx = nd->hi_x[i];
+    hy = nd->hi_y[i];
+    hz = nd->hi_z[i];
+    ref = nd->child[i];
+  }
+
+  // The quantized slab test of Walk8: whether the ray enters child i before
+  // `limit`, and where.  The planes of a child are ordered, so the smaller
+  // of its two distances is the near plane's.
+  BJ_D bool enters(const v3& o, const v3& rcp, float limit, float& tin) const {
+    const uint32_t meta = h.w;
+    const float bx = __builtin_bit_cast(float, (meta & 0xFFu) << 23) * rcp.x;
+    const float by = __builtin_bit_cast(float, ((meta >> 8) & 0xFFu) << 23) * rcp.y;
+    const float bz = __builtin_bit_cast(float, ((meta >> 16) & 0xFFu) << 23) * rcp.z;
+    const float ax = (__builtin_bit_cast(float, h.x) - o.x) * rcp.x;
+    const float ay = (__builtin_bit_cast(float, h.y) - o.y) * rcp.y;
+    const float az = (__builtin_bit_cast(float, h.z) - o.z) * rcp.z;
+    const float x0 = fmaf((float)lx, bx, ax), x1 = fmaf((float)hx, bx, ax);
+    const float y0 = fmaf((float)ly, by, ay), y1 = fmaf((float)hy, by, ay);
+    const float z0 = fmaf((float)lz, bz, az), z1 = fmaf((float)hz, bz, az);
+    tin = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), fmaxf(fminf(z0, z1), 0.0f));
+    const float tout = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fminf(fmaxf(z0, z1), limit));
+    return (lane_id() & 7u) < (meta >> 24) && tin <= tout;
+  }
+};
+
+// Writes the records of the entered leaves of a group (`is_leaf`, reference
+// `cref`) to the group's LDS list in lane order and returns their number.
+// Positions come from one ballot per count bit: a shuffle scan would wait on
+// LDS log2(G) times.
 template <int G>
-struct GroupClosest {
-  static constexpr int kStack = 16 * G;  // entries of (node, entry distance); 18 levels fit, as GroupWalk
-  static constexpr int kRecs = 8 * G;
-  static constexpr float kMargin = 4e-6f;
+BJ_D uint32_t list_records(bool is_leaf, uint32_t cref, uint32_t prim_count, uint32_t gl, uint32_t* recs) {
+  const GroupBits<G> leaves = group_ballot<G>(is_leaf);
+  if (leaves == 0) return 0;
+  const GroupBits<G> below = ((GroupBits<G>)1 << gl) - 1;
+  uint32_t start = 0, k = 0;
+  if (is_leaf) {
+    start = cref & kWideLeafStartMask;
+    const uint32_t e = start + ((cref >> 28) & 7u) + 1u;
+    k = (e > prim_count ? prim_count : e) - (start < prim_count ? start : prim_count);
+  }
+  uint32_t first = 0, total = 0;
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const GroupBits<G> m = group_ballot<G>((k >> b) & 1u);
+    first += bit_count(m & below) << b;
+    total += bit_count(m) << b;
+  }
+  for (uint32_t m = 0; m < k; ++m) recs[first + m] = start + m;
+  return total;
+}
+
+// Scaled test of a record held in registers.
+BJ_D bool rec_scaled(const LeafRec& rec, const Ray& r, float t_max, float& ad, float& ts) {
+  const TriData tr{mk(rec.a.x, rec.a.y, rec.a.z), mk(rec.b.x, rec.b.y, rec.b.z), mk(rec.c.x, rec.c.y, rec.c.z),
+                   __builtin_bit_cast(uint32_t, rec.a.w)};
+  float us, vs;
+  return tri_scaled(r, tr, t_max, ad, ts, us, vs);
+}
+
+// The closest hit's record from its leaf record: the test that accepted it in
+// the walk, done again.
+BJ_D Hit record_hit(const BjTri* __restrict__ tris, uint32_t best, const Ray& ray) {
+  Closest c = no_closest(ray.tmax);
+  if (best != kEmpty) rec_closest<false>(load_rec<false>(tris, best), best, ray, c);
+  return closest_hit_p<false>(tris, c, ray);
+}
+
+BJ_D Hit shadow_record(bool occluded, float tmax) {
+  return occluded ? Hit{0.0f, 0.0f, kEmpty, kEmpty, mk(0, 0, 0), 0.0f} : miss(tmax);
+}
+
+// One ray walked by 8 lanes in exactly Walk8's order: lane i tests child i of
+// the current node, records are tested one per lane and accepted in slot
+// order, the nearest inner child comes next and the others go on the stack,
+// farthest first.  So the hit is Walk8's by construction, at an eighth of its
+// serial instructions per step.  While the records are tested the expected
+// next node (the nearest entered child, else the stack's top) is loaded.
+template <bool kAny>
+struct OrderedWalk8 {
+  static constexpr int G = 8;
+  static constexpr int kStackWords = kMaxStack;
+  static constexpr int kRecs = 64;
   Ray ray;
   v3 rcp;
-  bool px, py, pz;
+  float best_t;
+  uint32_t best, cur, steps;
   int sp;
-  uint32_t steps;
-  float t1, t2;
-  uint32_t best;  // record of t1 (kEmpty: no candidate)
+  bool occluded;
+  ChildLane nd;
 
-  BJ_D uint64_t group_mask() const {
-    const uint32_t lane = lane_id();
-    return (G == 64 ? ~0ull : ((1ull << G) - 1ull)) << ((lane / G) * G);
-  }
-  BJ_D float cull() const { return fminf(ray.tmax, t1 * (1.0f + kMargin)); }
-
-  BJ_D void begin(const WideView& wv, const Ray& r, uint32_t* stack) {
+  BJ_D void begin(const WideView& wv, const Ray& r) {
     ray = r;
     rcp = rcp_dir(r.d);
-    px = rcp.x >= 0.0f;
-    py = rcp.y >= 0.0f;
-    pz = rcp.z >= 0.0f;
-    steps = 0;
-    t1 = t2 = kFltMax;
+    best_t = r.tmax;
     best = kEmpty;
-    sp = wv.node_count == 0 ? 0 : 1;
-    if (lane_id() % G == 0) {
-      stack[0] = wv.root;
-      stack[1] = __builtin_bit_cast(uint32_t, 0.0f);
-    }
-    wave_lds_sync();
+    occluded = false;
+    steps = 0;
+    sp = 0;
+    cur = wv.node_count == 0 ? kSentinel : wv.root;
+    if (cur < wv.node_count) nd.load(wv.nodes, cur);
   }
 
   // One step; true once the walk is finished (or ended by an error).
   BJ_D bool step(const WideView& wv, uint32_t* stack, uint32_t* recs, uint32_t& visits, uint32_t& tests) {
-    if (sp == 0) return true;
-    const uint32_t gl = lane_id() % G, j = gl >> 3, i = gl & 7;
-    const uint64_t gm = group_mask();
-    const int nf = sp < G / 8 ? sp : G / 8;
-    const float limit = cull();
-    uint32_t node = 0;
-    bool mine = false;
-    if ((int)j < nf) {
-      node = stack[2 * (sp - 1 - (int)j)];
-      mine = __builtin_bit_cast(float, stack[2 * (sp - 1 - (int)j) + 1]) <= limit;
+    if (cur == kSentinel) return true;
+    const uint32_t gl = lane_id() & 7u;
+    if (cur >= wv.node_count || steps > wv.node_count) {
+      if (gl == 0) atomicOr(wv.status, (uint32_t)BAJO_STATUS_BAD_NODE);
+      return true;
+    }
+    ++steps;
+    ++visits;
+    float tin;
+    const bool hit = nd.enters(ray.o, rcp, kAny ? ray.tmax : best_t, tin);
+    const uint32_t cref = nd.ref;
+    const bool is_inner = hit && (cref & kLeafFlag) == 0;
+    const uint32_t total = list_records<G>(hit && (cref & kLeafFlag) != 0, cref, wv.prim_count, gl, recs);
+    const uint32_t rank = far_rank8(is_inner ? __builtin_bit_cast(uint32_t, tin) + 1u : 0u);
+    const uint32_t inner = group_ballot<G>(is_inner);
+    const uint32_t n_inner = bit_count(inner);
+    wave_lds_sync();
+    LeafRec rec;
+    uint32_t s = 0;
+    if (gl < total) {
+      s = recs[gl];
+      rec = load_rec<false>(wv.tris, s);
+    }
+    // the node to visit next unless a record drops it
+    uint32_t next = kSentinel;
+    if (n_inner) {
+      const uint32_t p = low_bit(group_ballot<G>(is_inner && rank + 1u == n_inner));
+      next = (uint32_t)__shfl((int)cref, (int)((lane_id() & 56u) + p), 64);
+    } else if (sp > 0) {
+      next = stack[sp - 1];
+    }
+    if (next < wv.node_count) nd.load(wv.nodes, next);
+    bool closer = false;
+    for (uint32_t base = 0; base < total; base += G) {
+      const bool go = base + gl < total;
+      if (base > 0 && go) {
+        s = recs[base + gl];
+        rec = load_rec<false>(wv.tris, s);
+      }
+      float ad = 0.0f, ts = 0.0f;
+      const bool cand = go && rec_scaled(rec, ray, kAny ? ray.tmax : best_t, ad, ts);
+      uint32_t m = group_ballot<G>(cand);
+      tests += total - base < G ? total - base : G;
+      if constexpr (kAny) {
+        if (m) {
+          occluded = true;
+          return true;
+        }
+      } else {
+        const float t = cand ? ts * (1.0f / ad) : 0.0f;
+        for (; m; m &= m - 1) {
+          const int p = (int)((lane_id() & 56u) + low_bit(m));
+          if (__shfl(ts, p, 64) < best_t * __shfl(ad, p, 64)) {
+            best_t = __shfl(t, p, 64);
+            best = (uint32_t)__shfl((int)s, p, 64);
+            closer = true;
+          }
+        }
+      }
+    }
+    if (n_inner) {
+      // children entered beyond the closest hit are dropped: the farthest ones
+      uint32_t kept = n_inner;
+      bool keep = is_inner;
+      if (!kAny && closer) {
+        keep = is_inner && !(tin > best_t);
+        kept = bit_count(group_ballot<G>(keep));
+      }
+      if (kept > 1 && sp + (int)kept - 1 > kMaxStack) {
+        if (gl == 0) atomicOr(wv.status, (uint32_t)BAJO_STATUS_STACK_OVERFLOW);
+        return true;
+      }
+      if (keep && rank + 1u < n_inner) stack[sp + (int)(rank - (n_inner - kept))] = cref;
+      wave_lds_sync();
+      if (kept) {
+        sp += (int)kept - 1;
+        cur = next;
+        return false;
+      }
+      if (sp == 0) {
+        cur = kSentinel;
+        return true;
+      }
+      cur = stack[--sp];
+      if (cur < wv.node_count) nd.load(wv.nodes, cur);
+      return false;
     }
     wave_lds_sync();
-    sp -= nf;
-    visits += (uint32_t)__builtin_popcountll(__ballot(mine && i == 0) & gm);
-    if ((__ballot(mine && node >= wv.node_count) & gm) != 0 || ++steps > wv.node_count) {
-      if (gl == 0) atomicOr(wv.status, (uint32_t)BAJO_STATUS_BAD_NODE);
-      sp = 0;
-      return true;
+    cur = next;
+    if (sp > 0) --sp;
+    return cur == kSentinel;
+  }
+
+  BJ_D Hit finish(const WideView& wv, uint32_t*, uint32_t*, uint32_t&, uint32_t&) const {
+    if constexpr (kAny) return shadow_record(occluded, ray.tmax);
+    else return record_hit(wv.tris, best, ray);
+  }
+};
+
+// One ray walked by G lanes (any hit: 8 to 64, closest hit: 16 to 64) over the
+// 8-wide layout: the walk of rays whose chains are long and serial when one
+// lane carries a ray (shadow rays, the last paths of a chunk, and launches
+// with fewer rays than the chip has lanes).  A step holds up to G/8 nodes of
+// the frontier, lane 8j + i tests child i of node j, entered inner children
+// are pushed on the group's LDS stack, each node's farthest first and the
+// nearest node's last, and the records of all entered leaves are tested one
+// per lane.  The first round of record loads and the next frontier's node
+// loads are issued before the records are tested, so a step waits for one
+// round of memory whatever its width.
+//
+// Any hit: occlusion does not depend on the order of the tests.  Closest hit:
+// see NearTwo; stack entries carry their entry distance, and entries beyond
+// the nearest candidate are dropped as they come off the stack.
+//
+// `fallback` set at the end asks for the ordered walk (a near tie, or a
+// frontier larger than the group's stack): finish() runs it on the group's
+// first eight lanes.  With kFallback off (any hit in the renderer, whose
+// shadow kernel would lose a resident wave to the code: 0.87 -> 1.09 ms for
+// 416 K rays) a full stack ends the ray with a status word.  Every lane of a group holds the same state, and the
+// group's lanes call together; other groups of the wave may be on rays of
+// their own.
+template <int G, bool kAny, bool kFallback = true>
+struct GroupWalk8 {
+  static_assert(kAny || kFallback, "closest hits need the ordered walk at near ties");
+  static_assert(kAny || G > 8, "eight lanes walk closest hits in order (OrderedWalk8)");
+  using Bits = GroupBits<G>;
+  static constexpr int kEntry = kAny ? 1 : 2;           // words: node (, entry distance)
+  static constexpr int kStackWords = 16 * G;            // per group
+  static constexpr int kStack = kStackWords / kEntry;
+  static constexpr int kRecs = 8 * G;                   // G entered leaves of up to 8 records
+  static constexpr uint32_t kNodes = G / 8;
+  static_assert(kStackWords >= OrderedWalk8<kAny>::kStackWords && kRecs >= OrderedWalk8<kAny>::kRecs,
+                "the ordered walk uses the group's LDS area");
+  Ray ray;
+  v3 rcp;
+  bool occluded, fallback;
+  int sp;
+  uint32_t steps;
+  NearTwo near;
+  // The frontier of the next step, taken off the stack and loaded while the
+  // previous step's records were tested: how many nodes it holds, whether
+  // this lane's node is one of them, its entry distance and this lane's child.
+  // Lanes without a node load their group's first one (the same cache lines),
+  // so the loads are unconditional and stay in flight across the record tests.
+  uint32_t nf;
+  bool mine;
+  float te;
+  ChildLane nd;
+
+  // Starts a ray with the root as its first frontier (loaded here); a root
+  // outside the hierarchy ends the ray at once with a status word.
+  BJ_D void begin(const WideView& wv, const Ray& r) {
+    ray = r;
+    rcp = rcp_dir(r.d);
+    occluded = fallback = false;
+    steps = 1;
+    sp = 0;
+    near.clear(r);
+    const bool ok = wv.node_count != 0 && wv.root < wv.node_count;
+    if (wv.node_count != 0 && !ok && lane_id() % G == 0) atomicOr(wv.status, (uint32_t)BAJO_STATUS_BAD_NODE);
+    nf = ok ? 1u : 0u;
+    te = 0.0f;
+    mine = ok && (lane_id() % G) < 8;
+    if (ok) nd.load(wv.nodes, wv.root);
+  }
+
+  // Takes the next frontier off the stack and issues its loads.
+  BJ_D bool pop(const WideView& wv, const uint32_t* stack, uint32_t gl) {
+    const uint32_t j = gl >> 3;
+    uint32_t node = 0;
+    if constexpr (kAny) {
+      nf = sp < (int)kNodes ? (uint32_t)sp : kNodes;
+      mine = j < nf;
+      const int at = sp - 1 - (mine ? (int)j : 0);
+      node = stack[at > 0 ? at : 0];
+      sp -= (int)nf;
+    } else {
+      const float limit = near.cull(ray.tmax);
+      nf = 0;
+      while (sp > 0) {
+        // the top G entries, one per lane; the nearest kNodes still in reach
+        const int at = sp - 1 - (int)gl;
+        const bool live = at >= 0 && __builtin_bit_cast(float, stack[2 * (at < 0 ? 0 : at) + 1]) <= limit;
+        Bits b = group_ballot<G>(live);
+        if (b == 0) {
+          sp = sp > G ? sp - G : 0;
+          continue;
+        }
+        uint32_t own = low_bit(b), last = own;
+        nf = 1;
+#pragma unroll
+        for (uint32_t q = 1; q < kNodes; ++q) {
+          b &= b - 1;
+          if (b) {
+            last = low_bit(b);
+            own = j >= q ? last : own;
+            nf = q + 1;
+          }
+        }
+        mine = j < nf;
+        const int e = 2 * (sp - 1 - (int)(mine ? own : 0u));
+        node = stack[e > 0 ? e : 0];
+        te = __builtin_bit_cast(float, stack[e > 0 ? e + 1 : 1]);
+        sp -= (int)last + 1;
+        break;
+      }
+      if (nf == 0) mine = false;
     }
-    bool hit = false;
-    uint32_t ref = 0;
+    const bool bad = group_ballot<G>(mine && node >= wv.node_count) != 0 || (nf > 0 && ++steps > wv.node_count);
+    nd.load(wv.nodes, mine && node < wv.node_count ? node : 0u);
+    return bad;
+  }
+
+  // One step; true once the walk is finished (or ended by an error).
+  BJ_D bool step(const WideView& wv, uint32_t* stack, uint32_t* recs, uint32_t& visits, uint32_t& tests) {
+    if (nf == 0) return true;
+    const uint32_t gl = lane_id() % G, j = gl >> 3, i = gl & 7;
+    const float limit = kAny ? ray.tmax : near.cull(ray.tmax);
+    const bool on = mine && (kAny || te <= limit);
+    visits += kAny ? nf : bit_count(group_ballot<G>(on && i == 0));
     float tin = 0.0f;
-    if (mine) {
-      const uint4* np = reinterpret_cast<const uint4*>(wv.nodes + node);
-      const uint4 w0 = np[0], w1 = np[1], w2 = np[2], w3 = np[3];
-      ref = reinterpret_cast<const uint32_t*>(wv.nodes + node)[16 + i];
-      const uint32_t meta = w0.w;
-      const uint32_t n = meta >> 24;
-      const float sx = __builtin_bit_cast(float, (meta & 0xFFu) << 23);
-      const float sy = __builtin_bit_cast(float, ((meta >> 8) & 0xFFu) << 23);
-      const float sz = __builtin_bit_cast(float, ((meta >> 16) & 0xFFu) << 23);
-      const float ax = (__builtin_bit_cast(float, w0.x) - ray.o.x) * rcp.x;
-      const float ay = (__builtin_bit_cast(float, w0.y) - ray.o.y) * rcp.y;
-      const float az = (__builtin_bit_cast(float, w0.z) - ray.o.z) * rcp.z;
-      const float bx = sx * rcp.x, by = sy * rcp.y, bz = sz * rcp.z;
-      const bool hiw = i >= 4;
-      const int bt = (int)(i & 3u);
-      const uint32_t lox = hiw ? w1.y : w1.x, loy = hiw ? w1.w : w1.z, loz = hiw ? w2.y : w2.x;
-      const uint32_t hix = hiw ? w2.w : w2.z, hiy = hiw ? w3.y : w3.x, hiz = hiw ? w3.w : w3.z;
-      const uint32_t qnx = px ? lox : hix, qfx = px ? hix : lox;
-      const uint32_t qny = py ? loy : hiy, qfy = py ? hiy : loy;
-      const uint32_t qnz = pz ? loz : hiz, qfz = pz ? hiz : loz;
-      const float tnx = fmaf(ubyte_f(qnx, bt), bx, ax), tfx = fmaf(ubyte_f(qfx, bt), bx, ax);
-      const float tny = fmaf(ubyte_f(qny, bt), by, ay), tfy = fmaf(ubyte_f(qfy, bt), by, ay);
-      const float tnz = fmaf(ubyte_f(qnz, bt), bz, az), tfz = fmaf(ubyte_f(qfz, bt), bz, az);
-      tin = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, 0.0f));
-      const float tout = fminf(fminf(tfx, tfy), fminf(tfz, limit));
-      hit = i < n && tin <= tout;
-    }
-    const bool is_leaf = hit && (ref & kLeafFlag) != 0;
-    const bool is_inner = hit && (ref & kLeafFlag) == 0;
-    const uint64_t inner = __ballot(is_inner) & gm;
-    const int n_inner = __builtin_popcountll(inner);
+    const bool hit = nd.enters(ray.o, rcp, limit, tin) && on;
+    const uint32_t cref = nd.ref;
+    const bool is_inner = hit && (cref & kLeafFlag) == 0;
+    // entered inner children onto the group's stack
+    const Bits inner = group_ballot<G>(is_inner);
+    const int n_inner = (int)bit_count(inner);
     if (sp + n_inner > kStack) {
-      if (gl == 0) atomicOr(wv.status, (uint32_t)BAJO_STATUS_STACK_OVERFLOW);
-      sp = 0;
+      if constexpr (kFallback) fallback = true;
+      else if (gl == 0) atomicOr(wv.status, (uint32_t)BAJO_STATUS_STACK_OVERFLOW);
+      nf = 0;
       return true;
     }
+    if constexpr (kAny) {
+      if (is_inner) stack[sp + (int)bit_count(inner & (((Bits)1 << gl) - 1))] = cref;
+    } else {
+      const uint32_t rank = far_rank8(is_inner ? __builtin_bit_cast(uint32_t, tin) + 1u : 0u);
+      if (is_inner) {
+        // nodes off the stack's top come first in the frontier and go back last
+        const Bits later = j + 1u < kNodes ? inner >> (8u * (j + 1u)) : 0;
+        const int at = sp + (int)(bit_count(later) + rank);
+        stack[2 * at] = cref;
+        stack[2 * at + 1] = __builtin_bit_cast(uint32_t, tin);
+      }
+    }
+    sp += n_inner;
+    // the entered leaves' records, one per lane
+    const uint32_t total = list_records<G>(hit && (cref & kLeafFlag) != 0, cref, wv.prim_count, gl, recs);
+    wave_lds_sync();
+    tests += total;
+    LeafRec rec;
+    uint32_t s = 0;
+    if (gl < total) {
+      s = recs[gl];
+      rec = load_rec<false>(wv.tris, s);
+    }
+    const bool bad = pop(wv, stack, gl);
+    wave_lds_sync();
+    for (uint32_t base = 0; base < total; base += G) {
+      const bool go = base + gl < total;
+      if (base > 0 && go) {
+        s = recs[base + gl];
+        rec = load_rec<false>(wv.tris, s);
+      }
+      float ad = 0.0f, ts = 0.0f;
+      const bool cand = go && rec_scaled(rec, ray, ray.tmax, ad, ts);
+      if constexpr (kAny) {
+        if (group_ballot<G>(cand) != 0) {
+          occluded = true;
+          nf = 0;
+          return true;
+        }
+      } else {
+        near.take<G>(cand, cand ? ts * (1.0f / ad) : 0.0f, s);
+      }
+    }
+    if (total > G) wave_lds_sync();
+    if (bad) {
+      if (gl == 0) atomicOr(wv.status, (uint32_t)BAJO_STATUS_BAD_NODE);
+      nf = 0;
+    }
+    if (nf == 0 && !kAny && near.tie()) fallback = true;
+    return nf == 0;
+  }
+
+  // The finished walk's hit record, in the group's first lanes.
+  BJ_D Hit finish(const WideView& wv, uint32_t* stack, uint32_t* recs, uint32_t& visits, uint32_t& tests) const {
+    if (kFallback && fallback) {
+      Hit h = miss(ray.tmax);
+      if (lane_id() % G < 8) {
+        OrderedWalk8<kAny> w;
+        w.begin(wv, ray);
+        while (!w.step(wv, stack, recs, visits, tests)) {
+        }
+        h = w.finish(wv, stack, recs, visits, tests);
+      }
+      return h;
+    }
+    if constexpr (kAny) return shadow_record(occluded, ray.tmax);
+    else return record_hit(wv.tris, near.best, ray);
+  }
+};
+
+// The group walk of G lanes over the 8-wide layout.
+template <int G, bool kAny>
+using Wide8 = std::conditional_t<G == 8 && !kAny, OrderedWalk8<false>, GroupWalk8<G == 8 && !kAny ? 16 : G, kAny>>;
+
+// One ray walked by G lanes over the binary layout, as GroupWalk8: a step
+// holds up to G/2 nodes, lane 2j + i tests child i of node j against its full
+// box (the slab test of traverse()) and, where that child is a leaf, its one
+// triangle, so no records are handed between lanes.
+template <int G, bool kAny>
+struct GroupWalk2 {
+  static constexpr int kStackWords = 16 * G;
+  static constexpr int kStack = kStackWords / 2;  // (node, entry distance)
+  static constexpr uint32_t kNodes = G / 2;
+  using Bits = GroupBits<G>;
+  Ray ray;
+  v3 rcp;
+  bool occluded, fallback;
+  int sp;
+  uint32_t steps;
+  NearTwo near;
+  uint32_t nf;
+  bool mine;
+  float te;
+  float2 b0, b1, b2;  // this lane's child box
+  uint32_t ref;
+
+  BJ_D void load(const BvhView& bv, uint32_t node) {
+    const uint32_t i = lane_id() & 1u;
+    const float* p = reinterpret_cast<const float*>(bv.nodes + node);
+    const float2* q = reinterpret_cast<const float2*>(p + 6 * i);
+    b0 = q[0];
+    b1 = q[1];
+    b2 = q[2];
+    ref = reinterpret_cast<const uint32_t*>(p)[13 + i];
+  }
+
+  BJ_D void begin(const BvhView& bv, const Ray& r) {
+    ray = r;
+    rcp = rcp_dir(r.d);
+    occluded = fallback = false;
+    steps = 1;
+    sp = 0;
+    near.clear(r);
+    const uint32_t root = bv.root_dev ? *bv.root_dev : bv.root;
+    // a hierarchy of one leaf, or a root the one-lane walk reports
+    fallback = root != kSentinel && ((root & kLeafFlag) != 0 || root >= bv.node_count);
+    const bool ok = root != kSentinel && !fallback;
+    nf = ok ? 1u : 0u;
+    te = 0.0f;
+    mine = ok && (lane_id() % G) < 2;
+    if (ok) load(bv, root);
+  }
+
+  BJ_D bool step(const BvhView& bv, uint32_t* stack) {
+    if (nf == 0) return true;
+    const uint32_t gl = lane_id() % G, j = gl >> 1;
+    const float limit = kAny ? ray.tmax : near.cull(ray.tmax);
+    const bool on = mine && te <= limit;
+    float tin = 0.0f;
+    bool hit = false;
+    if (on) hit = slab(ray.o, rcp, b0.x, b0.y, b1.x, b1.y, b2.x, b2.y, limit, tin);
+    const uint32_t cref = ref;
+    const uint32_t s = cref & kIndexMask;
+    const bool is_leaf = hit && (cref & kLeafFlag) != 0 && s < bv.prim_count;
+    const bool is_inner = hit && (cref & kLeafFlag) == 0;
+    const Bits inner = group_ballot<G>(is_inner);
+    const int n_inner = (int)bit_count(inner);
+    if (sp + n_inner > kStack) {
+      fallback = true;
+      nf = 0;
+      return true;
+    }
+    // the nearer of two entered children on top (child 0 at equal distances)
+    const uint32_t key = is_inner ? __builtin_bit_cast(uint32_t, tin) + 1u : 0u;
+    const uint32_t other = dpp_mov<0xB1>(key);
     if (is_inner) {
-      const int at = sp + (int)mask_rank(inner);
-      stack[2 * at] = ref;
+      const uint32_t rank = other >= key + (gl & 1u) ? 1u : 0u;
+      const Bits later = j + 1u < kNodes ? inner >> (2u * (j + 1u)) : 0;
+      const int at = sp + (int)(bit_count(later) + rank);
+      stack[2 * at] = cref;
       stack[2 * at + 1] = __builtin_bit_cast(uint32_t, tin);
     }
     sp += n_inner;
-    uint32_t start = 0, k = 0;
-    if (is_leaf) {
-      start = ref & kWideLeafStartMask;
-      const uint32_t e = start + ((ref >> 28) & 7u) + 1u;
-      k = (e > wv.prim_count ? wv.prim_count : e) - (start < wv.prim_count ? start : wv.prim_count);
-    }
-    uint32_t incl = k;
-#pragma unroll
-    for (int off = 1; off < G; off <<= 1) {
-      const uint32_t y = __shfl_up(incl, off, G);
-      if (gl >= (uint32_t)off) incl += y;
-    }
-    const uint32_t total = __shfl(incl, G - 1, G);
-    for (uint32_t m = 0; m < k; ++m) recs[incl - k + m] = start + m;
+    LeafRec rec;
+    if (is_leaf) rec = load_rec<false>(bv.tris, s);
     wave_lds_sync();
-    tests += total;
-    for (uint32_t base = 0; base < total; base += G) {
-      float t = kFltMax;
-      uint32_t s = kEmpty;
-      if (base + gl < total) {
-        s = recs[base + gl];
-        const LeafRec rec = load_rec<false>(wv.tris, s);
-        const TriData tr{mk(rec.a.x, rec.a.y, rec.a.z), mk(rec.b.x, rec.b.y, rec.b.z),
-                         mk(rec.c.x, rec.c.y, rec.c.z), __builtin_bit_cast(uint32_t, rec.a.w)};
-        float ad, ts, us, vs;
-        if (tri_scaled(ray, tr, ray.tmax, ad, ts, us, vs)) {
-          const float inv = 1.0f / ad;
-          t = ts * inv;
-        } else {
-          s = kEmpty;
-        }
+    // the next frontier: the nearest kNodes of the stack's top G entries still in reach
+    nf = 0;
+    uint32_t node = 0;
+    while (sp > 0) {
+      const int at = sp - 1 - (int)gl;
+      const bool live = at >= 0 && __builtin_bit_cast(float, stack[2 * (at < 0 ? 0 : at) + 1]) <= limit;
+      const Bits b = group_ballot<G>(live);
+      if (b == 0) {
+        sp = sp > G ? sp - G : 0;
+        continue;
       }
-      // the two smallest distances of this round (the lowest lane wins equal ones)
-      float m1 = t;
-      uint32_t r1 = s, l1 = gl;
+      // the j-th live entry belongs to lanes 2j and 2j + 1
+      uint32_t own = low_bit(b), last = own;
+      Bits m = b;
+      nf = 1;
 #pragma unroll
-      for (int off = 1; off < G; off <<= 1) {
-        const float om = __shfl_xor(m1, off, G);
-        const uint32_t orr = (uint32_t)__shfl_xor((int)r1, off, G);
-        const uint32_t ol = (uint32_t)__shfl_xor((int)l1, off, G);
-        if (om < m1 || (om == m1 && ol < l1)) {
-          m1 = om;
-          r1 = orr;
-          l1 = ol;
+      for (uint32_t q = 1; q < kNodes; ++q) {
+        m &= m - 1;
+        if (m) {
+          last = low_bit(m);
+          own = j >= q ? last : own;
+          nf = q + 1;
         }
       }
-      float m2 = gl == l1 ? kFltMax : t;
-#pragma unroll
-      for (int off = 1; off < G; off <<= 1) m2 = fminf(m2, __shfl_xor(m2, off, G));
-      if (r1 != kEmpty) {
-        if (m1 < t1) {
-          t2 = fminf(t1, m2);
-          t1 = m1;
-          best = r1;
-        } else {
-          t2 = fminf(t2, m1);
-        }
-      }
+      mine = j < nf;
+      const int e = 2 * (sp - 1 - (int)(mine ? own : 0u));
+      node = stack[e > 0 ? e : 0];
+      te = __builtin_bit_cast(float, stack[e > 0 ? e + 1 : 1]);
+      sp -= (int)last + 1;
+      break;
     }
+    if (nf == 0) mine = false;
+    const bool bad = group_ballot<G>(mine && node >= bv.node_count) != 0 || (nf > 0 && ++steps > bv.node_count);
+    load(bv, mine && node < bv.node_count ? node : 0u);
     wave_lds_sync();
-    return sp == 0;
+    if constexpr (kAny) {
+      if (group_ballot<G>(is_leaf && rec_any<false>(rec, ray)) != 0) {
+        occluded = true;
+        nf = 0;
+        return true;
+      }
+    } else {
+      float ad = 0.0f, ts = 0.0f;
+      const bool cand = is_leaf && rec_scaled(rec, ray, ray.tmax, ad, ts);
+      near.take<G>(cand, cand ? ts * (1.0f / ad) : 0.0f, s);
+    }
+    if (bad) {
+      if (gl == 0) atomicOr(bv.status, (uint32_t)BAJO_STATUS_BAD_NODE);
+      nf = 0;
+    }
+    if (nf == 0 && !kAny && near.tie()) fallback = true;
+    return nf == 0;
   }
 
-  // After the walk: whether Walk8 must decide (a near tie at the nearest
-  // candidate), else the hit record of the nearest candidate.
-  BJ_D bool near_tie() const { return best != kEmpty && t2 <= t1 * (1.0f + kMargin); }
-  BJ_D Hit finish(const WideView& wv) const {
-    Closest c = no_closest(ray.tmax);
-    if (best != kEmpty) {
-      const LeafRec rec = load_rec<false>(wv.tris, best);
-      rec_closest<false>(rec, best, ray, c);
+  BJ_D Hit finish(const BvhView& bv, uint32_t* stack) const {
+    if (fallback) {
+      Stack st{stack, nullptr, 0, 0, kMaxStack, 1};
+      return traverse<kAny ? BAJO_TRACE_ANY_HIT : BAJO_TRACE_CLOSEST_HIT, false>(bv, ray, st, nullptr);
     }
-    return closest_hit_p<false>(wv.tris, c, ray);
+    if constexpr (kAny) return shadow_record(occluded, ray.tmax);
+    else return record_hit(bv.tris, near.best, ray);
   }
 };
 

@@ -370,8 +370,8 @@ typedef struct bajo_scene bajo_scene;
  *     on-chip stack per lane against resident waves; used by PATH, NEE and
  *     MIS over 4- and 8-wide triangle and batch scenes (others ignore it);
  *   tail_paths: live paths at or below which the tail kernel finishes the
- *     chunk's remaining bounces in one launch (0 = the tail grid's resident
- *     threads);
+ *     chunk's remaining bounces in one launch (0 = 49,152 where the default
+ *     tail_group applies, else the tail grid's resident threads);
  *   shadow_walk: the 4- and 8-wide any-hit walk of the shadow-ray kernel:
  *     1 = one node per step with one leaf record loaded ahead, 2 = two nodes
  *     per step (the stack top with the current node), 3 = one node with leaf
@@ -382,13 +382,13 @@ typedef struct bajo_scene bajo_scene;
  *     never;
  *   shadow_group: lanes per shadow ray above that threshold: 1 = one lane
  *     per ray (shadow_walk applies), 8, 16 or 32 = that many lanes per ray
- *     (one node per 8 lanes per step); 0 = 16 lanes up to 2^20 rays and one
+ *     (one node per 8 lanes per step); 0 = 16 lanes up to 2^19 rays and one
  *     lane per ray beyond;
  *   tail_group: lanes per path in the tail kernel (4- and 8-wide triangle
  *     and batch scenes): 1 = one lane per path, 16, 32 or 64 = that many
  *     (extension rays by a group walk equal to the one-lane walk, shadow
  *     rays by group any hit; one node per 8 lanes per step); 0 = 32 up to
- *     2^15 live paths, one beyond. */
+ *     2,048 live paths, 16 up to 49,152, one beyond. */
 typedef struct {
   uint32_t image_width, image_height, samples_per_pixel, max_depth;
   uint64_t rng_seed;
