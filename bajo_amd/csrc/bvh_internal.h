@@ -114,9 +114,8 @@ struct bajo_bvh {
 namespace bj {
 // hp_ctl word holding H-PLOC's root reference.
 constexpr int kHpCtlRoot = 2;
-// Collapses h's binary hierarchy into h->wide (W-wide quantized nodes);
-// `largest_tree` bounds the leaves of one tree (a segment of a set); wide.hip.
-int32_t collapse_wide(bajo_ctx* ctx, bajo_bvh* h, uint64_t largest_tree);
+// Collapses h's binary hierarchy into h->wide (W-wide quantized nodes); wide.hip.
+int32_t collapse_wide(bajo_ctx* ctx, bajo_bvh* h);
 // The node count in a host copy of wide_ctl, clipped to the capacity.
 uint32_t collapse_read_count(const uint32_t* host_ctl, uint64_t capacity);
 // Reads back what a build left on the device (wide node count, H-PLOC root)

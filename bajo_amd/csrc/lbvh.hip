@@ -869,7 +869,7 @@ int32_t build_into(bajo_ctx* ctx, bajo_bvh* h, const float* vertices, uint64_t n
   }
   ev.record(5, st);
   if (wide_layout(h->node_width)) {
-    rc = collapse_wide(ctx, h, n);
+    rc = collapse_wide(ctx, h);
     if (rc) return rc;
   } else {
     h->wide_count = 0;
@@ -964,9 +964,6 @@ int32_t build_segmented(bajo_ctx* ctx, bajo_bvh* h, const float* vertices, const
   hipStream_t st = ctx->stream;
   rc = upload_segment_offsets(st, h, offsets, S);
   if (rc) return rc;
-  uint64_t largest = 0;
-  for (uint32_t s = 0; s < S; ++s)
-    if (offsets[s + 1] - offsets[s] > largest) largest = offsets[s + 1] - offsets[s];
   h->n = n;
   h->root_on_device = false;
   h->root_pending = false;
@@ -1026,7 +1023,7 @@ int32_t build_segmented(bajo_ctx* ctx, bajo_bvh* h, const float* vertices, const
   }
   ev.record(5, st);
   if (wide_layout(h->node_width)) {
-    rc = collapse_wide(ctx, h, largest);
+    rc = collapse_wide(ctx, h);
     if (rc) return rc;
   } else {
     h->wide_count = 0;

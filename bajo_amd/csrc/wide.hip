@@ -9,34 +9,40 @@
 // stored as 8-bit offsets on a per-axis power-of-two grid anchored at the
 // node's lower corner.
 //
-// Unlike bajo's persistent work queue with a spin fail-safe, the collapse here
-// is level-synchronous: level k processes the wide nodes allocated while
-// processing level k-1 (a contiguous index range), so no kernel ever waits on
-// another wave.  The host never reads the level sizes back: it enqueues a
-// depth-bounded number of full-grid level launches (each followed by a
-// one-thread launch that opens the next level; a launch past the last level
-// does nothing), then one single-block kernel that finishes any deeper
-// levels with block barriers.
-// The whole collapse is therefore enqueue-only and can be captured in a HIP
-// graph.  Leaf children reference ranges of the sorted triangle records that
-// the refit already wrote (an LBVH subtree covers a contiguous sorted range),
-// so no triangle data is copied.
+// Unlike bajo's persistent work queue with a spin fail-safe, no wave here
+// waits on another block.  Two launches build the whole hierarchy:
+//   - one block opens the first levels, one per barrier round, until a level
+//     holds more nodes than the block has threads;
+//   - one block per CU then takes every gridDim-th node of that level and
+//     finishes their subtrees by itself: it keeps the index ranges of its
+//     nodes still to be opened on an LDS stack and reserves the nodes of each
+//     batch's children (a contiguous range) with one atomic.
+// A node's children are opened through a chain of up to seven dependent loads,
+// so a level costs its latency however few nodes it has.  One launch per level
+// (each followed by a launch that opened the next, with four to five spare
+// ones for the depth) took 22 launches of 5-31 us: 0.40 ms at 4M triangles
+// (LBVH), 0.26 ms at 1M (H-PLOC).  The two launches take 0.24 and 0.15 ms.
+// The host reads nothing back, so the collapse is enqueue-only and can be
+// captured in a HIP graph.  Leaf children reference ranges of the sorted
+// triangle records that the refit already wrote (a subtree covers a contiguous
+// sorted range), so no triangle data is copied.
 #include "bvh_internal.h"
 
 namespace bj {
 namespace {
 
-constexpr int kCollapseBlock = 256;
-constexpr int kTailBlock = 1024;
-// Levels the single-block finishing kernel takes at most (a tree deeper than
-// the full-grid launches plus this raises BAJO_STATUS_COLLAPSE_FAILED).
-constexpr uint32_t kTailLevelCap = 4096;
+constexpr int kCollapseBlock = 1024;
+// Levels the first launch takes at most, and ranges a block of the second one
+// keeps (one per level of its subtrees): a deeper tree raises
+// BAJO_STATUS_COLLAPSE_FAILED.
+constexpr uint32_t kLevelCap = 4096;
 // wide_ctl words: node counter, level range, status
 constexpr int kCtlCount = 0, kCtlBegin = 1, kCtlEnd = 2, kCtlStatus = 3;
 constexpr uint32_t kStatusOutOfNodes = 1, kStatusTooDeep = 2, kStatusBadRoot = 4;
 
 struct Child {
   uint32_t ref, count;
+  uint32_t first;  // Karras hierarchies: the first sorted position below
   float b[6];
 };
 
@@ -45,8 +51,13 @@ BJ_D float half_area(const float* b) {
   return dx * dy + dx * dz + dy * dz;
 }
 
+// The children of binary node `node`.  In a Karras hierarchy the left child's
+// reference is the split position, so with the node's own range (`first`,
+// `count`) the children's ranges are known without another load; H-PLOC nodes
+// look their counts up.
+template <bool kKarras>
 BJ_D void load_children(const BjNode* __restrict__ bnodes, const uint32_t* __restrict__ leaf_counts, uint32_t node,
-                        Child& l, Child& r) {
+                        uint32_t first, uint32_t count, Child& l, Child& r) {
   const float4* p = reinterpret_cast<const float4*>(bnodes + node);
   const float4 a = p[0], b = p[1], c = p[2];
   const uint4 m = reinterpret_cast<const uint4*>(bnodes + node)[3];
@@ -54,8 +65,16 @@ BJ_D void load_children(const BjNode* __restrict__ bnodes, const uint32_t* __res
   r.b[0] = b.z; r.b[1] = b.w; r.b[2] = c.x; r.b[3] = c.y; r.b[4] = c.z; r.b[5] = c.w;
   l.ref = m.y;
   r.ref = m.z;
-  l.count = (l.ref & kLeafFlag) ? 1u : leaf_counts[l.ref];
-  r.count = (r.ref & kLeafFlag) ? 1u : leaf_counts[r.ref];
+  if constexpr (kKarras) {
+    l.first = first;
+    l.count = (m.y & kIndexMask) - first + 1u;
+    r.first = first + l.count;
+    r.count = count - l.count;
+  } else {
+    l.first = r.first = 0u;
+    l.count = (l.ref & kLeafFlag) ? 1u : leaf_counts[l.ref];
+    r.count = (r.ref & kLeafFlag) ? 1u : leaf_counts[r.ref];
+  }
 }
 
 // Smallest biased exponent e with o + 254 * 2^(e-127) >= hi (one spare step).
@@ -91,14 +110,14 @@ BJ_HD void quantize(float o, uint32_t e, float lo, float hi, uint8_t& qlo, uint8
   qhi = (uint8_t)fh;
 }
 
-// `root_dev` (H-PLOC: the root its clustering wrote) overrides `root_binary`;
-// a root outside the hierarchy leaves the level range empty and raises
-// BAJO_STATUS_COLLAPSE_FAILED.
-__global__ void collapse_root_kernel(const float* __restrict__ scene, uint32_t n, uint32_t root_binary,
-                                     const uint32_t* __restrict__ root_dev, BjWide* __restrict__ wide,
-                                     uint32_t* __restrict__ wide_src, uint32_t* __restrict__ ctl,
-                                     uint32_t* __restrict__ status) {
-  if (threadIdx.x != 0) return;
+// Wide node 0's source, written by one thread: the binary root.  `root_dev`
+// (H-PLOC: the root its clustering wrote) overrides `root_binary`; a root
+// outside the hierarchy raises BAJO_STATUS_COLLAPSE_FAILED and leaves nothing
+// to open.  Returns the nodes of level 0 still to be opened.
+BJ_D uint32_t collapse_root(const float* __restrict__ scene, uint32_t n, uint32_t root_binary,
+                            const uint32_t* __restrict__ root_dev, BjWide* __restrict__ wide,
+                            uint32_t* __restrict__ wide_src, uint32_t* __restrict__ ctl,
+                            uint32_t* __restrict__ status) {
   ctl[kCtlStatus] = 0;
   if (n == 1) {
     // single triangle: one wide node with one leaf child spanning the scene box
@@ -118,22 +137,16 @@ __global__ void collapse_root_kernel(const float* __restrict__ scene, uint32_t n
     quantize(scene[2], w.ez, scene[2], scene[5], w.lo_z[0], w.hi_z[0]);
     w.child[0] = kLeafFlag | 0u;
     wide[0] = w;
-    ctl[kCtlCount] = 1;
-    ctl[kCtlBegin] = 0;
-    ctl[kCtlEnd] = 0;
-    return;
+    return 0;
   }
   const uint32_t root = root_dev ? *root_dev : root_binary;
-  ctl[kCtlCount] = 1;
-  ctl[kCtlBegin] = 0;
   if ((root & kLeafFlag) || root >= n - 1) {
     ctl[kCtlStatus] = kStatusBadRoot;
-    ctl[kCtlEnd] = 0;
     atomicMax(status, (uint32_t)BAJO_STATUS_COLLAPSE_FAILED);
-    return;
+    return 0;
   }
   wide_src[0] = root;
-  ctl[kCtlEnd] = 1;
+  return 1;
 }
 
 // Segmented builds: wide node s is the root of segment s (S roots form level
@@ -177,76 +190,90 @@ __global__ void seg_collapse_root_kernel(const float* __restrict__ seg_scene, co
   }
 }
 
-// The next level is the nodes reserved by the last one, clipped to the
-// capacity; after a capacity failure the level range is left empty.  Run by
-// one thread once every wave of the level has reserved its nodes.
-BJ_D void level_advance(uint32_t* __restrict__ ctl, uint32_t capacity, uint32_t* __restrict__ status) {
-  const uint32_t end = ctl[kCtlEnd];
-  uint32_t next = __hip_atomic_load(ctl + kCtlCount, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (next > capacity) next = capacity;
-  if (__hip_atomic_load(ctl + kCtlStatus, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-    next = end;
-    atomicMax(status, (uint32_t)BAJO_STATUS_COLLAPSE_FAILED);
-  }
-  ctl[kCtlBegin] = end;
-  ctl[kCtlEnd] = next;
-}
-
-// LDS of one block's slot reservation: per-wave totals, then offsets.
-struct Reserve {
-  uint32_t wave_total[kTailBlock / 64];
-  uint32_t first;
+// LDS of one block's batch: per-wave totals, then offsets; the range reserved
+// for the batch's children.
+struct Batch {
+  uint32_t wave_total[kCollapseBlock / 64];
+  uint32_t first, total;
+  uint32_t failed;
 };
 
-// Collapses the wide nodes [begin, end) of one level.  The whole block steps
-// together (block `block` of `blocks`, `stride` threads apart) so that one
-// atomic per block and step reserves the nodes its children need: a
-// per-node atomic on the shared counter serializes (about 25 ns each).
-BJ_D void collapse_level(const BjNode* __restrict__ bnodes, const uint32_t* __restrict__ leaf_counts,
+// Opens the wide nodes begin + stride * threadIdx.x for threadIdx.x < len,
+// the whole block together: kShared reserves their children with one atomic on
+// the node counter (a per-node atomic serializes, about 25 ns each), a lone
+// block counts on in bt->first + bt->total.  Afterwards [bt->first,
+// bt->first + bt->total) are the children to be opened; bt->failed is set if
+// they do not fit.
+template <bool kKarras, bool kShared>
+BJ_D void collapse_batch(const BjNode* __restrict__ bnodes, const uint32_t* __restrict__ leaf_counts,
                          BjWide* __restrict__ wide, uint32_t* __restrict__ wide_src, uint32_t* __restrict__ ctl,
-                         uint32_t capacity, uint32_t max_leaf, int max_children, uint32_t begin, uint32_t end,
-                         uint32_t block_base, uint32_t stride, Reserve* __restrict__ rs) {
+                         uint32_t capacity, uint32_t max_leaf, int max_children, uint32_t begin, uint32_t stride,
+                         uint32_t len, Batch* __restrict__ bt) {
   const uint32_t lane = lane_id();
   const uint32_t wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
-  for (uint32_t bbase = begin + block_base; bbase < end; bbase += stride) {
-    const uint32_t w = bbase + threadIdx.x;
-    const bool active = w < end && wide_src[w] != kSentinel;
-    // The children live in registers: every index into ch[] below is a
-    // compile-time constant after unrolling (a data-dependent index would
-    // place the array in scratch memory).
+  {
+    const uint32_t w = begin + stride * threadIdx.x;
+    const uint32_t src = threadIdx.x < len ? wide_src[w] : kSentinel;
+    const bool active = src != kSentinel;
+    // The children live in registers: every index into ch[] is a compile-time
+    // constant (a data-dependent one would place the array in scratch memory).
+    // A lane that still opens children in step k has k + 2 of them, so the
+    // right child's slot is a constant and only the opened child's slot is
+    // selected.  A child's area is formed once, when it is loaded.
     Child ch[8];
+    float area[8];
     int n = 0;
     if (active) {
-      load_children(bnodes, leaf_counts, wide_src[w], ch[0], ch[1]);
+      uint32_t count = 0, first = 0;
+      if constexpr (kKarras) {
+        count = leaf_counts[src];
+        first = bnodes[src].fence + 1u - count;
+      }
+      load_children<kKarras>(bnodes, leaf_counts, src, first, count, ch[0], ch[1]);
+      area[0] = half_area(ch[0].b);
+      area[1] = half_area(ch[1].b);
       n = 2;
-      // open largest-area children: first those too big for a leaf, then any inner child
-      for (int phase = 0; phase < 2; ++phase) {
-        for (int step = 0; step < 6 && n < max_children; ++step) {
-          int pick = -1;
-          float best = -1.0f;
-          uint32_t pick_ref = 0;
+    }
 #pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            if (i < n) {
-              const bool inner = !(ch[i].ref & kLeafFlag);
-              const bool eligible = inner && (phase == 0 ? ch[i].count > max_leaf : ch[i].count >= 2);
-              const float a = half_area(ch[i].b);
-              if (eligible && a > best) {
-                best = a;
-                pick = i;
-                pick_ref = ch[i].ref;
-              }
+    for (int k = 2; k < 8; ++k) {
+      if (k < max_children && n == k) {
+        // the largest child too big for a leaf, else the largest inner child
+        // (the first of equal ones)
+        int pick = -1, pick1 = -1;
+        float best = -1.0f, best1 = -1.0f;
+#pragma unroll
+        for (int i = 0; i < k; ++i) {
+          const bool inner = !(ch[i].ref & kLeafFlag) && ch[i].count >= 2;
+          if (inner && ch[i].count > max_leaf && area[i] > best) {
+            best = area[i];
+            pick = i;
+          }
+          if (inner && area[i] > best1) {
+            best1 = area[i];
+            pick1 = i;
+          }
+        }
+        if (pick < 0) pick = pick1;
+        if (pick >= 0) {
+          uint32_t pick_ref = ch[0].ref, pick_first = ch[0].first, pick_count = ch[0].count;
+#pragma unroll
+          for (int i = 1; i < k; ++i) {
+            pick_ref = i == pick ? ch[i].ref : pick_ref;
+            pick_first = i == pick ? ch[i].first : pick_first;
+            pick_count = i == pick ? ch[i].count : pick_count;
+          }
+          Child l;
+          load_children<kKarras>(bnodes, leaf_counts, pick_ref, pick_first, pick_count, l, ch[k]);
+          const float al = half_area(l.b);
+          area[k] = half_area(ch[k].b);
+#pragma unroll
+          for (int i = 0; i < k; ++i) {
+            if (i == pick) {
+              ch[i] = l;
+              area[i] = al;
             }
           }
-          if (pick < 0) break;
-          Child l, r;
-          load_children(bnodes, leaf_counts, pick_ref, l, r);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            if (i == pick) ch[i] = l;
-            if (i == n) ch[i] = r;
-          }
-          ++n;
+          n = k + 1;
         }
       }
     }
@@ -261,24 +288,23 @@ BJ_D void collapse_level(const BjNode* __restrict__ bnodes, const uint32_t* __re
       const uint32_t y = __shfl_up(incl, off, 64);
       if (lane >= (uint32_t)off) incl += y;
     }
-    if (lane == 63) rs->wave_total[wave] = incl;
+    if (lane == 63) bt->wave_total[wave] = incl;
     __syncthreads();
     if (threadIdx.x == 0) {
       uint32_t sum = 0;
       for (uint32_t i = 0; i < waves; ++i) {
-        const uint32_t t = rs->wave_total[i];
-        rs->wave_total[i] = sum;
+        const uint32_t t = bt->wave_total[i];
+        bt->wave_total[i] = sum;
         sum += t;
       }
-      rs->first = sum ? atomicAdd(ctl + kCtlCount, sum) : 0u;
+      if constexpr (kShared) bt->first = sum ? atomicAdd(ctl + kCtlCount, sum) : 0u;
+      else bt->first += bt->total;
+      bt->total = sum;
+      bt->failed = (uint64_t)bt->first + sum > capacity ? 1u : 0u;
     }
     __syncthreads();
-    const uint32_t first = rs->first + rs->wave_total[wave] + (incl - k);
-    if (!active) continue;
-    if ((uint64_t)first + k > capacity) {
-      atomicOr(ctl + kCtlStatus, kStatusOutOfNodes);
-      continue;
-    }
+    if (!active || bt->failed) return;
+    const uint32_t first = bt->first + bt->wave_total[wave] + (incl - k);
     // node box and per-axis grids
     float box[6] = {kFltMax, kFltMax, kFltMax, -kFltMax, -kFltMax, -kFltMax};
 #pragma unroll
@@ -314,8 +340,8 @@ BJ_D void collapse_level(const BjNode* __restrict__ bnodes, const uint32_t* __re
           child[i] = kLeafFlag | (ref & kIndexMask);  // one triangle
         } else if (ch[i].count <= max_leaf) {
           // inner binary node over sorted range [fence - count + 1, fence]
-          const uint32_t fence = bnodes[ref].fence;
-          child[i] = kLeafFlag | ((ch[i].count - 1u) << 28) | (fence + 1u - ch[i].count);
+          const uint32_t start = kKarras ? ch[i].first : bnodes[ref].fence + 1u - ch[i].count;
+          child[i] = kLeafFlag | ((ch[i].count - 1u) << 28) | start;
         } else {
           child[i] = next;
           wide_src[next] = ref;
@@ -335,116 +361,136 @@ BJ_D void collapse_level(const BjNode* __restrict__ bnodes, const uint32_t* __re
   }
 }
 
-// One level over the whole grid; a launch whose level range is empty returns
-// at once, and blocks past the level's nodes return before any barrier.
-__global__ void __launch_bounds__(kCollapseBlock) collapse_level_kernel(const BjNode* __restrict__ bnodes,
-                                                                        const uint32_t* __restrict__ leaf_counts,
-                                                                        BjWide* __restrict__ wide,
-                                                                        uint32_t* __restrict__ wide_src,
-                                                                        uint32_t* __restrict__ ctl,
-                                                                        uint32_t capacity, uint32_t max_leaf,
-                                                                        int max_children) {
-  __shared__ Reserve rs;
-  const uint32_t begin = ctl[kCtlBegin], end = ctl[kCtlEnd];
-  if ((uint64_t)begin + (uint64_t)blockIdx.x * blockDim.x >= end) return;
-  collapse_level(bnodes, leaf_counts, wide, wide_src, ctl, capacity, max_leaf, max_children, begin, end,
-                 blockIdx.x * blockDim.x, gridDim.x * blockDim.x, &rs);
-}
-
-// Opens the next level once every block of the last one has finished.
-__global__ void level_advance_kernel(uint32_t* __restrict__ ctl, uint32_t capacity, uint32_t* __restrict__ status) {
-  if (threadIdx.x == 0 && ctl[kCtlBegin] != ctl[kCtlEnd]) level_advance(ctl, capacity, status);
-}
-
-// Every level left after the full-grid launches, in one block: level by level
-// with block barriers (no wait on another block), up to kTailLevelCap levels.
-__global__ void __launch_bounds__(kTailBlock) collapse_tail_kernel(const BjNode* __restrict__ bnodes,
-                                                                   const uint32_t* __restrict__ leaf_counts,
-                                                                   BjWide* __restrict__ wide,
-                                                                   uint32_t* __restrict__ wide_src,
-                                                                   uint32_t* __restrict__ ctl, uint32_t capacity,
-                                                                   uint32_t max_leaf, int max_children,
-                                                                   uint32_t* __restrict__ status) {
-  __shared__ uint32_t range[2];
-  __shared__ Reserve rs;
-  for (uint32_t level = 0;; ++level) {
-    if (threadIdx.x == 0) {
-      range[0] = ctl[kCtlBegin];
-      range[1] = ctl[kCtlEnd];
-    }
+// The first levels, in one block.  `segmented`: level 0 (the segment roots)
+// is already in ctl.  Leaves the first level larger than the block (or an
+// empty range) in ctl.
+template <bool kKarras>
+__global__ void __launch_bounds__(kCollapseBlock)
+collapse_top_kernel(const BjNode* __restrict__ bnodes, const uint32_t* __restrict__ leaf_counts,
+                    BjWide* __restrict__ wide, uint32_t* __restrict__ wide_src, uint32_t* __restrict__ ctl,
+                    uint32_t capacity, uint32_t max_leaf, int max_children, const float* __restrict__ scene,
+                    uint32_t n, uint32_t root_binary, const uint32_t* __restrict__ root_dev, int segmented,
+                    uint32_t* __restrict__ status) {
+  __shared__ Batch bt;
+  // the level being opened is [bt.first, bt.first + bt.total)
+  if (threadIdx.x == 0) {
+    bt.first = 0;
+    bt.total = segmented ? ctl[kCtlEnd] : collapse_root(scene, n, root_binary, root_dev, wide, wide_src, ctl, status);
+    bt.failed = 0;
+  }
+  __threadfence_block();
+  __syncthreads();
+  uint32_t level = 0;
+  while (bt.total != 0 && bt.total <= blockDim.x && !bt.failed && level < kLevelCap) {
+    const uint32_t begin = bt.first, len = bt.total;
+    ++level;
     __syncthreads();
-    const uint32_t begin = range[0], end = range[1];
-    if (begin == end) break;
-    if (level == kTailLevelCap) {
-      if (threadIdx.x == 0) {
-        atomicOr(ctl + kCtlStatus, kStatusTooDeep);
-        atomicMax(status, (uint32_t)BAJO_STATUS_COLLAPSE_FAILED);
-      }
-      break;
-    }
-    collapse_level(bnodes, leaf_counts, wide, wide_src, ctl, capacity, max_leaf, max_children, begin, end, 0u,
-                   blockDim.x, &rs);
-    __threadfence();
-    __syncthreads();
-    if (threadIdx.x == 0) level_advance(ctl, capacity, status);
+    collapse_batch<kKarras, false>(bnodes, leaf_counts, wide, wide_src, ctl, capacity, max_leaf, max_children, begin,
+                                   1u, len, &bt);
+    __threadfence_block();
     __syncthreads();
   }
+  if (threadIdx.x == 0) {
+    uint32_t end = bt.first + bt.total;
+    if (bt.failed || (bt.total != 0 && level == kLevelCap)) {
+      ctl[kCtlStatus] = bt.failed ? kStatusOutOfNodes : kStatusTooDeep;
+      atomicMax(status, (uint32_t)BAJO_STATUS_COLLAPSE_FAILED);
+      end = bt.first;
+    }
+    ctl[kCtlBegin] = bt.first;
+    ctl[kCtlEnd] = end;
+    // a build without nodes to open still has its root record
+    ctl[kCtlCount] = end > 0 ? end : 1u;
+  }
+}
+
+// Every level left, one subtree after another in each block.
+template <bool kKarras>
+__global__ void __launch_bounds__(kCollapseBlock)
+collapse_subtree_kernel(const BjNode* __restrict__ bnodes, const uint32_t* __restrict__ leaf_counts,
+                        BjWide* __restrict__ wide, uint32_t* __restrict__ wide_src, uint32_t* __restrict__ ctl,
+                        uint32_t capacity, uint32_t max_leaf, int max_children, uint32_t* __restrict__ status) {
+  __shared__ Batch bt;
+  __shared__ uint32_t s_first[kLevelCap], s_len[kLevelCap];
+  const uint32_t end = ctl[kCtlEnd];
+  for (uint32_t at = ctl[kCtlBegin] + blockIdx.x; at < end; at += gridDim.x * blockDim.x) {
+    const uint32_t left = (end - at + gridDim.x - 1) / gridDim.x;
+    uint32_t begin = at, stride = gridDim.x, len = left < blockDim.x ? left : blockDim.x;
+    int depth = 0;
+    for (;;) {
+      collapse_batch<kKarras, true>(bnodes, leaf_counts, wide, wide_src, ctl, capacity, max_leaf, max_children, begin,
+                                    stride, len, &bt);
+      __threadfence_block();
+      __syncthreads();
+      const bool full = bt.total != 0 && depth == (int)kLevelCap;
+      if (bt.failed || full) {
+        if (threadIdx.x == 0) {
+          atomicOr(ctl + kCtlStatus, full ? kStatusTooDeep : kStatusOutOfNodes);
+          atomicMax(status, (uint32_t)BAJO_STATUS_COLLAPSE_FAILED);
+        }
+        return;
+      }
+      if (bt.total != 0) {
+        if (threadIdx.x == 0) {
+          s_first[depth] = bt.first;
+          s_len[depth] = bt.total;
+        }
+        ++depth;
+      }
+      __syncthreads();
+      if (depth == 0) break;
+      // the next batch: up to a block's worth of the range on top
+      begin = s_first[depth - 1];
+      stride = 1;
+      const uint32_t range = s_len[depth - 1];
+      len = range < blockDim.x ? range : blockDim.x;
+      __syncthreads();
+      if (len == range) {
+        --depth;
+      } else if (threadIdx.x == 0) {
+        s_first[depth - 1] = begin + len;
+        s_len[depth - 1] = range - len;
+      }
+    }
+  }
+}
+
+template <bool kKarras>
+void launch_collapse(bajo_ctx* ctx, bajo_bvh* h, const uint32_t* root_dev, unsigned blocks) {
+  const uint32_t n = (uint32_t)h->n, capacity = (uint32_t)h->wide_capacity;
+  collapse_top_kernel<kKarras><<<1, kCollapseBlock, 0, ctx->stream>>>(
+      h->nodes, h->leaf_counts, h->wide, h->wide_src, h->wide_ctl, capacity, h->wide_leaf, h->node_width, h->scene, n,
+      n > 1 ? h->root : 0u, root_dev, h->seg_count ? 1 : 0, ctx->status);
+  if (n <= kCollapseBlock && !h->seg_count) return;  // no level can outgrow the first launch
+  collapse_subtree_kernel<kKarras><<<blocks, kCollapseBlock, 0, ctx->stream>>>(
+      h->nodes, h->leaf_counts, h->wide, h->wide_src, h->wide_ctl, capacity, h->wide_leaf, h->node_width, ctx->status);
 }
 
 }  // namespace
 
-// Full-grid level launches enqueued before the finishing kernel: the depth of
-// a W-wide tree over `leaves` leaf groups of max_leaf triangles plus the few
-// deeper levels an LBVH or H-PLOC tree adds (measured: 2-3 at W = 8, 4-5 at
-// W = 4 for 1M-16M triangles).  Launches past the last level return at once.
-uint32_t collapse_grid_levels(uint64_t leaves, uint32_t max_leaf, int width) {
-  const uint64_t groups = leaves / (max_leaf ? max_leaf : 1) + 1;
-  uint32_t depth = 0;
-  for (uint64_t span = 1; span < groups; span *= (uint64_t)width) ++depth;
-  return depth + (width == 4 ? 5u : 4u);
-}
-
 // Builds the W-wide layout of h from its binary hierarchy.  Enqueue-only: the
 // host reads nothing back (the node count is read at the first host query,
 // H-PLOC's root comes from the device).
-int32_t collapse_wide(bajo_ctx* ctx, bajo_bvh* h, uint64_t largest_tree) {
+int32_t collapse_wide(bajo_ctx* ctx, bajo_bvh* h) {
   hipStream_t st = ctx->stream;
   const uint32_t n = (uint32_t)h->n;
   int dev = 0, cus = 0;
   BJ_HIP(hipGetDevice(&dev));
   BJ_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  const uint32_t* root_dev = nullptr;
   if (h->seg_count) {
     const uint32_t S = h->seg_count;
     seg_collapse_root_kernel<<<div_up(S, 256u) < 1024u ? div_up(S, 256u) : 1024u, 256, 0, st>>>(
         h->seg_scene, h->seg_off, S, h->wide, h->wide_src, h->wide_ctl);
-  } else {
-    const uint32_t* root_dev = (n > 1 && h->root_on_device) ? h->hp_ctl + kHpCtlRoot : nullptr;
-    collapse_root_kernel<<<1, 64, 0, st>>>(h->scene, n, n > 1 ? h->root : 0u, root_dev, h->wide, h->wide_src,
-                                           h->wide_ctl, ctx->status);
+    BJ_HIP(hipGetLastError());
+  } else if (n > 1 && h->root_on_device) {
+    root_dev = h->hp_ctl + kHpCtlRoot;
   }
+  if (h->method == BAJO_BUILD_HPLOC) launch_collapse<false>(ctx, h, root_dev, (unsigned)cus);
+  else launch_collapse<true>(ctx, h, root_dev, (unsigned)cus);
   BJ_HIP(hipGetLastError());
-  h->wide_pending = false;
-  if (n == 1) {
-    h->wide_count = 1;
-    return BAJO_OK;
-  }
-  // grid: enough waves for the widest level (~n/3 nodes), capped at a few per CU
-  unsigned grid = div_up(n / 3 + 1, kCollapseBlock);
-  const unsigned cap_grid = (unsigned)cus * 8;
-  if (grid > cap_grid) grid = cap_grid;
-  if (grid < 1) grid = 1;
-  const uint32_t levels = collapse_grid_levels(largest_tree, h->wide_leaf, h->node_width);
-  for (uint32_t l = 0; l < levels; ++l) {
-    collapse_level_kernel<<<grid, kCollapseBlock, 0, st>>>(h->nodes, h->leaf_counts, h->wide, h->wide_src,
-                                                           h->wide_ctl, (uint32_t)h->wide_capacity,
-                                                           (uint32_t)h->wide_leaf, h->node_width);
-    level_advance_kernel<<<1, 64, 0, st>>>(h->wide_ctl, (uint32_t)h->wide_capacity, ctx->status);
-  }
-  collapse_tail_kernel<<<1, kTailBlock, 0, st>>>(h->nodes, h->leaf_counts, h->wide, h->wide_src, h->wide_ctl,
-                                                 (uint32_t)h->wide_capacity, (uint32_t)h->wide_leaf, h->node_width,
-                                                 ctx->status);
-  BJ_HIP(hipGetLastError());
-  h->wide_pending = true;
+  h->wide_pending = !(n == 1 && !h->seg_count);
+  if (!h->wide_pending) h->wide_count = 1;
   return BAJO_OK;
 }
 
