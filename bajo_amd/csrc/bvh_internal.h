@@ -53,7 +53,8 @@ struct bajo_bvh {
   uint64_t* keys;      // n
   uint32_t* leaf_parent;  // n
   uint32_t* leaf_counts;  // n-1
-  uint32_t* flags;        // n-1
+  uint32_t* flags;        // n: arrival words of the bottom-up passes
+  void* hands;            // LBVH: records handed between blocks of the climb
   uint32_t* acc;          // 12 ordered-int bounds accumulators
   float* scene;           // 12 floats
   void* sort_ws;

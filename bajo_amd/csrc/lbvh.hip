@@ -15,10 +15,13 @@
 //      order and the sort is stable, which yields the same order as a full
 //      64-bit sort (and as bajo's stable (segment, code) pair sort with
 //      value = index, lbvh.mojo:94-113) in 4 passes instead of 8.
-//   4. Karras topology (lbvh.mojo:164-329), one thread per internal node.
-//   5. atomic bottom-up refit (lbvh.mojo:116-161): the second arriver at a
-//      node merges both child boxes and climbs.  The same pass packs each
-//      sorted leaf's triangle (v0, e1, e2, prim) for traversal.
+//   4. topology (lbvh.mojo:164-329) and boxes (lbvh.mojo:116-161) in one
+//      bottom-up climb that also packs each sorted leaf's triangle (v0, e1,
+//      e2, prim) for traversal.  (The top-down Karras kernel below is H-PLOC's
+//      guide.)
+// The vertices are read three times; plain loads leave them in the Infinity
+// Cache for the next pass (non-temporal ones: the climb 376 us against 343 at
+// 4M triangles, 638 against 510 for a 512-mesh set of 6M).
 #include <string.h>
 
 #include <vector>
@@ -34,36 +37,12 @@ constexpr int kSortBeginBit = 32;
 constexpr int kSortEndBit = 64;
 constexpr int kSortPasses = (kSortEndBit - kSortBeginBit) / 8;
 
-BJ_D float ld(const float* p) { return __builtin_nontemporal_load(p); }
-
 BJ_D uint64_t pack2(float a, float b) {
   return (uint64_t)__builtin_bit_cast(uint32_t, a) | ((uint64_t)__builtin_bit_cast(uint32_t, b) << 32);
 }
 BJ_D void unpack2(uint64_t w, float& a, float& b) {
   a = __builtin_bit_cast(float, (uint32_t)w);
   b = __builtin_bit_cast(float, (uint32_t)(w >> 32));
-}
-
-BJ_D void load_tri(const float* __restrict__ v, uint64_t i, v3& a, v3& b, v3& c) {
-  const float* t = v + 9 * i;
-  a = mk(ld(t + 0), ld(t + 1), ld(t + 2));
-  b = mk(ld(t + 3), ld(t + 4), ld(t + 5));
-  c = mk(ld(t + 6), ld(t + 7), ld(t + 8));
-}
-
-// Leaf box with streaming (non-temporal) loads for the one-pass kernels.
-template <bool kBoxes>
-BJ_D void leaf_src(const float* __restrict__ src, uint64_t i, v3& lo, v3& hi) {
-  if constexpr (kBoxes) {
-    const float* b = src + 6 * i;
-    lo = mk(ld(b + 0), ld(b + 1), ld(b + 2));
-    hi = mk(ld(b + 3), ld(b + 4), ld(b + 5));
-  } else {
-    v3 a, b, c;
-    load_tri(src, i, a, b, c);
-    lo = vmin(vmin(a, b), c);
-    hi = vmax(vmax(a, b), c);
-  }
 }
 
 __global__ void __launch_bounds__(256) lbvh_init_kernel(uint32_t* acc, uint32_t* hist, uint32_t* tickets) {
@@ -98,7 +77,7 @@ __global__ void __launch_bounds__(kBlock) scene_bounds_kernel(const float* __res
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
     v3 lo, hi;
-    leaf_src<kBoxes>(vertices, i, lo, hi);
+    leaf_box<kBoxes>(vertices, i, lo, hi);
     v3 ce = scale(add(lo, hi), 0.5f);
     r[0] = fmin_sel(r[0], lo.x); r[1] = fmin_sel(r[1], lo.y); r[2] = fmin_sel(r[2], lo.z);
     r[3] = fmax_sel(r[3], hi.x); r[4] = fmax_sel(r[4], hi.y); r[5] = fmax_sel(r[5], hi.z);
@@ -127,7 +106,8 @@ template <bool kBoxes>
 __global__ void __launch_bounds__(kBlock) morton_kernel(const float* __restrict__ vertices, uint64_t n,
                                                         const uint32_t* __restrict__ acc, float* __restrict__ scene,
                                                         uint64_t* __restrict__ keys, uint32_t* __restrict__ hist,
-                                                        uint32_t* __restrict__ lookback, uint64_t lookback_words) {
+                                                        uint32_t* __restrict__ lookback, uint64_t lookback_words,
+                                                        uint32_t* __restrict__ meet) {
   __shared__ uint32_t s_hist[kBlock / 64][kSortPasses * 256];
   const uint32_t wave = threadIdx.x >> 6;
   for (uint32_t i = threadIdx.x; i < (kBlock / 64) * kSortPasses * 256; i += blockDim.x) (&s_hist[0][0])[i] = 0;
@@ -142,10 +122,11 @@ __global__ void __launch_bounds__(kBlock) morton_kernel(const float* __restrict_
   __syncthreads();
   for (uint64_t i = gtid; i < n; i += gstride) {
     v3 lo, hi;
-    leaf_src<kBoxes>(vertices, i, lo, hi);
+    leaf_box<kBoxes>(vertices, i, lo, hi);
     v3 q = mul(sub(scale(add(lo, hi), 0.5f), cmin), inv);
     uint32_t code = morton3(q.x, q.y, q.z);
     keys[i] = ((uint64_t)code << 32) | (uint64_t)(uint32_t)i;
+    meet[i] = 0;
 #pragma unroll
     for (int p = 0; p < kSortPasses; ++p) atomicAdd(&s_hist[wave][p * 256 + ((code >> (8 * p)) & 0xFFu)], 1u);
   }
@@ -275,151 +256,6 @@ __global__ void __launch_bounds__(kBlock) karras_kernel(const uint64_t* __restri
 
 namespace {
 
-// Bottom-up refit, one thread per sorted leaf.  Nodes whose leaf range lies
-// inside this block's 256 leaves are merged in LDS (arrival counters and
-// child boxes in shared memory; the second arriver writes the node's two
-// child boxes with plain stores).  Only nodes whose range crosses a block
-// boundary use the cross-XCD hand-off through global memory.
-// `gprim` (segmented builds) gives each sorted leaf's input index, whose low
-// key word is its index inside the segment; `node_total` bounds the climb.
-template <bool kBoxes>
-__global__ void __launch_bounds__(kBlock) refit_kernel(const float* __restrict__ vertices,
-                                                       const uint64_t* __restrict__ keys,
-                                                       const uint32_t* __restrict__ gprim, uint64_t n,
-                                                       uint64_t node_total, BjNode* __restrict__ nodes,
-                                                       uint32_t* __restrict__ leaf_parent,
-                                                       const uint32_t* __restrict__ leaf_counts,
-                                                       uint32_t* __restrict__ flags, BjTri* __restrict__ tris,
-                                                       uint32_t* __restrict__ status) {
-  __shared__ uint32_t s_flag[kBlock];
-  __shared__ float s_box[kBlock][2][6];
-  s_flag[threadIdx.x] = 0;
-  __syncthreads();
-  const uint64_t s = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= n) return;
-  const uint32_t prim = (uint32_t)keys[s];
-  const uint64_t src = gprim ? (uint64_t)gprim[s] : (uint64_t)prim;
-  v3 lo, hi;
-  if constexpr (kBoxes) {
-    leaf_src<true>(vertices, src, lo, hi);
-  } else {
-    v3 a, b, c;
-    load_tri(vertices, src, a, b, c);
-    v3 e1 = sub(b, a), e2 = sub(c, a);
-    float4* out = reinterpret_cast<float4*>(tris + s);
-    out[0] = make_float4(a.x, a.y, a.z, __builtin_bit_cast(float, prim));
-    out[1] = make_float4(e1.x, e1.y, e1.z, 0.0f);
-    out[2] = make_float4(e2.x, e2.y, e2.z, 0.0f);
-    // bvh/gpu/triangle_bvh.mojo:711-712: leaf box = vmin(vmin(v0,v1),v2).
-    lo = vmin(vmin(a, b), c);
-    hi = vmax(vmax(a, b), c);
-  }
-  if (n < 2) {
-    leaf_parent[0] = kSentinel;  // single-leaf segment, lbvh.mojo:246-248
-    return;
-  }
-  const uint64_t block_first = (uint64_t)blockIdx.x * blockDim.x;
-  const uint64_t block_last = block_first + blockDim.x - 1 < n - 1 ? block_first + blockDim.x - 1 : n - 1;
-  uint32_t cur = kLeafFlag | (uint32_t)s;
-  uint32_t parent = leaf_parent[s];
-  // A node's topology (parent, left, right, fence: its last 16 bytes) and leaf
-  // count were written by the topology launch and do not change here, so the
-  // next level's are loaded while this level's boxes are exchanged.
-  uint4 topo = make_uint4(kSentinel, kSentinel, kSentinel, 0u);
-  uint32_t count = 0;
-  if (parent < node_total) {
-    topo = reinterpret_cast<const uint4*>(nodes + parent)[3];
-    count = leaf_counts[parent];
-  }
-  // A Karras hierarchy over 64-bit keys is at most 64 levels deep; the index
-  // and depth checks only keep a corrupted hierarchy from leaving the arrays,
-  // and a climb they stop raises BAJO_STATUS_REFIT_CORRUPT.
-  int depth = 0;
-  for (; parent != kSentinel && depth < 128; ++depth) {
-    if (parent >= node_total) {
-      atomicMax(status, (uint32_t)BAJO_STATUS_REFIT_CORRUPT);
-      break;
-    }
-    BjNode* node = nodes + parent;
-    const uint32_t left = topo.y, right = topo.z;
-    const bool is_left = cur == left;
-    if (!is_left && cur != right) {
-      atomicMax(status, (uint32_t)BAJO_STATUS_REFIT_CORRUPT);
-      break;
-    }
-    // Karras node i is one end of its leaf range [fence + 1 - count, fence]
-    const uint64_t last = topo.w, first = last + 1 - count;
-    const uint32_t next = topo.x;
-    uint4 next_topo = make_uint4(kSentinel, kSentinel, kSentinel, 0u);
-    uint32_t next_count = 0;
-    if (next < node_total) {
-      next_topo = reinterpret_cast<const uint4*>(nodes + next)[3];
-      next_count = leaf_counts[next];
-    }
-    v3 olo, ohi;
-    if (first >= block_first && last <= block_last && parent >= block_first && parent - block_first < kBlock) {
-      // every leaf below this node belongs to this block
-      float* mine = s_box[parent - block_first][is_left ? 0 : 1];
-      mine[0] = lo.x; mine[1] = lo.y; mine[2] = lo.z; mine[3] = hi.x; mine[4] = hi.y; mine[5] = hi.z;
-      __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      __builtin_amdgcn_s_waitcnt(0xC07F);  // LDS writes done (lgkmcnt 0)
-      __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      const uint32_t old = atomicAdd(&s_flag[parent - block_first], 1u);
-      if (old == 0) break;
-      __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      const float* o = s_box[parent - block_first][is_left ? 1 : 0];
-      olo = mk(o[0], o[1], o[2]);
-      ohi = mk(o[3], o[4], o[5]);
-      // both child boxes of the node
-      float* l = node->b;
-      const v3 llo = is_left ? lo : olo, lhi = is_left ? hi : ohi;
-      const v3 rlo = is_left ? olo : lo, rhi = is_left ? ohi : hi;
-      reinterpret_cast<float4*>(l)[0] = make_float4(llo.x, llo.y, llo.z, lhi.x);
-      reinterpret_cast<float4*>(l)[1] = make_float4(lhi.y, lhi.z, rlo.x, rlo.y);
-      reinterpret_cast<float4*>(l)[2] = make_float4(rlo.z, rhi.x, rhi.y, rhi.z);
-    } else {
-      // Publish this child's box with write-through (agent-scope) stores and
-      // wait until they are performed before the arrival counter is bumped.
-      // This is the release half of the hand-off without an L2 writeback:
-      // the shared data itself never sits in a non-coherent cache line.
-      // Boxes move as three 8-byte words (child halves start at byte 0 and 24).
-      uint64_t* mine = reinterpret_cast<uint64_t*>(node->b + (is_left ? 0 : 6));
-      const uint64_t w0 = pack2(lo.x, lo.y), w1 = pack2(lo.z, hi.x), w2 = pack2(hi.y, hi.z);
-      __hip_atomic_store(mine + 0, w0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(mine + 1, w1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(mine + 2, w2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      __builtin_amdgcn_s_waitcnt(0);
-      __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      const uint32_t old = __hip_atomic_fetch_add(flags + parent, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (old == 0) break;
-      // Second arriver: the sibling's stores completed before its increment,
-      // which returned before ours; coherent loads read them.
-      __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      const uint64_t* other = reinterpret_cast<const uint64_t*>(node->b + (is_left ? 6 : 0));
-      float o[6];
-      unpack2(__hip_atomic_load(other + 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), o[0], o[1]);
-      unpack2(__hip_atomic_load(other + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), o[2], o[3]);
-      unpack2(__hip_atomic_load(other + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), o[4], o[5]);
-      olo = mk(o[0], o[1], o[2]);
-      ohi = mk(o[3], o[4], o[5]);
-    }
-    // _load_and_union_node_bounds (binary_layout.mojo:95-101): merge(left, right).
-    if (is_left) {
-      lo = vmin(lo, olo);
-      hi = vmax(hi, ohi);
-    } else {
-      lo = vmin(olo, lo);
-      hi = vmax(ohi, hi);
-    }
-    cur = parent;
-    parent = next;
-    topo = next_topo;
-    count = next_count;
-  }
-  if (depth == 128) atomicMax(status, (uint32_t)BAJO_STATUS_REFIT_CORRUPT);
-}
-
 // ---- segmented builds (bajo's BLAS sets) ------------------------------------
 // Segment s owns sorted leaves [off_s, off_{s+1}) (every segment nonempty)
 // and internal nodes [off_s, off_{s+1} - 1): its hierarchy is the
@@ -452,6 +288,221 @@ BJ_D uint32_t segment_at(const uint64_t* __restrict__ off, const uint32_t* __res
   uint32_t s = chunk[i >> 6];
   while (off[s + 1] <= i) ++s;
   return s;
+}
+
+// Topology and boxes of the LBVH in one bottom-up pass, one thread per sorted
+// leaf.  The common prefixes d(i) of neighbouring keys i, i + 1 decide the
+// hierarchy: the parent of the node over [l, r] splits at r if
+// d(r) > d(l - 1) (the node is its left child), else at l - 1; the two never
+// tie, because keys are unique ((code << 32) | sorted position).  Both
+// children meet at their split: the first leaves its box, outer end and outer
+// prefix there, the second forms the parent and climbs on, so a node's own
+// range and both its prefixes are always at hand and no key is read again.
+// A node's index is Karras's: the last position of its range if it is a left
+// child, the first if it is a right child or the root.
+//
+// Meetings inside a block's leaves go through LDS; a node whose sibling
+// reaches past the block is left for the second phase, where the meetings go
+// through global memory: the record is written with agent-scope write-through
+// stores, performed before the exchange that announces it (release without an
+// L2 writeback; the eight XCDs' L2s are not coherent otherwise), and the
+// second arriver reads it with coherent loads.  At most two nodes per level
+// of the hierarchy reach past a block (its prefixes grow along a path, so 62
+// levels at most), hence kHandSlots records per block.
+//
+// A topology launch (0.12 ms) and an atomic refit that read every level's
+// record, leaf count and parent from memory (0.45 ms) took 0.57 ms at 4M
+// triangles; this pass takes 0.34 ms, for 261 MB read and 572 MB written
+// (2.4 TB/s): the records leave the climb in 16-, 12- and 4-byte pieces.
+// (Gathered in LDS and stored in rows they took 0.48 ms: the 64 bytes per leaf
+// halve the resident waves.  Blocks of 256 / 512 / 1,024 leaves: 416, 376 and
+// 393 us with non-temporal loads.)
+constexpr int kClimbBlock = 512;
+constexpr uint32_t kHandSlots = 128;
+struct __attribute__((aligned(16))) HandOff {
+  float box[6];
+  uint32_t end, prefix;  // outer end of the range, and the prefix beyond it
+};
+
+// A node during the climb: its range, the prefixes beyond both ends (0 = the
+// end of the hierarchy, else 1 + the common prefix length) and its box.
+struct Climber {
+  uint32_t l, r, dl, dr;
+  v3 lo, hi;
+  BJ_D bool root() const { return (dl | dr) == 0; }
+  BJ_D bool is_left() const { return dr > dl; }
+  BJ_D HandOff hand() const {
+    const bool left = is_left();
+    return HandOff{{lo.x, lo.y, lo.z, hi.x, hi.y, hi.z}, left ? l : r, left ? dl : dr};
+  }
+  // Joins the sibling `o` and writes the parent's record; *this becomes the
+  // parent.
+  BJ_D void join(const HandOff& o, BjNode* __restrict__ nodes, uint32_t* __restrict__ leaf_parent,
+                 uint32_t* __restrict__ leaf_counts) {
+    const bool left = is_left();
+    const uint32_t split = left ? r : l - 1u;
+    const v3 olo = mk(o.box[0], o.box[1], o.box[2]), ohi = mk(o.box[3], o.box[4], o.box[5]);
+    const v3 llo = left ? lo : olo, lhi = left ? hi : ohi, rlo = left ? olo : lo, rhi = left ? ohi : hi;
+    if (left) {
+      r = o.end;
+      dr = o.prefix;
+    } else {
+      l = o.end;
+      dl = o.prefix;
+    }
+    // _load_and_union_node_bounds (binary_layout.mojo:95-101): merge(left, right).
+    lo = vmin(llo, rlo);
+    hi = vmax(lhi, rhi);
+    const uint32_t me = is_left() ? r : l;
+    const bool left_leaf = l == split, right_leaf = split + 1u == r;
+    BjNode* nd = nodes + me;
+    reinterpret_cast<float4*>(nd)[0] = make_float4(llo.x, llo.y, llo.z, lhi.x);
+    reinterpret_cast<float4*>(nd)[1] = make_float4(lhi.y, lhi.z, rlo.x, rlo.y);
+    reinterpret_cast<float4*>(nd)[2] = make_float4(rlo.z, rhi.x, rhi.y, rhi.z);
+    nd->left = left_leaf ? (kLeafFlag | split) : split;
+    *reinterpret_cast<uint2*>(&nd->right) = make_uint2(right_leaf ? (kLeafFlag | (split + 1u)) : split + 1u, r);
+    leaf_counts[me] = r - l + 1u;
+    if (left_leaf) leaf_parent[split] = me;
+    else nodes[split].parent = me;
+    if (right_leaf) leaf_parent[split + 1u] = me;
+    else nodes[split + 1u].parent = me;
+    if (root()) nd->parent = kSentinel;
+  }
+};
+
+// `gprim` (segmented builds) gives each sorted leaf's input index, whose low
+// key word is its index inside the segment; no prefix crosses a segment.
+template <bool kBoxes, bool kSeg>
+__global__ void __launch_bounds__(kClimbBlock)
+lbvh_climb_kernel(const float* __restrict__ vertices, const uint64_t* __restrict__ keys,
+                  const uint32_t* __restrict__ gprim, uint64_t n, const uint64_t* __restrict__ off,
+                  const uint32_t* __restrict__ chunk, BjNode* __restrict__ nodes, uint32_t* __restrict__ leaf_parent,
+                  uint32_t* __restrict__ leaf_counts, uint32_t* __restrict__ meet, HandOff* __restrict__ hands,
+                  BjTri* __restrict__ tris, uint32_t* __restrict__ status) {
+  __shared__ uint32_t s_code[kClimbBlock + 1];
+  __shared__ uint8_t s_prefix[kClimbBlock + 1];  // [t]: beyond position t - 1 of the block
+  __shared__ uint32_t s_meet[kClimbBlock];       // 1 + the thread waiting at a split
+  __shared__ HandOff s_hand[kClimbBlock];
+  __shared__ uint32_t s_slots;
+  const uint32_t t = threadIdx.x;
+  const uint64_t first = (uint64_t)blockIdx.x * kClimbBlock, i = first + t;
+  const uint32_t m = n - first < kClimbBlock ? (uint32_t)(n - first) : (uint32_t)kClimbBlock;
+  const bool live = t < m;
+  s_meet[t] = 0;
+  if (t == 0) s_slots = 0;
+  const uint64_t key = live ? keys[i] : 0ull;
+  s_code[t] = (uint32_t)(key >> 32);
+  if (t == 0) s_code[kClimbBlock] = first + kClimbBlock < n ? (uint32_t)(keys[first + kClimbBlock] >> 32) : 0u;
+  uint64_t seg_first = 0, seg_end = n;
+  if constexpr (kSeg) {
+    if (live) {
+      const uint32_t s = segment_at(off, chunk, i);
+      seg_first = off[s];
+      seg_end = off[s + 1];
+    }
+  }
+  // 1 + the common prefix of (code, position in the hierarchy)
+  auto prefix = [&](uint32_t ca, uint32_t cb, uint64_t a) {
+    const uint32_t x = ca ^ cb;
+    const uint32_t j = (uint32_t)(a - seg_first);
+    return (uint8_t)(1u + (x ? (uint32_t)__builtin_clz(x) : 32u + (uint32_t)__builtin_clz(j ^ (j + 1u))));
+  };
+  v3 lo = mk(0, 0, 0), hi = mk(0, 0, 0);
+  if (live) {
+    const uint32_t prim = (uint32_t)key;
+    const uint64_t src = gprim ? (uint64_t)gprim[i] : (uint64_t)prim;
+    if constexpr (kBoxes) {
+      leaf_box<true>(vertices, src, lo, hi);
+    } else {
+      v3 a, b, c;
+      load_tri_vertices(vertices, src, a, b, c);
+      const v3 e1 = sub(b, a), e2 = sub(c, a);
+      float4* out = reinterpret_cast<float4*>(tris + i);
+      out[0] = make_float4(a.x, a.y, a.z, __builtin_bit_cast(float, prim));
+      out[1] = make_float4(e1.x, e1.y, e1.z, 0.0f);
+      out[2] = make_float4(e2.x, e2.y, e2.z, 0.0f);
+      // bvh/gpu/triangle_bvh.mojo:711-712: leaf box = vmin(vmin(v0,v1),v2).
+      lo = vmin(vmin(a, b), c);
+      hi = vmax(vmax(a, b), c);
+    }
+  }
+  __syncthreads();
+  if (live) {
+    s_prefix[t + 1] = i + 1 < seg_end ? prefix(s_code[t], s_code[t + 1], i) : (uint8_t)0;
+    if (t == 0) s_prefix[0] = i > seg_first ? prefix((uint32_t)(keys[i - 1] >> 32), s_code[0], i - 1) : (uint8_t)0;
+  }
+  __syncthreads();
+
+  // phase 1: meetings inside the block
+  Climber c{(uint32_t)i, (uint32_t)i, live ? s_prefix[t] : 0u, live ? s_prefix[t + 1] : 0u, lo, hi};
+  const uint32_t base = (uint32_t)first;
+  bool done = !live, outside = false;
+  uint32_t at = 0;  // the split waited at
+  if (live && c.root()) {
+    leaf_parent[i] = kSentinel;  // single-leaf hierarchy, lbvh.mojo:246-248
+    done = true;
+  }
+  for (bool up = !done; up;) {
+    const bool left = c.is_left();
+    // the block-local split; m - 1 and -1 lie on the block's ends
+    const uint32_t split = (left ? c.r : c.l - 1u) - base;
+    if (split >= m - 1u) {
+      outside = true;
+      break;
+    }
+    s_hand[t] = c.hand();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // LDS writes done (lgkmcnt 0)
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    const uint32_t other = atomicExch(&s_meet[split], t + 1u);
+    if (other == 0) {
+      at = split;
+      break;
+    }
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    const HandOff o = s_hand[other - 1u];
+    c.join(o, nodes, leaf_parent, leaf_counts);
+    if (c.root()) {
+      done = true;
+      up = false;
+    }
+  }
+  __syncthreads();
+
+  // phase 2: siblings past the block
+  if (done || (!outside && s_meet[at] != t + 1u)) return;
+  const uint32_t k = atomicAdd(&s_slots, 1u);
+  if (k >= kHandSlots) {
+    atomicMax(status, (uint32_t)BAJO_STATUS_REFIT_CORRUPT);
+    return;
+  }
+  const uint32_t slot = blockIdx.x * kHandSlots + k;
+  while (!c.root()) {
+    const HandOff h = c.hand();
+    uint64_t* mine = reinterpret_cast<uint64_t*>(hands + slot);
+    const uint64_t w[4] = {pack2(h.box[0], h.box[1]), pack2(h.box[2], h.box[3]), pack2(h.box[4], h.box[5]),
+                           (uint64_t)h.end | ((uint64_t)h.prefix << 32)};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) __hip_atomic_store(mine + q, w[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    const uint32_t other = __hip_atomic_exchange(meet + (c.is_left() ? c.r : c.l - 1u), slot + 1u, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
+    if (other == 0) return;
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    const uint64_t* theirs = reinterpret_cast<const uint64_t*>(hands + (other - 1u));
+    uint64_t v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = __hip_atomic_load(theirs + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    HandOff o;
+    unpack2(v[0], o.box[0], o.box[1]);
+    unpack2(v[1], o.box[2], o.box[3]);
+    unpack2(v[2], o.box[4], o.box[5]);
+    o.end = (uint32_t)v[3];
+    o.prefix = (uint32_t)(v[3] >> 32);
+    c.join(o, nodes, leaf_parent, leaf_counts);
+  }
 }
 
 __global__ void __launch_bounds__(kBlock) seg_init_kernel(uint32_t* __restrict__ acc, uint32_t S) {
@@ -505,7 +556,7 @@ __global__ void __launch_bounds__(kBlock) seg_bounds_kernel(const float* __restr
       if (active) {
         seg = segment_at(off, chunk, i);
         v3 lo, hi;
-        leaf_src<kBoxes>(src, i, lo, hi);
+        leaf_box<kBoxes>(src, i, lo, hi);
         const v3 ce = scale(add(lo, hi), 0.5f);
         r[0] = f2ord(lo.x); r[1] = f2ord(lo.y); r[2] = f2ord(lo.z);
         r[3] = f2ord(hi.x); r[4] = f2ord(hi.y); r[5] = f2ord(hi.z);
@@ -568,7 +619,7 @@ __global__ void __launch_bounds__(kBlock) seg_morton_kernel(const float* __restr
     const v3 cmax = mk(ord2f(a[9]), ord2f(a[10]), ord2f(a[11]));
     const v3 inv = safe_inv(sub(cmax, cmin));
     v3 lo, hi;
-    leaf_src<kBoxes>(src, i, lo, hi);
+    leaf_box<kBoxes>(src, i, lo, hi);
     const v3 q = mul(sub(scale(add(lo, hi), 0.5f), cmin), inv);
     keys[i] = ((uint64_t)seg << 30) | (uint64_t)morton3(q.x, q.y, q.z);
     values[i] = (uint32_t)i;
@@ -580,9 +631,11 @@ __global__ void __launch_bounds__(kBlock) seg_morton_kernel(const float* __restr
 __global__ void __launch_bounds__(kBlock) seg_keys_kernel(uint64_t* __restrict__ keys,
                                                           const uint32_t* __restrict__ gprim, uint64_t n,
                                                           const uint64_t* __restrict__ off,
-                                                          uint32_t* __restrict__ leaf_parent) {
+                                                          uint32_t* __restrict__ leaf_parent,
+                                                          uint32_t* __restrict__ meet) {
   const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
+  meet[k] = 0;
   const uint64_t key = keys[k];
   const uint32_t seg = (uint32_t)(key >> 30);
   const uint64_t first = off[seg];
@@ -640,9 +693,9 @@ int32_t ensure_capacity(bajo_bvh* h, uint64_t n) {
   SortPlan plan = make_sort_plan(n, 8, 0, kSortBeginBit, kSortEndBit);
   if (n <= h->capacity && plan.total <= h->sort_ws_bytes) return BAJO_OK;
   (void)hipFree(h->nodes); (void)hipFree(h->tris); (void)hipFree(h->keys); (void)hipFree(h->leaf_parent); (void)hipFree(h->leaf_counts);
-  (void)hipFree(h->flags); (void)hipFree(h->acc); (void)hipFree(h->scene); (void)hipFree(h->sort_ws);
+  (void)hipFree(h->flags); (void)hipFree(h->hands); (void)hipFree(h->acc); (void)hipFree(h->scene); (void)hipFree(h->sort_ws);
   h->nodes = nullptr; h->tris = nullptr; h->keys = nullptr; h->leaf_parent = nullptr; h->leaf_counts = nullptr;
-  h->flags = nullptr; h->acc = nullptr; h->scene = nullptr; h->sort_ws = nullptr;
+  h->flags = nullptr; h->hands = nullptr; h->acc = nullptr; h->scene = nullptr; h->sort_ws = nullptr;
   h->capacity = 0;
   h->sort_ws_bytes = 0;
   uint64_t internal = n > 1 ? n - 1 : 1;
@@ -651,7 +704,8 @@ int32_t ensure_capacity(bajo_bvh* h, uint64_t n) {
   BJ_HIP(hipMalloc(&h->keys, n * sizeof(uint64_t)));
   BJ_HIP(hipMalloc(&h->leaf_parent, n * sizeof(uint32_t)));
   BJ_HIP(hipMalloc(&h->leaf_counts, internal * sizeof(uint32_t)));
-  BJ_HIP(hipMalloc(&h->flags, internal * sizeof(uint32_t)));
+  BJ_HIP(hipMalloc(&h->flags, n * sizeof(uint32_t)));
+  BJ_HIP(hipMalloc(&h->hands, (uint64_t)div_up(n, kClimbBlock) * kHandSlots * sizeof(HandOff)));
   BJ_HIP(hipMalloc(&h->acc, 16 * sizeof(uint32_t)));
   BJ_HIP(hipMalloc(&h->scene, 16 * sizeof(float)));
   BJ_HIP(hipMalloc(&h->sort_ws, plan.total));
@@ -771,7 +825,7 @@ void free_bvh(bajo_bvh* h) {
   free_segments(h);
   free_hploc(h);
   (void)hipFree(h->nodes); (void)hipFree(h->tris); (void)hipFree(h->keys); (void)hipFree(h->leaf_parent); (void)hipFree(h->leaf_counts);
-  (void)hipFree(h->flags); (void)hipFree(h->acc); (void)hipFree(h->scene); (void)hipFree(h->sort_ws);
+  (void)hipFree(h->flags); (void)hipFree(h->hands); (void)hipFree(h->acc); (void)hipFree(h->scene); (void)hipFree(h->sort_ws);
   free_wide(h);
   delete h;
 }
@@ -836,10 +890,10 @@ int32_t build_into(bajo_ctx* ctx, bajo_bvh* h, const float* vertices, uint64_t n
   ev.record(1, st);
   if (h->boxes)
     morton_kernel<true><<<stream_blocks, kBlock, 0, st>>>(vertices, n, h->acc, h->scene, h->keys, hist, lookback,
-                                                          lookback_words);
+                                                          lookback_words, h->flags);
   else
     morton_kernel<false><<<stream_blocks, kBlock, 0, st>>>(vertices, n, h->acc, h->scene, h->keys, hist, lookback,
-                                                           lookback_words);
+                                                           lookback_words, h->flags);
   BJ_HIP(hipGetLastError());
   ev.record(2, st);
   rc = onesweep_run(ctx, plan, h->keys, nullptr, ws, true);
@@ -851,20 +905,17 @@ int32_t build_into(bajo_ctx* ctx, bajo_bvh* h, const float* vertices, uint64_t n
     rc = build_hploc(ctx, h, vertices);
     if (rc) return rc;
   } else {
-    if (n > 1) {
-      karras_kernel<<<div_up(n - 1, kBlock), kBlock, 0, st>>>(h->keys, n, h->nodes, h->leaf_parent,
-                                                             h->leaf_counts, h->flags, nullptr);
-      BJ_HIP(hipGetLastError());
-    }
     ev.record(4, st);
+    const unsigned blocks = div_up(n, kClimbBlock);
+    HandOff* hands = static_cast<HandOff*>(h->hands);
     if (h->boxes)
-      refit_kernel<true><<<div_up(n, kBlock), kBlock, 0, st>>>(vertices, h->keys, nullptr, n, n - 1, h->nodes,
-                                                               h->leaf_parent, h->leaf_counts, h->flags, h->tris,
-                                                               ctx->status);
+      lbvh_climb_kernel<true, false><<<blocks, kClimbBlock, 0, st>>>(vertices, h->keys, nullptr, n, nullptr, nullptr,
+                                                                     h->nodes, h->leaf_parent, h->leaf_counts,
+                                                                     h->flags, hands, h->tris, ctx->status);
     else
-      refit_kernel<false><<<div_up(n, kBlock), kBlock, 0, st>>>(vertices, h->keys, nullptr, n, n - 1, h->nodes,
-                                                                h->leaf_parent, h->leaf_counts, h->flags, h->tris,
-                                                                ctx->status);
+      lbvh_climb_kernel<false, false><<<blocks, kClimbBlock, 0, st>>>(vertices, h->keys, nullptr, n, nullptr, nullptr,
+                                                                      h->nodes, h->leaf_parent, h->leaf_counts,
+                                                                      h->flags, hands, h->tris, ctx->status);
     BJ_HIP(hipGetLastError());
   }
   ev.record(5, st);
@@ -997,16 +1048,16 @@ int32_t build_segmented(bajo_ctx* ctx, bajo_bvh* h, const float* vertices, const
   ev.record(2, st);
   rc = onesweep_run(ctx, plan, h->keys, h->seg_prim, h->seg_sort_ws, false);
   if (rc) return rc;
-  seg_keys_kernel<<<div_up(n, kBlock), kBlock, 0, st>>>(h->keys, h->seg_prim, n, h->seg_off, h->leaf_parent);
+  seg_keys_kernel<<<div_up(n, kBlock), kBlock, 0, st>>>(h->keys, h->seg_prim, n, h->seg_off, h->leaf_parent,
+                                                        h->flags);
   BJ_HIP(hipGetLastError());
   ev.record(3, st);
   const bool hploc = h->method == BAJO_BUILD_HPLOC && n > S;
-  if (n > S) {
-    // the LBVH writes its nodes directly; H-PLOC's guide is the same forest
-    seg_karras_kernel<<<div_up(n - 1, kBlock), kBlock, 0, st>>>(h->keys, n, h->seg_off, h->seg_chunk,
-                                                                hploc ? h->hp_guide : h->nodes, h->leaf_parent,
-                                                                h->leaf_counts, h->flags,
-                                                                hploc ? h->hp_first : nullptr);
+  if (hploc) {
+    // H-PLOC's guide: the same forest
+    seg_karras_kernel<<<div_up(n - 1, kBlock), kBlock, 0, st>>>(h->keys, n, h->seg_off, h->seg_chunk, h->hp_guide,
+                                                                h->leaf_parent, h->leaf_counts, h->flags,
+                                                                h->hp_first);
     BJ_HIP(hipGetLastError());
   }
   ev.record(4, st);
@@ -1016,9 +1067,9 @@ int32_t build_segmented(bajo_ctx* ctx, bajo_bvh* h, const float* vertices, const
     rc = build_hploc_segmented(ctx, h, vertices);
     if (rc) return rc;
   } else {
-    refit_kernel<false><<<div_up(n, kBlock), kBlock, 0, st>>>(vertices, h->keys, h->seg_prim, n, n - 1, h->nodes,
-                                                              h->leaf_parent, h->leaf_counts, h->flags, h->tris,
-                                                              ctx->status);
+    lbvh_climb_kernel<false, true><<<div_up(n, kClimbBlock), kClimbBlock, 0, st>>>(
+        vertices, h->keys, h->seg_prim, n, h->seg_off, h->seg_chunk, h->nodes, h->leaf_parent, h->leaf_counts,
+        h->flags, static_cast<HandOff*>(h->hands), h->tris, ctx->status);
     BJ_HIP(hipGetLastError());
   }
   ev.record(5, st);

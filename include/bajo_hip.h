@@ -35,7 +35,7 @@ extern "C" {
  * TIMEOUT words, bvh/gpu/builder/hploc_layout.mojo:9-11,
  * wide_collapse.mojo:34-38,236-254): */
 #define BAJO_STATUS_SORT_LOOKBACK 4  /* a sort tile gave up waiting for its predecessor (spin cap) */
-#define BAJO_STATUS_REFIT_CORRUPT 5  /* the refit climb met an inconsistent hierarchy or passed the depth bound */
+#define BAJO_STATUS_REFIT_CORRUPT 5  /* the LBVH climb met an inconsistent hierarchy */
 #define BAJO_STATUS_HPLOC_FAILED 6   /* H-PLOC made no progress, met a corrupt cluster list or ended without one root */
 #define BAJO_STATUS_COLLAPSE_FAILED 7 /* the wide collapse ran out of nodes, met a bad root or passed its level bound */
 /* WAVE_STATUS words of the renderer, rt/wavefront_contract.mojo:25-29, offset by 10 */
@@ -92,8 +92,8 @@ typedef struct {
   uint64_t bounds_ns;   /* triangle + scene/centroid bounds           */
   uint64_t morton_ns;   /* Morton keys (and the fused key histogram)  */
   uint64_t sort_ns;     /* onesweep radix sort of the 64-bit keys     */
-  uint64_t topology_ns; /* Karras hierarchy (LBVH; H-PLOC: 0)         */
-  uint64_t refit_ns;    /* LBVH: bottom-up refit + triangle packing;
+  uint64_t topology_ns; /* sets: H-PLOC's guide hierarchies (else 0)   */
+  uint64_t refit_ns;    /* LBVH: topology, boxes and triangle packing;
                            H-PLOC: guide, clustering, leaf reorder      */
   uint64_t collapse_ns; /* binary -> 8-wide collapse (width 8 only)   */
   uint64_t total_ns;
