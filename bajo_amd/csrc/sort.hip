@@ -4,16 +4,25 @@
 // :102-118, digit_binning :121-327) and the reduce-then-scan sort of
 // bajo/sort/gpu/radix_sort.mojo:510-609 with one engine:
 //   1. one histogram pass computes the 256-bin digit histogram of every
-//      pass at once (per-wave LDS histograms, one global atomic per bin);
-//   2. one binning launch per 8-bit digit: a tile of 4096 keys is taken by
-//      atomic ticket (tickets are handed out in dispatch order, so every tile
-//      a block waits on is already resident), ranked stably with wave64
-//      ballot match masks, published to a decoupled look-back table, staged
-//      in LDS as full-width keys (64-bit keys stay 64-bit; bajo's
-//      onesweep.mojo:244,311 staged u32) and written out in digit-contiguous
-//      runs.
+//      pass at once (LDS histograms, one global atomic per bin and block; 4M
+//      64-bit keys 32.4 -> 17.3 us with one block per CU instead of four);
+//   2. one binning launch per 8-bit digit: a tile of 1,024 to 4,096 keys is
+//      taken by ticket, counted and published to a decoupled look-back table,
+//      ranked stably with wave64 ballot match masks, staged in LDS as
+//      full-width keys (64-bit keys stay 64-bit; bajo's onesweep.mojo:244,311
+//      staged u32) and written out in digit-contiguous runs.
 // The global exclusive digit offsets are recomputed by every tile from the
 // 256-bin histogram, so no separate scan launch is needed.
+//
+// What bounds a pass is a tile's serial chain, not its bytes: at 4M 64-bit
+// keys all 1,024 tiles are resident at once.  Hence a tile publishes its
+// counts before it ranks; looks back over the tiles of its group of 16 and
+// then over whole groups, each round's loads in flight together (tile by tile
+// four at a time the chain grew to 22 rounds); and draws its ticket from one
+// of eight counters (same-address atomics serialize).  A pass over 4M pairs
+// (100 MB moved) took 50.9 us and takes 38.5 (2.6 TB/s), over 4M keys 48.2 and
+// 31.7.  Lists of at most 8,192 keys are sorted by one block in LDS, all
+// passes in one launch (8,192 64-bit pairs: 109 -> 54 us).
 #include <mutex>
 
 #include "sort_internal.h"
@@ -57,15 +66,18 @@ __global__ void __launch_bounds__(256) sort_init_kernel(uint32_t* hist, uint32_t
   for (uint32_t i = threadIdx.x; i < ticket_words; i += blockDim.x) tickets[i] = 0;
 }
 
+// One block per CU: a block ends with one atomic per bin, so their number is
+// kept small; four histograms per block keep the waves' LDS atomics apart.
+constexpr int kHistBlock = 1024, kHistCopies = 4;
 template <typename K>
 __global__ void __launch_bounds__(kHistBlock) sort_hist_kernel(const K* __restrict__ keys, uint64_t n,
                                                                uint32_t begin_bit, uint32_t passes,
                                                                uint32_t* __restrict__ hist,
                                                                uint32_t* __restrict__ lookback,
                                                                uint64_t lookback_words) {
-  __shared__ uint32_t s_hist[kHistBlock / 64][8 * 256];
-  const uint32_t wave = threadIdx.x >> 6;
-  for (uint32_t i = threadIdx.x; i < (kHistBlock / 64) * 8 * 256; i += blockDim.x) (&s_hist[0][0])[i] = 0;
+  __shared__ uint32_t s_hist[kHistCopies][8 * 256];
+  uint32_t* mine = s_hist[(threadIdx.x >> 6) % kHistCopies];
+  for (uint32_t i = threadIdx.x; i < kHistCopies * 8 * 256; i += blockDim.x) (&s_hist[0][0])[i] = 0;
   // The look-back table of every pass starts NOT_READY.
   const uint64_t gtid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const uint64_t gstride = (uint64_t)gridDim.x * blockDim.x;
@@ -73,30 +85,142 @@ __global__ void __launch_bounds__(kHistBlock) sort_hist_kernel(const K* __restri
   __syncthreads();
   for (uint64_t i = gtid; i < n; i += gstride) {
     K k = keys[i];
-    for (uint32_t p = 0; p < passes; ++p) atomicAdd(&s_hist[wave][p * 256 + digit_of(k, begin_bit + 8 * p)], 1u);
+    for (uint32_t p = 0; p < passes; ++p) atomicAdd(&mine[p * 256 + digit_of(k, begin_bit + 8 * p)], 1u);
   }
   __syncthreads();
   for (uint32_t i = threadIdx.x; i < passes * 256; i += blockDim.x) {
     uint32_t c = 0;
 #pragma unroll
-    for (int w = 0; w < kHistBlock / 64; ++w) c += s_hist[w][i];
+    for (int w = 0; w < kHistCopies; ++w) c += s_hist[w][i];
     if (c) atomicAdd(&hist[i], c);
   }
 }
 
-template <typename K, bool kValues>
-__global__ void __launch_bounds__(kSortBlock) sort_bin_kernel(const K* __restrict__ in_keys, K* __restrict__ out_keys,
+// Stable rank of every key of a wave within its digit (kpt keys per lane, in
+// order of k, then lane): on return s_hist holds the wave's digit counts.
+// `valid` is a prefix of the wave's keys.
+template <typename K, int kKpt>
+BJ_D void rank_keys(const K (&key)[kKpt], uint32_t shift, uint32_t valid, uint32_t lane, uint32_t* __restrict__ s_hist,
+                    uint32_t (&rank)[kKpt]) {
+#pragma unroll
+  for (int k = 0; k < kKpt; ++k) {
+    const bool on = (uint32_t)k * 64u + lane < valid;
+    const uint32_t d = digit_of(key[k], shift);
+    uint64_t match = ballot(on);
+    uint32_t lo = (uint32_t)match, hi = (uint32_t)(match >> 32);
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+      // lanes whose bit b equals this lane's
+      const uint64_t m = ballot((d >> b) & 1u);
+      const uint32_t off = ((d >> b) & 1u) - 1u;  // 0 if set, else all ones
+      lo &= (uint32_t)m ^ off;
+      hi &= (uint32_t)(m >> 32) ^ off;
+    }
+    const uint32_t below = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+    const uint32_t total = (uint32_t)(__builtin_popcount(lo) + __builtin_popcount(hi));
+    const uint32_t base = on ? s_hist[d] : 0u;
+    rank[k] = base + below;
+    __builtin_amdgcn_wave_barrier();
+    if (on && below + 1u == total) s_hist[d] = base + total;
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// Sums of the look-back words at p[-256 j], j = 1..count (count <= kMost), once
+// all are published; their loads are in flight together.  Every predecessor
+// holds an earlier ticket and is resident, so it publishes; the cap only
+// bounds the wait if the table was corrupted (false then).
+template <uint32_t kMost>
+BJ_D bool sum_published(const uint32_t* p, uint32_t count, uint32_t spin_limit, uint32_t& sum) {
+  for (uint32_t spins = 0;; ++spins) {
+    uint32_t v[kMost];
+#pragma unroll
+    for (uint32_t j = 0; j < kMost; ++j)
+      v[j] = j < count ? __hip_atomic_load(p - 256 * (int64_t)(j + 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                       : kLookbackAgg;
+    uint32_t total = 0;
+    bool ready = true;
+#pragma unroll
+    for (uint32_t j = 0; j < kMost; ++j) {
+      total += v[j] & kLookbackMask;
+      ready = ready && (v[j] & ~kLookbackMask) != 0;
+    }
+    if (ready) {
+      sum += total;
+      return true;
+    }
+    if (spins >= spin_limit) return false;
+    __builtin_amdgcn_s_sleep(1);
+  }
+}
+
+// The number of keys with this thread's digit in all tiles before `tile`, from
+// the counts published per tile and per group of kSortGroup tiles.
+BJ_D uint32_t look_back(uint32_t* __restrict__ lookback, uint32_t tiles, uint32_t tile, uint32_t count, uint32_t t,
+                        uint32_t spin_limit, uint32_t* __restrict__ status) {
+  uint32_t* mine = lookback + (uint64_t)tile * 256 + t;
+  const uint32_t g = tile / kSortGroup, q = tile % kSortGroup;
+  const bool last = q == kSortGroup - 1;  // publishes its group's counts
+  uint32_t* group = lookback + ((uint64_t)tiles + g) * 256 + t;
+  uint32_t before = 0;
+  bool ok = q == 0 || sum_published<kSortGroup - 1>(mine, q, spin_limit, before);
+  if (last)
+    __hip_atomic_store(group, (g == 0 ? kLookbackInc : kLookbackAgg) | ((before + count) & kLookbackMask),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  // whole groups, eight loads in flight: aggregates are added up to an
+  // inclusive prefix, or to the first group not yet published, polled again
+  constexpr int kAhead = 8;
+  int64_t j = (int64_t)g - 1;
+  uint32_t spins = 0;
+  while (ok && j >= 0) {
+    uint32_t v[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k)
+      v[k] = j - k >= 0 ? __hip_atomic_load(lookback + ((uint64_t)tiles + (uint64_t)(j - k)) * 256 + t,
+                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                        : 0u;
+    int k = 0;
+    bool waiting = false, done = false;
+#pragma unroll
+    for (int q2 = 0; q2 < kAhead; ++q2) {
+      if (waiting || done || j - q2 < 0) continue;
+      const uint32_t flag = v[q2] & ~kLookbackMask;
+      if (flag == 0) {
+        waiting = true;
+      } else {
+        before += v[q2] & kLookbackMask;
+        done = flag == kLookbackInc;
+        ++k;
+      }
+    }
+    if (done) break;
+    j -= k;
+    if (waiting) {
+      if (++spins > spin_limit) ok = false;
+      else __builtin_amdgcn_s_sleep(1);
+    }
+  }
+  if (last && g > 0)
+    __hip_atomic_store(group, kLookbackInc | ((before + count) & kLookbackMask), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  if (!ok) atomicMax(status, (uint32_t)BAJO_STATUS_SORT_LOOKBACK);
+  return before;
+}
+
+template <typename K, bool kValues, int kKpt>
+__global__ void __launch_bounds__(kSortBlock) __attribute__((amdgpu_waves_per_eu(4))) sort_bin_kernel(const K* __restrict__ in_keys, K* __restrict__ out_keys,
                                                               const uint32_t* __restrict__ in_vals,
                                                               uint32_t* __restrict__ out_vals, uint64_t n,
                                                               uint32_t shift, const uint32_t* __restrict__ pass_hist,
                                                               uint32_t* __restrict__ lookback,
-                                                              uint32_t* __restrict__ ticket,
+                                                              uint32_t* __restrict__ tickets,
                                                               uint32_t* __restrict__ status, uint32_t spin_limit) {
-  __shared__ K s_keys[kSortTile];
-  __shared__ uint32_t s_vals[kValues ? kSortTile : 1];
+  constexpr uint32_t kTile = kSortBlock * kKpt;
+  // keys are staged first, then the values in the same words: four blocks of
+  // 4,096 pairs fit a CU instead of two
+  __shared__ K s_keys[kTile];
   __shared__ uint32_t s_wave_hist[kSortWaves][256];
-  __shared__ uint32_t s_digit_start[256];
-  __shared__ uint32_t s_adjust[256];
+  __shared__ uint32_t s_adjust[256];  // the tile's digit counts, then the offset from tile to global position
   __shared__ uint32_t s_tmp[kSortWaves];
   __shared__ uint32_t s_tile;
 
@@ -104,161 +228,211 @@ __global__ void __launch_bounds__(kSortBlock) sort_bin_kernel(const K* __restric
   const uint32_t lane = lane_id();
   const uint32_t wave = t >> 6;
 
-  if (t == 0) s_tile = atomicAdd(ticket, 1u);
-  for (uint32_t i = t; i < kSortWaves * 256; i += kSortBlock) (&s_wave_hist[0][0])[i] = 0;
+  // Blocks are dealt to the eight XCDs round robin and started in order within
+  // each, so the tiles drawn per class keep every predecessor of a started
+  // tile started or next in line on its own XCD.
+  if (t == 0) {
+    const uint32_t c = blockIdx.x % kTicketClasses;
+    s_tile = kTicketClasses * atomicAdd(tickets + c * kTicketStride, 1u) + c;
+  }
+#pragma unroll
+  for (int w = 0; w < kSortWaves; ++w) s_wave_hist[w][t] = 0;
+  s_adjust[t] = 0;
   __syncthreads();
   const uint32_t tile = s_tile;
-  const uint64_t tile_base = (uint64_t)tile * kSortTile;
+  const uint64_t tile_base = (uint64_t)tile * kTile;
+  const uint32_t tile_count = n - tile_base < kTile ? (uint32_t)(n - tile_base) : kTile;
 
   // ---- load (wave-striped: each load instruction covers 64 consecutive keys)
-  K key[kSortKpt];
-  uint32_t val[kValues ? kSortKpt : 1];
-  uint32_t rank[kSortKpt];
-  const uint64_t wave_base = tile_base + (uint64_t)wave * 64 * kSortKpt;
+  K key[kKpt];
+  const uint32_t wave_base = wave * 64 * kKpt;
+  const uint32_t valid = tile_count > wave_base ? (tile_count - wave_base < 64u * kKpt ? tile_count - wave_base : 64u * kKpt) : 0u;
 #pragma unroll
-  for (int k = 0; k < kSortKpt; ++k) {
-    uint64_t idx = wave_base + (uint64_t)k * 64 + lane;
-    bool valid = idx < n;
-    key[k] = valid ? in_keys[idx] : (K)0;
-    if constexpr (kValues) val[k] = valid ? in_vals[idx] : 0u;
+  for (int k = 0; k < kKpt; ++k) {
+    const uint32_t o = (uint32_t)k * 64 + lane;
+    key[k] = o < valid ? in_keys[tile_base + wave_base + o] : (K)0;
   }
 
-  // ---- stable wave-level ranking with ballot match masks
+  // ---- the tile's digit counts, published before the ranking
 #pragma unroll
-  for (int k = 0; k < kSortKpt; ++k) {
-    uint64_t idx = wave_base + (uint64_t)k * 64 + lane;
-    bool valid = idx < n;
-    uint32_t d = digit_of(key[k], shift);
-    uint64_t match = ballot(valid);
-#pragma unroll
-    for (int b = 0; b < 8; ++b) {
-      bool bit = (d >> b) & 1u;
-      uint64_t m = ballot(bit);
-      match &= bit ? m : ~m;
-    }
-    uint32_t below = mask_rank(match);
-    uint32_t base = valid ? s_wave_hist[wave][d] : 0u;
-    rank[k] = base + below;
-    bool last = valid && ((match >> lane) == 1ull);
-    __builtin_amdgcn_wave_barrier();
-    if (last) s_wave_hist[wave][d] = base + (uint32_t)__builtin_popcountll(match);
-    __builtin_amdgcn_wave_barrier();
-  }
+  for (int k = 0; k < kKpt; ++k)
+    if ((uint32_t)k * 64 + lane < valid) atomicAdd(&s_adjust[digit_of(key[k], shift)], 1u);
   __syncthreads();
+  const uint32_t count = s_adjust[t];
+  __hip_atomic_store(lookback + (uint64_t)tile * 256 + t, kLookbackAgg | count, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
 
-  // ---- per-digit block counts and per-wave exclusive offsets (thread t = digit t)
-  uint32_t run = 0;
+  // ---- stable wave-level ranking
+  uint32_t rank[kKpt];
+  rank_keys<K, kKpt>(key, shift, valid, lane, s_wave_hist[wave], rank);
+  const uint32_t digit_start = block_exclusive_scan_256(count, s_tmp, nullptr);
+  const uint32_t global_excl = block_exclusive_scan_256(pass_hist[t], s_tmp, nullptr);
+  // (the scans' barriers close the ranking) per-wave positions of digit t
+  uint32_t run = digit_start;
 #pragma unroll
   for (int w = 0; w < kSortWaves; ++w) {
-    uint32_t c = s_wave_hist[w][t];
+    const uint32_t c = s_wave_hist[w][t];
     s_wave_hist[w][t] = run;
     run += c;
   }
-  const uint32_t count = run;
-
-  // ---- decoupled look-back: publish this tile's count, then sum predecessors
-  uint32_t* my_entry = lookback + (uint64_t)tile * 256 + t;
-  uint32_t exclusive = 0;
-  if (tile == 0) {
-    __hip_atomic_store(my_entry, kLookbackInc | count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  } else {
-    __hip_atomic_store(my_entry, kLookbackAgg | count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // Predecessors' entries are read kLookAhead at a time (their loads in
-    // flight together) and consumed in order: aggregates are added until an
-    // inclusive prefix, or the first entry not yet published, which is polled
-    // again.
-    constexpr int kLookAhead = 4;
-    int64_t j = (int64_t)tile - 1;
-    uint32_t spins = 0;
-    bool done = false;
-    while (!done && j >= 0) {
-      uint32_t v[kLookAhead];
+  // the values' loads overlap the look-back's
+  uint32_t val[kValues ? kKpt : 1];
+  if constexpr (kValues) {
 #pragma unroll
-      for (int k = 0; k < kLookAhead; ++k)
-        v[k] = j - k >= 0 ? __hip_atomic_load(lookback + (uint64_t)(j - k) * 256 + t, __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT)
-                          : 0u;
-      int k = 0;
-      bool waiting = false;
-      for (; k < kLookAhead && j - k >= 0; ++k) {
-        const uint32_t flag = v[k] & ~kLookbackMask;
-        if (flag == 0) {
-          waiting = true;
-          break;
-        }
-        exclusive += v[k] & kLookbackMask;
-        if (flag == kLookbackInc) {
-          done = true;
-          break;
-        }
-      }
-      if (done) break;
-      j -= k;
-      if (waiting) {
-        // Every predecessor holds an earlier ticket and is resident, so it
-        // publishes; the cap only bounds the wait if the table was corrupted,
-        // and giving up is reported through the status word.
-        if (++spins > spin_limit) {
-          atomicMax(status, (uint32_t)BAJO_STATUS_SORT_LOOKBACK);
-          break;
-        }
-        __builtin_amdgcn_s_sleep(1);
-      }
+    for (int k = 0; k < kKpt; ++k) {
+      const uint32_t o = (uint32_t)k * 64 + lane;
+      val[k] = o < valid ? in_vals[tile_base + wave_base + o] : 0u;
     }
-    __hip_atomic_store(my_entry, kLookbackInc | (exclusive + count), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-
-  // ---- block-local digit starts and global destinations
-  uint32_t digit_start = block_exclusive_scan_256(count, s_tmp, nullptr);
-  uint32_t global_excl = block_exclusive_scan_256(pass_hist[t], s_tmp, nullptr);
-  s_digit_start[t] = digit_start;
+  const uint32_t exclusive = look_back(lookback, gridDim.x, tile, count, t, spin_limit, status);
   s_adjust[t] = global_excl + exclusive - digit_start;
   __syncthreads();
 
-  // ---- scatter into LDS in sorted order
+  // ---- keys into LDS in sorted order, then out in digit-contiguous runs
 #pragma unroll
-  for (int k = 0; k < kSortKpt; ++k) {
-    uint64_t idx = wave_base + (uint64_t)k * 64 + lane;
-    if (idx < n) {
-      uint32_t d = digit_of(key[k], shift);
-      uint32_t pos = s_digit_start[d] + s_wave_hist[wave][d] + rank[k];
-      s_keys[pos] = key[k];
-      if constexpr (kValues) s_vals[pos] = val[k];
+  for (int k = 0; k < kKpt; ++k) {
+    if ((uint32_t)k * 64 + lane < valid) {
+      rank[k] += s_wave_hist[wave][digit_of(key[k], shift)];
+      s_keys[rank[k]] = key[k];
     }
   }
   __syncthreads();
-
-  // ---- write digit-contiguous runs
-  const uint64_t rem = n - tile_base;
-  const uint32_t tile_count = rem < (uint64_t)kSortTile ? (uint32_t)rem : (uint32_t)kSortTile;
-  for (uint32_t i = t; i < tile_count; i += kSortBlock) {
-    K k = s_keys[i];
-    uint32_t pos = s_adjust[digit_of(k, shift)] + i;
-    if (pos < n) {
-      out_keys[pos] = k;
-      if constexpr (kValues) out_vals[pos] = s_vals[i];
+  uint32_t pos[kKpt];
+#pragma unroll
+  for (int k = 0; k < kKpt; ++k) {
+    const uint32_t i = (uint32_t)k * kSortBlock + t;
+    pos[k] = 0xFFFFFFFFu;
+    if (i < tile_count) {
+      const K x = s_keys[i];
+      pos[k] = s_adjust[digit_of(x, shift)] + i;
+      if (pos[k] < n) out_keys[pos[k]] = x;
     }
+  }
+  if constexpr (kValues) {
+    uint32_t* s_vals = reinterpret_cast<uint32_t*>(s_keys);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kKpt; ++k)
+      if ((uint32_t)k * 64 + lane < valid) s_vals[rank[k]] = val[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kKpt; ++k) {
+      const uint32_t i = (uint32_t)k * kSortBlock + t;
+      if (i < tile_count && pos[k] < n) out_vals[pos[k]] = s_vals[i];
+    }
+  }
+}
+
+// Every pass over a short list in one block: the keys (and values) live in
+// registers and LDS from the first pass to the last.
+constexpr int kSmallBlock = 1024, kSmallKpt = (int)(kSortSmall / kSmallBlock), kSmallWaves = kSmallBlock / 64;
+template <typename K, bool kValues>
+__global__ void __launch_bounds__(kSmallBlock) sort_small_kernel(K* __restrict__ keys, uint32_t* __restrict__ vals,
+                                                                 uint32_t n, uint32_t begin_bit, uint32_t passes) {
+  __shared__ K s_keys[kSortSmall];
+  __shared__ uint32_t s_vals[kValues ? kSortSmall : 1];
+  __shared__ uint32_t s_hist[kSmallWaves][256];
+  __shared__ uint32_t s_tmp[4];
+  const uint32_t t = threadIdx.x, lane = lane_id(), wave = t >> 6;
+  // a wave takes `span` consecutive keys, 64 at a time
+  const uint32_t span = (n + kSmallBlock - 1) / kSmallBlock * 64;
+  const uint32_t base = wave * span;
+  const uint32_t valid = n > base ? (n - base < span ? n - base : span) : 0u;
+  for (uint32_t i = t; i < n; i += kSmallBlock) {
+    s_keys[i] = keys[i];
+    if constexpr (kValues) s_vals[i] = vals[i];
+  }
+  for (uint32_t p = 0; p < passes; ++p) {
+    const uint32_t shift = begin_bit + 8 * p;
+    for (uint32_t i = t; i < kSmallWaves * 256; i += kSmallBlock) (&s_hist[0][0])[i] = 0;
+    __syncthreads();
+    K key[kSmallKpt];
+    uint32_t val[kValues ? kSmallKpt : 1], rank[kSmallKpt];
+#pragma unroll
+    for (int k = 0; k < kSmallKpt; ++k) {
+      const uint32_t o = (uint32_t)k * 64 + lane;
+      key[k] = o < valid ? s_keys[base + o] : (K)0;
+      if constexpr (kValues) val[k] = o < valid ? s_vals[base + o] : 0u;
+    }
+#pragma unroll
+    for (int k = 0; k < kSmallKpt; ++k) {
+      if ((uint32_t)k * 64 < valid) {
+        const K one[1] = {key[k]};
+        uint32_t r[1];
+        rank_keys<K, 1>(one, shift, valid - (uint32_t)k * 64, lane, s_hist[wave], r);
+        rank[k] = r[0];
+      }
+    }
+    __syncthreads();
+    // digit t's first position, then each wave's
+    uint32_t total = 0;
+    if (t < 256)
+      for (int w = 0; w < kSmallWaves; ++w) total += s_hist[w][t];
+    uint32_t x = total;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t y = __shfl_up(x, off, 64);
+      if (lane >= (uint32_t)off) x += y;
+    }
+    if (t < 256 && lane == 63) s_tmp[wave] = x;
+    __syncthreads();
+    if (t < 256) {
+      uint32_t run = x - total;
+      for (uint32_t w = 0; w < wave; ++w) run += s_tmp[w];
+      for (int w = 0; w < kSmallWaves; ++w) {
+        const uint32_t c = s_hist[w][t];
+        s_hist[w][t] = run;
+        run += c;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kSmallKpt; ++k) {
+      if ((uint32_t)k * 64 + lane < valid) {
+        const uint32_t at = s_hist[wave][digit_of(key[k], shift)] + rank[k];
+        s_keys[at] = key[k];
+        if constexpr (kValues) s_vals[at] = val[k];
+      }
+    }
+    __syncthreads();
+  }
+  for (uint32_t i = t; i < n; i += kSmallBlock) {
+    keys[i] = s_keys[i];
+    if constexpr (kValues) vals[i] = s_vals[i];
   }
 }
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-template <typename K>
+template <typename K, bool kValues, int kKpt>
+void launch_bin(bajo_ctx* ctx, const SortPlan& p, const K* src, K* dst, const uint32_t* vsrc, uint32_t* vdst,
+                uint32_t shift, const uint32_t* hist, uint32_t* lookback, uint32_t* tickets, uint32_t spin_limit) {
+  sort_bin_kernel<K, kValues, kKpt><<<p.tiles, kSortBlock, 0, ctx->stream>>>(
+      src, dst, vsrc, vdst, p.n, shift, hist, lookback, tickets, ctx->status, spin_limit);
+}
+
+template <typename K, bool kValues>
 int32_t run_typed(bajo_ctx* ctx, const SortPlan& p, K* keys, uint32_t* values, char* ws, bool hist_ready) {
+  if (p.n <= kSortSmall) {
+    sort_small_kernel<K, kValues><<<1, kSmallBlock, 0, ctx->stream>>>(keys, values, (uint32_t)p.n,
+                                                                      (uint32_t)p.begin_bit, (uint32_t)p.passes);
+    BJ_HIP(hipGetLastError());
+    return BAJO_OK;
+  }
   K* alt_keys = (K*)(ws + p.off_alt_keys);
-  uint32_t* alt_vals = p.has_values ? (uint32_t*)(ws + p.off_alt_vals) : nullptr;
+  uint32_t* alt_vals = kValues ? (uint32_t*)(ws + p.off_alt_vals) : nullptr;
   uint32_t* hist = (uint32_t*)(ws + p.off_hist);
   uint32_t* lookback = (uint32_t*)(ws + p.off_lookback);
   uint32_t* tickets = (uint32_t*)(ws + p.off_tickets);
-  const uint64_t lb_pass_words = (uint64_t)p.tiles * 256;
+  const uint64_t lb_pass_words = p.lookback_words / (uint64_t)p.passes;
   if (!hist_ready) {
-    sort_init_kernel<<<1, 256, 0, ctx->stream>>>(hist, (uint32_t)p.passes * 256, tickets, (uint32_t)p.passes);
+    sort_init_kernel<<<1, 256, 0, ctx->stream>>>(hist, (uint32_t)p.passes * 256, tickets,
+                                                 (uint32_t)p.passes * kTicketWords);
     BJ_HIP(hipGetLastError());
-    unsigned blocks = div_up(p.n, (uint64_t)kHistBlock * 16);
-    if (blocks > 2048) blocks = 2048;
-    if (blocks < 1) blocks = 1;
+    unsigned blocks = div_up(p.n, (uint64_t)kHistBlock * 4);
+    if (blocks > 256) blocks = 256;
     sort_hist_kernel<K><<<blocks, kHistBlock, 0, ctx->stream>>>(keys, p.n, (uint32_t)p.begin_bit, (uint32_t)p.passes,
-                                                                hist, lookback, lb_pass_words * p.passes);
+                                                                hist, lookback, p.lookback_words);
     BJ_HIP(hipGetLastError());
   }
   K* src = keys;
@@ -267,22 +441,20 @@ int32_t run_typed(bajo_ctx* ctx, const SortPlan& p, K* keys, uint32_t* values, c
   uint32_t* vdst = alt_vals;
   const uint32_t spin_limit = ctx->spin_limit ? ctx->spin_limit : kLookbackSpinLimit;
   for (int pass = 0; pass < p.passes; ++pass) {
-    uint32_t shift = (uint32_t)(p.begin_bit + 8 * pass);
-    if (p.has_values)
-      sort_bin_kernel<K, true><<<p.tiles, kSortBlock, 0, ctx->stream>>>(
-          src, dst, vsrc, vdst, p.n, shift, hist + pass * 256, lookback + lb_pass_words * pass, tickets + pass,
-          ctx->status, spin_limit);
-    else
-      sort_bin_kernel<K, false><<<p.tiles, kSortBlock, 0, ctx->stream>>>(
-          src, dst, nullptr, nullptr, p.n, shift, hist + pass * 256, lookback + lb_pass_words * pass, tickets + pass,
-          ctx->status, spin_limit);
+    const uint32_t shift = (uint32_t)(p.begin_bit + 8 * pass);
+    const uint32_t* h = hist + pass * 256;
+    uint32_t* lb = lookback + lb_pass_words * pass;
+    uint32_t* tk = tickets + (uint32_t)pass * kTicketWords;
+    if (p.kpt == 4) launch_bin<K, kValues, 4>(ctx, p, src, dst, vsrc, vdst, shift, h, lb, tk, spin_limit);
+    else if (p.kpt == 8) launch_bin<K, kValues, 8>(ctx, p, src, dst, vsrc, vdst, shift, h, lb, tk, spin_limit);
+    else launch_bin<K, kValues, 16>(ctx, p, src, dst, vsrc, vdst, shift, h, lb, tk, spin_limit);
     BJ_HIP(hipGetLastError());
-    K* tk = src; src = dst; dst = tk;
-    uint32_t* tv = vsrc; vsrc = vdst; vdst = tv;
+    K* sk = src; src = dst; dst = sk;
+    uint32_t* sv = vsrc; vsrc = vdst; vdst = sv;
   }
   if (src != keys) {
     BJ_HIP(hipMemcpyAsync(keys, src, p.n * sizeof(K), hipMemcpyDeviceToDevice, ctx->stream));
-    if (p.has_values) BJ_HIP(hipMemcpyAsync(values, vsrc, p.n * sizeof(uint32_t), hipMemcpyDeviceToDevice, ctx->stream));
+    if (kValues) BJ_HIP(hipMemcpyAsync(values, vsrc, p.n * sizeof(uint32_t), hipMemcpyDeviceToDevice, ctx->stream));
   }
   return BAJO_OK;
 }
@@ -297,7 +469,13 @@ SortPlan make_sort_plan(uint64_t n, int key_bytes, int has_values, int begin_bit
   p.begin_bit = begin_bit;
   p.end_bit = end_bit;
   p.passes = (end_bit - begin_bit + 7) / 8;
-  p.tiles = div_up(n ? n : 1, kSortTile);
+  // smaller tiles for shorter lists: a pass lasts as long as a tile's chain, so
+  // the keys are spread over the chip (64-bit pairs: 262,144 keys 105.9 us
+  // with 4 keys per thread, 115.3 with 8; 1M 163 with 8, 186 with 16; 2M 258
+  // and 262; 4M 451 and 402)
+  p.kpt = n <= 262144 ? 4 : (n <= 1310720 ? 8 : 16);
+  p.tiles = div_up(n ? n : 1, (uint64_t)kSortBlock * p.kpt);
+  p.lookback_words = (size_t)(p.passes ? p.passes : 1) * (p.tiles + div_up(p.tiles, kSortGroup)) * 256;
   size_t off = 0;
   p.off_alt_keys = off;
   off = align256(off + n * (size_t)key_bytes);
@@ -306,17 +484,21 @@ SortPlan make_sort_plan(uint64_t n, int key_bytes, int has_values, int begin_bit
   p.off_hist = off;
   off = align256(off + (size_t)(p.passes ? p.passes : 1) * 256 * sizeof(uint32_t));
   p.off_lookback = off;
-  off = align256(off + (size_t)(p.passes ? p.passes : 1) * p.tiles * 256 * sizeof(uint32_t));
+  off = align256(off + p.lookback_words * sizeof(uint32_t));
   p.off_tickets = off;
-  off = align256(off + 8 * sizeof(uint32_t));
+  off = align256(off + (size_t)(p.passes ? p.passes : 1) * kTicketWords * sizeof(uint32_t));
   p.total = off;
   return p;
 }
 
 int32_t onesweep_run(bajo_ctx* ctx, const SortPlan& plan, void* keys, uint32_t* values, void* ws, bool hist_ready) {
   if (plan.n <= 1 || plan.passes == 0) return BAJO_OK;
-  if (plan.key_bytes == 8) return run_typed<uint64_t>(ctx, plan, (uint64_t*)keys, values, (char*)ws, hist_ready);
-  return run_typed<uint32_t>(ctx, plan, (uint32_t*)keys, values, (char*)ws, hist_ready);
+  char* w = (char*)ws;
+  if (plan.key_bytes == 8)
+    return plan.has_values ? run_typed<uint64_t, true>(ctx, plan, (uint64_t*)keys, values, w, hist_ready)
+                           : run_typed<uint64_t, false>(ctx, plan, (uint64_t*)keys, values, w, hist_ready);
+  return plan.has_values ? run_typed<uint32_t, true>(ctx, plan, (uint32_t*)keys, values, w, hist_ready)
+                         : run_typed<uint32_t, false>(ctx, plan, (uint32_t*)keys, values, w, hist_ready);
 }
 
 }  // namespace bj
@@ -352,7 +534,7 @@ int32_t sort_entry(bajo_ctx* ctx, void* keys, uint32_t* values, uint64_t n, int 
 // code uses the address hipGetSymbolAddress returns for the current device,
 // never the array's name.
 constexpr uint64_t kNoAllocMaxKeys = 1ull << 20;
-constexpr size_t kNoAllocScratchBytes = 16ull << 20;
+constexpr size_t kNoAllocScratchBytes = 20ull << 20;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 constexpr int kNoAllocMaxDevices = 64;

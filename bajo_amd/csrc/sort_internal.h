@@ -5,11 +5,14 @@
 
 namespace bj {
 
-constexpr int kSortBlock = 256;                 // 4 waves of 64
+constexpr int kSortBlock = 256;             // 4 waves of 64
 constexpr int kSortWaves = kSortBlock / 64;
-constexpr int kSortKpt = 16;                    // keys per thread
-constexpr int kSortTile = kSortBlock * kSortKpt;  // 4096 keys per tile
-constexpr int kHistBlock = 256;
+constexpr uint32_t kSortGroup = 16;         // tiles per look-back group
+// Tile tickets are drawn from eight counters a cache line apart.
+constexpr uint32_t kTicketClasses = 8, kTicketStride = 32;
+constexpr uint32_t kTicketWords = kTicketClasses * kTicketStride;  // per pass
+// Lists one block sorts by itself, in LDS.
+constexpr uint64_t kSortSmall = 8192;
 constexpr uint32_t kLookbackAgg = 0x40000000u;
 constexpr uint32_t kLookbackInc = 0x80000000u;
 constexpr uint32_t kLookbackMask = 0x3FFFFFFFu;
@@ -22,7 +25,9 @@ struct SortPlan {
   int key_bytes = 8;
   int has_values = 0;
   int begin_bit = 0, end_bit = 64, passes = 0;
+  int kpt = 16;          // keys per thread of a tile
   unsigned tiles = 0;
+  size_t lookback_words = 0;  // all passes: 256 words per tile and per group of tiles
   size_t off_alt_keys = 0, off_alt_vals = 0, off_hist = 0, off_lookback = 0, off_tickets = 0, total = 0;
 };
 
@@ -32,6 +37,7 @@ SortPlan make_sort_plan(uint64_t n, int key_bytes, int has_values, int begin_bit
 // counters are cleared and the digit histogram is computed first; when true
 // the caller has already cleared the tickets, zeroed the look-back table and
 // filled the histogram (the LBVH Morton kernel does this in its own pass).
+// Lists of at most kSortSmall keys need none of them.
 // Sorted output always lands back in `keys` / `values`.
 int32_t onesweep_run(bajo_ctx* ctx, const SortPlan& plan, void* keys, uint32_t* values, void* ws, bool hist_ready);
 

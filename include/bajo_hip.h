@@ -174,7 +174,7 @@ int32_t bajo_onesweep_radix_sort_pairs_u64_u32(bajo_ctx* ctx, uint64_t* keys, ui
 /* No counterpart in bajo.  The same sort as
  * bajo_onesweep_radix_sort_pairs_u64_u32 for callers that cannot allocate
  * device memory (code under HIP graph capture, tight submission loops,
- * harnesses that forbid hipMalloc): its workspace is a fixed 16 MiB device
+ * harnesses that forbid hipMalloc): its workspace is a fixed 20 MiB device
  * array inside the library (one per GPU, held until the process ends), so
  * the call allocates nothing.  n is at most 2^20 pairs (larger n returns
  * BAJO_ERR_INVALID_ARGUMENT).  Every call on one GPU shares that array:

@@ -148,3 +148,25 @@ def test_lookback_give_up_is_reported_never_silent(gpu_ctx):
     np.testing.assert_array_equal(to_host(k, np.uint64), want)
     print(f"forced give-ups reported in {raised} of 3 sorts")
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [8191, 8192, 8193, 262144, 262145, 1310720, 1310721, 4096 * 16 * 9 + 5])
+@pytest.mark.parametrize("bits", [32, 64])
+def test_tile_size_edges(gpu_ctx, n, bits):
+    """The one-block sort, the tile sizes and the look-back groups at their edges (few distinct digits, so that
+    every digit spans tiles), stable against numpy."""
+    from bajo_amd import sort
+
+    announce(f"sort tile edges n={n} bits={bits}")
+    rng = np.random.default_rng(n + bits)
+    dtype = np.uint32 if bits == 32 else np.uint64
+    keys = (rng.integers(0, 7, n, dtype=np.uint64) * np.uint64(0x0101010101010101)).astype(dtype)
+    keys[::3] ^= rng.integers(0, 2**31, keys[::3].size, dtype=np.uint64).astype(dtype)
+    order = np.argsort(keys, kind="stable")
+    k, v = to_dev(keys), to_dev(np.arange(n, dtype=np.uint32))
+    sort.device_radix_sort_pairs(k, v)
+    np.testing.assert_array_equal(to_host(v, np.uint32), order)
+    np.testing.assert_array_equal(to_host(k, dtype), keys[order])
+    k = to_dev(keys)
+    sort.device_radix_sort_keys(k)
+    np.testing.assert_array_equal(to_host(k, dtype), keys[order])
