@@ -8,20 +8,26 @@
 // - Weights live in one device image: BF16 rows padded by 8 elements (so
 //   16 lanes reading one 16-byte column slice of 16 rows hit different LDS
 //   banks), transposed copies of W2..W4 for the backward pass, FP32 biases.
-//   A block copies the image into LDS once (55 KB forward, 83 KB training)
-//   and its waves loop over 16-sample tiles.
+//   A block copies the image into LDS once (55 KB forward, 83 KB training).
 // - MFMA operand layout (16x16x32): A[i][k] at lane i + 16 (k / 8), element
 //   k % 8; B[k][j] at lane j + 16 (k / 8); D[i][j] at lane j + 16 (i / 4),
-//   element i % 4.  A row of weights W[j][k..k+7] is one 16-byte LDS load,
-//   and so is a row of activations, so every operand is a ds_read_b128.
-// - The input encoding is computed straight into A fragments: lane (i, g)
-//   of k-step s needs features 32 s + 8 g .. + 7, i.e. four frequencies of
-//   one input, so layer 1 reads nothing but the sample's 9 inputs.
-// - Training writes activations and deltas transposed (batch-contiguous
-//   rows, BF16) and the weight gradient is a batch-reduction GEMM
-//   dW = D^T X with the batch as the MFMA K dimension: 111 output tiles x
-//   batch chunks of 2048, partial tiles summed in fixed order by the Adam
-//   kernel (deterministic, no atomics).
+//   element i % 4.  Weights are the A operand and samples the B operand's
+//   columns, so a lane's results are units 16 t + 4 g .. + 3 of one sample.
+//   The rows of W2..W4 hold their inputs in the order in which the lanes
+//   then have them (hidden_pos), so a layer's results, rounded to BF16 in
+//   registers, are the next layer's operand: activations never pass
+//   through LDS, and outputs leave as 16-byte stores.
+// - The input encoding is computed straight into the layer-1 operand: lane
+//   (i, g) of k-step s needs features 32 s + 8 g .. + 7, i.e. four
+//   frequencies of one input.
+// - A wave takes 32 samples (two operands) for each weight fragment it reads.
+// - Training is one launch: the operands of a product swapped give its
+//   transpose (lanes hold units, registers samples), which is the operand
+//   form of the weight gradient dW = D^T X with the batch as K.  The eight
+//   waves of a block exchange these fragments through LDS and each
+//   accumulates 12 to 14 of the 111 gradient tiles; one partial per block
+//   of 256 samples goes to memory, summed in fixed order by the Adam kernel
+//   (deterministic, no atomics).
 #include <math.h>
 #include <string.h>
 
@@ -52,11 +58,9 @@ constexpr size_t kPackBytes = (size_t)kPackAll * 2 + kBiasFloats * 4;
 static_assert((kPackAll * 2) % 16 == 0 && (kPackFwd * 2) % 16 == 0, "pack images are 16-byte aligned");
 
 // ---- training layout -----------------------------------------------------------
-constexpr int kX0Rows = kGuideK0;            // 224: features, row 216 = 1
-constexpr int kHRows = kGuideHidden + 16;    // 80: hidden units, row 64 = 1
-constexpr int kDRows = kGuideHidden;         // 64
-constexpr int kDoRows = kGuideOutPad;        // 48 (rows 40..47 zero)
-constexpr int kChunk = 2048;                 // batch samples per weight-gradient partial
+constexpr int kTrainWaves = 8;
+constexpr int kTrainSamples = kTrainWaves * 32;  // samples of one block and pass
+constexpr uint32_t kTrainBlocks = 256;           // at most one per CU; larger batches loop
 // gradient tiles (16 x 16 of dW[out][in], the bias in the column of the constant input)
 constexpr int kT1 = 0, kT2 = 4 * 14, kT3 = kT2 + 4 * 5, kT4 = kT3 + 4 * 5, kTiles = kT4 + 3 * 5;  // 111
 
@@ -70,43 +74,53 @@ BJ_HD float bf2f(uint16_t b) { return __builtin_bit_cast(float, (uint32_t)b << 1
 BJ_D bf16x8 frag16(const uint16_t* p) { return __builtin_bit_cast(bf16x8, *(const uint4*)p); }
 BJ_D f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 
-// Where parameter p lives: its gradient tile / element and its positions in
-// the weight image (forward and, for W2..W4, transposed; -1 = none; biases
-// go to the FP32 bias block).
+// Where input k of a 64-wide layer lives in its weight row: lane group g of
+// k-step s takes elements 32 s + 8 g .. + 7, and as B operand it has units
+// 16 (2 s) + 4 g .. + 3 and 16 (2 s + 1) + 4 g .. + 3 of the layer before.
+BJ_HD int hidden_pos(int k) { return 32 * (k >> 5) + 8 * ((k >> 2) & 3) + 4 * ((k >> 4) & 1) + (k & 3); }
+
+// Where parameter p lives in the weight image (forward and, for W2..W4,
+// transposed; -1 = none; biases go to the FP32 bias block).
 struct ParamSlot {
-  int tile, elem, fwd, tr, bias;
+  int fwd, tr, bias;
 };
 BJ_HD ParamSlot param_slot(int p) {
-  ParamSlot s{0, 0, -1, -1, -1};
-  int j, k, base_t, ntiles, fwd_base, fwd_stride, tr_base, bias_base;
+  ParamSlot s{-1, -1, -1};
   if (p < kGuideOffB1) {
-    j = p / kGuideFeatures; k = p - j * kGuideFeatures;
-    s.tile = kT1 + (j >> 4) * 14 + (k >> 4); s.elem = (j & 15) * 16 + (k & 15);
-    s.fwd = kPackW1 + j * kW1Stride + k;
+    const int j = p / kGuideFeatures;
+    s.fwd = kPackW1 + j * kW1Stride + (p - j * kGuideFeatures);
     return s;
   }
   if (p < kGuideOffW2) {
-    j = p - kGuideOffB1; k = kGuideFeatures;
-    s.tile = kT1 + (j >> 4) * 14 + (k >> 4); s.elem = (j & 15) * 16 + (k & 15);
-    s.bias = j;
+    s.bias = p - kGuideOffB1;
     return s;
   }
-  if (p < kGuideOffW3) { base_t = kT2; ntiles = 5; fwd_base = kPackW2; tr_base = kPackW2t; bias_base = 64; p -= kGuideOffW2; }
-  else if (p < kGuideOffW4) { base_t = kT3; ntiles = 5; fwd_base = kPackW3; tr_base = kPackW3t; bias_base = 128; p -= kGuideOffW3; }
-  else { base_t = kT4; ntiles = 5; fwd_base = kPackW4; tr_base = kPackW4t; bias_base = 192; p -= kGuideOffW4; }
-  fwd_stride = kRowStride;
-  const int rows = base_t == kT4 ? kGuideOut : kGuideHidden;
+  int fwd_base, tr_base, bias_base, rows = kGuideHidden;
+  if (p < kGuideOffW3) { fwd_base = kPackW2; tr_base = kPackW2t; bias_base = 64; p -= kGuideOffW2; }
+  else if (p < kGuideOffW4) { fwd_base = kPackW3; tr_base = kPackW3t; bias_base = 128; p -= kGuideOffW3; }
+  else { fwd_base = kPackW4; tr_base = kPackW4t; bias_base = 192; p -= kGuideOffW4; rows = kGuideOut; }
   if (p < rows * kGuideHidden) {
-    j = p / kGuideHidden; k = p - j * kGuideHidden;
-    s.fwd = fwd_base + j * fwd_stride + k;
-    s.tr = tr_base + k * kRowStride + j;
+    const int j = p / kGuideHidden, k = p - j * kGuideHidden;
+    s.fwd = fwd_base + j * kRowStride + hidden_pos(k);
+    s.tr = tr_base + k * kRowStride + hidden_pos(j);
   } else {
-    j = p - rows * kGuideHidden; k = kGuideHidden;
-    s.bias = bias_base + j;
+    s.bias = bias_base + p - rows * kGuideHidden;
   }
-  s.tile = base_t + (j >> 4) * ntiles + (k >> 4);
-  s.elem = (j & 15) * 16 + (k & 15);
   return s;
+}
+
+// The parameter of element e of gradient tile t (lane e / 4 holds four rows
+// of one column), or -1: the column after the inputs is the bias.
+BJ_HD int slot_param(int t, int e) {
+  int base, tiles, rows = kGuideHidden, inputs = kGuideHidden;
+  if (t < kT2) { base = kGuideOffW1; tiles = 14; inputs = kGuideFeatures; t -= kT1; }
+  else if (t < kT3) { base = kGuideOffW2; tiles = 5; t -= kT2; }
+  else if (t < kT4) { base = kGuideOffW3; tiles = 5; t -= kT3; }
+  else { base = kGuideOffW4; tiles = 5; rows = kGuideOut; t -= kT4; }
+  const int m = t / tiles;
+  const int j = 16 * m + 4 * (e >> 6) + (e & 3), k = 16 * (t - m * tiles) + ((e >> 2) & 15);
+  if (j >= rows || k > inputs) return -1;
+  return k == inputs ? base + rows * inputs + j : base + j * inputs + k;
 }
 
 BJ_D void pack_param(uint8_t* pack, const ParamSlot& s, float v) {
@@ -126,100 +140,105 @@ __global__ void __launch_bounds__(256) guide_pack_kernel(const float* __restrict
   if (p < kGuideParams) pack_param(pack, param_slot(p), params[p]);
 }
 
-// ---- layer-1 A fragments ---------------------------------------------------------
-// Chunk q (0..27) of a sample's features: input d = q / 3, frequencies
-// 4 (q % 3) .. + 3, (sin, cos) pairs; chunk 27 is padding (zeros).
-BJ_D bf16x8 encode_chunk(const float (&x)[kGuideInputs], int q) {
-  float s[4] = {0.0f, 0.0f, 0.0f, 0.0f}, c[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  if (q < 27) {
-    const int d = q / 3, fb = q - 3 * d;
-    float xd = x[0];
+// ---- layer-1 operand -------------------------------------------------------------
+// Chunk q = 4 s + g (0..27) of a sample's features: input d = q / 3,
+// frequencies 4 (q % 3) .. + 3, (sin, cos) pairs; chunk 27 is padding, whose
+// first element is the constant input (its weights are zero, its gradient is
+// the bias's).  The chunks of one k-step lie in two neighbouring inputs.
+BJ_D int chunk_input(int s, uint32_t g) {
+  const int q = 4 * s + (int)g;
+  return q < 27 ? q / 3 : kGuideInputs - 1;
+}
+
+// A lane's scales of its chunks' first frequencies: (q % 3) == (s + g) % 3.
+BJ_D void chunk_scales(uint32_t g, float (&sc)[3]) {
 #pragma unroll
-    for (int a = 1; a < kGuideInputs; ++a) xd = d == a ? x[a] : xd;
-    guide_encode_group(xd, fb, s, c);
-  }
+  for (int t = 0; t < 3; ++t) sc[t] = guide_freq_scale(4 * (int)((t + g) % 3));
+}
+
+BJ_D bf16x8 encode_chunk(float x, float scale, bool constant) {
+  float s[4], c[4];
+  guide_encode_scaled(x, scale, s, c);
   // round to nearest even (the hardware conversion equals f2bf for finite values)
-  return bf16x8{(__bf16)s[0], (__bf16)c[0], (__bf16)s[1], (__bf16)c[1],
-                (__bf16)s[2], (__bf16)c[2], (__bf16)s[3], (__bf16)c[3]};
+  bf16x8 f = {(__bf16)s[0], (__bf16)c[0], (__bf16)s[1], (__bf16)c[1],
+              (__bf16)s[2], (__bf16)c[2], (__bf16)s[3], (__bf16)c[3]};
+  if (constant) f = __builtin_bit_cast(bf16x8, uint4{0x3F80u, 0u, 0u, 0u});
+  return f;
 }
 
-// Bias + ReLU of a 16 x 64 layer result into a row-major BF16 tile.
-BJ_D void store_hidden(const f32x4 (&acc)[4], const float* bias, uint16_t* sh, uint32_t lane) {
-  const uint32_t col = lane & 15u, g = lane >> 4;
+// ---- layers ----------------------------------------------------------------------
+// ReLU (NaN to 0).
+BJ_D float relu(float v) { return __builtin_amdgcn_fmed3f(v, 0.0f, __builtin_inff()); }
+BJ_D f32x4 relu4(f32x4 v) { return f32x4{relu(v[0]), relu(v[1]), relu(v[2]), relu(v[3])}; }
+BJ_D bf16x8 to_frag(f32x4 a, f32x4 b) {
+  return bf16x8{(__bf16)a[0], (__bf16)a[1], (__bf16)a[2], (__bf16)a[3],
+                (__bf16)b[0], (__bf16)b[1], (__bf16)b[2], (__bf16)b[3]};
+}
+
+// acc[u][t] += (rows 16 t .. + 15 of a 64-wide layer) x (sample tile u).
+template <int kT>
+BJ_D void layer64(const uint16_t* sw, const bf16x8 (&in)[2][2], f32x4 (&acc)[2][kT], uint32_t lane) {
+  const uint32_t i = lane & 15u, g = lane >> 4;
 #pragma unroll
-  for (int jt = 0; jt < 4; ++jt)
+  for (int s = 0; s < 2; ++s)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float v = acc[jt][r] + bias[16 * jt + col];
-      sh[(4 * g + r) * kRowStride + 16 * jt + col] = f2bf(v > 0.0f ? v : 0.0f);
+    for (int t = 0; t < kT; ++t) {
+      const bf16x8 w = frag16(sw + (16 * t + i) * kRowStride + 32 * s + 8 * g);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) acc[u][t] = mfma(w, in[u][s], acc[u][t]);
     }
 }
 
-// One 64-wide layer: acc = H (16 x 64, row-major BF16 tile) x W^T rows.
-template <int kTiles>
-BJ_D void layer64(const uint16_t* sh, const uint16_t* sw, f32x4 (&acc)[kTiles], uint32_t lane) {
-  const uint32_t i = lane & 15u, g = lane >> 4;
+// Biases of a lane's units 16 t + 4 g .. + 3.
+template <int kT>
+BJ_D void start_bias(const float* bias, f32x4 (&acc)[2][kT], uint32_t g) {
 #pragma unroll
-  for (int jt = 0; jt < kTiles; ++jt) acc[jt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    const bf16x8 a = frag16(sh + i * kRowStride + 32 * s + 8 * g);
-#pragma unroll
-    for (int jt = 0; jt < kTiles; ++jt) acc[jt] = mfma(a, frag16(sw + (16 * jt + i) * kRowStride + 32 * s + 8 * g), acc[jt]);
-  }
+  for (int t = 0; t < kT; ++t) acc[0][t] = acc[1][t] = *(const f32x4*)(bias + 16 * t + 4 * g);
 }
 
-// Layer 1 from the encoded inputs: lane (i, g) holds sample i's inputs.
-BJ_D void layer1(const float (&x)[kGuideInputs], const uint16_t* sw, f32x4 (&acc)[4], uint32_t lane,
-                 uint16_t* x0t = nullptr, uint64_t ldb = 0, uint64_t col = 0) {
-  const uint32_t i = lane & 15u, g = lane >> 4;
+// Activations as the next layer's operand.
+BJ_D void hidden_frags(const f32x4 (&acc)[2][4], bf16x8 (&h)[2][2]) {
 #pragma unroll
-  for (int jt = 0; jt < 4; ++jt) acc[jt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int u = 0; u < 2; ++u)
 #pragma unroll
-  for (int s = 0; s < 7; ++s) {
-    const bf16x8 a = encode_chunk(x, 4 * s + (int)g);
-    if (x0t) {
-      // training: the transposed features, with the constant input 1 at row 216
-      const uint4 w = __builtin_bit_cast(uint4, a);
-      const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
-      const uint32_t k0 = 32u * s + 8u * g;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        uint16_t h = (uint16_t)(ww[e >> 1] >> (16 * (e & 1)));
-        if (k0 + e == (uint32_t)kGuideFeatures) h = 0x3F80u;
-        x0t[(uint64_t)(k0 + e) * ldb + col + i] = h;
-      }
-    }
-#pragma unroll
-    for (int jt = 0; jt < 4; ++jt) acc[jt] = mfma(a, frag16(sw + (16 * jt + i) * kW1Stride + 32 * s + 8 * g), acc[jt]);
-  }
+    for (int s = 0; s < 2; ++s) h[u][s] = to_frag(relu4(acc[u][2 * s]), relu4(acc[u][2 * s + 1]));
+}
+
+// A value that the compiler takes for a new one: what depends on it is
+// computed where it stands.  Loops over sample tiles use it for the lane:
+// the weights' addresses and fragments, hoisted out of the loop, would take
+// more registers than there are.
+BJ_D uint32_t fresh(uint32_t v) {
+  asm volatile("" : "+v"(v));
+  return v;
 }
 
 // Block-wide copy of the first `elems` BF16 weights and the biases into LDS.
-BJ_D void load_pack(const uint8_t* __restrict__ pack, uint16_t* sw, int elems, float* sb) {
+BJ_D void load_pack(const uint8_t* __restrict__ pack, uint16_t* sw, int elems, float* sb, uint32_t tid) {
   const uint4* src = (const uint4*)pack;
   uint4* dst = (uint4*)sw;
-  for (int i = threadIdx.x; i < elems / 8; i += blockDim.x) dst[i] = src[i];
+  for (uint32_t i = tid; i < (uint32_t)elems / 8; i += blockDim.x) dst[i] = src[i];
   const float* bsrc = (const float*)(pack + (size_t)kPackAll * 2);
-  for (int i = threadIdx.x; i < kBiasFloats; i += blockDim.x) sb[i] = bsrc[i];
+  for (uint32_t i = tid; i < (uint32_t)kBiasFloats; i += blockDim.x) sb[i] = bsrc[i];
   __syncthreads();
 }
 
 // ---- forward ---------------------------------------------------------------------
 // Inputs: explicit f32[9 n], or render vertices (their position, normal and
 // ray direction planes) normalized against the scene box.
+// load: the inputs of row r's seven chunks of lane group g.
 struct InputRows {
   const float* x;
-  BJ_D void load(uint64_t r, float (&v)[kGuideInputs]) const {
+  BJ_D void load(uint64_t r, uint32_t g, float (&v)[7]) const {
 #pragma unroll
-    for (int a = 0; a < kGuideInputs; ++a) v[a] = x[r * kGuideInputs + a];
+    for (int s = 0; s < 7; ++s) v[s] = x[r * kGuideInputs + chunk_input(s, g)];
   }
 };
 
 struct VertexRows {
   const float* f;
   const float* bounds;  // scene box lo.xyz, hi.xyz
-  BJ_D void load(uint64_t r, float (&v)[kGuideInputs]) const {
+  BJ_D void load(uint64_t r, uint32_t g, float (&v)[7]) const {
     const v3 lo = mk(bounds[0], bounds[1], bounds[2]);
     const v3 hi = mk(bounds[3], bounds[4], bounds[5]);
     const v3 ext = sub(hi, lo);
@@ -228,78 +247,107 @@ struct VertexRows {
     const v3 p = mk(f[vplane(r, 0)], f[vplane(r, 1)], f[vplane(r, 2)]);
     const v3 n = mk(f[vplane(r, 3)], f[vplane(r, 4)], f[vplane(r, 5)]);
     const v3 d = mk(f[vplane(r, 6)], f[vplane(r, 7)], f[vplane(r, 8)]);
-    const GuideInput g = guide_input(p, n, normalize(mk(-d.x, -d.y, -d.z)), lo, inv);
+    const GuideInput gi = guide_input(p, n, normalize(mk(-d.x, -d.y, -d.z)), lo, inv);
 #pragma unroll
-    for (int a = 0; a < kGuideInputs; ++a) v[a] = g.v[a];
+    for (int s = 0; s < 7; ++s) {
+      const int first = 4 * s / 3, next = first + 1 < kGuideInputs ? first + 1 : first;
+      v[s] = chunk_input(s, g) == first ? gi.v[first] : gi.v[next];
+    }
   }
 };
 
+// Bound by the encoding's arithmetic (about 400 instructions per lane and 16
+// samples) beside the outputs' 160 bytes per sample; 524,309 inputs take
+// 48 us, 102 with activations staged through LDS 16 samples at a time,
+// element by element.
+constexpr int kForwardBlock = 512;
+
 template <typename Rows>
-__global__ void __launch_bounds__(256) guide_forward_kernel(const uint8_t* __restrict__ pack, Rows rows,
-                                                            const uint32_t* __restrict__ count_dev, uint64_t count,
-                                                            float* __restrict__ out) {
+__global__ void __launch_bounds__(kForwardBlock) guide_forward_kernel(const uint8_t* __restrict__ pack, Rows rows,
+                                                                      const uint32_t* __restrict__ count_dev,
+                                                                      uint64_t count, float* __restrict__ out) {
+  // outputs may start at any float
+  typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4_any;
   __shared__ __attribute__((aligned(16))) uint16_t s_w[kPackFwd];
-  __shared__ float s_b[kBiasFloats];
-  __shared__ __attribute__((aligned(16))) uint16_t s_h[4][16 * kRowStride];
+  __shared__ __attribute__((aligned(16))) float s_b[kBiasFloats];
+  constexpr uint32_t kWaves = kForwardBlock / 64;
   uint64_t n = count;
   if (count_dev) n = *count_dev < count ? *count_dev : count;
-  const uint64_t tiles = (n + 15) / 16;
-  if ((uint64_t)blockIdx.x * 4 >= tiles) return;  // uniform per block: before the barrier
-  load_pack(pack, s_w, kPackFwd, s_b);
-  const uint32_t lane = lane_id(), wave = threadIdx.x >> 6;
-  const uint32_t i = lane & 15u, g = lane >> 4;
-  uint16_t* sh = s_h[wave];
-  for (uint64_t tile = (uint64_t)blockIdx.x * 4 + wave; tile < tiles; tile += (uint64_t)gridDim.x * 4) {
-    const uint64_t r = tile * 16 + i;
-    float x[kGuideInputs];
-    if (r < n) rows.load(r, x);
-    else
+  const uint64_t pairs = (n + 31) / 32;
+  if ((uint64_t)blockIdx.x >= pairs) return;  // uniform per block: before the barrier
+  load_pack(pack, s_w, kPackFwd, s_b, threadIdx.x);
+  const uint32_t wave = threadIdx.x >> 6;
+  // waves take neighbouring pairs across the grid, so that a short list spreads over the blocks
+  for (uint64_t pair = (uint64_t)wave * gridDim.x + blockIdx.x; pair < pairs; pair += (uint64_t)gridDim.x * kWaves) {
+    const uint32_t lane = fresh(lane_id());
+    const uint32_t i = lane & 15u, g = lane >> 4;
+    float sc[3];
+    chunk_scales(g, sc);
+    float x[2][7];
 #pragma unroll
-      for (int a = 0; a < kGuideInputs; ++a) x[a] = 0.0f;
-    f32x4 acc[4];
-    layer1(x, s_w + kPackW1, acc, lane);
-    store_hidden(acc, s_b, sh, lane);
-    __builtin_amdgcn_wave_barrier();
-    layer64<4>(sh, s_w + kPackW2, acc, lane);
-    __builtin_amdgcn_wave_barrier();
-    store_hidden(acc, s_b + 64, sh, lane);
-    __builtin_amdgcn_wave_barrier();
-    layer64<4>(sh, s_w + kPackW3, acc, lane);
-    __builtin_amdgcn_wave_barrier();
-    store_hidden(acc, s_b + 128, sh, lane);
-    __builtin_amdgcn_wave_barrier();
-    f32x4 o[3];
-    layer64<3>(sh, s_w + kPackW4, o, lane);
-    __builtin_amdgcn_wave_barrier();
+    for (int u = 0; u < 2; ++u) {
+      const uint64_t r = pair * 32 + 16 * u + i;
+      rows.load(r < n ? r : n - 1, g, x[u]);
+    }
+    f32x4 acc[2][4];
+    start_bias<4>(s_b, acc, g);
 #pragma unroll
-    for (int jt = 0; jt < 3; ++jt) {
-      const uint32_t col = 16u * jt + i;
+    for (int s = 0; s < 7; ++s) {
+      bf16x8 f[2];
 #pragma unroll
-      for (int rr = 0; rr < 4; ++rr) {
-        const uint64_t row = tile * 16 + 4 * g + rr;
-        if (col < (uint32_t)kGuideOut && row < n) out[row * kGuideOut + col] = o[jt][rr] + s_b[192 + col];
+      for (int u = 0; u < 2; ++u) f[u] = encode_chunk(x[u][s], sc[s % 3], s == 6 && g == 3);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const bf16x8 w = frag16(s_w + kPackW1 + (16 * t + i) * kW1Stride + 32 * s + 8 * g);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) acc[u][t] = mfma(w, f[u], acc[u][t]);
       }
+    }
+    bf16x8 h[2][2];
+    hidden_frags(acc, h);
+    start_bias<4>(s_b + 64, acc, g);
+    layer64<4>(s_w + kPackW2, h, acc, lane);
+    hidden_frags(acc, h);
+    start_bias<4>(s_b + 128, acc, g);
+    layer64<4>(s_w + kPackW3, h, acc, lane);
+    hidden_frags(acc, h);
+    f32x4 o[2][3];
+    start_bias<3>(s_b + 192, o, g);
+    layer64<3>(s_w + kPackW4, h, o, lane);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const uint64_t r = pair * 32 + 16 * u + i;
+      if (r >= n) continue;
+      float* row = out + r * kGuideOut + 4 * g;
+      *(f32x4_any*)row = o[u][0];
+      *(f32x4_any*)(row + 16) = o[u][1];
+      if (g < 2) *(f32x4_any*)(row + 32) = o[u][2];
     }
   }
 }
 
 // ---- loss gradient of one sample (outputs -> d loss / d outputs) ------------------
-// Loss -w ln q(dir), q = sum_j pi_j vMF_j(dir) in log space; returns the
-// weighted loss.
-BJ_D float output_gradient(const float* o, v3 dir, float w, float* d) {
-  float lp[kGuideLobes], lc[kGuideLobes], kap[kGuideLobes], mdw[kGuideLobes], len[kGuideLobes], e2v[kGuideLobes];
-  v3 mu[kGuideLobes];
-  bool inside[kGuideLobes];
-  float amax = o[4];
+// Sum and maximum over the four lanes of a sample (the same in each).
+BJ_D float sample_sum(float v) {
+  v += __shfl_xor(v, 16, 64);
+  return v + __shfl_xor(v, 32, 64);
+}
+BJ_D float sample_max(float v) {
+  v = fmax_sel(v, __shfl_xor(v, 16, 64));
+  return fmax_sel(v, __shfl_xor(v, 32, 64));
+}
+
+// Loss -w ln q(dir), q = sum_j pi_j vMF_j(dir) in log space; each of a
+// sample's four lanes takes two lobes (`o`: their 10 outputs, `d`: the
+// gradients).  Returns the sample's weighted loss.
+BJ_D float output_gradient(const float (&o)[10], v3 dir, float w, float (&d)[10]) {
+  float lp[2], lc[2], kap[2], mdw[2], len[2], e2v[2];
+  v3 mu[2];
+  bool inside[2];
+  const float amax = sample_max(fmax_sel(o[4], o[9]));
+  const float lse_a = amax + ln_f(sample_sum(exp_f(o[4] - amax) + exp_f(o[9] - amax)));
 #pragma unroll
-  for (int j = 1; j < kGuideLobes; ++j) amax = fmax_sel(amax, o[5 * j + 4]);
-  float se = 0.0f;
-#pragma unroll
-  for (int j = 0; j < kGuideLobes; ++j) se += exp_f(o[5 * j + 4] - amax);
-  const float lse_a = amax + ln_f(se);
-  float cmax = -kFltMax;
-#pragma unroll
-  for (int j = 0; j < kGuideLobes; ++j) {
+  for (int j = 0; j < 2; ++j) {
     const float* oj = o + 5 * j;
     const float l2 = oj[0] * oj[0] + oj[1] * oj[1] + oj[2] * oj[2];
     len[j] = sqrtf(l2);
@@ -311,14 +359,11 @@ BJ_D float output_gradient(const float* o, v3 dir, float w, float* d) {
     mdw[j] = dot(mu[j], dir);
     lp[j] = oj[4] - lse_a;
     lc[j] = lp[j] + (s - kLn2Pi - ln_f(1.0f - e2v[j])) + kap[j] * (mdw[j] - 1.0f);
-    cmax = fmax_sel(cmax, lc[j]);
   }
-  float sc = 0.0f;
+  const float cmax = sample_max(fmax_sel(lc[0], lc[1]));
+  const float lq = cmax + ln_f(sample_sum(exp_f(lc[0] - cmax) + exp_f(lc[1] - cmax)));
 #pragma unroll
-  for (int j = 0; j < kGuideLobes; ++j) sc += exp_f(lc[j] - cmax);
-  const float lq = cmax + ln_f(sc);
-#pragma unroll
-  for (int j = 0; j < kGuideLobes; ++j) {
+  for (int j = 0; j < 2; ++j) {
     const float r = exp_f(lc[j] - lq);
     const float pi = exp_f(lp[j]);
     d[5 * j + 4] = w * (pi - r);
@@ -332,40 +377,77 @@ BJ_D float output_gradient(const float* o, v3 dir, float w, float* d) {
   return -w * lq;
 }
 
-// Masked backward step: acc (16 x 64 D fragments) times the ReLU mask of
-// the forward activations `sh`, to BF16 in `sd` (row-major) .
-BJ_D void store_delta(const f32x4 (&acc)[4], const uint16_t* sh, uint16_t* sd, uint32_t lane) {
-  const uint32_t col = lane & 15u, g = lane >> 4;
-#pragma unroll
-  for (int jt = 0; jt < 4; ++jt)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int at = (4 * g + r) * kRowStride + 16 * jt + col;
-      sd[at] = sh[at] != 0 ? f2bf(acc[jt][r]) : (uint16_t)0;
-    }
+// ---- training: forward, backward and the weight gradient ----------------------------
+// Where the activation was 0 the delta is 0.
+BJ_D bf16x8 masked(bf16x8 d, bf16x8 h) {
+  const uint4 hw = __builtin_bit_cast(uint4, h);
+  uint4 dw = __builtin_bit_cast(uint4, d);
+  const auto keep = [](uint32_t v) { return ((v & 0xFFFFu) ? 0xFFFFu : 0u) | ((v >> 16) ? 0xFFFF0000u : 0u); };
+  dw.x &= keep(hw.x);
+  dw.y &= keep(hw.y);
+  dw.z &= keep(hw.z);
+  dw.w &= keep(hw.w);
+  return __builtin_bit_cast(bf16x8, dw);
 }
 
-// Writes rows [0, rows) of a row-major 16 x 72 tile transposed: lane l
-// writes row l's 16 samples (32 contiguous bytes) at dst[l * ldb + col].
-BJ_D void store_transposed(const uint16_t* st, int rows, uint16_t* dst, uint64_t ldb, uint64_t col, uint32_t lane) {
-  if ((int)lane < rows) {
-    uint32_t w[8];
+// The products of row tile k of a 64-wide layer with both sample tiles, in
+// both orientations: n as layer64, t its transpose (lane: unit 16 k + i,
+// elements: samples 4 g .. + 3).
+BJ_D void tile_both(const uint16_t* sw, int k, const bf16x8 (&in)[2][2], f32x4 (&n)[2], f32x4 (&t)[2], uint32_t lane) {
+  const uint32_t i = lane & 15u, g = lane >> 4;
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-      w[e] = (uint32_t)st[(2 * e) * kRowStride + lane] | ((uint32_t)st[(2 * e + 1) * kRowStride + lane] << 16);
-    uint4* p = (uint4*)(dst + (uint64_t)lane * ldb + col);
-    p[0] = uint4{w[0], w[1], w[2], w[3]};
-    p[1] = uint4{w[4], w[5], w[6], w[7]};
+  for (int s = 0; s < 2; ++s) {
+    const bf16x8 w = frag16(sw + (16 * k + i) * kRowStride + 32 * s + 8 * g);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      n[u] = mfma(w, in[u][s], n[u]);
+      t[u] = mfma(in[u][s], w, t[u]);
+    }
   }
 }
 
-// Constant rows 64..79 of a hidden-activation buffer: 1 at row 64, 0 below.
-BJ_D void store_bias_rows(uint16_t* dst, uint64_t ldb, uint64_t col, uint32_t lane) {
-  if (lane < 16) {
-    const uint32_t v = lane == 0 ? 0x3F803F80u : 0u;
-    uint4* p = (uint4*)(dst + (uint64_t)(kGuideHidden + lane) * ldb + col);
-    p[0] = uint4{v, v, v, v};
-    p[1] = uint4{v, v, v, v};
+// A hidden layer forward: h the next operand, ht the transposed activations:
+// unit 16 k + i of samples 4 g .. + 3 of both sample tiles, one operand of
+// the weight gradient (its K order is the same for both operands).  Row tile
+// by row tile, so that few products are live beside what the gradient needs.
+BJ_D void forward_both(const uint16_t* sw, const float* bias, const bf16x8 (&in)[2][2], bf16x8 (&h)[2][2],
+                       bf16x8 (&ht)[4], uint32_t lane) {
+  const uint32_t i = lane & 15u, g = lane >> 4;
+#pragma unroll
+  for (int kp = 0; kp < 2; ++kp) {
+    f32x4 n[2][2];
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const int k = 2 * kp + half;
+      const float b = bias[16 * k + i];
+      f32x4 t[2] = {f32x4{b, b, b, b}, f32x4{b, b, b, b}};
+      n[half][0] = n[half][1] = *(const f32x4*)(bias + 16 * k + 4 * g);
+      tile_both(sw, k, in, n[half], t, lane);
+      ht[k] = to_frag(relu4(t[0]), relu4(t[1]));
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) h[u][kp] = to_frag(relu4(n[0][u]), relu4(n[1][u]));
+  }
+}
+
+// A layer backward: the deltas of its inputs, masked by their activations
+// (h, ht), as the next operand and transposed.
+BJ_D void backward_both(const uint16_t* sw, const bf16x8 (&in)[2][2], const bf16x8 (&h)[2][2], const bf16x8 (&ht)[4],
+                        bf16x8 (&d)[2][2], bf16x8 (&dt)[4], uint32_t lane) {
+#pragma unroll
+  for (int kp = 0; kp < 2; ++kp) {
+    f32x4 n[2][2];
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const int k = 2 * kp + half;
+      const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+      f32x4 t[2] = {zero, zero};
+      n[half][0] = n[half][1] = zero;
+      tile_both(sw, k, in, n[half], t, lane);
+      dt[k] = masked(to_frag(t[0], t[1]), ht[k]);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) d[u][kp] = masked(to_frag(n[0][u], n[1][u]), h[u][kp]);
   }
 }
 
@@ -374,135 +456,250 @@ struct TrainArgs {
   // batch row r is sample (src_offset + r * src_stride) % src_count
   uint64_t src_count, src_offset, src_stride;
   uint64_t n;            // samples
-  uint64_t n_pad;        // n rounded up to a whole chunk (padded rows carry weight 0)
-  uint64_t ldb;          // row stride of the transposed buffers
-  uint16_t *x0t, *h1t, *h2t, *h3t, *d1t, *d2t, *d3t, *dot;
-  float* tile_part;      // per tile: sum w, weighted loss
+  float* part;           // [block][kTiles][256] weight gradients
+  double* loss_part;     // per block: sum of weights, weighted loss
 };
 
-// Forward + backward of 16-sample tiles: activations and deltas of every
-// layer written transposed for the weight gradient.
-__global__ void __launch_bounds__(256) guide_train_kernel(const uint8_t* __restrict__ pack, TrainArgs ta) {
-  __shared__ __attribute__((aligned(16))) uint16_t s_w[kPackAll];
-  __shared__ float s_b[kBiasFloats];
-  __shared__ __attribute__((aligned(16))) uint16_t s_h[4][3][16 * kRowStride];
-  __shared__ __attribute__((aligned(16))) uint16_t s_d[4][16 * kRowStride];
-  __shared__ float s_o[4][16 * kGuideOutPad];
-  const uint64_t tiles = ta.n_pad / 16;
-  if ((uint64_t)blockIdx.x * 4 >= tiles) return;
-  load_pack(pack, s_w, kPackAll, s_b);
-  const uint32_t lane = lane_id(), wave = threadIdx.x >> 6;
-  const uint32_t i = lane & 15u, g = lane >> 4;
-  uint16_t* h1 = s_h[wave][0];
-  uint16_t* h2 = s_h[wave][1];
-  uint16_t* h3 = s_h[wave][2];
-  uint16_t* sd = s_d[wave];
-  float* so = s_o[wave];
-  for (uint64_t tile = (uint64_t)blockIdx.x * 4 + wave; tile < tiles; tile += (uint64_t)gridDim.x * 4) {
-    const uint64_t col = tile * 16;
-    const uint64_t r = col + i;
-    float x[kGuideInputs];
-    const float* sp = ta.samples + ((ta.src_offset + r * ta.src_stride) % ta.src_count) * kGuideSampleFloats;
+// Fragments of the weight gradient in LDS: [fragment][wave of the samples][lane].
+constexpr int kExchangeFrags = 14 + 4;  // layer 1, the largest: features and deltas
+constexpr size_t kExchangeBytes = (size_t)kExchangeFrags * kTrainWaves * 64 * 16;
+constexpr int kOutRow = 44;             // floats of a sample's outputs (16-byte rows)
+constexpr size_t kOutBytes = (size_t)kTrainWaves * 32 * kOutRow * 4;
+static_assert((size_t)kPackAll * 2 + kOutBytes <= kExchangeBytes, "weights and outputs share the exchange's LDS");
+
+// kN gradient tiles (first, first + 1, ...) over the block's samples: deltas
+// at fragment `a`, inputs at fragments `b`, `b` + 1, ...; fragment index -1 is
+// the constant input in column `i == 0`.
+template <int kN>
+BJ_D void gradient_tiles(const uint4* ex, int a, const int (&b)[kN], float* part, int first, bool add, uint32_t lane) {
+  f32x4 acc[kN];
+  float* at = part + (size_t)first * 256 + lane * 4;
 #pragma unroll
-    for (int a = 0; a < kGuideInputs; ++a) x[a] = r < ta.n ? sp[a] : 0.0f;
-    f32x4 acc[4];
-    layer1(x, s_w + kPackW1, acc, lane, ta.x0t, ta.ldb, col);
-    store_hidden(acc, s_b, h1, lane);
-    __builtin_amdgcn_wave_barrier();
-    layer64<4>(h1, s_w + kPackW2, acc, lane);
-    store_hidden(acc, s_b + 64, h2, lane);
-    __builtin_amdgcn_wave_barrier();
-    layer64<4>(h2, s_w + kPackW3, acc, lane);
-    store_hidden(acc, s_b + 128, h3, lane);
-    __builtin_amdgcn_wave_barrier();
-    f32x4 o[3];
-    layer64<3>(h3, s_w + kPackW4, o, lane);
+  for (int t = 0; t < kN; ++t) acc[t] = add ? *(const f32x4*)(at + 256 * t) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const uint32_t one = (lane & 15u) == 0 ? 0x3F803F80u : 0u;
+#pragma unroll 2
+  for (int w = 0; w < kTrainWaves; ++w) {
+    const bf16x8 d = __builtin_bit_cast(bf16x8, ex[(a * kTrainWaves + w) * 64 + lane]);
 #pragma unroll
-    for (int jt = 0; jt < 3; ++jt)
-#pragma unroll
-      for (int rr = 0; rr < 4; ++rr) so[(4 * g + rr) * kGuideOutPad + 16 * jt + i] = o[jt][rr] + s_b[192 + 16 * jt + i];
-    store_transposed(h1, kGuideHidden, ta.h1t, ta.ldb, col, lane);
-    store_transposed(h2, kGuideHidden, ta.h2t, ta.ldb, col, lane);
-    store_transposed(h3, kGuideHidden, ta.h3t, ta.ldb, col, lane);
-    store_bias_rows(ta.h1t, ta.ldb, col, lane);
-    store_bias_rows(ta.h2t, ta.ldb, col, lane);
-    store_bias_rows(ta.h3t, ta.ldb, col, lane);
-    __builtin_amdgcn_wave_barrier();
-    // loss gradient of the outputs: lane i < 16 takes sample i
-    float wsum = 0.0f, lsum = 0.0f;
-    if (lane < 16) {
-      float d[kGuideOut];
-      float w = 0.0f;
-      v3 dir = mk(0.0f, 0.0f, 1.0f);
-      if (r < ta.n) {
-        dir = mk(sp[9], sp[10], sp[11]);
-        w = sp[12];
-      }
-      const float loss = output_gradient(so + lane * kGuideOutPad, dir, w, d);
-      wsum = w;
-      lsum = w > 0.0f ? loss : 0.0f;
-#pragma unroll
-      for (int c = 0; c < kGuideOut; ++c) sd[lane * kRowStride + c] = f2bf(d[c]);
-#pragma unroll
-      for (int c = kGuideOut; c < kGuideHidden; ++c) sd[lane * kRowStride + c] = 0;
+    for (int t = 0; t < kN; ++t) {
+      const uint4 x = b[t] >= 0 ? ex[(b[t] * kTrainWaves + w) * 64 + lane] : uint4{one, one, one, one};
+      acc[t] = mfma(d, __builtin_bit_cast(bf16x8, x), acc[t]);
     }
-#pragma unroll
-    for (int off = 8; off >= 1; off >>= 1) {
-      wsum += __shfl_xor(wsum, off, 64);
-      lsum += __shfl_xor(lsum, off, 64);
-    }
-    if (lane == 0) {
-      ta.tile_part[2 * tile] = wsum;
-      ta.tile_part[2 * tile + 1] = lsum;
-    }
-    __builtin_amdgcn_wave_barrier();
-    store_transposed(sd, kDoRows, ta.dot, ta.ldb, col, lane);
-    // backward: d3 = dO W4 (B rows from W4^T), masked by h3; then d2, d1
-    layer64<4>(sd, s_w + kPackW4t, acc, lane);
-    __builtin_amdgcn_wave_barrier();
-    store_delta(acc, h3, sd, lane);
-    __builtin_amdgcn_wave_barrier();
-    store_transposed(sd, kDRows, ta.d3t, ta.ldb, col, lane);
-    layer64<4>(sd, s_w + kPackW3t, acc, lane);
-    __builtin_amdgcn_wave_barrier();
-    store_delta(acc, h2, sd, lane);
-    __builtin_amdgcn_wave_barrier();
-    store_transposed(sd, kDRows, ta.d2t, ta.ldb, col, lane);
-    layer64<4>(sd, s_w + kPackW2t, acc, lane);
-    __builtin_amdgcn_wave_barrier();
-    store_delta(acc, h1, sd, lane);
-    __builtin_amdgcn_wave_barrier();
-    store_transposed(sd, kDRows, ta.d1t, ta.ldb, col, lane);
-    __builtin_amdgcn_wave_barrier();
   }
+#pragma unroll
+  for (int t = 0; t < kN; ++t) *(f32x4*)(at + 256 * t) = acc[t];
 }
 
-// ---- weight gradient: dW[out][in] = sum over the batch of D[out] X[in] ----------
-struct WgradArgs {
-  const uint16_t *x0t, *h1t, *h2t, *h3t, *d1t, *d2t, *d3t, *dot;
-  uint64_t ldb;
-  float* part;  // [chunk][kTiles][256]
-};
-
-__global__ void __launch_bounds__(64) guide_wgrad_kernel(WgradArgs wa) {
-  const uint32_t t = blockIdx.x, chunk = blockIdx.y;
-  const uint32_t lane = lane_id();
-  const uint32_t i = lane & 15u, g = lane >> 4;
-  const uint16_t *dsrc, *xsrc;
-  uint32_t mt, nt;
-  if (t < (uint32_t)kT2) { mt = t / 14; nt = t % 14; dsrc = wa.d1t; xsrc = wa.x0t; }
-  else if (t < (uint32_t)kT3) { mt = (t - kT2) / 5; nt = (t - kT2) % 5; dsrc = wa.d2t; xsrc = wa.h1t; }
-  else if (t < (uint32_t)kT4) { mt = (t - kT3) / 5; nt = (t - kT3) % 5; dsrc = wa.d3t; xsrc = wa.h2t; }
-  else { mt = (t - kT4) / 5; nt = (t - kT4) % 5; dsrc = wa.dot; xsrc = wa.h3t; }
-  const uint64_t b0 = (uint64_t)chunk * kChunk;
-  const uint16_t* a_row = dsrc + (uint64_t)(16 * mt + i) * wa.ldb + b0 + 8 * g;
-  const uint16_t* b_row = xsrc + (uint64_t)(16 * nt + i) * wa.ldb + b0 + 8 * g;
-  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 4
-  for (int s = 0; s < kChunk / 32; ++s) acc = mfma(frag16(a_row + 32 * s), frag16(b_row + 32 * s), acc);
-  float* out = wa.part + ((uint64_t)chunk * kTiles + t) * 256;
+// One launch per batch, 256 samples per block and pass.  Latency bound: one
+// wave's chain of four layers, the loss and three layers back, then three
+// exchanges.  65,521 samples: 38 us; 85 + 62 us as a pass that wrote
+// every activation and delta to memory in BF16 (92 MB) and a batch-reduction
+// kernel that read them.
+__global__ void __launch_bounds__(kTrainWaves * 64) guide_train_kernel(const uint8_t* __restrict__ pack, TrainArgs ta) {
+  __shared__ __attribute__((aligned(16))) uint8_t s_mem[kExchangeBytes];
+  __shared__ __attribute__((aligned(16))) float s_b[kBiasFloats];
+  __shared__ float s_loss[kTrainWaves * 2][2];
+  uint16_t* s_w = (uint16_t*)s_mem;
+  uint4* ex = (uint4*)s_mem;
+  float* part = ta.part + (size_t)blockIdx.x * kTiles * 256;
+  double block_w = 0.0, block_l = 0.0;
+  for (uint64_t base = (uint64_t)blockIdx.x * kTrainSamples; base < ta.n; base += (uint64_t)gridDim.x * kTrainSamples) {
+    const bool add = base != (uint64_t)blockIdx.x * kTrainSamples;
+    const uint32_t tid = fresh(threadIdx.x), lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t i = lane & 15u, g = lane >> 4;
+    float* s_out = (float*)(s_mem + (size_t)kPackAll * 2) + wave * 32 * kOutRow;
+    float sc[3];
+    chunk_scales(g, sc);
+    load_pack(pack, s_w, kPackAll, s_b, tid);
+    const float* sp[2];
+    bool real[2];
+    float x[2][7];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) out[(4 * g + r) * 16 + i] = acc[r];
+    for (int u = 0; u < 2; ++u) {
+      const uint64_t r = base + wave * 32 + 16 * u + i;
+      real[u] = r < ta.n;
+      const uint64_t row = real[u] ? (ta.src_offset + r * ta.src_stride) % ta.src_count : 0;
+      sp[u] = ta.samples + row * kGuideSampleFloats;
+#pragma unroll
+      for (int s = 0; s < 7; ++s) x[u][s] = real[u] ? sp[u][chunk_input(s, g)] : 0.0f;
+    }
+    bf16x8 h1t[4], h2t[4], h3t[4];
+    bf16x8 h1[2][2], h2[2][2], h3[2][2];
+    {
+      f32x4 n[2][4], t[2][4];
+      start_bias<4>(s_b, n, g);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float b = s_b[16 * k + i];
+        t[0][k] = t[1][k] = f32x4{b, b, b, b};
+      }
+#pragma unroll
+      for (int s = 0; s < 7; ++s) {
+        bf16x8 f[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) f[u] = encode_chunk(x[u][s], sc[s % 3], s == 6 && g == 3);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const bf16x8 w = frag16(s_w + kPackW1 + (16 * k + i) * kW1Stride + 32 * s + 8 * g);
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            n[u][k] = mfma(w, f[u], n[u][k]);
+            t[u][k] = mfma(f[u], w, t[u][k]);
+          }
+        }
+      }
+      hidden_frags(n, h1);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) h1t[k] = to_frag(relu4(t[0][k]), relu4(t[1][k]));
+    }
+    forward_both(s_w + kPackW2, s_b + 64, h1, h2, h2t, lane);
+    forward_both(s_w + kPackW3, s_b + 128, h2, h3, h3t, lane);
+    f32x4 o[2][3];
+    start_bias<3>(s_b + 192, o, g);
+    layer64<3>(s_w + kPackW4, h3, o, lane);
+__builtin_amdgcn_sched_barrier(0);
+    // outputs to rows of samples; a sample's four lanes take two lobes each
+    bf16x8 dof[2][2], dot[3], d3t[4], d2t[4], d1t[4];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      float* row = s_out + (16 * u + i) * kOutRow;
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        if (k < 2 || g < 2) *(f32x4*)(row + 16 * k + 4 * g) = o[u][k];
+      __builtin_amdgcn_wave_barrier();
+      float lobe[10], d[10];
+#pragma unroll
+      for (int k = 0; k < 10; ++k) lobe[k] = row[10 * g + k];
+      const v3 dir = real[u] ? mk(sp[u][9], sp[u][10], sp[u][11]) : mk(0.0f, 0.0f, 1.0f);
+      const float w = real[u] ? sp[u][12] : 0.0f;
+      const float loss = output_gradient(lobe, dir, w, d);
+#pragma unroll
+      for (int k = 0; k < 10; ++k) row[10 * g + k] = d[k];
+      float wsum = w, lsum = w > 0.0f ? loss : 0.0f;
+#pragma unroll
+      for (int off = 8; off >= 1; off >>= 1) {
+        wsum += __shfl_xor(wsum, off, 64);
+        lsum += __shfl_xor(lsum, off, 64);
+      }
+      if (lane == 0) {
+        s_loss[2 * wave + u][0] = wsum;
+        s_loss[2 * wave + u][1] = lsum;
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+    {
+      const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const float* row = s_out + (16 * u + i) * kOutRow + 4 * g;
+        dof[u][0] = to_frag(*(const f32x4*)row, *(const f32x4*)(row + 16));
+        dof[u][1] = to_frag(g < 2 ? *(const f32x4*)(row + 32) : zero, zero);
+      }
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        f32x4 c[2] = {zero, zero};
+        if (k < 2 || i < 8)
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) c[u][r] = s_out[(16 * u + 4 * g + r) * kOutRow + 16 * k + i];
+        dot[k] = to_frag(c[0], c[1]);
+      }
+    }
+__builtin_amdgcn_sched_barrier(0);
+    // backward: d3 = W4^T dO, masked by h3; then d2, d1 (its transpose only)
+    bf16x8 d3[2][2], d2[2][2];
+    backward_both(s_w + kPackW4t, dof, h3, h3t, d3, d3t, lane);
+    backward_both(s_w + kPackW3t, d3, h2, h2t, d2, d2t, lane);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+      f32x4 t[2] = {zero, zero};
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const bf16x8 w = frag16(s_w + kPackW2t + (16 * k + i) * kRowStride + 32 * s + 8 * g);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) t[u] = mfma(d2[u][s], w, t[u]);
+      }
+      d1t[k] = masked(to_frag(t[0], t[1]), h1t[k]);
+    }
+__builtin_amdgcn_sched_barrier(0);
+    // weight gradients; each exchange waits for the last one's readers
+    const auto put = [&](int f, bf16x8 v) { ex[(f * kTrainWaves + wave) * 64 + lane] = __builtin_bit_cast(uint4, v); };
+    __syncthreads();
+    if (threadIdx.x == 0)
+      for (int k = 0; k < 2 * kTrainWaves; ++k) {
+        block_w += (double)s_loss[k][0];
+        block_l += (double)s_loss[k][1];
+      }
+    // the features' transpose is their product with unit columns (encoded
+    // again: kept from layer 1 they would not fit the registers)
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int s = 0; s < 7; ++s) asm volatile("" : "+v"(x[u][s]));
+    bf16x8 unit[2];
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) unit[half][e] = (__bf16)(8 * g + e == 16 * half + i ? 1.0f : 0.0f);
+#pragma unroll
+    for (int s = 0; s < 7; ++s) {
+      bf16x8 f[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) f[u] = encode_chunk(x[u][s], sc[s % 3], s == 6 && g == 3);
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+        put(2 * s + half, to_frag(mfma(f[0], unit[half], zero), mfma(f[1], unit[half], zero)));
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) put(14 + k, d1t[k]);
+    __syncthreads();
+    {  // layer 1: wave w takes rows 16 (w % 4) .. + 15, seven of the 14 column tiles
+      const int m = (int)wave & 3, c = 7 * ((int)wave >> 2);
+      const int b[7] = {c, c + 1, c + 2, c + 3, c + 4, c + 5, c + 6};
+      gradient_tiles<7>(ex, 14 + m, b, part, kT1 + 14 * m + c, add, lane);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      __builtin_amdgcn_sched_barrier(0);
+put(k, h1t[k]);
+      put(4 + k, h2t[k]);
+      put(8 + k, d2t[k]);
+      put(12 + k, d3t[k]);
+    }
+    __syncthreads();
+    {  // layers 2 and 3: one row of five tiles (the last holds the biases) per wave
+      const int m = (int)wave & 3, c = 4 * ((int)wave >> 2);
+      const int b[5] = {c, c + 1, c + 2, c + 3, -1};
+      gradient_tiles<5>(ex, 8 + c + m, b, part, (wave < 4 ? kT2 : kT3) + 5 * m, add, lane);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) put(k, h3t[k]);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) put(4 + k, dot[k]);
+    __syncthreads();
+    if (wave < 6) {  // layer 4: three rows of five tiles, two waves per row
+      const int m = (int)wave >> 1;
+      if (wave & 1u) {
+        const int b[2] = {3, -1};
+        gradient_tiles<2>(ex, 4 + m, b, part, kT4 + 5 * m + 3, add, lane);
+      } else {
+        const int b[3] = {0, 1, 2};
+        gradient_tiles<3>(ex, 4 + m, b, part, kT4 + 5 * m, add, lane);
+      }
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    ta.loss_part[2 * blockIdx.x] = block_w;
+    ta.loss_part[2 * blockIdx.x + 1] = block_l;
+  }
 }
 
 // ---- reduce + Adam ----------------------------------------------------------------
@@ -515,41 +712,44 @@ struct AdamArgs {
   uint8_t* infer_pack;
   float ema_decay;
   const float* part;
-  uint32_t chunks;
-  const float* tile_part;
-  uint32_t tiles;
+  const double* loss_part;
+  uint32_t blocks;       // partials
   float lr, beta1, beta2, eps, bias1, bias2;  // bias1/2 = 1 - beta^t
   float* grad_out;  // gradient mode: write the gradient, no update
 };
-
-// Sum over the batch's tiles of per-tile values (stride 2), fixed order.
-BJ_D float block_sum(const float* v, uint32_t count, float* s_tmp) {
-  float acc = 0.0f;
-  for (uint32_t k = threadIdx.x; k < count; k += blockDim.x) acc += v[2 * k];
-  s_tmp[threadIdx.x] = acc;
-  __syncthreads();
-  for (uint32_t w = blockDim.x / 2; w > 0; w >>= 1) {
-    if (threadIdx.x < w) s_tmp[threadIdx.x] += s_tmp[threadIdx.x + w];
-    __syncthreads();
-  }
-  const float total = s_tmp[0];
-  __syncthreads();
-  return total;
-}
 
 // Decay of the weights' moving average that renders sample from: the last
 // steps of a frame are noisy (lr 1e-2 on one frame's samples), and the
 // average over about 100 steps is the steadier guide.
 constexpr float kEmaDecay = 0.99f;
 
-__global__ void __launch_bounds__(256) guide_adam_kernel(AdamArgs aa) {
-  __shared__ float s_tmp[256];
-  const float wsum = block_sum(aa.tile_part, aa.tiles, s_tmp);
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= kGuideParams) return;
-  const ParamSlot sl = param_slot(p);
+// One block per 64 elements of a gradient tile (elements that are no
+// parameter's are skipped at the end): its 16 waves sum every 16th partial
+// each, so that up to 256 partials (29 MB) are read with 16 loads in flight
+// per wave; 7.7 us, 16.5 with one thread per parameter over 32 partials.
+constexpr int kAdamWaves = 16;
+
+__global__ void __launch_bounds__(kAdamWaves * 64) guide_adam_kernel(AdamArgs aa) {
+  __shared__ float s_sum[kAdamWaves][64];
+  const uint32_t lane = lane_id(), wave = threadIdx.x >> 6;
+  const uint32_t at = blockIdx.x * 64 + lane;  // tile * 256 + element
+  float acc = 0.0f;
+#pragma unroll 16
+  for (uint32_t b = wave; b < aa.blocks; b += kAdamWaves) acc += aa.part[(uint64_t)b * (kTiles * 256) + at];
+  s_sum[wave][lane] = acc;
+  __syncthreads();
+  if (wave) return;
+  double weights = 0.0;
+  for (uint32_t b = lane; b < aa.blocks; b += 64) weights += aa.loss_part[2 * b];
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) weights += __shfl_xor(weights, off, 64);
+  const float wsum = (float)weights;
+  const int p = slot_param((int)(at >> 8), (int)(at & 255u));
+  if (p < 0) return;
   float gsum = 0.0f;
-  for (uint32_t c = 0; c < aa.chunks; ++c) gsum += aa.part[((uint64_t)c * kTiles + sl.tile) * 256 + sl.elem];
+#pragma unroll
+  for (int w = 0; w < kAdamWaves; ++w) gsum += s_sum[w][lane];
+  const ParamSlot sl = param_slot(p);
   const float grad = wsum > 0.0f ? gsum / wsum : 0.0f;
   if (aa.grad_out) {
     aa.grad_out[p] = grad;
@@ -633,9 +833,7 @@ void free_guide(bajo_guide* g) {
   if (!g) return;
   (void)hipFree(g->params); (void)hipFree(g->adam_m); (void)hipFree(g->adam_v); (void)hipFree(g->pack);
   (void)hipFree(g->ema); (void)hipFree(g->infer_pack);
-  (void)hipFree(g->x0t); (void)hipFree(g->h1t); (void)hipFree(g->h2t); (void)hipFree(g->h3t);
-  (void)hipFree(g->d1t); (void)hipFree(g->d2t); (void)hipFree(g->d3t); (void)hipFree(g->dot);
-  (void)hipFree(g->tile_part); (void)hipFree(g->grad_part);
+  (void)hipFree(g->loss_part); (void)hipFree(g->grad_part);
   (void)hipFree(g->records); (void)hipFree(g->contrib); (void)hipFree(g->samples); (void)hipFree(g->sample_count);
   (void)hipFree(g->block_counts);
   (void)hipFree(g->vertices); (void)hipFree(g->outputs);
@@ -647,35 +845,42 @@ int32_t blocks_per_cu(K kernel, int* out) {
   int dev = 0, cus = 0, per_cu = 0;
   BJ_HIP(hipGetDevice(&dev));
   BJ_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  BJ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 256, 0));
+  BJ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kForwardBlock, 0));
   *out = cus * (per_cu < 1 ? 1 : per_cu);
   return BAJO_OK;
 }
 
-// Forward + backward + weight-gradient partials of one batch (n <= batch_cap).
+// Blocks of one training pass over n samples.
+uint32_t train_blocks(uint64_t n) {
+  const uint64_t need = (n + kTrainSamples - 1) / kTrainSamples;
+  return (uint32_t)(need < kTrainBlocks ? need : kTrainBlocks);
+}
+
+// Weight-gradient and loss partials of one batch (n <= batch_cap), one per block.
 int32_t run_backward(hipStream_t stream, bajo_guide* g, const float* samples, uint64_t src_count, uint64_t src_offset,
-                     uint64_t src_stride, uint64_t n, uint64_t* ldb_out, uint32_t* chunks_out) {
-  const uint64_t ldb = (n + kChunk - 1) / kChunk * kChunk;  // padded batch
-  const uint32_t chunks = (uint32_t)(ldb / kChunk);
-  TrainArgs ta{samples, src_count, src_offset, src_stride, n, ldb, g->batch_cap, g->x0t, g->h1t, g->h2t, g->h3t,
-               g->d1t, g->d2t, g->d3t, g->dot, g->tile_part};
-  const uint64_t tiles = ldb / 16;
-  int grid = 0;
-  int32_t rc = blocks_per_cu(guide_train_kernel, &grid);
-  if (rc) return rc;
-  const uint64_t need = (tiles + 3) / 4;
-  if ((uint64_t)grid > need) grid = (int)need;
-  guide_train_kernel<<<grid, 256, 0, stream>>>(g->pack, ta);
+                     uint64_t src_stride, uint64_t n, uint32_t* blocks) {
+  *blocks = train_blocks(n);
+  TrainArgs ta{samples, src_count, src_offset, src_stride, n, g->grad_part, g->loss_part};
+  guide_train_kernel<<<*blocks, kTrainWaves * 64, 0, stream>>>(g->pack, ta);
   BJ_HIP(hipGetLastError());
-  WgradArgs wa{g->x0t, g->h1t, g->h2t, g->h3t, g->d1t, g->d2t, g->d3t, g->dot, g->batch_cap, g->grad_part};
-  guide_wgrad_kernel<<<dim3(kTiles, chunks), 64, 0, stream>>>(wa);
-  BJ_HIP(hipGetLastError());
-  *ldb_out = ldb;
-  *chunks_out = chunks;
   return BAJO_OK;
 }
 
-int32_t run_adam(hipStream_t stream, bajo_guide* g, uint64_t ldb, uint32_t chunks, float* grad_out) {
+// The batch's mean loss from its partials (synchronizes).
+int32_t read_loss(hipStream_t stream, const bajo_guide* g, uint32_t blocks, float* loss) {
+  double part[2 * kTrainBlocks];
+  BJ_HIP(hipMemcpyAsync(part, g->loss_part, 2 * blocks * sizeof(double), hipMemcpyDeviceToHost, stream));
+  BJ_HIP(hipStreamSynchronize(stream));
+  double ws = 0.0, ls = 0.0;
+  for (uint32_t k = 0; k < blocks; ++k) {
+    ws += part[2 * k];
+    ls += part[2 * k + 1];
+  }
+  *loss = ws > 0.0 ? (float)(ls / ws) : 0.0f;
+  return BAJO_OK;
+}
+
+int32_t run_adam(hipStream_t stream, bajo_guide* g, uint32_t blocks, float* grad_out) {
   AdamArgs aa;
   aa.params = g->params;
   aa.m = g->adam_m;
@@ -684,9 +889,8 @@ int32_t run_adam(hipStream_t stream, bajo_guide* g, uint64_t ldb, uint32_t chunk
   aa.ema = g->ema;
   aa.infer_pack = g->infer_pack;
   aa.part = g->grad_part;
-  aa.chunks = chunks;
-  aa.tile_part = g->tile_part;
-  aa.tiles = (uint32_t)(ldb / 16);
+  aa.loss_part = g->loss_part;
+  aa.blocks = blocks;
   aa.lr = g->opt.learning_rate;
   aa.beta1 = g->opt.beta1;
   aa.beta2 = g->opt.beta2;
@@ -703,7 +907,7 @@ int32_t run_adam(hipStream_t stream, bajo_guide* g, uint64_t ldb, uint32_t chunk
   } else {
     aa.bias1 = aa.bias2 = 1.0f;
   }
-  guide_adam_kernel<<<div_up(kGuideParams, 256), 256, 0, stream>>>(aa);
+  guide_adam_kernel<<<kTiles * 4, kAdamWaves * 64, 0, stream>>>(aa);
   BJ_HIP(hipGetLastError());
   return BAJO_OK;
 }
@@ -713,11 +917,10 @@ int32_t run_adam(hipStream_t stream, bajo_guide* g, uint64_t ldb, uint32_t chunk
 int32_t guide_train_samples(hipStream_t stream, bajo_guide* g, const float* samples, uint64_t n) {
   for (uint64_t b = 0; b < n; b += g->batch_cap) {
     const uint64_t m = n - b < g->batch_cap ? n - b : g->batch_cap;
-    uint64_t ldb = 0;
-    uint32_t chunks = 0;
-    int32_t rc = run_backward(stream, g, samples, n, b, 1, m, &ldb, &chunks);
+    uint32_t blocks = 0;
+    int32_t rc = run_backward(stream, g, samples, n, b, 1, m, &blocks);
     if (rc) return rc;
-    rc = run_adam(stream, g, ldb, chunks, nullptr);
+    rc = run_adam(stream, g, blocks, nullptr);
     if (rc) return rc;
   }
   return BAJO_OK;
@@ -865,9 +1068,9 @@ int32_t guide_infer_vertices(hipStream_t stream, const bajo_guide* g, const floa
   int grid = 0;
   int32_t rc = blocks_per_cu(guide_forward_kernel<VertexRows>, &grid);
   if (rc) return rc;
-  const uint64_t need = (cap + 63) / 64;
+  const uint64_t need = (cap + 31) / 32;
   if ((uint64_t)grid > need) grid = (int)need;
-  guide_forward_kernel<VertexRows><<<grid, 256, 0, stream>>>(g->infer_pack, VertexRows{vertex_fields, scene_bounds},
+  guide_forward_kernel<VertexRows><<<grid, kForwardBlock, 0, stream>>>(g->infer_pack, VertexRows{vertex_fields, scene_bounds},
                                                              count_dev, cap, outputs);
   BJ_HIP(hipGetLastError());
   return BAJO_OK;
@@ -941,26 +1144,16 @@ int32_t guide_train_collected(hipStream_t stream, bajo_guide* g, uint64_t* sampl
   uint64_t stride = total / n;
   if (stride < 1) stride = 1;
   while (gcd_u64(stride, total) != 1) ++stride;
-  uint64_t ldb = 0;
+  uint32_t blocks = 0;
   for (uint32_t k = 0; k < g->opt.steps_per_frame; ++k) {
-    uint32_t chunks = 0;
     const uint64_t offset = g->sample_cursor++ % total;
-    int32_t rc = run_backward(stream, g, g->samples, total, offset, stride, n, &ldb, &chunks);
+    int32_t rc = run_backward(stream, g, g->samples, total, offset, stride, n, &blocks);
     if (rc) return rc;
-    rc = run_adam(stream, g, ldb, chunks, nullptr);
+    rc = run_adam(stream, g, blocks, nullptr);
     if (rc) return rc;
     *steps_out += 1;
   }
-  std::vector<float> part(ldb / 16 * 2);
-  BJ_HIP(hipMemcpyAsync(part.data(), g->tile_part, part.size() * sizeof(float), hipMemcpyDeviceToHost, stream));
-  BJ_HIP(hipStreamSynchronize(stream));
-  double ws = 0.0, ls = 0.0;
-  for (size_t i = 0; i < part.size(); i += 2) {
-    ws += part[i];
-    ls += part[i + 1];
-  }
-  *loss_out = ws > 0.0 ? (float)(ls / ws) : 0.0f;
-  return BAJO_OK;
+  return read_loss(stream, g, blocks, loss_out);
 }
 
 }  // namespace bj
@@ -984,8 +1177,8 @@ int32_t bajo_guide_create(bajo_ctx* ctx, const bajo_guide_options* options, bajo
   bajo_guide* g = new bajo_guide();
   g->device = ctx->device;
   g->opt = o;
-  g->batch_cap = (o.batch_size + bj::kChunk - 1) / bj::kChunk * bj::kChunk;
-  const uint64_t cap = g->batch_cap;
+  g->batch_cap = (o.batch_size + 2047) / 2048 * 2048;
+  const uint32_t blocks = bj::train_blocks(g->batch_cap);
   auto fail = [&](hipError_t e, const char* what) {
     bj::free_guide(g);
     return bj::hip_fail(e, what, __FILE__, __LINE__);
@@ -997,16 +1190,8 @@ int32_t bajo_guide_create(bajo_ctx* ctx, const bajo_guide_options* options, bajo
   if (e == hipSuccess) e = hipMalloc(&g->pack, bj::kPackBytes);
   if (e == hipSuccess) e = hipMalloc(&g->ema, bj::kGuideParams * sizeof(float));
   if (e == hipSuccess) e = hipMalloc(&g->infer_pack, bj::kPackBytes);
-  if (e == hipSuccess) e = hipMalloc(&g->x0t, (size_t)bj::kX0Rows * cap * 2);
-  if (e == hipSuccess) e = hipMalloc(&g->h1t, (size_t)bj::kHRows * cap * 2);
-  if (e == hipSuccess) e = hipMalloc(&g->h2t, (size_t)bj::kHRows * cap * 2);
-  if (e == hipSuccess) e = hipMalloc(&g->h3t, (size_t)bj::kHRows * cap * 2);
-  if (e == hipSuccess) e = hipMalloc(&g->d1t, (size_t)bj::kDRows * cap * 2);
-  if (e == hipSuccess) e = hipMalloc(&g->d2t, (size_t)bj::kDRows * cap * 2);
-  if (e == hipSuccess) e = hipMalloc(&g->d3t, (size_t)bj::kDRows * cap * 2);
-  if (e == hipSuccess) e = hipMalloc(&g->dot, (size_t)bj::kDoRows * cap * 2);
-  if (e == hipSuccess) e = hipMalloc(&g->tile_part, (size_t)(cap / 16) * 2 * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&g->grad_part, (size_t)(cap / bj::kChunk) * bj::kTiles * 256 * sizeof(float));
+  if (e == hipSuccess) e = hipMalloc(&g->loss_part, (size_t)blocks * 2 * sizeof(double));
+  if (e == hipSuccess) e = hipMalloc(&g->grad_part, (size_t)blocks * bj::kTiles * 256 * sizeof(float));
   if (e == hipSuccess) e = hipMalloc(&g->sample_count, 4 * sizeof(uint32_t));
   if (e != hipSuccess) return fail(e, "hipMalloc(guide)");
   // padding entries of the weight image stay zero
@@ -1059,9 +1244,9 @@ int32_t bajo_guide_forward(bajo_ctx* ctx, const bajo_guide* guide, const float* 
   int grid = 0;
   int32_t rc = bj::blocks_per_cu(bj::guide_forward_kernel<bj::InputRows>, &grid);
   if (rc) return rc;
-  const uint64_t need = (n + 63) / 64;
+  const uint64_t need = (n + 31) / 32;
   if ((uint64_t)grid > need) grid = (int)need;
-  bj::guide_forward_kernel<bj::InputRows><<<grid, 256, 0, ctx->stream>>>(guide->pack, bj::InputRows{inputs}, nullptr,
+  bj::guide_forward_kernel<bj::InputRows><<<grid, bj::kForwardBlock, 0, ctx->stream>>>(guide->pack, bj::InputRows{inputs}, nullptr,
                                                                          n, outputs);
   BJ_HIP(hipGetLastError());
   return BAJO_OK;
@@ -1073,25 +1258,12 @@ int32_t bajo_guide_gradient(bajo_ctx* ctx, bajo_guide* guide, const float* sampl
   BJ_REQUIRE(n > 0 && samples, "bajo_guide_gradient: empty batch");
   BJ_REQUIRE(n <= guide->batch_cap, "bajo_guide_gradient: %llu samples exceed the batch size %u",
              (unsigned long long)n, guide->batch_cap);
-  uint64_t ldb = 0;
-  uint32_t chunks = 0;
-  int32_t rc = bj::run_backward(ctx->stream, guide, samples, n, 0, 1, n, &ldb, &chunks);
+  uint32_t blocks = 0;
+  int32_t rc = bj::run_backward(ctx->stream, guide, samples, n, 0, 1, n, &blocks);
   if (rc) return rc;
-  rc = bj::run_adam(ctx->stream, guide, ldb, chunks, gradient);
+  rc = bj::run_adam(ctx->stream, guide, blocks, gradient);
   if (rc) return rc;
-  if (loss) {
-    std::vector<float> part(ldb / 16 * 2);
-    BJ_HIP(hipMemcpyAsync(part.data(), guide->tile_part, part.size() * sizeof(float), hipMemcpyDeviceToHost,
-                          ctx->stream));
-    BJ_HIP(hipStreamSynchronize(ctx->stream));
-    double ws = 0.0, ls = 0.0;
-    for (size_t k = 0; k < part.size(); k += 2) {
-      ws += part[k];
-      ls += part[k + 1];
-    }
-    *loss = ws > 0.0 ? (float)(ls / ws) : 0.0f;
-  }
-  return BAJO_OK;
+  return loss ? bj::read_loss(ctx->stream, guide, blocks, loss) : BAJO_OK;
 }
 
 int32_t bajo_guide_train(bajo_ctx* ctx, bajo_guide* guide, const float* samples, uint64_t n) {

@@ -14,18 +14,10 @@ struct bajo_guide {
   uint8_t* pack = nullptr;       // bf16 weight images (forward + transposed) and f32 biases
   float* ema = nullptr;          // exponential moving average of the weights (what renders sample from)
   uint8_t* infer_pack = nullptr; // the same images of `ema`
-  // training batch buffers (bf16, batch-contiguous rows), for `batch_cap` samples
+  // training partials of a batch of at most `batch_cap` samples, per block
   uint32_t batch_cap = 0;
-  uint16_t* x0t = nullptr;       // [224][batch_cap] encoded inputs, row 216 = 1
-  uint16_t* h1t = nullptr;       // [80][batch_cap] hidden activations, row 64 = 1
-  uint16_t* h2t = nullptr;
-  uint16_t* h3t = nullptr;
-  uint16_t* d1t = nullptr;       // [64][batch_cap] loss gradients of the hidden layers
-  uint16_t* d2t = nullptr;
-  uint16_t* d3t = nullptr;
-  uint16_t* dot = nullptr;       // [48][batch_cap] loss gradients of the outputs
-  float* tile_part = nullptr;    // per 16-sample tile: sum of weights, weighted loss
-  float* grad_part = nullptr;    // per batch chunk and gradient tile: 16 x 16 partial sums
+  double* loss_part = nullptr;   // sum of weights, weighted loss
+  float* grad_part = nullptr;    // per gradient tile: 16 x 16 partial sums
   // rendering: training records of one frame and the samples made from them
   uint64_t record_cap = 0;       // path-bounce slots
   float* records = nullptr;      // kRecordPlanes floats per slot

@@ -71,21 +71,18 @@ BJ_HD float exp_f(float x) {
 // ln x for x > 0 (log2_pos times ln 2).
 BJ_HD float ln_f(float x) { return log2_pos(x) * 0.693147180559945309417f; }
 
-// Encoded pair (sin, cos)(pi 2^f x) of one input value: the argument in
-// turns, x 2^(f-1), is reduced to its fraction first (exact scaling).
-BJ_HD void guide_encode_pair(float x, int f, float& s, float& c) {
-  const float y = x * __builtin_bit_cast(float, (uint32_t)(f - 1 + 127) << 23);
-  const float u = y - floorf(y);
-  sincos_turns(u, s, c);
-}
+// Scale from an input to turns at frequency f: pi 2^f x radians = 2^(f - 1) x turns.
+BJ_HD float guide_freq_scale(int f) { return __builtin_bit_cast(float, (uint32_t)(f - 1 + 127) << 23); }
 
-// The four pairs of frequencies 4 b .. 4 b + 3: the first from the series,
-// the next three by the double-angle formulas sin 2a = 2 sin a cos a,
-// cos 2a = (cos a - sin a)(cos a + sin a), in this order of FP32 operations
-// (each doubling at most doubles the first pair's error, well below the
-// BF16 features' precision).
-BJ_HD void guide_encode_group(float x, int b, float (&s)[4], float (&c)[4]) {
-  guide_encode_pair(x, 4 * b, s[0], c[0]);
+// The four (sin, cos) pairs from the frequency of `scale` on: the first from
+// the series (the argument in turns reduced to its fraction first, exact
+// scaling), the next three by the double-angle formulas
+// sin 2a = 2 sin a cos a, cos 2a = (cos a - sin a)(cos a + sin a), in this
+// order of FP32 operations (each doubling at most doubles the first pair's
+// error, well below the BF16 features' precision).
+BJ_HD void guide_encode_scaled(float x, float scale, float (&s)[4], float (&c)[4]) {
+  const float y = x * scale;
+  sincos_turns(y - floorf(y), s[0], c[0]);
 #pragma unroll
   for (int t = 1; t < 4; ++t) {
     s[t] = 2.0f * s[t - 1] * c[t - 1];

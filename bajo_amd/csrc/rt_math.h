@@ -94,13 +94,12 @@ BJ_HD void sincos_turns(float u, float& s, float& c) {
   pc = fmaf(x2, pc, 4.16666666666666666667e-2f);
   pc = fmaf(x2, pc, -0.5f);
   const float cs = fmaf(x2, pc, 1.0f);
-  const int quadrant = ((int)q) & 3;
-  switch (quadrant) {
-    case 0: s = sn; c = cs; break;
-    case 1: s = cs; c = -sn; break;
-    case 2: s = -sn; c = -cs; break;
-    default: s = -cs; c = sn; break;
-  }
+  // quadrant 0: (sn, cs), 1: (cs, -sn), 2: (-sn, -cs), 3: (-cs, sn), by
+  // selects and sign bits (a switch becomes divergent branches)
+  const uint32_t quadrant = (uint32_t)(int)q;
+  const bool odd = (quadrant & 1u) != 0u;
+  s = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, odd ? cs : sn) ^ ((quadrant & 2u) << 30));
+  c = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, odd ? sn : cs) ^ (((quadrant + 1u) & 2u) << 30));
 }
 
 // ---- small helpers of bajo's renderer -----------------------------------------

@@ -125,3 +125,52 @@ def test_mixture_sampler_bit_exact(gpu_ctx):
         d, pdf = oracle.guide_mixture_sample(outs[r], u[r])
         assert np.array_equal(dirs[r].view(np.uint32), d.view(np.uint32)), r
         assert np.float32(pdf).view(np.uint32) == pdfs[r].view(np.uint32), r
+
+
+@pytest.mark.parametrize("n", [1, 15, 17, 31, 33, 255, 257, 8192 + 31])
+def test_sample_tile_edges(gpu_ctx, n):
+    """Partial wave (32) and block (256) tiles of the forward and training kernels against the oracle; the outputs
+    start one float into their buffer (no 16-byte alignment) and nothing around them is written."""
+    from bajo_amd import _lib
+
+    announce(f"guide tiles n={n}")
+    rng = np.random.default_rng(n)
+    p = random_params(rng).astype(np.float32)
+    s = random_samples(n, rng)
+    g = make_guide(gpu_ctx, batch_size=16384)
+    g.set_params(p)
+    buf = torch.full((n * 40 + 41,), 7.0, device="cuda")
+    out = buf[1:1 + n * 40].view(n, 40)
+    x = torch.from_numpy(s[:, :9].copy()).cuda()
+    _lib.check(_lib.lib().bajo_guide_forward(gpu_ctx.handle, g._handle, x.data_ptr(), n, out.data_ptr()))
+    torch.cuda.synchronize()
+    assert float(buf[0]) == 7.0 and bool((buf[1 + n * 40:] == 7.0).all())
+    want = oracle.guide_forward(p.astype(np.float64), s[:, :9].copy(), emulate_bf16=True)
+    np.testing.assert_allclose(out.cpu().numpy(), want, rtol=2e-2, atol=5e-3)
+    grad, loss = g.gradient(torch.from_numpy(s).cuda())
+    got = grad.cpu().numpy().astype(np.float64)
+    want_loss, want = oracle.guide_loss_grad(p.astype(np.float64), s, emulate_bf16=True)
+    assert abs(loss - want_loss) < 1e-3 * abs(want_loss) + 1e-5
+    # a few BF16 roundings per sample fall the other way: 2^-8 of the gradient, more where one sample is all of it
+    assert np.linalg.norm(got - want) <= (1e-2 if n > 64 else 2e-2) * np.linalg.norm(want)
+    g.free()
+
+
+def test_gradient_of_a_batch_in_several_passes(gpu_ctx):
+    """Above 65,536 samples the blocks loop: the gradient is the weighted mean of its halves' (each one pass), in
+    FP32 sums of the same BF16 products (2^-24 times the square root of their number, with room)."""
+    announce("guide gradient in two passes")
+    rng = np.random.default_rng(3)
+    n, m = 66_000, 33_000
+    g = make_guide(gpu_ctx, batch_size=n // 32 * 32 + 32)
+    g.set_params(random_params(rng).astype(np.float32))
+    s = random_samples(n, rng)
+    parts = []
+    for rows in (s, s[:m], s[m:]):
+        grad, loss = g.gradient(torch.from_numpy(rows.copy()).cuda())
+        parts.append((grad.cpu().numpy().astype(np.float64), loss, rows[:, 12].sum(dtype=np.float64)))
+    (whole, loss, w), (ga, la, wa), (gb, lb, wb) = parts
+    want = (ga * wa + gb * wb) / w
+    assert np.linalg.norm(whole - want) < 1e-5 * np.linalg.norm(want)
+    assert abs(loss - (la * wa + lb * wb) / w) < 1e-6 * abs(loss)
+    g.free()
