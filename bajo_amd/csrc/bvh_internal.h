@@ -79,7 +79,6 @@ struct bajo_bvh {
   BjNode* hp_guide;       // n-1 guide nodes (Karras over the sorted keys)
   uint32_t* hp_first;     // n-1 first sorted position of each guide node
   void* hp_clusters;      // n cluster entries of 32 bytes
-  uint32_t* hp_counts;    // n-1 cluster list lengths
   uint32_t* hp_pos;       // n depth-first leaf positions
   uint32_t* hp_ctl;       // node counter, status, root
   uint32_t* host_hp_ctl;  // pinned host mirror of hp_ctl

@@ -14,16 +14,22 @@
 //
 // MI355X design:
 //   - one thread per sorted leaf climbs the guide hierarchy; arrival is a
-//     relaxed agent-scope counter per guide node, and every datum handed to
-//     another wave (cluster lists, their counts, output nodes) is written
+//     relaxed agent-scope word per guide node, which hands the length of the
+//     first arrival's list to the second, and every datum handed to
+//     another wave (the cluster lists) is written
 //     with write-through stores and read with coherent loads, so no L2
 //     writeback or invalidate is needed across the 8 XCDs;
 //   - a guide node that needs merging is processed by its whole wave: up to
-//     2 x threshold (64) clusters sit one per lane, neighbour boxes move by lane shuffles,
-//     mutual pairs are found with one ballot, a new node takes the index
-//     (retired leaf position - 1) of the larger lowest leaf position of its
-//     two clusters (no shared counter), and the list is compacted with a
-//     forward lane permute (ds_permute);
+//     2 x threshold (64) clusters sit one per lane, neighbour boxes move by
+//     the vector unit's wave shifts and each merged area is computed once for
+//     its two clusters, mutual pairs are found with one ballot, a new node
+//     takes the index (retired leaf position - 1) of the larger lowest leaf
+//     position of its two clusters (no shared counter), and the list is
+//     compacted with a forward lane permute (ds_permute).  Bound by the
+//     chains of upper nodes (arrival, list load, rounds, publication) and by
+//     the rounds' instructions: 1M triangles 751 -> 372 us (lane shuffles for
+//     every neighbour 751, wave shifts 493, one area per pair and list
+//     lengths in the arrival words 372; 64 registers for 8 waves: 505);
 //   - a segmented build (a BLAS set) runs every segment's H-PLOC in the same
 //     launch: the guide is the per-segment Karras forest, a guide node whose
 //     parent is the sentinel is its segment's root (merged down to one
@@ -116,6 +122,19 @@ BJ_D float merged_area(const HpEntry& a, const float* o) {
   return 2.0f * (dx * dy + dx * dz + dy * dz);
 }
 
+// Minimum and maximum of values that are not NaN, one instruction each.
+BJ_D float min_ordered(float a, float b) {
+  float r;
+  asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+BJ_D float max_ordered(float a, float b) {
+  float r;
+  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
+BJ_D uint32_t read_lane(uint32_t v, int src) { return (uint32_t)__builtin_amdgcn_readlane((int)v, src); }
 BJ_D uint32_t shfl_u(uint32_t v, int src) { return (uint32_t)__shfl((int)v, src, 64); }
 
 // Segment of sorted position i (off: u64[S + 1]), by binary search.
@@ -136,62 +155,122 @@ BJ_D float permute_f(uint32_t dst_lane, float v) {
   return __builtin_bit_cast(float, permute_u(dst_lane, __builtin_bit_cast(uint32_t, v)));
 }
 
-// Writes output node `idx` = (a, b) with write-through stores; sets the
-// children's parent links (inner children; leaves keep theirs in the
-// per-position parent array).
+// Writes output node `idx` = (a, b) and its children's parent links (inner
+// children; leaves keep theirs in the per-position parent array).  Plain
+// stores: only later launches read them.
 BJ_D void write_node(BjNode* __restrict__ nodes, uint32_t* __restrict__ leaf_counts,
                      uint32_t* __restrict__ leaf_parent, uint32_t idx, const HpEntry& a, const HpEntry& b) {
   BjNode* nd = nodes + idx;
-  for (int k = 0; k < 3; ++k) {
-    store_wt(&nd->b[k], a.lo[k]);
-    store_wt(&nd->b[3 + k], a.hi[k]);
-    store_wt(&nd->b[6 + k], b.lo[k]);
-    store_wt(&nd->b[9 + k], b.hi[k]);
-  }
-  store_wt(&nd->left, a.ref);
-  store_wt(&nd->right, b.ref);
-  store_wt(leaf_counts + idx, a.cnt + b.cnt);
-  if (a.ref & kLeafFlag) store_wt(leaf_parent + (a.ref & kIndexMask), idx);
-  else store_wt(&nodes[a.ref].parent, idx);
-  if (b.ref & kLeafFlag) store_wt(leaf_parent + (b.ref & kIndexMask), idx);
-  else store_wt(&nodes[b.ref].parent, idx);
+  float4* box = reinterpret_cast<float4*>(nd);
+  box[0] = make_float4(a.lo[0], a.lo[1], a.lo[2], a.hi[0]);
+  box[1] = make_float4(a.hi[1], a.hi[2], b.lo[0], b.lo[1]);
+  box[2] = make_float4(b.lo[2], b.hi[0], b.hi[1], b.hi[2]);
+  nd->left = a.ref;
+  nd->right = b.ref;
+  leaf_counts[idx] = a.cnt + b.cnt;
+  if (a.ref & kLeafFlag) leaf_parent[a.ref & kIndexMask] = idx;
+  else nodes[a.ref].parent = idx;
+  if (b.ref & kLeafFlag) leaf_parent[b.ref & kIndexMask] = idx;
+  else nodes[b.ref].parent = idx;
 }
 
-// The wave processes guide node `g` (all 64 lanes call this together).
-BJ_D void process_node(uint32_t g, uint64_t n, const BjNode* __restrict__ guide,
-                       const uint32_t* __restrict__ range_first, HpEntry* __restrict__ clusters,
-                       uint32_t* __restrict__ ids, uint32_t* __restrict__ counts, BjNode* __restrict__ nodes, uint32_t* __restrict__ leaf_counts,
-                       uint32_t* __restrict__ leaf_parent, uint32_t* __restrict__ ctl,
+// The value of the next lane, by the vector unit's wave shift; the last lane's is 0.
+BJ_D float next_lane(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x130, 0xF, 0xF, true));
+}
+
+BJ_D bool has_nan(const HpEntry& e) {
+  bool nan = false;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) nan = nan || e.lo[k] != e.lo[k] || e.hi[k] != e.hi[k];
+  return nan;
+}
+
+// The cluster within the radius whose merged box with lane's has the least
+// area, among c clusters one per lane (right before left, nearer first,
+// strict '<'), or -1.
+BJ_D int nearest_any(const HpEntry& e, uint32_t c, uint32_t lane) {
+  float best_area = kFltMax;
+  int best = -1;
+#pragma unroll 1
+  for (int r = 1; r <= kHpRadius; ++r) {
+#pragma unroll 1
+    for (int side = 0; side < 2; ++side) {
+      const int o = (int)lane + (side ? -r : r);
+      float box[6];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        box[k] = shfl_f(e.lo[k], o & 63);
+        box[3 + k] = shfl_f(e.hi[k], o & 63);
+      }
+      const float area = merged_area(e, box);
+      if (lane < c && o >= 0 && o < (int)c && area < best_area) {
+        best_area = area;
+        best = o;
+      }
+    }
+  }
+  return best;
+}
+
+// The same of boxes without NaN: their merged box is the same from either
+// side, so a lane computes its right neighbours' areas, by plain minima and
+// maxima of boxes that move by the vector unit's wave shifts, and takes its
+// left neighbours' areas from them.
+BJ_D int nearest_ordered(const HpEntry& e, uint32_t c, uint32_t lane) {
+  float best_area = kFltMax;
+  int best = -1;
+  float o[6] = {e.lo[0], e.lo[1], e.lo[2], e.hi[0], e.hi[1], e.hi[2]};
+#pragma unroll
+  for (int r = 1; r <= kHpRadius; ++r) {
+    const int rs = (int)lane + r, ls = (int)lane - r;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) o[k] = next_lane(o[k]);
+    const float dx = max_ordered(e.hi[0], o[3]) - min_ordered(e.lo[0], o[0]);
+    const float dy = max_ordered(e.hi[1], o[4]) - min_ordered(e.lo[1], o[1]);
+    const float dz = max_ordered(e.hi[2], o[5]) - min_ordered(e.lo[2], o[2]);
+    const float to_right = rs < (int)c ? 2.0f * (dx * dy + dx * dz + dy * dz) : kFltMax;
+    // a lane without a left neighbour reads one without a right neighbour
+    const float to_left = shfl_f(to_right, ls & 63);
+    if (to_right < best_area) {
+      best_area = to_right;
+      best = rs;
+    }
+    if (to_left < best_area) {
+      best_area = to_left;
+      best = ls;
+    }
+  }
+  return best;
+}
+
+// A guide node's topology and the lengths of its two lists (0: not a list).
+struct GuideNode {
+  uint32_t first, split, last, cl, cr;
+  bool root;  // of the hierarchy or the segment: no parent in the guide
+};
+
+BJ_D bool lists_ok(const GuideNode& t, uint64_t n, uint32_t threshold) {
+  return t.cl >= 1 && t.cr >= 1 && t.cl <= threshold && t.cr <= threshold && t.first <= t.split && t.split < t.last &&
+         (uint64_t)t.last < n && t.cl <= t.split - t.first + 1 && t.cr <= t.last - t.split;
+}
+
+// The wave processes a guide node (all 64 lanes call this together with the
+// same node).  Returns the length of its list, 0 after a failure.
+BJ_D uint32_t process_node(const GuideNode& t, uint64_t n, HpEntry* __restrict__ clusters,
+                       uint32_t* __restrict__ ids, BjNode* __restrict__ nodes,
+                       uint32_t* __restrict__ leaf_counts, uint32_t* __restrict__ leaf_parent, uint32_t* __restrict__ ctl,
                        const uint64_t* __restrict__ seg_off, uint32_t S, uint32_t* __restrict__ seg_roots,
                        uint32_t threshold) {
   const uint32_t lane = lane_id();
-  const uint32_t first = range_first[g], last = guide[g].fence;
-  const uint32_t gl = guide[g].left, gr = guide[g].right;
-  const uint32_t split = gl & kIndexMask;
-  const uint32_t cl = (gl & kLeafFlag) ? 1u : load_co(counts + split);
-  const uint32_t cr = (gr & kLeafFlag) ? 1u : load_co(counts + (gr & kIndexMask));
+  const uint32_t first = t.first, split = t.split, cl = t.cl, cr = t.cr;
+  const bool root = t.root;
   uint32_t c = cl + cr;
-  if (cl > threshold || cr > threshold || cl == 0 || cr == 0 || first > split || split >= last ||
-      (uint64_t)last >= n || cl > split - first + 1 || cr > last - split) {
+  if (!lists_ok(t, n, threshold)) {
     if (lane == 0) atomicOr(ctl + kHpStatus, kHpStatusBadList);
-    return;
+    return 0u;
   }
-  // the hierarchy's (or the segment's) root: no parent in the guide
-  const bool root = guide[g].parent == kSentinel;
   const uint32_t thr = root ? 1u : threshold;
-  if (c <= thr) {
-    // no merging: the list is the left list (already at `first`) followed by
-    // the right list, which moves only if the left one is shorter than its range
-    if (split + 1 != first + cl && lane < cr) {
-      const HpEntry m = load_entry(clusters + split + 1 + lane);
-      const uint32_t mid = load_co(ids + split + 1 + lane);
-      store_entry(clusters + first + cl + lane, m);
-      store_wt(ids + first + cl + lane, mid);
-    }
-    if (lane == 0) store_wt(counts + g, c);
-    publish_fence();
-    return;
-  }
   HpEntry e{};
   uint32_t id = 0;
   if (lane < cl) {
@@ -203,35 +282,7 @@ BJ_D void process_node(uint32_t g, uint64_t n, const BjNode* __restrict__ guide,
   }
   for (int round = 0; c > thr && round < 64; ++round) {
     const bool live = lane < c;
-    float best_area = kFltMax;
-    int best = -1;
-    for (int r = 1; r <= kHpRadius; ++r) {
-      float o[6];
-      const int rs = (int)lane + r;  // right neighbour
-      for (int k = 0; k < 3; ++k) {
-        o[k] = shfl_f(e.lo[k], rs & 63);
-        o[3 + k] = shfl_f(e.hi[k], rs & 63);
-      }
-      if (live && rs < (int)c) {
-        const float a = merged_area(e, o);
-        if (a < best_area) {
-          best_area = a;
-          best = rs;
-        }
-      }
-      const int ls = (int)lane - r;  // left neighbour
-      for (int k = 0; k < 3; ++k) {
-        o[k] = shfl_f(e.lo[k], ls & 63);
-        o[3 + k] = shfl_f(e.hi[k], ls & 63);
-      }
-      if (live && ls >= 0) {
-        const float a = merged_area(e, o);
-        if (a < best_area) {
-          best_area = a;
-          best = ls;
-        }
-      }
-    }
+    int best = ballot(live && has_nan(e)) == 0 ? nearest_ordered(e, c, lane) : nearest_any(e, c, lane);
     const int nb_best = (int)shfl_u((uint32_t)best, best < 0 ? (int)lane : best);
     bool mutual = live && best >= 0 && nb_best == (int)lane;
     uint64_t mergers = ballot(mutual && (int)lane < best);
@@ -289,20 +340,18 @@ BJ_D void process_node(uint32_t g, uint64_t n, const BjNode* __restrict__ guide,
   }
   if (c > thr) {
     if (lane == 0) atomicOr(ctl + kHpStatus, kHpStatusNoProgress);
-    return;
+    return 0u;
   }
   if (lane < c) {
     store_entry(clusters + first + lane, e);
     store_wt(ids + first + lane, id);
   }
-  if (lane == 0) {
-    store_wt(counts + g, c);
-    if (root) {
-      if (seg_roots) store_wt(seg_roots + seg_of(seg_off, S, first), e.ref);
-      else store_wt(ctl + kHpRoot, e.ref);
-    }
+  if (lane == 0 && root) {
+    if (seg_roots) store_wt(seg_roots + seg_of(seg_off, S, first), e.ref);
+    else store_wt(ctl + kHpRoot, e.ref);
   }
   publish_fence();
+  return c;
 }
 
 template <bool kBoxes>
@@ -312,8 +361,7 @@ __global__ void __launch_bounds__(kHpBlock) hploc_kernel(const float* __restrict
                                                          const uint32_t* __restrict__ range_first,
                                                          uint32_t* __restrict__ leaf_parent,
                                                          uint32_t* __restrict__ flags, HpEntry* __restrict__ clusters,
-                                                         uint32_t* __restrict__ ids,
-                                                         uint32_t* __restrict__ counts, BjNode* __restrict__ nodes,
+                                                         uint32_t* __restrict__ ids, BjNode* __restrict__ nodes,
                                                          uint32_t* __restrict__ leaf_counts,
                                                          uint32_t* __restrict__ ctl,
                                                          const uint32_t* __restrict__ gprim,
@@ -338,7 +386,9 @@ __global__ void __launch_bounds__(kHpBlock) hploc_kernel(const float* __restrict
   // constant here, so a parent's are loaded together with the arrival atomic.
   uint4 topo = make_uint4(kSentinel, 0u, 0u, 0u);
   uint32_t topo_first = 0;
+  uint32_t count = 1;  // clusters in the list of `cur`
   for (int it = 0; it < kHpMaxLoop; ++it) {
+    GuideNode t{};
     if (active && !pending) {
       const uint32_t parent = (cur & kLeafFlag) ? leaf_parent[cur & kIndexMask] : topo.x;
       if (parent == kSentinel || (uint64_t)parent >= n - 1) {
@@ -346,10 +396,15 @@ __global__ void __launch_bounds__(kHpBlock) hploc_kernel(const float* __restrict
       } else {
         const uint4 ptopo = reinterpret_cast<const uint4*>(guide + parent)[3];
         const uint32_t pfirst = range_first[parent];
-        const uint32_t old = __hip_atomic_fetch_add(flags + parent, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint32_t old = __hip_atomic_fetch_add(flags + parent, (count << 1) | 1u, __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_AGENT);
         if (old == 0) {
           active = false;
         } else {
+          const bool is_left = ptopo.y == cur;
+          const uint32_t other = old >> 1;
+          t.cl = is_left ? count : other;
+          t.cr = is_left ? other : count;
           cur = parent;
           pending = true;
           topo = ptopo;
@@ -362,22 +417,17 @@ __global__ void __launch_bounds__(kHpBlock) hploc_kernel(const float* __restrict
     // merging: each lane finishes its own (appending the right list after
     // the left one) and keeps climbing.  Only merging nodes take the wave.
     if (pending) {
-      const uint32_t g = cur;
-      const uint32_t first = topo_first, last = topo.w;
-      const uint32_t gl = topo.y, gr = topo.z;
-      const uint32_t split = gl & kIndexMask;
-      const uint32_t cl = (gl & kLeafFlag) ? 1u : load_co(counts + split);
-      const uint32_t cr = (gr & kLeafFlag) ? 1u : load_co(counts + (gr & kIndexMask));
-      const bool root = topo.x == kSentinel;
-      const bool sane = cl >= 1 && cr >= 1 && cl <= threshold && cr <= threshold && first <= split &&
-                        split < last && (uint64_t)last < n && cl <= split - first + 1 && cr <= last - split;
-      if (sane && !root && cl + cr <= threshold) {
-        if (split + 1 != first + cl)
-          for (uint32_t k = 0; k < cr; ++k) {
-            store_entry(clusters + first + cl + k, load_entry(clusters + split + 1 + k));
-            store_wt(ids + first + cl + k, load_co(ids + split + 1 + k));
+      t.first = topo_first;
+      t.last = topo.w;
+      t.split = topo.y & kIndexMask;
+      t.root = topo.x == kSentinel;
+      if (!t.root && t.cl + t.cr <= threshold && lists_ok(t, n, threshold)) {
+        if (t.split + 1 != t.first + t.cl)
+          for (uint32_t k = 0; k < t.cr; ++k) {
+            store_entry(clusters + t.first + t.cl + k, load_entry(clusters + t.split + 1 + k));
+            store_wt(ids + t.first + t.cl + k, load_co(ids + t.split + 1 + k));
           }
-        store_wt(counts + g, cl + cr);
+        count = t.cl + t.cr;
         pending = false;
       }
     }
@@ -386,10 +436,12 @@ __global__ void __launch_bounds__(kHpBlock) hploc_kernel(const float* __restrict
     while (todo) {
       const int leader = __builtin_ctzll(todo);
       todo &= todo - 1;
-      const uint32_t g = shfl_u(cur, leader);
-      process_node(g, n, guide, range_first, clusters, ids, counts, nodes, leaf_counts, leaf_parent, ctl, seg_off, S,
-                   seg_roots, threshold);
+      const GuideNode w{read_lane(t.first, leader), read_lane(t.split, leader), read_lane(t.last, leader),
+                        read_lane(t.cl, leader),    read_lane(t.cr, leader),    read_lane(t.root, leader) != 0u};
+      const uint32_t left = process_node(w, n, clusters, ids, nodes, leaf_counts, leaf_parent, ctl, seg_off, S,
+                                         seg_roots, threshold);
       if ((int)lane_id() == leader) {
+        count = left;
         pending = false;
         if (topo.x == kSentinel) active = false;  // the leader's own node g
       }
@@ -578,12 +630,12 @@ int32_t build_hploc(bajo_ctx* ctx, bajo_bvh* h, const float* vertices) {
   if (h->boxes)
     hploc_kernel<true><<<div_up(n, kHpBlock), kHpBlock, 0, st>>>(vertices, h->keys, n, h->hp_guide, h->hp_first,
                                                                  h->leaf_parent, h->flags, clusters, h->hp_pos,
-                                                                 h->hp_counts, h->nodes, h->leaf_counts, h->hp_ctl,
+                                                                 h->nodes, h->leaf_counts, h->hp_ctl,
                                                                  nullptr, nullptr, 0u, nullptr, threshold);
   else
     hploc_kernel<false><<<div_up(n, kHpBlock), kHpBlock, 0, st>>>(vertices, h->keys, n, h->hp_guide, h->hp_first,
                                                                   h->leaf_parent, h->flags, clusters, h->hp_pos,
-                                                                  h->hp_counts, h->nodes, h->leaf_counts, h->hp_ctl,
+                                                                  h->nodes, h->leaf_counts, h->hp_ctl,
                                                                   nullptr, nullptr, 0u, nullptr, threshold);
   hploc_root_kernel<<<1, 64, 0, st>>>(h->nodes, n, h->leaf_counts, h->hp_ctl, ctx->status);
   BJ_HIP(hipGetLastError());
@@ -627,7 +679,7 @@ int32_t build_hploc_segmented(bajo_ctx* ctx, bajo_bvh* h, const float* vertices)
   seg_roots_init_kernel<<<div_up(S, kHpBlock), kHpBlock, 0, st>>>(seg_roots, S);
   hploc_kernel<false><<<div_up(n, kHpBlock), kHpBlock, 0, st>>>(vertices, h->keys, n, h->hp_guide, h->hp_first,
                                                                 h->leaf_parent, h->flags, clusters, h->hp_pos,
-                                                                h->hp_counts, h->nodes, h->leaf_counts, h->hp_ctl,
+                                                                h->nodes, h->leaf_counts, h->hp_ctl,
                                                                 h->seg_prim, h->seg_off, S, seg_roots, threshold);
   seg_root_fix_kernel<<<div_up(S, kHpBlock), kHpBlock, 0, st>>>(h->nodes, h->leaf_counts, h->leaf_parent, h->seg_off,
                                                                S, seg_roots, h->hp_ctl);

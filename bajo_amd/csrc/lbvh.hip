@@ -742,16 +742,16 @@ int32_t ensure_wide_capacity(bajo_bvh* h, uint64_t n) {
 }
 
 void free_hploc(bajo_bvh* h) {
-  (void)hipFree(h->hp_guide); (void)hipFree(h->hp_first); (void)hipFree(h->hp_clusters); (void)hipFree(h->hp_counts); (void)hipFree(h->hp_pos);
+  (void)hipFree(h->hp_guide); (void)hipFree(h->hp_first); (void)hipFree(h->hp_clusters); (void)hipFree(h->hp_pos);
   (void)hipFree(h->hp_ctl); (void)hipHostFree(h->host_hp_ctl);
-  h->hp_guide = nullptr; h->hp_first = nullptr; h->hp_clusters = nullptr; h->hp_counts = nullptr;
+  h->hp_guide = nullptr; h->hp_first = nullptr; h->hp_clusters = nullptr;
   h->hp_pos = nullptr; h->hp_ctl = nullptr; h->host_hp_ctl = nullptr;
   h->hp_capacity = 0;
 }
 
 // H-PLOC workspace: the guide hierarchy, range starts, 32-byte cluster
-// entries (later reused for the depth-first keys and parents), list
-// lengths and leaf positions.
+// entries (later reused for the depth-first keys and parents) and leaf
+// positions.
 int32_t ensure_hploc_capacity(bajo_bvh* h, uint64_t n) {
   if (n <= h->hp_capacity) return BAJO_OK;
   free_hploc(h);
@@ -759,7 +759,6 @@ int32_t ensure_hploc_capacity(bajo_bvh* h, uint64_t n) {
   BJ_HIP(hipMalloc(&h->hp_guide, internal * sizeof(BjNode)));
   BJ_HIP(hipMalloc(&h->hp_first, internal * sizeof(uint32_t)));
   BJ_HIP(hipMalloc(&h->hp_clusters, n * 32));
-  BJ_HIP(hipMalloc(&h->hp_counts, internal * sizeof(uint32_t)));
   BJ_HIP(hipMalloc(&h->hp_pos, n * sizeof(uint32_t)));
   BJ_HIP(hipMalloc(&h->hp_ctl, 16 * sizeof(uint32_t)));
   BJ_HIP(hipHostMalloc(&h->host_hp_ctl, 16 * sizeof(uint32_t), hipHostMallocDefault));

@@ -161,6 +161,25 @@ def test_hploc_threshold32_equals_reference(gpu_ctx, name, n):
     bvh.free()
 
 
+@pytest.mark.parametrize("threshold", [16, 32])
+@pytest.mark.parametrize("n", [33, 64, 65, 1000])
+def test_hploc_of_boxes_that_are_not_finite(gpu_ctx, n, threshold):
+    """Lists with NaN boxes compare merged boxes side by side, lists with infinite ones (areas inf and NaN) take the
+    ordered search: the layout is the oracle's in both."""
+    announce(f"hploc not finite n={n} threshold={threshold}")
+    v = soup(n, n).reshape(n, 9)
+    v[n // 5::97, 2] = np.nan   # first vertex: the box's running minimum starts from it
+    v[n // 3::89, 7] = np.nan
+    v[n // 2::31, 4] = np.inf
+    v = v.reshape(-1)
+    bvh, got, _ = device_hploc(v, merging_threshold=threshold)
+    want = oracle.build_hploc(v, merging_threshold=threshold)
+    assert got["root"] == want["root"]
+    for key in ("node_meta", "leaf_ids", "leaf_counts", "leaf_parent"):
+        np.testing.assert_array_equal(got[key], want[key], err_msg=key)
+    bvh.free()
+
+
 def test_hploc_threshold_is_validated(gpu_ctx):
     from bajo_amd.bvh import build_triangle_bvh
 
