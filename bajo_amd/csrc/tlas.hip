@@ -9,11 +9,17 @@
 //   - the top level is this library's box builder (bajo_build_binary_bounds)
 //     over the instances' world boxes, so it is the same LBVH / H-PLOC
 //     layout the parity tests already pin;
-//   - one persistent grid walks the top level near-first; at an instance
+//   - one persistent grid takes 64 rays per wave at a time from a counter and
+//     walks the top level near-first; at an instance
 //     leaf the ray is mapped into BLAS space with the inverse transform (t is
 //     unchanged) and the BLAS, binary or 8-wide, is traversed with the same
 //     code as a plain launch, its stack in LDS; the top-level stack is a
 //     per-thread column in global memory (few top-level nodes per ray);
+//   - bound by the walks' latency at few waves and by lanes waiting for each
+//     other: with one BLAS visit in the code (it stood at three places), the
+//     all-wide-triangles case compiled by itself and six waves per SIMD (the
+//     stacks' LDS allows no more) 256 instances and 691,200 rays take 354 us
+//     (697 at two waves; 440 at three, 426 at five);
 //   - instance transforms, BLAS views and instance-to-BLAS indices live in
 //     device arrays uploaded once at creation; the BLAS handles stay owned
 //     by the caller.
@@ -31,6 +37,7 @@ struct TlasBlas {
 struct bajo_tlas {
   int device = 0;
   uint32_t instance_count = 0, blas_count = 0;
+  bool plain8 = true;             // every BLAS is a wide triangle hierarchy
   bajo_bvh* top = nullptr;        // boxes hierarchy over the instance world boxes
   float* boxes = nullptr;         // f32[6 I] instance world boxes
   float* inv = nullptr;           // f32[12 I] world -> BLAS transforms
@@ -77,7 +84,9 @@ BJ_D v3 normal_from_inverse(const float* m, v3 n) {
 // the closest hit so far; a closer BLAS hit is promoted with inst = the
 // instance (bvh/tlas_common.mojo:8-30); the winning normal is transformed
 // once at the end.  Any hit: bajo's shadow hit carrying the instance.
-template <int kMode>
+// kPlain8: every BLAS is an 8- or 4-wide triangle hierarchy, and the other
+// three traversals (and the registers they hold) are left out.
+template <int kMode, bool kPlain8>
 BJ_D Hit tlas_trace(const TlasView& tv, const Ray& ray, Stack& st, uint32_t* ts, uint64_t ts_stride) {
   Hit hit = miss(ray.tmax);
   uint32_t occ_inst = kEmpty;
@@ -97,7 +106,8 @@ BJ_D Hit tlas_trace(const TlasView& tv, const Ray& ray, Stack& st, uint32_t* ts,
     lr.tmin = ray.tmin;
     lr.tmax = kMode == BAJO_TRACE_ANY_HIT ? ray.tmax : hit.t;
     Hit lh;
-    if (b.is_sphere)
+    if constexpr (kPlain8) lh = traverse8<kMode, false>(b.wide, lr, st, nullptr);
+    else if (b.is_sphere)
       lh = b.is_wide ? traverse8<kMode, false, true>(b.wide, lr, st, nullptr)
                      : traverse<kMode, false, true>(b.bin, lr, st, nullptr);
     else
@@ -116,14 +126,46 @@ BJ_D Hit tlas_trace(const TlasView& tv, const Ray& ray, Stack& st, uint32_t* ts,
       return false;
     }
   };
-  bool done = false;
+  // A lane walks the top level until it has an instance to visit, and only
+  // then do the wave's lanes enter their BLASes together: one visit in the
+  // code, and lanes still between instances do not wait for each other's.
+  bool done = false, tested = false, v0 = false, v1 = false;
+  uint32_t cur = tv.root, n_visit = 0, c0 = kSentinel, c1 = kSentinel;
+  uint32_t pend = 0;  // children 0 / 1 (bits) that are hit instances, not yet visited
+  float t0 = 0.0f, t1 = 0.0f;
+  int sp = 0;
+  const v3 rcp = rcp_dir(ray.d);
   if (tv.root & kLeafFlag) {
-    done = visit(tv.root & kIndexMask);
-  } else if (tv.root != kSentinel) {
-    const v3 rcp = rcp_dir(ray.d);
-    uint32_t cur = tv.root, n_visit = 0;
-    int sp = 0;
-    for (;;) {
+    c0 = tv.root;
+    pend = tv.root != kSentinel ? 1u : 0u;
+  }
+  for (;;) {
+    while (pend == 0u) {
+      if (tv.root & kLeafFlag) break;
+      if (tested) {  // the node's inner children: the nearer next, the other on the stack
+        int near = -1;
+        float near_t = kFltMax;
+        if (v0) { near = 0; near_t = t0; }
+        if (v1 && (near == -1 || t1 < near_t)) { near = 1; near_t = t1; }
+        const float bound = kMode == BAJO_TRACE_ANY_HIT ? ray.tmax : hit.t;
+        bool overflow = false;
+        if (v0 && near != 0 && t0 <= bound) {
+          if (sp >= kTlasStack) overflow = true; else ts[(uint64_t)(sp++) * ts_stride] = c0;
+        }
+        if (v1 && near != 1 && t1 <= bound) {
+          if (sp >= kTlasStack) overflow = true; else ts[(uint64_t)(sp++) * ts_stride] = c1;
+        }
+        if (overflow) {
+          atomicOr(tv.status, (uint32_t)BAJO_STATUS_STACK_OVERFLOW);
+          break;
+        }
+        if (near != -1 && near_t <= bound) {
+          cur = near == 0 ? c0 : c1;
+        } else {
+          if (sp == 0) break;
+          cur = ts[(uint64_t)(--sp) * ts_stride];
+        }
+      }
       if (cur >= tv.node_count || ++n_visit > tv.node_count) {
         atomicOr(tv.status, (uint32_t)BAJO_STATUS_BAD_NODE);
         break;
@@ -132,43 +174,20 @@ BJ_D Hit tlas_trace(const TlasView& tv, const Ray& ray, Stack& st, uint32_t* ts,
       const float4 q0 = np[0], q1 = np[1], q2 = np[2];
       const uint4 m = reinterpret_cast<const uint4*>(tv.nodes + cur)[3];
       const float node_tmax = kMode == BAJO_TRACE_ANY_HIT ? ray.tmax : hit.t;
-      float t0, t1;
       const bool h0 = slab(ray.o, rcp, q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, node_tmax, t0);
       const bool h1 = slab(ray.o, rcp, q1.z, q1.w, q2.x, q2.y, q2.z, q2.w, node_tmax, t1);
-      const uint32_t c0 = m.y, c1 = m.z;
-      bool v0 = false, v1 = false;
-      if (h0) {
-        if (c0 & kLeafFlag) done = visit(c0 & kIndexMask);
-        else v0 = true;
-      }
-      if (!done && h1) {
-        if (c1 & kLeafFlag) done = visit(c1 & kIndexMask);
-        else v1 = true;
-      }
-      if (done) break;
-      int near = -1;
-      float near_t = kFltMax;
-      if (v0) { near = 0; near_t = t0; }
-      if (v1 && (near == -1 || t1 < near_t)) { near = 1; near_t = t1; }
-      const float bound = kMode == BAJO_TRACE_ANY_HIT ? ray.tmax : hit.t;
-      bool overflow = false;
-      if (v0 && near != 0 && t0 <= bound) {
-        if (sp >= kTlasStack) overflow = true; else ts[(uint64_t)(sp++) * ts_stride] = c0;
-      }
-      if (v1 && near != 1 && t1 <= bound) {
-        if (sp >= kTlasStack) overflow = true; else ts[(uint64_t)(sp++) * ts_stride] = c1;
-      }
-      if (overflow) {
-        atomicOr(tv.status, (uint32_t)BAJO_STATUS_STACK_OVERFLOW);
-        break;
-      }
-      if (near != -1 && near_t <= bound) {
-        cur = near == 0 ? c0 : c1;
-        continue;
-      }
-      if (sp == 0) break;
-      cur = ts[(uint64_t)(--sp) * ts_stride];
+      c0 = m.y;
+      c1 = m.z;
+      v0 = h0 && !(c0 & kLeafFlag);
+      v1 = h1 && !(c1 & kLeafFlag);
+      pend = (h0 && (c0 & kLeafFlag) ? 1u : 0u) | (h1 && (c1 & kLeafFlag) ? 2u : 0u);
+      tested = true;
     }
+    if (pend == 0u) break;
+    const bool second = (pend & 1u) == 0u;
+    pend = second ? 0u : pend & 2u;
+    done = visit((second ? c1 : c0) & kIndexMask);
+    if (done) break;
   }
   if constexpr (kMode == BAJO_TRACE_ANY_HIT) {
     if (done) return Hit{0.0f, 0.0f, kEmpty, occ_inst, mk(0, 0, 0), 0.0f};
@@ -179,17 +198,46 @@ BJ_D Hit tlas_trace(const TlasView& tv, const Ray& ray, Stack& st, uint32_t* ts,
   }
 }
 
-template <int kMode, bool kCamera>
-__global__ void __launch_bounds__(kTraceBlock) tlas_kernel(const TlasView tv, const float* __restrict__ rays,
+// The pixel that index r of a camera launch of R rays traces: views in order,
+// a view in tiles of 8 x 8 pixels (narrower and lower ones at its right and
+// bottom edges), so that a wave's rays stay close together and walk the same
+// nodes (256 instances of a 67,280-triangle mesh, three 640 x 360 views: 426
+// us against 482 row by row).  A view that the launch cuts short is traced
+// row by row.
+BJ_D uint64_t camera_pixel(uint64_t r, uint64_t R, uint32_t w, uint32_t h) {
+  const uint64_t ppv = (uint64_t)w * h;
+  const uint64_t start = r / ppv * ppv;
+  if (start + ppv > R) return r;
+  uint32_t k = (uint32_t)(r - start);
+  const uint32_t band = k / (8u * w);
+  k -= band * 8u * w;
+  const uint32_t rows = h - 8u * band < 8u ? h - 8u * band : 8u;
+  const uint32_t tile = k / (8u * rows);
+  k -= tile * 8u * rows;
+  const uint32_t cols = w - 8u * tile < 8u ? w - 8u * tile : 8u;
+  const uint32_t y = k / cols, x = k - y * cols;
+  return start + (uint64_t)(8u * band + y) * w + 8u * tile + x;
+}
+
+template <int kMode, bool kCamera, bool kPlain8>
+__global__ void __attribute__((amdgpu_waves_per_eu(6))) __launch_bounds__(kTraceBlock) tlas_kernel(const TlasView tv, const float* __restrict__ rays,
                                                            const float* __restrict__ cams, uint32_t cam_w,
                                                            uint32_t cam_h, float inv_height, float* __restrict__ hits,
-                                                           uint64_t R, uint32_t* __restrict__ tstack,
+                                                           uint64_t R, uint32_t* __restrict__ counter,
+                                                           uint32_t* __restrict__ tstack,
                                                            uint32_t* __restrict__ spill) {
   __shared__ uint32_t s_stack[kLdsStack * kTraceBlock];
   const uint64_t gtid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const uint64_t threads = (uint64_t)gridDim.x * blockDim.x;
   Stack st{s_stack + threadIdx.x, spill + gtid, threads, 0};
-  for (uint64_t r = gtid; r < R; r += threads) {
+  for (;;) {
+    uint32_t base = 0;
+    if (lane_id() == 0) base = atomicAdd(counter, 64u);
+    base = __shfl(base, 0, 64);
+    if ((uint64_t)base >= R) break;
+    const uint64_t k = (uint64_t)base + lane_id();
+    if (k >= R) continue;
+    const uint64_t r = kCamera ? camera_pixel(k, R, cam_w, cam_h) : k;
     Ray ray;
     if constexpr (kCamera) {
       ray = camera_ray(cams, r, cam_w, cam_h, inv_height);
@@ -199,12 +247,12 @@ __global__ void __launch_bounds__(kTraceBlock) tlas_kernel(const TlasView tv, co
       ray.d = mk(rays[4 * R + r], rays[5 * R + r], rays[6 * R + r]);
       ray.tmax = rays[7 * R + r];
     }
-    store_hit(hits, r, tlas_trace<kMode>(tv, ray, st, tstack + gtid, threads));
+    store_hit(hits, r, tlas_trace<kMode, kPlain8>(tv, ray, st, tstack + gtid, threads));
   }
 }
 
-__global__ void tlas_status_kernel(uint32_t* status) {
-  if (threadIdx.x == 0) *status = 0;
+__global__ void tlas_init_kernel(uint32_t* status, uint32_t* counter) {
+  if (threadIdx.x == 0) { *status = 0; *counter = 0; }
 }
 
 // Affine3.inverse (core/transform.mojo:290-340): adjugate over the
@@ -258,15 +306,15 @@ void free_tlas(bajo_tlas* t) {
   delete t;
 }
 
-template <int kMode, bool kCamera>
-int32_t launch_tlas(bajo_ctx* ctx, const bajo_tlas* t, const float* rays, const float* cams, uint32_t w, uint32_t hh,
+template <int kMode, bool kCamera, bool kPlain8>
+int32_t launch_tlas_as(bajo_ctx* ctx, const bajo_tlas* t, const float* rays, const float* cams, uint32_t w, uint32_t hh,
                     float* hits, uint64_t R) {
   static unsigned cached = 0;
   if (!cached) {
     int dev = 0, cus = 0, per_cu = 0;
     BJ_HIP(hipGetDevice(&dev));
     BJ_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    BJ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, tlas_kernel<kMode, kCamera>, kTraceBlock, 0));
+    BJ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, tlas_kernel<kMode, kCamera, kPlain8>, kTraceBlock, 0));
     cached = (unsigned)(cus * (per_cu < 1 ? 1 : per_cu));
   }
   unsigned grid = cached;
@@ -275,18 +323,26 @@ int32_t launch_tlas(bajo_ctx* ctx, const bajo_tlas* t, const float* rays, const 
   if (grid < 1) grid = 1;
   const uint64_t threads = (uint64_t)grid * kTraceBlock;
   void* scratch = nullptr;
-  int32_t rc = ctx_scratch(ctx, threads * (kSpill + kTlasStack) * sizeof(uint32_t), &scratch);
+  int32_t rc = ctx_scratch(ctx, (64 + threads * (kSpill + kTlasStack)) * sizeof(uint32_t), &scratch);
   if (rc) return rc;
-  uint32_t* spill = (uint32_t*)scratch;
+  uint32_t* counter = (uint32_t*)scratch;
+  uint32_t* spill = counter + 64;
   uint32_t* tstack = spill + threads * kSpill;
   const bajo_bvh* top = t->top;
   TlasView tv{top->nodes, top->keys, top->root, (uint32_t)(top->n - 1), t->instance_count, t->inv, t->inst_blas,
               t->blas, t->status};
-  tlas_status_kernel<<<1, 64, 0, ctx->stream>>>(t->status);
-  tlas_kernel<kMode, kCamera><<<grid, kTraceBlock, 0, ctx->stream>>>(tv, rays, cams, w, hh, hh ? 1.0f / (float)hh : 0.0f,
-                                                                    hits, R, tstack, spill);
+  tlas_init_kernel<<<1, 64, 0, ctx->stream>>>(t->status, counter);
+  tlas_kernel<kMode, kCamera, kPlain8><<<grid, kTraceBlock, 0, ctx->stream>>>(tv, rays, cams, w, hh, hh ? 1.0f / (float)hh : 0.0f,
+                                                                    hits, R, counter, tstack, spill);
   BJ_HIP(hipGetLastError());
   return BAJO_OK;
+}
+
+template <int kMode, bool kCamera>
+int32_t launch_tlas(bajo_ctx* ctx, const bajo_tlas* t, const float* rays, const float* cams, uint32_t w, uint32_t hh,
+                    float* hits, uint64_t R) {
+  return t->plain8 ? launch_tlas_as<kMode, kCamera, true>(ctx, t, rays, cams, w, hh, hits, R)
+                   : launch_tlas_as<kMode, kCamera, false>(ctx, t, rays, cams, w, hh, hits, R);
 }
 
 }  // namespace
@@ -347,6 +403,7 @@ int32_t bajo_tlas_create(bajo_ctx* ctx, const bajo_bvh* const* blases, uint32_t 
     const AccelView av = accel_view(blases[b], t->status);
     views[b] = TlasBlas{av.bin, av.wide, wide_layout(blases[b]->node_width) ? 1u : 0u,
                         blases[b]->spheres ? 1u : 0u, (uint32_t)blases[b]->n};
+    t->plain8 = t->plain8 && views[b].is_wide && !views[b].is_sphere;
   }
   TL_HIP(hipMalloc(&t->boxes, t->host_boxes.size() * sizeof(float)));
   TL_HIP(hipMalloc(&t->inv, inv.size() * sizeof(float)));

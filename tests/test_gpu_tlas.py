@@ -142,3 +142,23 @@ def test_tlas_rejects_bad_arguments(gpu_ctx):
     boxes = build_binary_bvh(to_dev(np.array([0, 0, 0, 1, 1, 1], np.float32)))
     with pytest.raises(BajoError, match="not a triangle or sphere BVH"):
         build_triangle_tlas([boxes], [Instance(translation(), 0)])
+
+
+@pytest.mark.parametrize("widths,n_inst", [((8, 8), 1), ((8, 8, 8), 60), ((8, 2, 8), 60)])
+@pytest.mark.parametrize("w,h,cut", [(64, 16, 0), (37, 21, 0), (5, 3, 0), (9, 8, 0), (8, 9, 5), (70, 30, 1000), (1, 200, 0)])
+def test_tlas_camera_tiles(gpu_ctx, widths, n_inst, w, h, cut):
+    """Camera launches walk a view in 8 x 8 tiles: whole and partial tiles, two views, and a second view cut short by
+    `cut` rays, over all-wide and mixed BLASes and one instance (the top level is a leaf)."""
+    from bajo_amd.bvh import Camera
+
+    announce(f"tlas camera tiles {w}x{h} cut={cut} widths={widths} instances={n_inst}")
+    tlas, blases, xf, idx, boxes = scene(widths, n_inst, 43)
+    cams = np.concatenate([Camera((0.0, 2.0, z), (0.0, 0.0, 0.0), (0.0, 1.0, 0.0), 0.6).flatten() for z in (-14.0, 9.0)])
+    R = 2 * w * h - cut
+    hits = torch.full((8 * R + 64,), 7.0, dtype=torch.float32, device="cuda:0")
+    tlas.launch_camera(to_dev(cams), hits[:8 * R], R, w, h)
+    got = to_host(hits, np.float32)
+    assert (got[8 * R:] == 7.0).all()
+    want = oracle.tlas_trace(blases, xf, idx, oracle.build_lbvh_bounds(boxes), oracle.camera_rays(cams, R, w, h))
+    np.testing.assert_array_equal(got[:8 * R].view(np.uint32), want.reshape(-1).view(np.uint32))
+    assert tlas.status() == 0
