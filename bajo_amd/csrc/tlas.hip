@@ -18,8 +18,9 @@
 //   - bound by the walks' latency at few waves and by lanes waiting for each
 //     other: with one BLAS visit in the code (it stood at three places), the
 //     all-wide-triangles case compiled by itself and six waves per SIMD (the
-//     stacks' LDS allows no more) 256 instances and 691,200 rays take 354 us
-//     (697 at two waves; 440 at three, 426 at five);
+//     stacks' LDS allows no more) 256 instances and 691,200 rays take 391 us
+//     (697 at two waves; 440 at three, 420 at five; the counter measured the
+//     same as a grid stride here, 391 against 397);
 //   - instance transforms, BLAS views and instance-to-BLAS indices live in
 //     device arrays uploaded once at creation; the BLAS handles stay owned
 //     by the caller.
