@@ -41,7 +41,7 @@ class DeviceContext:
         return word.value
 
     def set_spin_limit(self, spin_limit: int) -> None:
-        """Spin cap of the sort's look-back wait (0 = default); a tile past it raises BAJO_STATUS_SORT_LOOKBACK."""
+        """Spin cap of the sort's look-back wait (0 = default); a tile past it counts its predecessors' keys itself."""
         _lib.check(_lib.lib().bajo_ctx_set_spin_limit(self._handle, int(spin_limit)))
 
     def name(self) -> str:

@@ -19,7 +19,10 @@
 // counts before it ranks; looks back over the tiles of its group of 16 and
 // then over whole groups, each round's loads in flight together (tile by tile
 // four at a time the chain grew to 22 rounds); and draws its ticket from one
-// of eight counters (same-address atomics serialize).  A pass over 4M pairs
+// of eight counters (same-address atomics serialize).  With eight counters a
+// predecessor may not have started (another stream's kernel can hold its XCD),
+// so a tile waits for a bounded time and then counts the missing tiles itself:
+// a sort ends whatever else runs on the chip.  A pass over 4M pairs
 // (100 MB moved) took 50.9 us and takes 38.5 (2.6 TB/s), over 4M keys 48.2 and
 // 31.7.  Lists of at most 8,192 keys are sorted by one block in LDS, all
 // passes in one launch (8,192 64-bit pairs: 109 -> 54 us).
@@ -127,11 +130,10 @@ BJ_D void rank_keys(const K (&key)[kKpt], uint32_t shift, uint32_t valid, uint32
 }
 
 // Sums of the look-back words at p[-256 j], j = 1..count (count <= kMost), once
-// all are published; their loads are in flight together.  Every predecessor
-// holds an earlier ticket and is resident, so it publishes; the cap only
-// bounds the wait if the table was corrupted (false then).
+// all are published; their loads are in flight together.  False if one stayed
+// unpublished for more than `patience` polls.
 template <uint32_t kMost>
-BJ_D bool sum_published(const uint32_t* p, uint32_t count, uint32_t spin_limit, uint32_t& sum) {
+BJ_D bool sum_published(const uint32_t* p, uint32_t count, uint32_t patience, uint32_t& sum) {
   for (uint32_t spins = 0;; ++spins) {
     uint32_t v[kMost];
 #pragma unroll
@@ -149,21 +151,23 @@ BJ_D bool sum_published(const uint32_t* p, uint32_t count, uint32_t spin_limit, 
       sum += total;
       return true;
     }
-    if (spins >= spin_limit) return false;
+    if (spins >= patience) return false;
     __builtin_amdgcn_s_sleep(1);
   }
 }
 
-// The number of keys with this thread's digit in all tiles before `tile`, from
-// the counts published per tile and per group of kSortGroup tiles.
-BJ_D uint32_t look_back(uint32_t* __restrict__ lookback, uint32_t tiles, uint32_t tile, uint32_t count, uint32_t t,
-                        uint32_t spin_limit, uint32_t* __restrict__ status) {
+// The number of keys with this thread's digit in all tiles before `tile`
+// (`before`), from the counts published per tile and per group of kSortGroup
+// tiles.  False if a count stayed unpublished for `patience` polls: then
+// count_back finds the number.
+BJ_D bool look_back(uint32_t* __restrict__ lookback, uint32_t tiles, uint32_t tile, uint32_t count, uint32_t t,
+                    uint32_t patience, uint32_t& before) {
   uint32_t* mine = lookback + (uint64_t)tile * 256 + t;
   const uint32_t g = tile / kSortGroup, q = tile % kSortGroup;
   const bool last = q == kSortGroup - 1;  // publishes its group's counts
   uint32_t* group = lookback + ((uint64_t)tiles + g) * 256 + t;
-  uint32_t before = 0;
-  bool ok = q == 0 || sum_published<kSortGroup - 1>(mine, q, spin_limit, before);
+  before = 0;
+  if (q != 0 && !sum_published<kSortGroup - 1>(mine, q, patience, before)) return false;
   if (last)
     __hip_atomic_store(group, (g == 0 ? kLookbackInc : kLookbackAgg) | ((before + count) & kLookbackMask),
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -172,7 +176,7 @@ BJ_D uint32_t look_back(uint32_t* __restrict__ lookback, uint32_t tiles, uint32_
   constexpr int kAhead = 8;
   int64_t j = (int64_t)g - 1;
   uint32_t spins = 0;
-  while (ok && j >= 0) {
+  while (j >= 0) {
     uint32_t v[kAhead];
 #pragma unroll
     for (int k = 0; k < kAhead; ++k)
@@ -196,14 +200,68 @@ BJ_D uint32_t look_back(uint32_t* __restrict__ lookback, uint32_t tiles, uint32_
     if (done) break;
     j -= k;
     if (waiting) {
-      if (++spins > spin_limit) ok = false;
-      else __builtin_amdgcn_s_sleep(1);
+      if (++spins > patience) return false;
+      __builtin_amdgcn_s_sleep(1);
     }
   }
   if (last && g > 0)
     __hip_atomic_store(group, kLookbackInc | ((before + count) & kLookbackMask), __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
-  if (!ok) atomicMax(status, (uint32_t)BAJO_STATUS_SORT_LOOKBACK);
+  return true;
+}
+
+// look_back's number without waiting, by the whole block: a predecessor whose
+// counts are not published (its block may not have started, and need not start
+// before this one ends) is counted from its keys, which no tile of the pass
+// writes, and published in its place -- the same words that it would write.
+// s_count: 256 words of LDS that nothing else uses now.
+template <typename K>
+BJ_D uint32_t count_back(const K* __restrict__ keys, uint32_t tile_keys, uint32_t shift,
+                         uint32_t* __restrict__ lookback, uint32_t tiles, uint32_t tile, uint32_t count, uint32_t t,
+                         uint32_t* __restrict__ s_count) {
+  const uint32_t g = tile / kSortGroup;
+  auto tile_count = [&](uint32_t p) {
+    uint32_t* at = lookback + (uint64_t)p * 256 + t;
+    uint32_t v = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!__syncthreads_and(v != 0u)) {
+      s_count[t] = 0;
+      __syncthreads();
+      const K* first = keys + (uint64_t)p * tile_keys;  // a predecessor's tile is full
+      for (uint32_t i = t; i < tile_keys; i += kSortBlock) atomicAdd(&s_count[digit_of(first[i], shift)], 1u);
+      __syncthreads();
+      v = kLookbackAgg | s_count[t];
+      __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    return v & kLookbackMask;
+  };
+  uint32_t before = 0;
+  for (uint32_t p = tile; p > g * kSortGroup;) before += tile_count(--p);
+  // a group's word only ever grows: unpublished, aggregate, inclusive prefix
+  auto publish = [&](uint32_t group, uint32_t word) {
+    __hip_atomic_fetch_max(lookback + ((uint64_t)tiles + group) * 256 + t, word, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+  };
+  const bool last = tile % kSortGroup == kSortGroup - 1;
+  if (last) publish(g, (g == 0 ? kLookbackInc : kLookbackAgg) | ((before + count) & kLookbackMask));
+  bool done = false;
+  for (uint32_t j = g; j-- > 0;) {
+    uint32_t v = __hip_atomic_load(lookback + ((uint64_t)tiles + j) * 256 + t, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+    if (!__syncthreads_and(done || v != 0u)) {
+      uint32_t sum = 0;
+      for (uint32_t p = j * kSortGroup; p < (j + 1) * kSortGroup; ++p) sum += tile_count(p);
+      if (v == 0u) {
+        v = (j == 0 ? kLookbackInc : kLookbackAgg) | sum;
+        publish(j, v);
+      }
+    }
+    if (!done) {
+      before += v & kLookbackMask;
+      done = (v & kLookbackInc) != 0u;
+    }
+    if (__syncthreads_and(done)) break;
+  }
+  if (last && g > 0) publish(g, kLookbackInc | ((before + count) & kLookbackMask));
   return before;
 }
 
@@ -213,8 +271,7 @@ __global__ void __launch_bounds__(kSortBlock) __attribute__((amdgpu_waves_per_eu
                                                               uint32_t* __restrict__ out_vals, uint64_t n,
                                                               uint32_t shift, const uint32_t* __restrict__ pass_hist,
                                                               uint32_t* __restrict__ lookback,
-                                                              uint32_t* __restrict__ tickets,
-                                                              uint32_t* __restrict__ status, uint32_t spin_limit) {
+                                                              uint32_t* __restrict__ tickets, uint32_t patience) {
   constexpr uint32_t kTile = kSortBlock * kKpt;
   // keys are staged first, then the values in the same words: four blocks of
   // 4,096 pairs fit a CU instead of two
@@ -222,18 +279,18 @@ __global__ void __launch_bounds__(kSortBlock) __attribute__((amdgpu_waves_per_eu
   __shared__ uint32_t s_wave_hist[kSortWaves][256];
   __shared__ uint32_t s_adjust[256];  // the tile's digit counts, then the offset from tile to global position
   __shared__ uint32_t s_tmp[kSortWaves];
-  __shared__ uint32_t s_tile;
+  __shared__ uint32_t s_tile, s_late;
 
   const uint32_t t = threadIdx.x;
   const uint32_t lane = lane_id();
   const uint32_t wave = t >> 6;
 
-  // Blocks are dealt to the eight XCDs round robin and started in order within
-  // each, so the tiles drawn per class keep every predecessor of a started
-  // tile started or next in line on its own XCD.
+  // Tiles are drawn in order within a class.  Of another class a predecessor
+  // may not have started yet: where it stays out, count_back does without it.
   if (t == 0) {
     const uint32_t c = blockIdx.x % kTicketClasses;
     s_tile = kTicketClasses * atomicAdd(tickets + c * kTicketStride, 1u) + c;
+    s_late = 0;
   }
 #pragma unroll
   for (int w = 0; w < kSortWaves; ++w) s_wave_hist[w][t] = 0;
@@ -284,9 +341,16 @@ __global__ void __launch_bounds__(kSortBlock) __attribute__((amdgpu_waves_per_eu
       val[k] = o < valid ? in_vals[tile_base + wave_base + o] : 0u;
     }
   }
-  const uint32_t exclusive = look_back(lookback, gridDim.x, tile, count, t, spin_limit, status);
+  uint32_t exclusive = 0;
+  if (!look_back(lookback, gridDim.x, tile, count, t, patience, exclusive)) s_late = 1;
   s_adjust[t] = global_excl + exclusive - digit_start;
   __syncthreads();
+  if (s_late) {
+    exclusive = count_back(in_keys, kTile, shift, lookback, gridDim.x, tile, count, t,
+                           reinterpret_cast<uint32_t*>(s_keys));
+    s_adjust[t] = global_excl + exclusive - digit_start;
+    __syncthreads();
+  }
 
   // ---- keys into LDS in sorted order, then out in digit-contiguous runs
 #pragma unroll
@@ -406,9 +470,9 @@ size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 template <typename K, bool kValues, int kKpt>
 void launch_bin(bajo_ctx* ctx, const SortPlan& p, const K* src, K* dst, const uint32_t* vsrc, uint32_t* vdst,
-                uint32_t shift, const uint32_t* hist, uint32_t* lookback, uint32_t* tickets, uint32_t spin_limit) {
+                uint32_t shift, const uint32_t* hist, uint32_t* lookback, uint32_t* tickets, uint32_t patience) {
   sort_bin_kernel<K, kValues, kKpt><<<p.tiles, kSortBlock, 0, ctx->stream>>>(
-      src, dst, vsrc, vdst, p.n, shift, hist, lookback, tickets, ctx->status, spin_limit);
+      src, dst, vsrc, vdst, p.n, shift, hist, lookback, tickets, patience);
 }
 
 template <typename K, bool kValues>
@@ -439,15 +503,15 @@ int32_t run_typed(bajo_ctx* ctx, const SortPlan& p, K* keys, uint32_t* values, c
   K* dst = alt_keys;
   uint32_t* vsrc = values;
   uint32_t* vdst = alt_vals;
-  const uint32_t spin_limit = ctx->spin_limit ? ctx->spin_limit : kLookbackSpinLimit;
+  const uint32_t patience = ctx->spin_limit ? ctx->spin_limit : kLookbackPatience;
   for (int pass = 0; pass < p.passes; ++pass) {
     const uint32_t shift = (uint32_t)(p.begin_bit + 8 * pass);
     const uint32_t* h = hist + pass * 256;
     uint32_t* lb = lookback + lb_pass_words * pass;
     uint32_t* tk = tickets + (uint32_t)pass * kTicketWords;
-    if (p.kpt == 4) launch_bin<K, kValues, 4>(ctx, p, src, dst, vsrc, vdst, shift, h, lb, tk, spin_limit);
-    else if (p.kpt == 8) launch_bin<K, kValues, 8>(ctx, p, src, dst, vsrc, vdst, shift, h, lb, tk, spin_limit);
-    else launch_bin<K, kValues, 16>(ctx, p, src, dst, vsrc, vdst, shift, h, lb, tk, spin_limit);
+    if (p.kpt == 4) launch_bin<K, kValues, 4>(ctx, p, src, dst, vsrc, vdst, shift, h, lb, tk, patience);
+    else if (p.kpt == 8) launch_bin<K, kValues, 8>(ctx, p, src, dst, vsrc, vdst, shift, h, lb, tk, patience);
+    else launch_bin<K, kValues, 16>(ctx, p, src, dst, vsrc, vdst, shift, h, lb, tk, patience);
     BJ_HIP(hipGetLastError());
     K* sk = src; src = dst; dst = sk;
     uint32_t* sv = vsrc; vsrc = vdst; vdst = sv;

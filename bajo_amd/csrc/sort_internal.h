@@ -17,7 +17,9 @@ constexpr uint32_t kLookbackAgg = 0x40000000u;
 constexpr uint32_t kLookbackInc = 0x80000000u;
 constexpr uint32_t kLookbackMask = 0x3FFFFFFFu;
 constexpr uint64_t kSortMaxKeys = (1ull << 30) - 1;
-constexpr uint32_t kLookbackSpinLimit = 1u << 24;
+// Polls of the look-back table (about a microsecond each) before a tile counts
+// its missing predecessors itself; a pass alone on the chip waits some tens.
+constexpr uint32_t kLookbackPatience = 512;
 
 // Workspace layout of one sort.  All offsets are 256-byte aligned.
 struct SortPlan {

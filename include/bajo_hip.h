@@ -34,7 +34,7 @@ extern "C" {
  * word, reported at its sync points, like bajo's HPLOC_STATUS / collapse
  * TIMEOUT words, bvh/gpu/builder/hploc_layout.mojo:9-11,
  * wide_collapse.mojo:34-38,236-254): */
-#define BAJO_STATUS_SORT_LOOKBACK 4  /* a sort tile gave up waiting for its predecessor (spin cap) */
+#define BAJO_STATUS_SORT_LOOKBACK 4  /* reserved: a sort tile no longer gives up, see bajo_ctx_set_spin_limit */
 #define BAJO_STATUS_REFIT_CORRUPT 5  /* the LBVH climb met an inconsistent hierarchy */
 #define BAJO_STATUS_HPLOC_FAILED 6   /* H-PLOC made no progress, met a corrupt cluster list or ended without one root */
 #define BAJO_STATUS_COLLAPSE_FAILED 7 /* the wide collapse ran out of nodes, met a bad root or passed its level bound */
@@ -133,12 +133,12 @@ int32_t bajo_ctx_synchronize(bajo_ctx* ctx);
 /* Synchronizes and reads the context status word into *status (0 = none
  * raised), then clears it.  Returns BAJO_OK unless the read itself fails. */
 int32_t bajo_ctx_status(bajo_ctx* ctx, uint32_t* status);
-/* Spin cap of the sort's decoupled look-back wait (0 = the default 2^24):
- * a tile that waits longer gives up and raises BAJO_STATUS_SORT_LOOKBACK
- * instead of waiting forever on a corrupted look-back table.  bajo's wide
- * collapse has the same kind of fail-safe (a 10M-spin cap,
+/* Spin cap of the sort's decoupled look-back wait (0 = the default 512 polls):
+ * a tile that waits longer counts its missing predecessors' keys itself and
+ * goes on, so a sort ends with the right order whatever else runs on the
+ * GPU.  bajo's wide collapse has a spin cap that fails (10M spins,
  * bvh/gpu/builder/wide_collapse.mojo:236-254); a tiny cap lets tests force
- * the status path from the host. */
+ * the counting path from the host. */
 int32_t bajo_ctx_set_spin_limit(bajo_ctx* ctx, uint32_t spin_limit);
 const char* bajo_last_error(void);
 const char* bajo_status_string(int32_t status);

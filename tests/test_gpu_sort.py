@@ -170,3 +170,54 @@ def test_tile_size_edges(gpu_ctx, n, bits):
     k = to_dev(keys)
     sort.device_radix_sort_keys(k)
     np.testing.assert_array_equal(to_host(k, dtype), keys[order])
+
+
+@pytest.mark.parametrize("n", [8193, 4096 * 5 + 3, 262145, 1310721 + 4096 * 40])
+@pytest.mark.parametrize("bits", [32, 64])
+def test_a_tile_that_does_not_wait_counts_its_predecessors(gpu_ctx, n, bits):
+    """A tile past the cap of its look-back wait counts the missing tiles' keys itself: with the cap forced to one
+    poll from the host, every sort is right and raises nothing (few distinct digits, so that every count matters)."""
+    from bajo_amd import sort
+    from bajo_amd.context import DeviceContext
+
+    announce(f"sort without waiting n={n} bits={bits}")
+    ctx = DeviceContext(0)
+    ctx.set_spin_limit(1)
+    rng = np.random.default_rng(n + bits)
+    dtype = np.uint32 if bits == 32 else np.uint64
+    keys = (rng.integers(0, 9, n, dtype=np.uint64) * np.uint64(0x0101010101010101)).astype(dtype)
+    keys[::2] ^= rng.integers(0, 2**31, keys[::2].size, dtype=np.uint64).astype(dtype)
+    order = np.argsort(keys, kind="stable")
+    for _ in range(4):
+        k, v = to_dev(keys), to_dev(np.arange(n, dtype=np.uint32))
+        sort.device_radix_sort_pairs(k, v, ctx=ctx)
+        assert ctx.status() == 0
+        np.testing.assert_array_equal(to_host(v, np.uint32), order)
+        np.testing.assert_array_equal(to_host(k, dtype), keys[order])
+        k = to_dev(keys)
+        sort.device_radix_sort_keys(k, ctx=ctx)
+        assert ctx.status() == 0
+        np.testing.assert_array_equal(to_host(k, dtype), keys[order])
+    ctx.close()
+
+
+def test_a_build_that_does_not_wait(gpu_ctx):
+    """The LBVH's key sort, whose histogram the Morton kernel fills, under the same cap: the layout is the oracle's."""
+    import torch
+
+    import oracle
+    from bajo_amd import scenes
+    from bajo_amd.bvh import build_triangle_bvh
+    from bajo_amd.context import DeviceContext
+
+    announce("build without waiting in the sort")
+    ctx = DeviceContext(0)
+    ctx.set_spin_limit(1)
+    v = scenes.soup(300_000, initstate=8, initseq=5)
+    bvh = build_triangle_bvh(torch.from_numpy(v).to("cuda:0"), ctx=ctx)
+    got, want = bvh.binary(), oracle.build_lbvh(v)
+    assert ctx.status() == 0
+    for key in ("sorted_keys", "leaf_ids", "node_meta", "leaf_parent"):
+        np.testing.assert_array_equal(got[key], want[key], err_msg=key)
+    bvh.free()
+    ctx.close()
