@@ -16,7 +16,7 @@
 //
 // What bounds a pass is a tile's serial chain, not its bytes: at 4M 64-bit
 // keys all 1,024 tiles are resident at once.  Hence a tile publishes its
-// counts before it ranks; looks back over the tiles of its group of 16 and
+// counts before it ranks; looks back over the tiles of its group (8 or 16) and
 // then over whole groups, each round's loads in flight together (tile by tile
 // four at a time the chain grew to 22 rounds); and draws its ticket from one
 // of eight counters (same-address atomics serialize).  With eight counters a
@@ -157,23 +157,26 @@ BJ_D bool sum_published(const uint32_t* p, uint32_t count, uint32_t patience, ui
 }
 
 // The number of keys with this thread's digit in all tiles before `tile`
-// (`before`), from the counts published per tile and per group of kSortGroup
-// tiles.  False if a count stayed unpublished for `patience` polls: then
+// (`before`), from the counts published per tile and per group of kGroup tiles.
+// False if a count stayed unpublished for `patience` polls: then
 // count_back finds the number.
+template <uint32_t kGroup>
 BJ_D bool look_back(uint32_t* __restrict__ lookback, uint32_t tiles, uint32_t tile, uint32_t count, uint32_t t,
                     uint32_t patience, uint32_t& before) {
   uint32_t* mine = lookback + (uint64_t)tile * 256 + t;
-  const uint32_t g = tile / kSortGroup, q = tile % kSortGroup;
-  const bool last = q == kSortGroup - 1;  // publishes its group's counts
+  const uint32_t g = tile / kGroup, q = tile % kGroup;
+  const bool last = q == kGroup - 1;  // publishes its group's counts
   uint32_t* group = lookback + ((uint64_t)tiles + g) * 256 + t;
   before = 0;
-  if (q != 0 && !sum_published<kSortGroup - 1>(mine, q, patience, before)) return false;
+  if (q != 0 && !sum_published<kGroup - 1>(mine, q, patience, before)) return false;
   if (last)
     __hip_atomic_store(group, (g == 0 ? kLookbackInc : kLookbackAgg) | ((before + count) & kLookbackMask),
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  // whole groups, eight loads in flight: aggregates are added up to an
-  // inclusive prefix, or to the first group not yet published, polled again
-  constexpr int kAhead = 8;
+  // whole groups, two loads in flight: aggregates are added up to an
+  // inclusive prefix, or to the first group not yet published, polled again.
+  // (The words come from memory, past the L2s, and the prefix is mostly near:
+  // 47.5M 64-bit pairs 3.60 ms, 3.65 with three and 3.69 with four in flight.)
+  constexpr int kAhead = 2;
   int64_t j = (int64_t)g - 1;
   uint32_t spins = 0;
   while (j >= 0) {
@@ -215,11 +218,11 @@ BJ_D bool look_back(uint32_t* __restrict__ lookback, uint32_t tiles, uint32_t ti
 // before this one ends) is counted from its keys, which no tile of the pass
 // writes, and published in its place -- the same words that it would write.
 // s_count: 256 words of LDS that nothing else uses now.
-template <typename K>
+template <typename K, uint32_t kGroup>
 BJ_D uint32_t count_back(const K* __restrict__ keys, uint32_t tile_keys, uint32_t shift,
                          uint32_t* __restrict__ lookback, uint32_t tiles, uint32_t tile, uint32_t count, uint32_t t,
                          uint32_t* __restrict__ s_count) {
-  const uint32_t g = tile / kSortGroup;
+  const uint32_t g = tile / kGroup;
   auto tile_count = [&](uint32_t p) {
     uint32_t* at = lookback + (uint64_t)p * 256 + t;
     uint32_t v = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -235,13 +238,13 @@ BJ_D uint32_t count_back(const K* __restrict__ keys, uint32_t tile_keys, uint32_
     return v & kLookbackMask;
   };
   uint32_t before = 0;
-  for (uint32_t p = tile; p > g * kSortGroup;) before += tile_count(--p);
+  for (uint32_t p = tile; p > g * kGroup;) before += tile_count(--p);
   // a group's word only ever grows: unpublished, aggregate, inclusive prefix
   auto publish = [&](uint32_t group, uint32_t word) {
     __hip_atomic_fetch_max(lookback + ((uint64_t)tiles + group) * 256 + t, word, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
   };
-  const bool last = tile % kSortGroup == kSortGroup - 1;
+  const bool last = tile % kGroup == kGroup - 1;
   if (last) publish(g, (g == 0 ? kLookbackInc : kLookbackAgg) | ((before + count) & kLookbackMask));
   bool done = false;
   for (uint32_t j = g; j-- > 0;) {
@@ -249,7 +252,7 @@ BJ_D uint32_t count_back(const K* __restrict__ keys, uint32_t tile_keys, uint32_
                                    __HIP_MEMORY_SCOPE_AGENT);
     if (!__syncthreads_and(done || v != 0u)) {
       uint32_t sum = 0;
-      for (uint32_t p = j * kSortGroup; p < (j + 1) * kSortGroup; ++p) sum += tile_count(p);
+      for (uint32_t p = j * kGroup; p < (j + 1) * kGroup; ++p) sum += tile_count(p);
       if (v == 0u) {
         v = (j == 0 ? kLookbackInc : kLookbackAgg) | sum;
         publish(j, v);
@@ -272,7 +275,7 @@ __global__ void __launch_bounds__(kSortBlock) __attribute__((amdgpu_waves_per_eu
                                                               uint32_t shift, const uint32_t* __restrict__ pass_hist,
                                                               uint32_t* __restrict__ lookback,
                                                               uint32_t* __restrict__ tickets, uint32_t patience) {
-  constexpr uint32_t kTile = kSortBlock * kKpt;
+  constexpr uint32_t kTile = kSortBlock * kKpt, kGroup = sort_group(kKpt);
   // keys are staged first, then the values in the same words: four blocks of
   // 4,096 pairs fit a CU instead of two
   __shared__ K s_keys[kTile];
@@ -342,12 +345,12 @@ __global__ void __launch_bounds__(kSortBlock) __attribute__((amdgpu_waves_per_eu
     }
   }
   uint32_t exclusive = 0;
-  if (!look_back(lookback, gridDim.x, tile, count, t, patience, exclusive)) s_late = 1;
+  if (!look_back<kGroup>(lookback, gridDim.x, tile, count, t, patience, exclusive)) s_late = 1;
   s_adjust[t] = global_excl + exclusive - digit_start;
   __syncthreads();
   if (s_late) {
-    exclusive = count_back(in_keys, kTile, shift, lookback, gridDim.x, tile, count, t,
-                           reinterpret_cast<uint32_t*>(s_keys));
+    exclusive = count_back<K, kGroup>(in_keys, kTile, shift, lookback, gridDim.x, tile, count, t,
+                                      reinterpret_cast<uint32_t*>(s_keys));
     s_adjust[t] = global_excl + exclusive - digit_start;
     __syncthreads();
   }
@@ -539,7 +542,7 @@ SortPlan make_sort_plan(uint64_t n, int key_bytes, int has_values, int begin_bit
   // and 262; 4M 451 and 402)
   p.kpt = n <= 262144 ? 4 : (n <= 1310720 ? 8 : 16);
   p.tiles = div_up(n ? n : 1, (uint64_t)kSortBlock * p.kpt);
-  p.lookback_words = (size_t)(p.passes ? p.passes : 1) * (p.tiles + div_up(p.tiles, kSortGroup)) * 256;
+  p.lookback_words = (size_t)(p.passes ? p.passes : 1) * (p.tiles + div_up(p.tiles, sort_group(p.kpt))) * 256;
   size_t off = 0;
   p.off_alt_keys = off;
   off = align256(off + n * (size_t)key_bytes);

@@ -7,7 +7,12 @@ namespace bj {
 
 constexpr int kSortBlock = 256;             // 4 waves of 64
 constexpr int kSortWaves = kSortBlock / 64;
-constexpr uint32_t kSortGroup = 16;         // tiles per look-back group
+// Tiles per look-back group.  A tile reads the counts of half a group on
+// average, and at 16 keys per thread the registers of 15 loads in flight
+// spill: 64-bit pairs, 4M 314 us with 16 tiles and 262 with 8, 47.5M 4.16 and
+// 3.60 ms.  Shorter lists have registers to spare and fewer, smaller tiles:
+// 300K 107 and 110 us.
+constexpr uint32_t sort_group(int kpt) { return kpt == 16 ? 8u : 16u; }
 // Tile tickets are drawn from eight counters a cache line apart.
 constexpr uint32_t kTicketClasses = 8, kTicketStride = 32;
 constexpr uint32_t kTicketWords = kTicketClasses * kTicketStride;  // per pass
