@@ -57,8 +57,7 @@ struct bajo_bvh {
   void* hands;            // LBVH: records handed between blocks of the climb
   uint32_t* acc;          // 12 ordered-int bounds accumulators
   float* scene;           // 12 floats
-  void* sort_ws;
-  size_t sort_ws_bytes;
+  void* sort_ws;          // of every key sort of at most `capacity` keys
   // 8-wide layout (node_width == 8): collapsed from the binary LBVH
   int node_width;
   BjWide* wide;

@@ -697,14 +697,12 @@ __global__ void __launch_bounds__(kBlock) pack_spheres_kernel(const float* __res
 }
 
 int32_t ensure_capacity(bajo_bvh* h, uint64_t n) {
-  SortPlan plan = make_sort_plan(n, 8, 0, kSortBeginBit, kSortEndBit);
-  if (n <= h->capacity && plan.total <= h->sort_ws_bytes) return BAJO_OK;
+  if (n <= h->capacity) return BAJO_OK;  // (the sort workspace holds every shorter list's)
   (void)hipFree(h->nodes); (void)hipFree(h->tris); (void)hipFree(h->keys); (void)hipFree(h->leaf_parent); (void)hipFree(h->leaf_counts);
   (void)hipFree(h->flags); (void)hipFree(h->hands); (void)hipFree(h->acc); (void)hipFree(h->scene); (void)hipFree(h->sort_ws);
   h->nodes = nullptr; h->tris = nullptr; h->keys = nullptr; h->leaf_parent = nullptr; h->leaf_counts = nullptr;
   h->flags = nullptr; h->hands = nullptr; h->acc = nullptr; h->scene = nullptr; h->sort_ws = nullptr;
   h->capacity = 0;
-  h->sort_ws_bytes = 0;
   uint64_t internal = n > 1 ? n - 1 : 1;
   BJ_HIP(hipMalloc(&h->nodes, internal * sizeof(BjNode)));
   BJ_HIP(hipMalloc(&h->tris, n * sizeof(BjTri)));
@@ -715,9 +713,8 @@ int32_t ensure_capacity(bajo_bvh* h, uint64_t n) {
   BJ_HIP(hipMalloc(&h->hands, (uint64_t)div_up(n, kClimbBlock) * kHandSlots * sizeof(HandOff)));
   BJ_HIP(hipMalloc(&h->acc, 16 * sizeof(uint32_t)));
   BJ_HIP(hipMalloc(&h->scene, 16 * sizeof(float)));
-  BJ_HIP(hipMalloc(&h->sort_ws, plan.total));
+  BJ_HIP(hipMalloc(&h->sort_ws, sort_workspace_bound(n, 8, 0, kSortBeginBit, kSortEndBit)));
   h->capacity = n;
-  h->sort_ws_bytes = plan.total;
   return BAJO_OK;
 }
 
@@ -1015,7 +1012,7 @@ int32_t build_segmented(bajo_ctx* ctx, bajo_bvh* h, const float* vertices, const
   int seg_bits = 0;
   while ((1ull << seg_bits) < S) ++seg_bits;
   const SortPlan plan = make_sort_plan(n, 8, 1, 0, 30 + seg_bits);
-  rc = ensure_segment_capacity(h, n, S, plan.total);
+  rc = ensure_segment_capacity(h, n, S, sort_workspace_bound(n, 8, 1, 0, 30 + seg_bits));
   if (rc) return rc;
   hipStream_t st = ctx->stream;
   rc = upload_segment_offsets(st, h, offsets, S);

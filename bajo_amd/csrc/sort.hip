@@ -536,11 +536,7 @@ SortPlan make_sort_plan(uint64_t n, int key_bytes, int has_values, int begin_bit
   p.begin_bit = begin_bit;
   p.end_bit = end_bit;
   p.passes = (end_bit - begin_bit + 7) / 8;
-  // smaller tiles for shorter lists: a pass lasts as long as a tile's chain, so
-  // the keys are spread over the chip (64-bit pairs: 262,144 keys 105.9 us
-  // with 4 keys per thread, 115.3 with 8; 1M 163 with 8, 186 with 16; 2M 258
-  // and 262; 4M 451 and 402)
-  p.kpt = n <= 262144 ? 4 : (n <= 1310720 ? 8 : 16);
+  p.kpt = n <= kSortKpt4Keys ? 4 : (n <= kSortKpt8Keys ? 8 : 16);
   p.tiles = div_up(n ? n : 1, (uint64_t)kSortBlock * p.kpt);
   p.lookback_words = (size_t)(p.passes ? p.passes : 1) * (p.tiles + div_up(p.tiles, sort_group(p.kpt))) * 256;
   size_t off = 0;
@@ -556,6 +552,16 @@ SortPlan make_sort_plan(uint64_t n, int key_bytes, int has_values, int begin_bit
   off = align256(off + (size_t)(p.passes ? p.passes : 1) * kTicketWords * sizeof(uint32_t));
   p.total = off;
   return p;
+}
+
+size_t sort_workspace_bound(uint64_t n, int key_bytes, int has_values, int begin_bit, int end_bit) {
+  size_t most = make_sort_plan(n, key_bytes, has_values, begin_bit, end_bit).total;
+  for (const uint64_t m : {kSortKpt4Keys, kSortKpt8Keys}) {
+    if (n <= m) break;
+    const size_t b = make_sort_plan(m, key_bytes, has_values, begin_bit, end_bit).total;
+    if (b > most) most = b;
+  }
+  return most;
 }
 
 int32_t onesweep_run(bajo_ctx* ctx, const SortPlan& plan, void* keys, uint32_t* values, void* ws, bool hist_ready) {
@@ -587,7 +593,8 @@ int32_t sort_entry(bajo_ctx* ctx, void* keys, uint32_t* values, uint64_t n, int 
     BJ_REQUIRE(workspace_bytes >= plan.total, "%s: workspace of %llu bytes is below the %llu required", name,
                (unsigned long long)workspace_bytes, (unsigned long long)plan.total);
   } else {
-    int32_t rc = bj::ctx_scratch(ctx, plan.total, &ws);
+    const size_t bytes = bj::sort_workspace_bound(n, key_bytes, values != nullptr, begin_bit, end_bit);
+    int32_t rc = bj::ctx_scratch(ctx, bytes, &ws);
     if (rc) return rc;
   }
   return bj::onesweep_run(ctx, plan, keys, values, ws, false);
@@ -635,7 +642,7 @@ extern "C" {
 
 uint64_t bajo_sort_workspace_bytes(uint64_t n, int32_t key_bytes, int32_t has_values) {
   if (key_bytes != 4 && key_bytes != 8) return 0;
-  return bj::make_sort_plan(n, key_bytes, has_values != 0, 0, key_bytes * 8).total;
+  return bj::sort_workspace_bound(n, key_bytes, has_values != 0, 0, key_bytes * 8);
 }
 
 int32_t bajo_device_radix_sort_pairs_u64_u32(bajo_ctx* ctx, uint64_t* keys, uint32_t* values, uint64_t n,

@@ -38,7 +38,18 @@ struct SortPlan {
   size_t off_alt_keys = 0, off_alt_vals = 0, off_hist = 0, off_lookback = 0, off_tickets = 0, total = 0;
 };
 
+// Longest lists of tiles with 4 and with 8 keys per thread (longer ones: 16).
+// Smaller tiles for shorter lists: a pass lasts as long as a tile's chain, so
+// the keys are spread over the chip (64-bit pairs with 16 tiles per group:
+// 262,144 keys 105.9 us with 4 keys per thread, 115.3 with 8; 1M 163 with 8,
+// 186 with 16; 2M 258 and 262; 4M 451 and 402).
+constexpr uint64_t kSortKpt4Keys = 262144, kSortKpt8Keys = 1310720;
+
 SortPlan make_sort_plan(uint64_t n, int key_bytes, int has_values, int begin_bit, int end_bit);
+
+// Bytes that hold the workspace of every list of at most n keys: the look-back
+// table shrinks where the tiles grow, so a shorter list can need more.
+size_t sort_workspace_bound(uint64_t n, int key_bytes, int has_values, int begin_bit, int end_bit);
 
 // Runs the digit-binning passes.  When `hist_ready` is false the plan's
 // counters are cleared and the digit histogram is computed first; when true

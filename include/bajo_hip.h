@@ -147,7 +147,9 @@ int32_t bajo_device_name(int32_t device, char* out, int32_t cap);
 /* ---- sort: bajo/sort/gpu ------------------------------------------------
  * Stable ascending LSD radix sort (8-bit digits) of device buffers, result
  * in place.  `workspace` may be NULL (the context's scratch arena is used);
- * otherwise it must hold bajo_sort_workspace_bytes(n, key_bytes, has_values).
+ * otherwise it must hold bajo_sort_workspace_bytes(n, key_bytes, has_values),
+ * which never falls as n grows: a workspace of the longest list serves every
+ * shorter one.
  */
 uint64_t bajo_sort_workspace_bytes(uint64_t n, int32_t key_bytes, int32_t has_values);
 

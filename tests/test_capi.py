@@ -74,3 +74,14 @@ def test_icosphere_is_crack_free():
     assert set(keys.values()) == {2}
     r = np.linalg.norm(tris.reshape(-1, 3), axis=1)
     assert r.min() > 0.94 and r.max() < 1.06
+
+
+def test_sort_workspace_serves_every_shorter_list():
+    from bajo_amd.sort import sort_workspace_bytes
+
+    edges = [e + d for e in (1, 4096, 8192, 65536, 262144, 300_000, 400_000, 1310720, 1_500_000, 1 << 22, 1 << 24)
+             for d in (-1, 0, 1)]
+    for key_bytes in (4, 8):
+        for values in (False, True):
+            sizes = [sort_workspace_bytes(n, key_bytes, values) for n in edges]
+            assert sizes == sorted(sizes), (key_bytes, values)

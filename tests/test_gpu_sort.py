@@ -221,3 +221,49 @@ def test_a_build_that_does_not_wait(gpu_ctx):
         np.testing.assert_array_equal(got[key], want[key], err_msg=key)
     bvh.free()
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [262144, 1310720])
+def test_workspace_of_a_longer_list(gpu_ctx, n):
+    """Tiles grow with the list, so a shorter list can have the larger look-back table: a workspace sized for the
+    longest list serves it, and so does what the context and a hierarchy have allocated -- a smaller sort or rebuild
+    allocates nothing (it can be captured) and moves no buffer."""
+    import torch
+
+    from bajo_amd import scenes, sort
+    from bajo_amd.bvh import build_triangle_bvh
+    from bajo_amd.context import DeviceContext
+
+    announce(f"sort and rebuild one shorter than {n + 1}")
+    rng = np.random.default_rng(n)
+    keys = rng.integers(0, 2**64 - 1, n, dtype=np.uint64, endpoint=True)
+    ws = torch.empty(sort.sort_workspace_bytes(n + 1, 8, True), dtype=torch.uint8, device="cuda:0")
+    k, v = to_dev(keys), to_dev(np.arange(n, dtype=np.uint32))
+    sort.device_radix_sort_pairs(k, v, workspace=ws)
+    np.testing.assert_array_equal(to_host(v, np.uint32), np.argsort(keys, kind="stable"))
+
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        ctx = DeviceContext(0, stream)
+        mesh = torch.from_numpy(scenes.soup(n + 1, initstate=n, initseq=3)).to("cuda:0")
+        buf, small = mesh.clone(), to_dev(keys)
+        sort.device_radix_sort_keys(torch.cat([small, small[:1]]), ctx=ctx)
+        bvh = build_triangle_bvh(buf, ctx=ctx)
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            bvh.rebuild(buf[:9 * n])
+            sort.device_radix_sort_keys(small, ctx=ctx)
+        for step in range(3):
+            buf.copy_(mesh * (1.0 + 0.5 * step))
+            small.copy_(to_dev(np.roll(keys, step)))
+            graph.replay()
+            ctx.synchronize()
+            fresh = build_triangle_bvh(buf[:9 * n].clone(), ctx=ctx)
+            got, want = bvh.binary(), fresh.binary()
+            for key in ("sorted_keys", "leaf_ids", "node_meta", "leaf_parent", "node_bounds"):
+                np.testing.assert_array_equal(got[key], want[key], err_msg=f"{key}, replay {step}")
+            np.testing.assert_array_equal(to_host(small, np.uint64), np.sort(keys))
+            fresh.free()
+        bvh.free()
+        ctx.close()
