@@ -12,16 +12,26 @@
 // Unlike bajo's persistent work queue with a spin fail-safe, no wave here
 // waits on another block.  Two launches build the whole hierarchy:
 //   - one block opens the first levels, one per barrier round, until a level
-//     holds more nodes than the block has threads;
-//   - one block per CU then takes every gridDim-th node of that level and
-//     finishes their subtrees by itself: it keeps the index ranges of its
-//     nodes still to be opened on an LDS stack and reserves the nodes of each
-//     batch's children (a contiguous range) with one atomic.
+//     holds more nodes than the block has threads, then nodes with more leaves
+//     than a block's share, and deals out the nodes still to be opened: every
+//     gridDim-th to a block if that spreads the leaves evenly, else a run of
+//     them with a share of the leaves;
+//   - one block per CU then finishes its nodes' subtrees by itself: it keeps
+//     the index ranges of its nodes still to be opened on an LDS stack and
+//     reserves the nodes of each batch's children (a contiguous range) with
+//     one atomic.
+// No block of the second launch gets more than two shares, whatever the
+// geometry.  With 80 % of 4M triangles in a cube of 5 % of the scene's width a
+// deal by node number alone left 40 % of the nodes to one block: 7.62 ms, now
+// 0.28; 4,096 environments of 256 to 65,536 triangles 1.86 -> 1.24 ms.  Opening
+// and dealing costs an even mesh 5 us (4M: 177 -> 182; nearly all of it is code
+// fetched once: scans unrolled or with LDS atomics took 3 us more, leaf counts
+// read from memory instead of kept as nodes are reserved 5 us more).
 // A node's children are opened through a chain of up to seven dependent loads,
 // so a level costs its latency however few nodes it has.  One launch per level
 // (each followed by a launch that opened the next, with four to five spare
 // ones for the depth) took 22 launches of 5-31 us: 0.40 ms at 4M triangles
-// (LBVH), 0.26 ms at 1M (H-PLOC).  The two launches take 0.24 and 0.15 ms.
+// (LBVH), 0.26 ms at 1M (H-PLOC), where the two launches took 0.24 and 0.15.
 // The host reads nothing back, so the collapse is enqueue-only and can be
 // captured in a HIP graph.  Leaf children reference ranges of the sorted
 // triangle records that the refit already wrote (a subtree covers a contiguous
@@ -36,8 +46,14 @@ constexpr int kCollapseBlock = 1024;
 // keeps (one per level of its subtrees): a deeper tree raises
 // BAJO_STATUS_COLLAPSE_FAILED.
 constexpr uint32_t kLevelCap = 4096;
-// wide_ctl words: node counter, level range, status
-constexpr int kCtlCount = 0, kCtlBegin = 1, kCtlEnd = 2, kCtlStatus = 3;
+// Leaves of a subtree that one block finishes in a few batches: smaller ones
+// are not opened to spread them.
+constexpr uint32_t kSmallSubtree = 4096;
+// Blocks of the second launch at most: their runs are kept in one hand-over
+// slot block of the climb, which is free by then (kHandSlots 32-byte records).
+constexpr unsigned kMostBlocks = 1023;
+// wide_ctl words: node counter, range still to be opened, status, how the range is dealt
+constexpr int kCtlCount = 0, kCtlBegin = 1, kCtlEnd = 2, kCtlStatus = 3, kCtlRuns = 4;
 constexpr uint32_t kStatusOutOfNodes = 1, kStatusTooDeep = 2, kStatusBadRoot = 4;
 
 struct Child {
@@ -198,22 +214,50 @@ struct Batch {
   uint32_t failed;
 };
 
-// Opens the wide nodes begin + stride * threadIdx.x for threadIdx.x < len,
-// the whole block together: kShared reserves their children with one atomic on
+// Inclusive scan of one value per thread over the block.
+BJ_D uint32_t block_inclusive_scan(uint32_t v, uint32_t* __restrict__ wave_total) {
+  const uint32_t lane = lane_id(), wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t y = __shfl_up(v, off, 64);
+    if (lane >= (uint32_t)off) v += y;
+  }
+  if (lane == 63) wave_total[wave] = v;
+  __syncthreads();
+  for (uint32_t i = 0; i < wave; ++i) v += wave_total[i];
+  __syncthreads();
+  return v;
+}
+
+// Leaves below a wide node still to be opened (0: opened, or a segment's lone leaf).
+BJ_D uint32_t open_leaves(const uint32_t* __restrict__ wide_src, const uint32_t* __restrict__ leaf_counts, uint32_t w) {
+  const uint32_t src = wide_src[w];
+  return src != kSentinel ? leaf_counts[src] : 0u;
+}
+
+// Leaves below the nodes [origin, origin + kKnown) that the first launch has
+// reserved, kept in LDS as they are reserved; later ones are looked up.
+constexpr uint32_t kKnown = 12288;
+struct Leaves {
+  uint32_t of[kKnown];
+};
+
+// Opens each thread's wide node `w` (where `have`), the whole block together:
+// kShared reserves their children with one atomic on
 // the node counter (a per-node atomic serializes, about 25 ns each), a lone
-// block counts on in bt->first + bt->total.  Afterwards [bt->first,
+// block counts on in bt->first + bt->total and keeps the children's leaves in
+// `known`, from `origin` on.  Afterwards [bt->first,
 // bt->first + bt->total) are the children to be opened; bt->failed is set if
 // they do not fit.
 template <bool kKarras, bool kShared>
 BJ_D void collapse_batch(const BjNode* __restrict__ bnodes, const uint32_t* __restrict__ leaf_counts,
                          BjWide* __restrict__ wide, uint32_t* __restrict__ wide_src, uint32_t* __restrict__ ctl,
-                         uint32_t capacity, uint32_t max_leaf, int max_children, uint32_t begin, uint32_t stride,
-                         uint32_t len, Batch* __restrict__ bt) {
+                         uint32_t capacity, uint32_t max_leaf, int max_children, uint32_t w, bool have,
+                         Batch* __restrict__ bt, Leaves* __restrict__ known = nullptr, uint32_t origin = 0) {
   const uint32_t lane = lane_id();
   const uint32_t wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
   {
-    const uint32_t w = begin + stride * threadIdx.x;
-    const uint32_t src = threadIdx.x < len ? wide_src[w] : kSentinel;
+    const uint32_t src = have ? wide_src[w] : kSentinel;
     const bool active = src != kSentinel;
     // The children live in registers: every index into ch[] is a compile-time
     // constant (a data-dependent one would place the array in scratch memory).
@@ -345,6 +389,8 @@ BJ_D void collapse_batch(const BjNode* __restrict__ bnodes, const uint32_t* __re
         } else {
           child[i] = next;
           wide_src[next] = ref;
+          if constexpr (!kShared)
+            if (next - origin < kKnown) known->of[next - origin] = ch[i].count;
           ++next;
         }
       }
@@ -362,43 +408,125 @@ BJ_D void collapse_batch(const BjNode* __restrict__ bnodes, const uint32_t* __re
 }
 
 // The first levels, in one block.  `segmented`: level 0 (the segment roots)
-// is already in ctl.  Leaves the first level larger than the block (or an
-// empty range) in ctl.
+// is already in ctl.  Opens whole levels until one holds more nodes than the
+// block has threads, then nodes with more than `share` leaves (their subtrees
+// are disjoint, so fewer than n / share at a time).  Leaves the range that
+// holds the nodes still to be opened (or an empty range) in ctl, and how it is
+// dealt: every `blocks`-th node to a block if that is even (kCtlRuns 0), else
+// runs of equal numbers of leaves, in deal[0 .. blocks].
 template <bool kKarras>
 __global__ void __launch_bounds__(kCollapseBlock)
 collapse_top_kernel(const BjNode* __restrict__ bnodes, const uint32_t* __restrict__ leaf_counts,
                     BjWide* __restrict__ wide, uint32_t* __restrict__ wide_src, uint32_t* __restrict__ ctl,
                     uint32_t capacity, uint32_t max_leaf, int max_children, const float* __restrict__ scene,
                     uint32_t n, uint32_t root_binary, const uint32_t* __restrict__ root_dev, int segmented,
-                    uint32_t* __restrict__ status) {
+                    uint32_t share, uint32_t* __restrict__ deal, uint32_t blocks, uint32_t* __restrict__ status) {
   __shared__ Batch bt;
+  __shared__ Leaves known;
+  __shared__ uint32_t s_list[kCollapseBlock], s_word;
+  const uint32_t t = threadIdx.x;
   // the level being opened is [bt.first, bt.first + bt.total)
-  if (threadIdx.x == 0) {
+  if (t == 0) {
     bt.first = 0;
     bt.total = segmented ? ctl[kCtlEnd] : collapse_root(scene, n, root_binary, root_dev, wide, wide_src, ctl, status);
     bt.failed = 0;
   }
   __threadfence_block();
   __syncthreads();
-  uint32_t level = 0;
-  while (bt.total != 0 && bt.total <= blockDim.x && !bt.failed && level < kLevelCap) {
-    const uint32_t begin = bt.first, len = bt.total;
+  uint32_t level = 0, begin = 0;  // begin: of the nodes still to be opened
+  bool levels = true;             // whole levels so far
+  const auto leaves_of = [&](uint32_t i) {
+    return i < kKnown ? known.of[i] : open_leaves(wide_src, leaf_counts, begin + i);
+  };
+  for (;;) {
+    const uint32_t first = bt.first, len = bt.total;
+    if (len == 0 || bt.failed || level == kLevelCap) break;
+    uint32_t w = first + t, origin = first + len;
+    bool have = t < len;
+    if (levels && len > kCollapseBlock) {
+      levels = false;
+      begin = first;
+      if (level == 0)  // segment roots
+#pragma unroll 1
+        for (uint32_t i = t; i < len && i < kKnown; i += kCollapseBlock)
+          known.of[i] = open_leaves(wide_src, leaf_counts, begin + i);
+    }
+    if (!levels) {
+      // the last range's nodes above a share
+      if (t == 0) s_word = 0;
+      __syncthreads();
+#pragma unroll 1
+      for (uint32_t i = t; i < len; i += kCollapseBlock)
+        if (leaves_of(first - begin + i) > share) {
+          const uint32_t at = atomicAdd(&s_word, 1u);
+          if (at < kCollapseBlock) s_list[at] = first + i;
+        }
+      __syncthreads();
+      if (s_word == 0) break;
+      have = t < s_word;
+      w = have ? s_list[t] : first;
+      origin = begin;
+    }
     ++level;
     __syncthreads();
-    collapse_batch<kKarras, false>(bnodes, leaf_counts, wide, wide_src, ctl, capacity, max_leaf, max_children, begin,
-                                   1u, len, &bt);
+    collapse_batch<kKarras, false>(bnodes, leaf_counts, wide, wide_src, ctl, capacity, max_leaf, max_children, w,
+                                   have, &bt, &known, origin);
+    if (!levels && have) {
+      wide_src[w] = kSentinel;
+      if (w - begin < kKnown) known.of[w - begin] = 0;
+    }
     __threadfence_block();
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    uint32_t end = bt.first + bt.total;
-    if (bt.failed || (bt.total != 0 && level == kLevelCap)) {
+  if (levels) begin = bt.first;
+  const bool failed = bt.failed || (bt.total != 0 && level == kLevelCap);
+  const uint32_t len = failed ? 0u : bt.first + bt.total - begin;  // from `begin` on
+  // whether a block's share is too large when the nodes are dealt by number
+  uint32_t load = 0;
+  if (t < blocks)
+#pragma unroll 1
+    for (uint32_t i = t; i < len; i += blocks) load += leaves_of(i);
+  const bool runs = __syncthreads_or(load > share + share / 8) != 0;
+  if (runs) {
+    // node i belongs to block (leaves before i) * blocks / n
+    constexpr uint32_t kEach = 8;
+    uint32_t carry = 0;
+    for (uint32_t base = 0; base < len; base += kEach * kCollapseBlock) {
+      const uint32_t mine = base + kEach * t;
+      uint32_t leaves[kEach], sum = 0;
+#pragma unroll
+      for (uint32_t i = 0; i < kEach; ++i) {
+        leaves[i] = mine + i < len ? leaves_of(mine + i) : 0u;
+        sum += leaves[i];
+      }
+      const uint32_t incl = block_inclusive_scan(sum, bt.wave_total);
+      uint32_t before = carry + incl - sum;
+#pragma unroll
+      for (uint32_t i = 0; i < kEach; ++i) {
+        const uint32_t a = (uint32_t)((uint64_t)before * blocks / n);
+        const uint32_t b = (uint32_t)((uint64_t)(before + leaves[i]) * blocks / n);
+        for (uint32_t k = a + 1; k <= b && k <= blocks; ++k) deal[k] = begin + mine + i + 1;
+        before += leaves[i];
+      }
+      if (t == kCollapseBlock - 1) s_word = before;
+      __syncthreads();
+      carry = s_word;
+      __syncthreads();
+    }
+    if (t == 0) {
+      deal[0] = begin;
+      for (uint32_t k = (uint32_t)((uint64_t)carry * blocks / n) + 1; k <= blocks; ++k) deal[k] = begin + len;
+    }
+  }
+  if (t == 0) {
+    if (failed) {
       ctl[kCtlStatus] = bt.failed ? kStatusOutOfNodes : kStatusTooDeep;
       atomicMax(status, (uint32_t)BAJO_STATUS_COLLAPSE_FAILED);
-      end = bt.first;
     }
-    ctl[kCtlBegin] = bt.first;
+    const uint32_t end = failed ? bt.first : begin + len;
+    ctl[kCtlBegin] = end - len;
     ctl[kCtlEnd] = end;
+    ctl[kCtlRuns] = runs ? 1u : 0u;
     // a build without nodes to open still has its root record
     ctl[kCtlCount] = end > 0 ? end : 1u;
   }
@@ -409,61 +537,78 @@ template <bool kKarras>
 __global__ void __launch_bounds__(kCollapseBlock)
 collapse_subtree_kernel(const BjNode* __restrict__ bnodes, const uint32_t* __restrict__ leaf_counts,
                         BjWide* __restrict__ wide, uint32_t* __restrict__ wide_src, uint32_t* __restrict__ ctl,
-                        uint32_t capacity, uint32_t max_leaf, int max_children, uint32_t* __restrict__ status) {
+                        uint32_t capacity, uint32_t max_leaf, int max_children, const uint32_t* __restrict__ deal,
+                        uint32_t* __restrict__ status) {
   __shared__ Batch bt;
   __shared__ uint32_t s_first[kLevelCap], s_len[kLevelCap];
-  const uint32_t end = ctl[kCtlEnd];
-  for (uint32_t at = ctl[kCtlBegin] + blockIdx.x; at < end; at += gridDim.x * blockDim.x) {
-    const uint32_t left = (end - at + gridDim.x - 1) / gridDim.x;
-    uint32_t begin = at, stride = gridDim.x, len = left < blockDim.x ? left : blockDim.x;
-    int depth = 0;
-    for (;;) {
-      collapse_batch<kKarras, true>(bnodes, leaf_counts, wide, wide_src, ctl, capacity, max_leaf, max_children, begin,
-                                    stride, len, &bt);
-      __threadfence_block();
-      __syncthreads();
-      const bool full = bt.total != 0 && depth == (int)kLevelCap;
-      if (bt.failed || full) {
-        if (threadIdx.x == 0) {
-          atomicOr(ctl + kCtlStatus, full ? kStatusTooDeep : kStatusOutOfNodes);
-          atomicMax(status, (uint32_t)BAJO_STATUS_COLLAPSE_FAILED);
-        }
-        return;
-      }
-      if (bt.total != 0) {
-        if (threadIdx.x == 0) {
-          s_first[depth] = bt.first;
-          s_len[depth] = bt.total;
-        }
-        ++depth;
-      }
-      __syncthreads();
-      if (depth == 0) break;
-      // the next batch: up to a block's worth of the range on top
-      begin = s_first[depth - 1];
-      stride = 1;
-      const uint32_t range = s_len[depth - 1];
-      len = range < blockDim.x ? range : blockDim.x;
-      __syncthreads();
-      if (len == range) {
-        --depth;
-      } else if (threadIdx.x == 0) {
-        s_first[depth - 1] = begin + len;
-        s_len[depth - 1] = range - len;
-      }
+  const uint32_t begin = ctl[kCtlBegin], end = ctl[kCtlEnd];
+  if (begin == end) return;
+  // the block's nodes: share + stride * i, i < count; the bottom of the stack
+  // holds the range of i still to be opened, what lies above it node ranges
+  uint32_t share = begin + blockIdx.x, stride = gridDim.x, count = 0;
+  if (ctl[kCtlRuns]) {
+    share = deal[blockIdx.x];
+    stride = 1;
+    count = deal[blockIdx.x + 1] - share;
+  } else if (share < end) {
+    count = (end - share + stride - 1) / stride;
+  }
+  if (count == 0) return;
+  if (threadIdx.x == 0) {
+    s_first[0] = 0;
+    s_len[0] = count;
+  }
+  __syncthreads();
+  int depth = 1, bottom = 1;
+  while (depth > 0) {
+    // the next batch: up to a block's worth of the range on top
+    const uint32_t first = s_first[depth - 1], range = s_len[depth - 1];
+    const uint32_t len = range < blockDim.x ? range : blockDim.x;
+    const uint32_t w = depth == bottom ? share + stride * (first + threadIdx.x) : first + threadIdx.x;
+    __syncthreads();
+    if (len == range) {
+      if (depth == bottom) bottom = 0;
+      --depth;
+    } else if (threadIdx.x == 0) {
+      s_first[depth - 1] = first + len;
+      s_len[depth - 1] = range - len;
     }
+    collapse_batch<kKarras, true>(bnodes, leaf_counts, wide, wide_src, ctl, capacity, max_leaf, max_children, w,
+                                  threadIdx.x < len, &bt);
+    __threadfence_block();
+    __syncthreads();
+    const bool full = bt.total != 0 && depth == (int)kLevelCap;
+    if (bt.failed || full) {
+      if (threadIdx.x == 0) {
+        atomicOr(ctl + kCtlStatus, full ? kStatusTooDeep : kStatusOutOfNodes);
+        atomicMax(status, (uint32_t)BAJO_STATUS_COLLAPSE_FAILED);
+      }
+      return;
+    }
+    if (bt.total != 0) {
+      if (threadIdx.x == 0) {
+        s_first[depth] = bt.first;
+        s_len[depth] = bt.total;
+      }
+      ++depth;
+    }
+    __syncthreads();
   }
 }
 
 template <bool kKarras>
 void launch_collapse(bajo_ctx* ctx, bajo_bvh* h, const uint32_t* root_dev, unsigned blocks) {
   const uint32_t n = (uint32_t)h->n, capacity = (uint32_t)h->wide_capacity;
+  // a subtree of up to kSmallSubtree leaves is a few batches of one block
+  const uint32_t share = n / blocks > kSmallSubtree ? n / blocks : kSmallSubtree;
+  uint32_t* deal = static_cast<uint32_t*>(h->hands);  // free once the binary hierarchy stands
   collapse_top_kernel<kKarras><<<1, kCollapseBlock, 0, ctx->stream>>>(
       h->nodes, h->leaf_counts, h->wide, h->wide_src, h->wide_ctl, capacity, h->wide_leaf, h->node_width, h->scene, n,
-      n > 1 ? h->root : 0u, root_dev, h->seg_count ? 1 : 0, ctx->status);
+      n > 1 ? h->root : 0u, root_dev, h->seg_count ? 1 : 0, share, deal, blocks, ctx->status);
   if (n <= kCollapseBlock && !h->seg_count) return;  // no level can outgrow the first launch
   collapse_subtree_kernel<kKarras><<<blocks, kCollapseBlock, 0, ctx->stream>>>(
-      h->nodes, h->leaf_counts, h->wide, h->wide_src, h->wide_ctl, capacity, h->wide_leaf, h->node_width, ctx->status);
+      h->nodes, h->leaf_counts, h->wide, h->wide_src, h->wide_ctl, capacity, h->wide_leaf, h->node_width, deal,
+      ctx->status);
 }
 
 }  // namespace
@@ -486,8 +631,9 @@ int32_t collapse_wide(bajo_ctx* ctx, bajo_bvh* h) {
   } else if (n > 1 && h->root_on_device) {
     root_dev = h->hp_ctl + kHpCtlRoot;
   }
-  if (h->method == BAJO_BUILD_HPLOC) launch_collapse<false>(ctx, h, root_dev, (unsigned)cus);
-  else launch_collapse<true>(ctx, h, root_dev, (unsigned)cus);
+  const unsigned blocks = (unsigned)cus < kMostBlocks ? (unsigned)cus : kMostBlocks;
+  if (h->method == BAJO_BUILD_HPLOC) launch_collapse<false>(ctx, h, root_dev, blocks);
+  else launch_collapse<true>(ctx, h, root_dev, blocks);
   BJ_HIP(hipGetLastError());
   h->wide_pending = !(n == 1 && !h->seg_count);
   if (!h->wide_pending) h->wide_count = 1;

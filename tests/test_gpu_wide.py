@@ -252,3 +252,57 @@ def test_wide4_render_matches_oracle(gpu_ctx, name):
     assert rmse <= 1e-3 and exact > 0.99
     assert res.stats["extension_rays"] == rays[0] and res.stats["shadow_rays"] == rays[1]
     g.free()
+
+
+def clustered(n, width, seed):
+    """80 % of the triangles in a cube of `width` times the scene's, with edges to match."""
+    rng = np.random.default_rng(seed)
+    v0 = rng.random((n, 3), dtype=np.float32)
+    e = (rng.random((n, 2, 3), dtype=np.float32) - 0.5) * 0.02
+    m = n * 4 // 5
+    v0[:m] = 0.37 + width * v0[:m]
+    e[:m] *= width
+    order = rng.permutation(n)
+    return np.concatenate([v0, v0 + e[:, 0], v0 + e[:, 1]], axis=1).astype(np.float32)[order].reshape(-1)
+
+
+@pytest.mark.parametrize("width", [0.05, 0.01])
+@pytest.mark.parametrize("method", [0, 1], ids=["lbvh", "hploc"])
+def test_wide_structure_of_a_mesh_with_a_dense_part(gpu_ctx, width, method):
+    """Subtrees of very different sizes: the first launch opens those above a block's share and deals the rest out by
+    leaves; whichever block finishes which, the layout is the oracle's."""
+    from bajo_amd.bvh import build_triangle_bvh
+
+    n = 200_000
+    announce(f"wide build with a dense part, width {width}, method {method}")
+    v = clustered(n, width, 17)
+    bvh = build_triangle_bvh(to_dev(v), node_width=8, leaf_size=4, method=method,
+                             merging_threshold=16 if method else 0)
+    binary = oracle.build_hploc(v, 16) if method else oracle.build_lbvh(v)
+    got, want = bvh.wide(), oracle.collapse_wide(binary, 4)
+    assert len(got) == len(want)
+    assert oracle.canonical_wide(got).tobytes() == oracle.canonical_wide(want).tobytes()
+    gpu_ctx.synchronize()
+    bvh.free()
+
+
+@pytest.mark.parametrize("count", [5, 1023, 1024, 1025, 3000])
+def test_wide_sets_with_one_large_segment(gpu_ctx, count):
+    """More and fewer segments than the first launch has threads, one of them with most of the triangles."""
+    from bajo_amd.bvh import build_triangle_blas_set_flat
+
+    announce(f"wide set of {count} segments, one large")
+    rng = np.random.default_rng(count)
+    sizes = rng.integers(1, 40, count)
+    sizes[count // 3] = 60_000
+    offsets = np.concatenate([[0], np.cumsum(sizes)]).astype(np.uint64)
+    v = soup(int(offsets[-1]), count)
+    bset = build_triangle_blas_set_flat(to_dev(v), offsets, node_width=8, leaf_size=4)
+    gpu_ctx.synchronize()
+    for s in (0, count // 3 - 1, count // 3, count // 3 + 1, count - 1):
+        mine = v[9 * int(offsets[s]):9 * int(offsets[s + 1])]
+        got = bset.blas(s).wide()
+        want = oracle.collapse_wide(oracle.build_lbvh(mine), 4)
+        assert len(got) == len(want), s
+        assert oracle.canonical_wide(got).tobytes() == oracle.canonical_wide(want).tobytes(), s
+    bset.free()
