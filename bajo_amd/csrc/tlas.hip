@@ -26,6 +26,7 @@
 //     by the caller.
 #include <vector>
 
+#include "pixel_order.h"
 #include "traverse.h"
 
 struct TlasBlas {
@@ -197,27 +198,6 @@ BJ_D Hit tlas_trace(const TlasView& tv, const Ray& ray, Stack& st, uint32_t* ts,
     if (hit.prim != kEmpty) hit.n = normal_from_inverse(tv.inv + 12 * (uint64_t)hit.inst, hit.n);
     return hit;
   }
-}
-
-// The pixel that index r of a camera launch of R rays traces: views in order,
-// a view in tiles of 8 x 8 pixels (narrower and lower ones at its right and
-// bottom edges), so that a wave's rays stay close together and walk the same
-// nodes (256 instances of a 67,280-triangle mesh, three 640 x 360 views: 426
-// us against 482 row by row).  A view that the launch cuts short is traced
-// row by row.
-BJ_D uint64_t camera_pixel(uint64_t r, uint64_t R, uint32_t w, uint32_t h) {
-  const uint64_t ppv = (uint64_t)w * h;
-  const uint64_t start = r / ppv * ppv;
-  if (start + ppv > R) return r;
-  uint32_t k = (uint32_t)(r - start);
-  const uint32_t band = k / (8u * w);
-  k -= band * 8u * w;
-  const uint32_t rows = h - 8u * band < 8u ? h - 8u * band : 8u;
-  const uint32_t tile = k / (8u * rows);
-  k -= tile * 8u * rows;
-  const uint32_t cols = w - 8u * tile < 8u ? w - 8u * tile : 8u;
-  const uint32_t y = k / cols, x = k - y * cols;
-  return start + (uint64_t)(8u * band + y) * w + 8u * tile + x;
 }
 
 template <int kMode, bool kCamera, bool kPlain8>
