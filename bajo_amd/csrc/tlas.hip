@@ -26,8 +26,8 @@
 //     by the caller.
 #include <vector>
 
-#include "pixel_order.h"
 #include "traverse.h"
+#include "pixel_order.h"
 
 struct TlasBlas {
   bj::BvhView bin;
