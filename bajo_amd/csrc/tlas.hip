@@ -9,8 +9,11 @@
 //   - the top level is this library's box builder (bajo_build_binary_bounds)
 //     over the instances' world boxes, so it is the same LBVH / H-PLOC
 //     layout the parity tests already pin;
-//   - one persistent grid takes 64 rays per wave at a time from a counter and
-//     walks the top level near-first; at an instance
+//   - one resident grid strides over the rays and walks the top level
+//     near-first (64 rays per wave at a time from a counter cost an atomic on
+//     one word per 64 rays, 0.27 ms under 691,200 rays of any length: 64
+//     instances of which the view hits few took 0.27 ms, now 0.10); at an
+//     instance
 //     leaf the ray is mapped into BLAS space with the inverse transform (t is
 //     unchanged) and the BLAS, binary or 8-wide, is traversed with the same
 //     code as a plain launch, its stack in LDS; the top-level stack is a
@@ -18,9 +21,8 @@
 //   - bound by the walks' latency at few waves and by lanes waiting for each
 //     other: with one BLAS visit in the code (it stood at three places), the
 //     all-wide-triangles case compiled by itself and six waves per SIMD (the
-//     stacks' LDS allows no more) 256 instances and 691,200 rays take 391 us
-//     (697 at two waves; 440 at three, 420 at five; the counter measured the
-//     same as a grid stride here, 391 against 397);
+//     stacks' LDS allows no more) 256 instances and 691,200 rays take 380 us
+//     (697 at two waves; 440 at three, 420 at five);
 //   - instance transforms, BLAS views and instance-to-BLAS indices live in
 //     device arrays uploaded once at creation; the BLAS handles stay owned
 //     by the caller.
@@ -204,20 +206,13 @@ template <int kMode, bool kCamera, bool kPlain8>
 __global__ void __attribute__((amdgpu_waves_per_eu(6))) __launch_bounds__(kTraceBlock) tlas_kernel(const TlasView tv, const float* __restrict__ rays,
                                                            const float* __restrict__ cams, uint32_t cam_w,
                                                            uint32_t cam_h, float inv_height, float* __restrict__ hits,
-                                                           uint64_t R, uint32_t* __restrict__ counter,
-                                                           uint32_t* __restrict__ tstack,
+                                                           uint64_t R, uint32_t* __restrict__ tstack,
                                                            uint32_t* __restrict__ spill) {
   __shared__ uint32_t s_stack[kLdsStack * kTraceBlock];
   const uint64_t gtid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const uint64_t threads = (uint64_t)gridDim.x * blockDim.x;
   Stack st{s_stack + threadIdx.x, spill + gtid, threads, 0};
-  for (;;) {
-    uint32_t base = 0;
-    if (lane_id() == 0) base = atomicAdd(counter, 64u);
-    base = __shfl(base, 0, 64);
-    if ((uint64_t)base >= R) break;
-    const uint64_t k = (uint64_t)base + lane_id();
-    if (k >= R) continue;
+  for (uint64_t k = gtid; k < R; k += threads) {
     const uint64_t r = kCamera ? camera_pixel(k, R, cam_w, cam_h) : k;
     Ray ray;
     if constexpr (kCamera) {
@@ -232,8 +227,8 @@ __global__ void __attribute__((amdgpu_waves_per_eu(6))) __launch_bounds__(kTrace
   }
 }
 
-__global__ void tlas_init_kernel(uint32_t* status, uint32_t* counter) {
-  if (threadIdx.x == 0) { *status = 0; *counter = 0; }
+__global__ void tlas_status_kernel(uint32_t* status) {
+  if (threadIdx.x == 0) *status = 0;
 }
 
 // Affine3.inverse (core/transform.mojo:290-340): adjugate over the
@@ -304,17 +299,16 @@ int32_t launch_tlas_as(bajo_ctx* ctx, const bajo_tlas* t, const float* rays, con
   if (grid < 1) grid = 1;
   const uint64_t threads = (uint64_t)grid * kTraceBlock;
   void* scratch = nullptr;
-  int32_t rc = ctx_scratch(ctx, (64 + threads * (kSpill + kTlasStack)) * sizeof(uint32_t), &scratch);
+  int32_t rc = ctx_scratch(ctx, threads * (kSpill + kTlasStack) * sizeof(uint32_t), &scratch);
   if (rc) return rc;
-  uint32_t* counter = (uint32_t*)scratch;
-  uint32_t* spill = counter + 64;
+  uint32_t* spill = (uint32_t*)scratch;
   uint32_t* tstack = spill + threads * kSpill;
   const bajo_bvh* top = t->top;
   TlasView tv{top->nodes, top->keys, top->root, (uint32_t)(top->n - 1), t->instance_count, t->inv, t->inst_blas,
               t->blas, t->status};
-  tlas_init_kernel<<<1, 64, 0, ctx->stream>>>(t->status, counter);
+  tlas_status_kernel<<<1, 64, 0, ctx->stream>>>(t->status);
   tlas_kernel<kMode, kCamera, kPlain8><<<grid, kTraceBlock, 0, ctx->stream>>>(tv, rays, cams, w, hh, hh ? 1.0f / (float)hh : 0.0f,
-                                                                    hits, R, counter, tstack, spill);
+                                                                    hits, R, tstack, spill);
   BJ_HIP(hipGetLastError());
   return BAJO_OK;
 }
