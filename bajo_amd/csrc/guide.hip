@@ -490,6 +490,9 @@ BJ_D void gradient_tiles(const uint4* ex, int a, const int (&b)[kN], float* part
   for (int t = 0; t < kN; ++t) *(f32x4*)(at + 256 * t) = acc[t];
 }
 
+// Inputs below this have finite features at every frequency.
+constexpr float kLargeInput = 1e30f;
+
 // One launch per batch, 256 samples per block and pass.  Latency bound: one
 // wave's chain of four layers, the loss and three layers back, then three
 // exchanges.  65,521 samples: 38 us; 85 + 62 us as a pass that wrote
@@ -499,6 +502,8 @@ __global__ void __launch_bounds__(kTrainWaves * 64) guide_train_kernel(const uin
   __shared__ __attribute__((aligned(16))) uint8_t s_mem[kExchangeBytes];
   __shared__ __attribute__((aligned(16))) float s_b[kBiasFloats];
   __shared__ float s_loss[kTrainWaves * 2][2];
+  __shared__ uint32_t s_nan;  // chunks of the features that were not numbers
+  if (threadIdx.x == 0) s_nan = 0;
   uint16_t* s_w = (uint16_t*)s_mem;
   uint4* ex = (uint4*)s_mem;
   float* part = ta.part + (size_t)blockIdx.x * kTiles * 256;
@@ -523,6 +528,22 @@ __global__ void __launch_bounds__(kTrainWaves * 64) guide_train_kernel(const uin
       sp[u] = ta.samples + row * kGuideSampleFloats;
 #pragma unroll
       for (int s = 0; s < 7; ++s) x[u][s] = real[u] ? sp[u][chunk_input(s, g)] : 0.0f;
+    }
+    // Chunks of features that are not numbers are marked.  Their sample's
+    // hidden units are off (ReLU of a NaN is 0), so nothing but the weights of
+    // the chunk's own columns depends on them.
+    bool large = false;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int s = 0; s < 7; ++s) large = large || !(fabsf(x[u][s]) < kLargeInput);
+    if (ballot(large) != 0) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int s = 0; s < 7; ++s)
+          if (!(fabsf(x[u][s] * sc[s % 3]) < __builtin_inff()) && 4 * s + (int)g < 27)
+            atomicOr(&s_nan, 1u << (4 * s + g));
     }
     bf16x8 h1t[4], h2t[4], h3t[4];
     bf16x8 h1[2][2], h2[2][2], h3[2][2];
@@ -558,7 +579,7 @@ __global__ void __launch_bounds__(kTrainWaves * 64) guide_train_kernel(const uin
     f32x4 o[2][3];
     start_bias<3>(s_b + 192, o, g);
     layer64<3>(s_w + kPackW4, h3, o, lane);
-__builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_sched_barrier(0);
     // outputs to rows of samples; a sample's four lanes take two lobes each
     bf16x8 dof[2][2], dot[3], d3t[4], d2t[4], d1t[4];
 #pragma unroll
@@ -607,7 +628,7 @@ __builtin_amdgcn_sched_barrier(0);
         dot[k] = to_frag(c[0], c[1]);
       }
     }
-__builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_sched_barrier(0);
     // backward: d3 = W4^T dO, masked by h3; then d2, d1 (its transpose only)
     bf16x8 d3[2][2], d2[2][2];
     backward_both(s_w + kPackW4t, dof, h3, h3t, d3, d3t, lane);
@@ -624,7 +645,7 @@ __builtin_amdgcn_sched_barrier(0);
       }
       d1t[k] = masked(to_frag(t[0], t[1]), h1t[k]);
     }
-__builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_sched_barrier(0);
     // weight gradients; each exchange waits for the last one's readers
     const auto put = [&](int f, bf16x8 v) { ex[(f * kTrainWaves + wave) * 64 + lane] = __builtin_bit_cast(uint4, v); };
     __syncthreads();
@@ -634,11 +655,17 @@ __builtin_amdgcn_sched_barrier(0);
         block_l += (double)s_loss[k][1];
       }
     // the features' transpose is their product with unit columns (encoded
-    // again: kept from layer 1 they would not fit the registers)
+    // again: kept from layer 1 they would not fit the registers).  It would
+    // spread a feature that is not a number over its block of 32: an input
+    // that has some counts as 0 here (from 2^24 turns on the finite features
+    // are those of 0), and the columns marked above are set below.
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int s = 0; s < 7; ++s) asm volatile("" : "+v"(x[u][s]));
+      for (int s = 0; s < 7; ++s) {
+        asm volatile("" : "+v"(x[u][s]));
+        x[u][s] = fabsf(x[u][s]) < kLargeInput ? x[u][s] : 0.0f;
+      }
     bf16x8 unit[2];
 #pragma unroll
     for (int half = 0; half < 2; ++half)
@@ -662,12 +689,17 @@ __builtin_amdgcn_sched_barrier(0);
       const int m = (int)wave & 3, c = 7 * ((int)wave >> 2);
       const int b[7] = {c, c + 1, c + 2, c + 3, c + 4, c + 5, c + 6};
       gradient_tiles<7>(ex, 14 + m, b, part, kT1 + 14 * m + c, add, lane);
+      const uint32_t nans = s_nan;
+      if (nans)
+        for (int t = 0; t < 7; ++t)
+          if ((nans >> (2u * (uint32_t)(c + t) + (i >> 3))) & 1u)  // chunk of column 16 (c + t) + i
+            for (int r = 0; r < 4; ++r) part[(size_t)(kT1 + 14 * m + c + t) * 256 + lane * 4 + r] = __builtin_nanf("");
     }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       __builtin_amdgcn_sched_barrier(0);
-put(k, h1t[k]);
+      put(k, h1t[k]);
       put(4 + k, h2t[k]);
       put(8 + k, d2t[k]);
       put(12 + k, d3t[k]);

@@ -174,3 +174,22 @@ def test_gradient_of_a_batch_in_several_passes(gpu_ctx):
     assert np.linalg.norm(whole - want) < 1e-5 * np.linalg.norm(want)
     assert abs(loss - (la * wa + lb * wb) / w) < 1e-6 * abs(loss)
     g.free()
+
+
+@pytest.mark.parametrize("column", [0, 3, 8])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_gradient_with_an_input_that_is_not_finite(gpu_ctx, column, value):
+    """One sample's input is not a number: its 24 features' columns of the first layer are not numbers, the rest of
+    the gradient is (the sample's hidden units are off, ReLU of a NaN being 0)."""
+    announce(f"guide gradient, input {column} = {value}")
+    rng = np.random.default_rng(5)
+    g = make_guide(gpu_ctx, batch_size=2048)
+    g.set_params(random_params(rng).astype(np.float32))
+    s = random_samples(700, rng)
+    s[333, column] = value
+    grad, _ = g.gradient(torch.from_numpy(s).cuda())
+    bad = ~np.isfinite(grad.cpu().numpy())
+    want = np.zeros(bad.size, bool)
+    want[:64 * 216].reshape(64, 216)[:, 24 * column:24 * column + 24] = True
+    np.testing.assert_array_equal(bad, want)
+    g.free()
