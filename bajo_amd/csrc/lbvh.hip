@@ -297,8 +297,9 @@ BJ_D uint32_t segment_at(const uint64_t* __restrict__ off, const uint32_t* __res
   return s;
 }
 
-// Topology and boxes of the LBVH in one bottom-up pass, one thread per sorted
-// leaf.  The common prefixes d(i) of neighbouring keys i, i + 1 decide the
+// Topology and boxes of the LBVH in one bottom-up pass (the construction of
+// Apetrei, "Fast and Simple Agglomerative LBVH Construction", 2014), one
+// thread per sorted leaf.  The common prefixes d(i) of neighbouring keys i, i + 1 decide the
 // hierarchy: the parent of the node over [l, r] splits at r if
 // d(r) > d(l - 1) (the node is its left child), else at l - 1; the two never
 // tie, because keys are unique ((code << 32) | sorted position).  Both

@@ -1360,6 +1360,9 @@ __global__ void __launch_bounds__(kRtBlock) shadow_group_kernel(SceneView sc, Qu
   for (;;) {
     if (!have && idx < count) {
       // the ray's planes now, its radiance planes (8..10) and id after the walk
+      // (frames without a tail, against every plane first and the earlier walk:
+      // ambient occlusion of a 600,000-triangle mesh, 640 x 360 x 2, 422 us and
+      // 435; next-event estimation to depth 1 321 and 319)
       float f[8];
 #pragma unroll
       for (int p = 0; p < 8; ++p) f[p] = q.shadow_fields[plane_at<kShadowPlanes>(idx, p)];

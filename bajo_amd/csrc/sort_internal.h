@@ -42,7 +42,8 @@ struct SortPlan {
 // Smaller tiles for shorter lists: a pass lasts as long as a tile's chain, so
 // the keys are spread over the chip (64-bit pairs with 16 tiles per group:
 // 262,144 keys 105.9 us with 4 keys per thread, 115.3 with 8; 1M 163 with 8,
-// 186 with 16; 2M 258 and 262; 4M 451 and 402).
+// 186 with 16; 2M 258 and 262; 4M 451 and 402; the call's own figures are
+// lower by now, 4M 262).
 constexpr uint64_t kSortKpt4Keys = 262144, kSortKpt8Keys = 1310720;
 
 SortPlan make_sort_plan(uint64_t n, int key_bytes, int has_values, int begin_bit, int end_bit);

@@ -199,10 +199,10 @@ int32_t bajo_build_triangle_bvh(bajo_ctx* ctx, const float* vertices, uint64_t n
  * triangle records), child boxes are stored on a per-axis power-of-two grid
  * and padded by one grid step.  Every build is enqueue-only: nothing is read
  * back and the host never waits (without `timings`), so a rebuild can be
- * captured into a HIP graph once its buffers are allocated.  The collapse
- * runs a depth-bounded number of level launches (a launch past the last
- * level does nothing) and a single-block kernel for any deeper levels; the
- * wide node count is read back at the first bajo_bvh_get_info.  Failures
+ * captured into a HIP graph once its buffers are allocated (they serve every
+ * build of no more triangles).  The collapse is two launches: one block opens
+ * the first levels and the largest subtrees, one block per CU finishes the
+ * rest; the wide node count is read back at the first bajo_bvh_get_info.  Failures
  * raise BAJO_STATUS_* into the context status word.  `options` NULL =
  * binary LBVH.  n < 2^28 for widths 4 and 8. */
 int32_t bajo_build_triangle_bvh_ex(bajo_ctx* ctx, const float* vertices, uint64_t n,

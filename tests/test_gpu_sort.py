@@ -115,10 +115,10 @@ def test_sort_with_caller_workspace(gpu_ctx):
 
 
 def test_lookback_give_up_is_reported_never_silent(gpu_ctx):
-    """The look-back wait is capped; a tile past the cap raises BAJO_STATUS_SORT_LOOKBACK.
-    With the cap forced to 1 spin from the host (every kernel still exits normally), a
-    multi-tile sort either comes out right or reports the status: never silently wrong.
-    With the default cap the same sort is right and reports nothing."""
+    """The look-back wait is capped; a tile past the cap counts its predecessors itself (it
+    used to raise BAJO_STATUS_SORT_LOOKBACK).  With the cap forced to 1 spin from the host
+    (every kernel still exits normally), a multi-tile sort is never silently wrong; with the
+    default cap the same sort is right and reports nothing."""
     from bajo_amd import sort
     from bajo_amd._lib import BAJO_STATUS_SORT_LOOKBACK
     from bajo_amd.context import DeviceContext

@@ -1,9 +1,9 @@
 """The lane-group tail gives the per-lane tail's images bit for bit.
 
 The tail kernel carries a chunk's last paths through its remaining bounces.  With `tail_group = 16`
-(or 32, 64) each path gets that many lanes: the extension ray through GroupClosest (which defers to Walk8 when two
-candidates lie within rounding of each other, since Walk8's winner can then depend on test order),
-shading on the group's leader, the shadow ray through GroupWalk.  Images must equal the one-lane
+(or 32, 64) each path gets that many lanes: the extension ray through GroupWalk8 (which defers to the
+ordered walk, OrderedWalk8, when two candidates lie within rounding of each other, since the winner can then
+depend on test order), shading on the group's leader, the shadow ray through its any-hit form.  Images must equal the one-lane
 tail's, and the ray counts the oracle's (bajo's wavefront protocol, test/rt/test_gpu.mojo:346-730).
 A scene whose every triangle is duplicated with a different albedo makes every hit an exact tie,
 so the deferred path decides every pixel there."""
