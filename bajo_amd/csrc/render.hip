@@ -87,8 +87,26 @@ constexpr uint32_t kGroupShadowRays = 1u << 19;
 // and 5.45 (5.91 one lane per path, 6.48 wavefront).  With 149,294 paths the
 // one-lane tail took 1.54 ms a frame against 1.00 with the bounce traced by
 // the wavefront and the tail taking the 959 paths left.)
+//
+// Small chunks can stay between for whole bounces.  In a chunk of at most six
+// times the paths the tail takes (one launch more per bounce, so not in one
+// whose paths are hardly ever more than kLanePerPath after a bounce), one lane
+// per path follows on 16 at kLanePerPath: in PATH renders, whose tails have no
+// shadow rays (600,000 triangles, 66,000 camera paths to depth 6 685 us with
+// 16 lanes, 584 with one; NEE to depth 4 712 and 767), and in scenes of few
+// triangles, whose walks are short, and there up to kSmallScenePaths, if at
+// the first bounce or with kSmallSceneBounces to go.  (us, 16 lanes or wavefront against one lane:
+// material box, MIS to depth 3, 52,272 paths 644 and 325, depth 8 757 and 556;
+// 131,000 to depth 8, after a bounce, 1,050 and 752, to depth 3 452 and 502;
+// box, PATH, 98,000: 531 and 208; 2,500 triangles, PATH, 131,000 camera paths
+// 379 and 244; 20,000 triangles, 98,000 camera paths to depth 5, NEE: 405, 610.
+// Below kLanePerPath 16 lanes: material box, depth 8, 20,000: 442 and 515.)
 constexpr uint32_t kWideTailPaths = 2048;
 constexpr uint32_t kGroupTailPaths = 49152;
+constexpr uint32_t kLanePerPath = 32768;
+constexpr uint64_t kSmallScene = 8192;
+constexpr uint32_t kSmallScenePaths = 98304;
+constexpr uint32_t kSmallSceneBounces = 3;
 constexpr int kCounterWords = 16;
 constexpr uint32_t kStatusPathOverflow = 1, kStatusShadowOverflow = 3;
 constexpr int kMaxBounces = 64;
@@ -1921,6 +1939,11 @@ int32_t run_render(bajo_ctx* ctx, bajo_scene* s, RenderArena& a, const bajo_rend
   const uint32_t depth = (kAlg == BAJO_RENDER_NORMALS || kAlg == BAJO_RENDER_AO) ? 1u : st->max_depth;
   for (uint64_t begin = 0; begin < total; begin += cap) {
     const uint32_t chunk = (uint32_t)((total - begin) < cap ? (total - begin) : cap);
+    const bool small_scene = s->n <= kSmallScene;
+    const uint32_t most = small_scene ? kSmallScenePaths : kGroupTailPaths;
+    const bool lane_per_path = kGroupTail && st->tail_group == 0 && !st->tail_paths && chunk <= 6u * most &&
+                               chunk > kLanePerPath + kLanePerPath / 4 &&
+                               (small_scene || kAlg == BAJO_RENDER_PATH);
     init_counters_kernel<<<1, 64, 0, stream>>>(a.counters, chunk, a.stats, begin == 0);
     BJ_HIP(hipGetLastError());
     for (uint32_t b = 0; b < depth; ++b) {
@@ -1934,6 +1957,11 @@ int32_t run_render(bajo_ctx* ctx, bajo_scene* s, RenderArena& a, const bajo_rend
       if (ev) { ev->mark(ev->ext, stream); }
       if constexpr (kTail) {
         if (b > 0) {
+          uint32_t tail_paths = tail_threshold, group_paths = group_hi;
+          if (lane_per_path) {
+            tail_paths = b == 1 || depth - b >= kSmallSceneBounces ? most : kGroupTailPaths;
+            group_paths = kLanePerPath;
+          }
           if constexpr (kGroupTail) {
             constexpr int kTG = kGroupTail ? kGeo : kGeoTriangles;
             if (wide_hi && wide_lanes == 32)
@@ -1943,18 +1971,18 @@ int32_t run_render(bajo_ctx* ctx, bajo_scene* s, RenderArena& a, const bajo_rend
               tail_group_kernel<kAlg, kTG, 64><<<g_tgroup, kRtBlock, 0, stream>>>(sv, q, st->rng_seed, b, depth, 0u,
                                                                                  wide_hi, a.stats);
             const uint32_t lo16 = wide_lanes == 16 ? 0u : wide_hi;
-            if (group_hi > lo16)
+            if (group_paths > lo16)
               tail_group_kernel<kAlg, kTG, 16><<<g_tgroup, kRtBlock, 0, stream>>>(sv, q, st->rng_seed, b, depth, lo16,
-                                                                                 group_hi, a.stats);
+                                                                                 group_paths, a.stats);
           }
-          if (tail_threshold > group_hi)
-            tail_kernel<kAlg, kWide, kGeo><<<g_tail, kRtBlock, 0, stream>>>(sv, q, st->rng_seed, b, depth, group_hi,
-                                                                      tail_threshold, simds, a.stats, a.spill);
+          if (tail_paths > group_paths)
+            tail_kernel<kAlg, kWide, kGeo><<<g_tail, kRtBlock, 0, stream>>>(sv, q, st->rng_seed, b, depth, group_paths,
+                                                                      tail_paths, simds, a.stats, a.spill);
           BJ_HIP(hipGetLastError());
           // a chunk no larger than the threshold ends in this tail: nothing is
           // left to launch for its later bounces (the material box at
           // 160 x 120 x 2 spp, depth 8, launched 48 kernels that returned at once)
-          if (chunk <= tail_threshold) {
+          if (chunk <= tail_paths) {
             if (ev) {
               // the event pairs of the launches left out
               const bool shadows = kAlg != BAJO_RENDER_PATH && kAlg != BAJO_RENDER_NORMALS;

@@ -53,7 +53,8 @@ class RenderSettings:
     max_depth: int = 8
     path_capacity: int = 0  # paths in flight per chunk; 0 = the whole frame
     extend_waves: int = 0  # occupancy of the bounce >= 1 extension kernel: 4, 6 or 8 waves per SIMD; 0 = 6
-    # live paths at which the tail kernel takes over; 0 = 49,152 with the default tail_group, else its resident threads
+    # live paths at which the tail kernel takes over; 0 = 49,152 (98,304 in small scenes) with the default
+    # tail_group, else its resident threads
     tail_paths: int = 0
     shadow_walk: int = 0  # shadow any-hit walk: 1 one node, 2 two nodes, 3 / 4 with 4-record leaf loads; 0 = default
     sparse_shadow_rays: int = 0  # shadow rays per bounce traced one per wave at or below; 0 = 8192, 2**32-1 never

@@ -373,7 +373,9 @@ typedef struct bajo_scene bajo_scene;
  *     MIS over 4- and 8-wide triangle and batch scenes (others ignore it);
  *   tail_paths: live paths at or below which the tail kernel finishes the
  *     chunk's remaining bounces in one launch (0 = 49,152 where the default
- *     tail_group applies, else the tail grid's resident threads);
+ *     tail_group applies, 98,304 in scenes of at most 8,192 triangles and
+ *     chunks of at most six times that, else the tail grid's resident
+ *     threads);
  *   shadow_walk: the 4- and 8-wide any-hit walk of the shadow-ray kernel:
  *     1 = one node per step with one leaf record loaded ahead, 2 = two nodes
  *     per step (the stack top with the current node), 3 = one node with leaf
@@ -390,7 +392,9 @@ typedef struct bajo_scene bajo_scene;
  *     and batch scenes): 1 = one lane per path, 16, 32 or 64 = that many
  *     (extension rays by a group walk equal to the one-lane walk, shadow
  *     rays by group any hit; one node per 8 lanes per step); 0 = 32 up to
- *     2,048 live paths, 16 up to 49,152, one beyond. */
+ *     2,048 live paths, 16 up to 49,152 (32,768 in PATH renders and small
+ *     scenes, in chunks of at most six times the paths the tail takes), one
+ *     beyond. */
 typedef struct {
   uint32_t image_width, image_height, samples_per_pixel, max_depth;
   uint64_t rng_seed;

@@ -98,3 +98,31 @@ def test_tail_groups_icosphere_and_batch(gpu_ctx):
         b = enqueue_render_gpu(replace(base, tail_group=tg), bcam, gb, NEE).numpy()
         np.testing.assert_array_equal(a, b, err_msg=f"tail_group {tg}")
     gb.free()
+
+
+@pytest.mark.parametrize("scene", ["materials", "mesh"])
+@pytest.mark.parametrize("w,h,spp", [(128, 128, 2), (54, 121, 8), (128, 96, 8), (160, 100, 7), (256, 193, 8)])
+def test_default_tail_at_its_edges(gpu_ctx, scene, w, h, spp):
+    """Chunks of 32,768 to 395,264 paths, about where the default tail changes from 16 lanes to one lane per path and
+    to the wavefront, in a scene of few triangles and one of many: the wavefront's image."""
+    from bajo_amd import scenes
+    from bajo_amd.bvh import Camera
+    from bajo_amd.rt import MAT, GpuScene, RenderSettings, SceneData, enqueue_render_gpu
+
+    announce(f"default tail {scene} {w}x{h}x{spp}")
+    if scene == "materials":
+        data = scenes.material_box_scene()
+        cam = Camera((0.0, 1.0, -3.0), (0.0, 0.9, 0.0), (0.0, 1.0, 0.0), 0.5).flatten()
+    else:
+        v = scenes.soup(9000, initstate=4, edge_min=0.02, edge_max=0.1)
+        light = scenes.quad((0.2, 1.5, 0.2), (0.8, 1.5, 0.2), (0.8, 1.5, 0.8), (0.2, 1.5, 0.8))
+        surf = np.concatenate([np.full(9000, MAT.LAMBERTIAN << 28, np.uint32), np.full(2, MAT.EMISSIVE << 28, np.uint32)])
+        data = SceneData(np.concatenate([v, light]), surf, np.full(3, 0.7, np.float32), np.full(3, 9.0, np.float32))
+        cam = Camera((0.5, 0.5, -1.5), (0.5, 0.5, 0.5), (0.0, 1.0, 0.0), 0.41421356).flatten()
+    g = GpuScene(data, gpu_ctx, node_width=8)
+    for alg, depth in ((NEE, 4), (PATH, 6)):
+        base = RenderSettings(w, h, spp, 99, depth)
+        got = enqueue_render_gpu(base, cam, g, alg).numpy()
+        want = enqueue_render_gpu(replace(base, tail_paths=1), cam, g, alg).numpy()
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    g.free()
