@@ -291,14 +291,25 @@ int32_t occupancy_grid(unsigned* grid) {
 // 8-wide any 16,384: 194 -> 31, 131,072: 214 -> 165, 262,144: 289 -> 306;
 // binary closest 4,096: 377 -> 43, 16,384: 395 -> 66, 65,536: 405 -> 160,
 // 131,072: 437 -> 306, 262,144: 515 -> 475, 524,288: 471 -> 622 (camera).
-int lanes_per_ray(bool wide, bool any, uint64_t R) {
+// Rays through few triangles have short chains, and the wider form stops
+// paying earlier: 22,000 camera rays over a 300-triangle ball 36 us with one
+// lane, 46 with 64 and 17 with 8 (12,000 triangles 99, 66 and 34; a million
+// scattered 582, 98 and 175); binary, 95,000 rays, 57 us with one lane, 75
+// with 8 and 58 with 4 (12,000 triangles 145, 127, 116; a million 907, 361,
+// 616 closest).  The last limits are a mean over the hierarchies' sizes: just
+// below them 30,000 scattered triangles lose (8-wide, 190,000 rays 275 us with
+// one lane, 309 with 8; binary, 290,000 camera rays 280 and 307) and small and
+// large ones gain (500: 80 and 42; a million, binary: 966 and 717).
+constexpr uint64_t kFewTriangles = 16384;
+int lanes_per_ray(bool wide, bool any, uint64_t R, uint64_t triangles) {
+  const bool few = triangles <= kFewTriangles;
   if (wide) {
-    if (R <= (any ? 32768u : 24576u)) return 64;
+    if (R <= (any ? 32768u : few ? 12288u : 24576u)) return 64;
     return R <= 196608u ? (any ? 16 : 8) : 1;
   }
   if (R <= 8192u) return 32;
   if (R <= 32768u) return 16;
-  if (R <= 98304u) return 8;
+  if (R <= (few ? 65536u : 98304u)) return 8;
   return R <= (any ? 196608u : 294912u) ? 4 : 1;
 }
 
@@ -331,7 +342,7 @@ template <int kMode, bool kStats, bool kCamera, bool kWide, bool kSeg = false, b
 int32_t launch_width(bajo_ctx* ctx, const bajo_bvh* h, const float* rays, const float* cams, uint32_t w, uint32_t hh,
                      float* hits, uint64_t R, uint32_t* stats) {
   if constexpr (!kStats && !kSph) {
-    switch (lanes_per_ray(kWide, kMode == BAJO_TRACE_ANY_HIT, R)) {
+    switch (lanes_per_ray(kWide, kMode == BAJO_TRACE_ANY_HIT, R, h->n)) {
       case 4:
         if constexpr (!kWide) return launch_groups<kMode, kCamera, kWide, kSeg, 4>(ctx, h, rays, cams, w, hh, hits, R);
         break;

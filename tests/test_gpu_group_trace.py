@@ -66,6 +66,23 @@ def test_group_walks_equal_per_lane(gpu_ctx, width, mesh):
         assert np.all(got[:, 2:4] == -1)
 
 
+@pytest.mark.parametrize("width,n", [(2, 65536), (2, 65537), (8, 12288), (8, 12289)])
+@pytest.mark.parametrize("triangles", [16384, 16385])
+def test_lanes_by_the_number_of_triangles(gpu_ctx, width, n, triangles):
+    """Hierarchies of few triangles change the lanes per ray at fewer rays."""
+    announce(f"group trace of {triangles} triangles, width {width}, rays {n}")
+    v = scenes.soup(triangles, initstate=6, edge_min=0.01, edge_max=0.1)
+    bvh = build_triangle_bvh(torch.from_numpy(v).to("cuda:0"), node_width=width)
+    rays = _rays(n, n + triangles)
+    hits = torch.full((8 * n,), 7.0, device="cuda:0")
+    want = torch.full((8 * n,), 7.0, device="cuda:0")
+    bvh.launch_rays(rays, want, stats=torch.empty(5 * n, dtype=torch.int32, device="cuda:0"))
+    bvh.launch_rays(rays, hits)
+    torch.cuda.synchronize()
+    assert np.array_equal(_bits(hits), _bits(want))
+    bvh.free()
+
+
 @pytest.mark.parametrize("width", [2, 8])
 def test_group_walks_of_set_cameras(gpu_ctx, width):
     sets = [torch.from_numpy(scenes.soup(n, initstate=5, initseq=n, edge_min=0.05, edge_max=0.3)).to("cuda:0")
